@@ -2,9 +2,9 @@
 // with weights stored [out, in] row-major as in the checkpoint (reference:
 // src/model/linear.cuh:9-37 calls a library product with fp32 accumulation).
 //
-//  * gemm_tiled_kernel: LDS-tiled product with scalar float FMAs, any element
-//    type, any size.  It is the whole 32-bit engine's product (true fp32: no
-//    matrix-core path with reduced inputs), and the plain twin of the bf16 ones.
+//  * gemm_tiled_kernel: LDS-tiled product with scalar float FMAs, any size: the plain twin of the bf16 products.
+//  * gemm_f32_mfma_kernel, gemm_f32_rows_kernel: the whole 32-bit engine's product, on the matrix cores' float
+//    instruction (true fp32: no reduced inputs), any size.
 #include "common.h"
 
 #define GT_BM 64
@@ -57,6 +57,160 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const XT* __restrict__ 
     }
 }
 
+// ---------------------------------------------------------------------------
+// The 32-bit product on the matrix cores: v_mfma_f32_16x16x4_f32 takes float operands as they are and adds in float,
+// so nothing is reduced; a lane's FMAs of the scalar kernel had the vector units and their LDS reads as bound (13
+// TFLOP/s), this instruction does 64 multiply-adds a cycle and SIMD (157 TFLOP/s on the chip).
+//
+// gemm_f32_mfma_kernel: 256 threads, 2 x 2 wavefronts of 16 TM x 16 TN outputs each; BK columns of both operands go
+// through LDS in two buffers, the next ones on their way to registers meanwhile, one barrier a piece.  A row of a piece
+// is BK / 4 chunks of 16 bytes, chunk c of row r at place c ^ (r % 8), so that 8 neighbouring lanes (8 rows, one chunk)
+// read all banks.  A lane's 16 bytes serve four instructions: in instruction s, lane group g stands for column 4 g + s
+// of the 16, in both operands alike (a sum over columns may take them in any order).
+// Measured (us, scalar kernel -> this one; rows x outputs x columns): 523 x 8,192 x 1,024 246 -> 109 (56 at 157
+// TFLOP/s), 523 x 1,024 x 4,096 557 -> 75, 2,048 x 4,096 x 4,096 1,650 -> 540, 1 x 8,192 x 1,024 144 -> 11,
+// 16 x 73,448 x 1,024 267 -> 70; its distance from a product in double is the scalar kernel's (5.7e-7 at 1,024
+// columns, 1.1e-6 at 4,096) or, at up to 16 rows, a third of it.
+// ---------------------------------------------------------------------------
+typedef float gfloatx4_t __attribute__((ext_vector_type(4)));
+
+// columns k .. k + 3 of a row of K, zero beyond its end; VEC: K % 4 == 0 and rows on 16-byte borders
+template <bool VEC>
+__device__ inline gfloatx4_t f32_piece(const float* __restrict__ row, int k, int K) {
+    gfloatx4_t v = {0.f, 0.f, 0.f, 0.f};
+    if (VEC) {
+        const gfloatx4_t in = *(const gfloatx4_t*)(row + min(k, K - 4));     // no branch around the load
+        if (k < K) v = in;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (k + i < K) v[i] = row[k + i];
+    }
+    return v;
+}
+
+template <int TM, int TN, int BK, bool VEC>
+__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ X, long ldx,
+                                                            const float* __restrict__ W, long ldw, float* __restrict__ Y,
+                                                            long ldy, int M, int N, int K, float alpha) {
+    constexpr int BM = 32 * TM, BN = 32 * TN, CH = BK / 4, PIECES = (BM + BN) * CH / 256;
+    __shared__ float lds[2][(BM + BN) * BK];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    // rows beyond the matrices read the last one; their results are not stored
+    const float* src[PIECES];
+    int place[PIECES];
+    const int chunk = threadIdx.x % CH;
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) {
+        const int row = threadIdx.x / CH + 256 / CH * i;
+        src[i] = row < BM ? X + (long)min(m0 + row, M - 1) * ldx : W + (long)min(n0 + row - BM, N - 1) * ldw;
+        place[i] = row * BK + ((chunk ^ (row & 7)) << 2);
+    }
+    gfloatx4_t next[PIECES];
+#pragma unroll
+    for (int i = 0; i < PIECES; ++i) next[i] = f32_piece<VEC>(src[i], chunk * 4, K);
+    gfloatx4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    const int row_a = (wave & 1) * 16 * TM + r, row_b = BM + (wave >> 1) * 16 * TN + r;
+    int buf = 0;
+    for (int k0 = 0; k0 < K; k0 += BK, buf ^= 1) {
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) *(gfloatx4_t*)&lds[buf][place[i]] = next[i];
+        __syncthreads();
+        if (k0 + BK < K) {
+#pragma unroll
+            for (int i = 0; i < PIECES; ++i) next[i] = f32_piece<VEC>(src[i], k0 + BK + chunk * 4, K);
+        }
+#pragma unroll
+        for (int kb = 0; kb < BK / 16; ++kb) {
+            const int at = ((kb * 4 + g) ^ (r & 7)) << 2;
+            gfloatx4_t a[TM], b[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[i] = *(const gfloatx4_t*)&lds[buf][(row_a + 16 * i) * BK + at];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[j] = *(const gfloatx4_t*)&lds[buf][(row_b + 16 * j) * BK + at];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][s], b[j][s], acc[i][j], 0, 0, 0);
+        }
+    }
+    // lane (column r, g): acc[i][j][e] is row 4 g + e of its 16 x 16 outputs
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + (wave & 1) * 16 * TM + 16 * i + 4 * g + e;
+            if (m >= M) continue;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int n = n0 + (wave >> 1) * 16 * TN + 16 * j + r;
+                if (n < N) Y[(long)m * ldy + n] = alpha * acc[i][j][e];
+            }
+        }
+}
+
+// The same for at most 16 rows (decode steps), where the weight's bytes are the bound: a workgroup owns 16 outputs a row
+// over all of K, its NW wavefronts take 16 columns each in turn, operands straight from memory, and add up through LDS.
+template <int NW, bool VEC>
+__global__ __launch_bounds__(NW * 64) void gemm_f32_rows_kernel(const float* __restrict__ X, long ldx,
+                                                                const float* __restrict__ W, long ldw,
+                                                                float* __restrict__ Y, long ldy, int M, int N, int K,
+                                                                float alpha) {
+    __shared__ gfloatx4_t part[NW][64];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * 16;
+    const float* xr = X + (long)min(r, M - 1) * ldx;
+    const float* wr = W + (long)min(n0 + r, N - 1) * ldw;
+    gfloatx4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int k = wave * 16 + 4 * g; k < K + 4 * g; k += NW * 16) {
+        const gfloatx4_t a = f32_piece<VEC>(xr, k, K), b = f32_piece<VEC>(wr, k, K);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc, 0, 0, 0);
+    }
+    part[wave][lane] = acc;
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+        for (int w = 1; w < NW; ++w) acc += part[w][lane];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = 4 * g + e;
+            if (m < M && n0 + r < N) Y[(long)m * ldy + n0 + r] = alpha * acc[e];
+        }
+    }
+}
+
+template <bool VEC>
+static void gemm_f32_launch(const float* X, long ldx, const float* W, long ldw, float* Y, long ldy, int M, int N, int K,
+                            float alpha, hipStream_t stream) {
+    const auto up = [](int a, int b) { return (a + b - 1) / b; };
+    // Up to 16 rows the weight's bytes bound the product: every workgroup takes 16 outputs over all of K (1 x 1,024 x
+    // 4,096: 12 us, 43 us in tiles of 32 x 32).  Beyond 32,768 outputs there are tiles enough, and those read x once for
+    // 32 outputs instead of 16 (16 x 73,448 x 1,024: 70 against 83 us).
+    if (M <= 16 && N <= 32768) {
+        gemm_f32_rows_kernel<16, VEC><<<up(N, 16), 1024, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
+        return;
+    }
+    // The largest tile that the rows fill and that still gives every CU two workgroups (whose waits then overlap):
+    // 2,048 x 4,096 x 4,096 540 us in tiles of 128 against 595 (64) and 776 (32), 2,048 x 1,024 x 4,096 289 / 153 / 191,
+    // 523 x 1,024 x 4,096 291 / 95 / 75.
+#define TILES(TM, TN, BK)                                                                                        \
+    gemm_f32_mfma_kernel<TM, TN, BK, VEC><<<dim3(up(N, 32 * TN), up(M, 32 * TM)), 256, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha)
+    if (M > 64 && (long)up(M, 128) * up(N, 128) >= 512) TILES(4, 4, 32);
+    else if (M > 32 && (long)up(M, 64) * up(N, 64) >= 512) TILES(2, 2, 32);
+    else TILES(1, 1, 64);
+#undef TILES
+}
+
 extern "C" const char* cpmcu_gemm_nt_plain(const void* X, long ldx, const void* W, long ldw, void* Y, long ldy,
                                            int in_dtype, int out_dtype, int M, int N, int K, float alpha,
                                            hipStream_t stream) {
@@ -65,11 +219,18 @@ extern "C" const char* cpmcu_gemm_nt_plain(const void* X, long ldx, const void* 
                   ldx, ldw, ldy, K, N);
     dim3 grid((N + GT_BN - 1) / GT_BN, (M + GT_BM - 1) / GT_BM);
     CPMCU_REQUIRE(grid.y <= 65535, "gemm: M=%d too large for one launch", M);
+    if (in_dtype == CPMCU_F32 && out_dtype == CPMCU_F32) {
+        const bool vec = K % 4 == 0 && ldx % 4 == 0 && ldw % 4 == 0 && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0;
+        const float *x = (const float*)X, *w = (const float*)W;
+        if (vec) gemm_f32_launch<true>(x, ldx, w, ldw, (float*)Y, ldy, M, N, K, alpha, stream);
+        else gemm_f32_launch<false>(x, ldx, w, ldw, (float*)Y, ldy, M, N, K, alpha, stream);
+        CPMCU_LAUNCH_CHECK("gemm_nt_plain");
+        return nullptr;
+    }
 #define LAUNCH(T, OT)                                                                                     \
     gemm_tiled_kernel<T, T, OT><<<grid, 256, 0, stream>>>((const T*)X, ldx, (const T*)W, ldw, (OT*)Y, ldy, \
                                                           M, N, K, alpha)
-    if (in_dtype == CPMCU_F32 && out_dtype == CPMCU_F32) LAUNCH(float, float);
-    else if (in_dtype == CPMCU_BF16 && out_dtype == CPMCU_BF16) LAUNCH(bf16_t, bf16_t);
+    if (in_dtype == CPMCU_BF16 && out_dtype == CPMCU_BF16) LAUNCH(bf16_t, bf16_t);
     else if (in_dtype == CPMCU_BF16 && out_dtype == CPMCU_F32) LAUNCH(bf16_t, float);
     else CPMCU_FAIL("gemm: unsupported dtypes in=%d out=%d", in_dtype, out_dtype);
 #undef LAUNCH
