@@ -5,8 +5,8 @@
 // P.V, float softmax with a running maximum.  It takes any head size up to 256,
 // any number of heads and groups, both element types, prompts and single
 // tokens alike, and an optional list of key blocks per (token, kv head) for
-// block-sparse attention.  It is the 32-bit engine's attention and the twin
-// against which the tuned bf16 kernels are checked.
+// block-sparse attention.  It is the twin against which the tuned bf16 kernels are
+// checked, and the 32-bit engine's attention where attention_f32_mfma_kernel does not fit.
 //
 // Formula (reference: src/model/attn.cuh:200-227, src/flash_attn/flash_api.hpp:294-394):
 // s_j = (q.k_j) * scale for keys j <= position of the query, softmax over j in
@@ -91,6 +91,161 @@ __global__ __launch_bounds__(64) void attention_paged_kernel(
     }
 }
 
+// The same on the matrix cores for head sizes that are multiples of 16 up to 128, with float operands as they are
+// (v_mfma_f32_16x16x4_f32): one workgroup a query token, one kv head and up to 16 of its query heads; its 4 wavefronts
+// take chunks of 32 keys in turn and merge their running results through LDS.  The plain kernel above walks the keys
+// of P.V one dependent 4-byte load after the other; here every operand is a 16-byte load in the order of the pages:
+//   S^T = K . Q^T      lane (key slot or head, g) holds features 16 j + 4 g .. + 3: instruction s of block j takes
+//                      feature 4 g + s of the 16 in both operands
+//   O^T += V^T . P^T   instruction (u, i) takes keys 8 g + 4 u + i, which is where the scores' lanes hold them
+// Two prompts of 333 and 190 tokens, 16 heads of 64 in 2 groups: 323 -> 17 us a layer.
+typedef float ffloatx4_t __attribute__((ext_vector_type(4)));
+#define ATT_F32_WAVES 4
+
+template <int DT>
+__global__ __launch_bounds__(ATT_F32_WAVES * 64) void attention_f32_mfma_kernel(
+    const float* __restrict__ q, float* __restrict__ out, const float* __restrict__ kpool, const float* __restrict__ vpool,
+    PagedView pv, const int* __restrict__ positions, const int* __restrict__ tok_slot, int nh, int nkv, float scale,
+    const int* __restrict__ sel_blocks, const int* __restrict__ sel_count, int max_sel, int block_size,
+    const float* __restrict__ head_slopes) {
+    constexpr int HD = 16 * DT, NW = ATT_F32_WAVES;
+    __shared__ ffloatx4_t part[NW][DT][64];
+    __shared__ float part_m[NW][16], part_l[NW][16];
+    const int t = blockIdx.x, kvh = blockIdx.y % nkv, ht = blockIdx.y / nkv;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int G = nh / nkv, head = kvh * G + ht * 16 + n;
+    const bool head_ok = ht * 16 + n < G;
+    const int pos = positions[t], slot = tok_slot[t];
+    const float slope = head_slopes && head_ok ? head_slopes[head] : 0.f;
+    ffloatx4_t qf[DT], acc[DT];
+#pragma unroll
+    for (int j = 0; j < DT; ++j) {
+        qf[j] = acc[j] = ffloatx4_t{0.f, 0.f, 0.f, 0.f};
+        if (head_ok) qf[j] = *(const ffloatx4_t*)(q + ((long)t * nh + head) * HD + 16 * j + 4 * g);
+    }
+    const int* sel = nullptr;
+    int chunks = pos / 32 + 1, cpb = 1;
+    if (sel_count) {
+        const int cnt = sel_count[(long)t * nkv + kvh];
+        if (cnt >= 0) {
+            sel = sel_blocks + ((long)t * nkv + kvh) * max_sel;
+            cpb = block_size / 32;
+            chunks = cnt * cpb;
+        }
+    }
+    const int lane_k = (g >> 1) * 128 + n * 8 + (g & 1) * 4, lane_v = g * 128 + n * 8;
+    float m = -INFINITY, l = 0.f;
+    for (int c = wave; c < chunks; c += NW) {
+        const int key0 = sel ? sel[c / cpb] * block_size + (c % cpb) * 32 : c * 32;
+        if (key0 > pos) continue;                                   // a listed block may reach beyond the token
+        const long base = ((paged_row(pv, slot, key0) >> 5) * nkv + kvh) * (32L * HD);
+        const float *kp = kpool + base + lane_k, *vp = vpool + base + lane_v;
+        ffloatx4_t kf[2][DT], vf[2][DT];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int j = 0; j < DT; ++j) kf[u][j] = *(const ffloatx4_t*)(kp + u * HD * 16 + j * 256);
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int j = 0; j < DT; ++j) vf[u][j] = *(const ffloatx4_t*)(vp + j * 512 + u * 4);
+        if (key0 + 31 > pos) {
+            // what lies behind the token in its page may be anything: a weight of zero would not silence an infinity
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (key0 + 8 * g + 4 * u + i > pos)
+#pragma unroll
+                        for (int j = 0; j < DT; ++j) vf[u][j][i] = 0.f;
+        }
+        ffloatx4_t st[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            st[u] = ffloatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int j = 0; j < DT; ++j)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) st[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u][j][s], qf[j][s], st[u], 0, 0, 0);
+        }
+        // lane (head n, g): st[u][i] is the score of key key0 + 8 g + 4 u + i
+        float mx = -INFINITY;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int back = pos - (key0 + 8 * g + 4 * u + i);
+                st[u][i] = back < 0 ? -INFINITY : st[u][i] * scale - slope * (float)back;
+                mx = fmaxf(mx, st[u][i]);
+            }
+        const float m_new = fmaxf(m, rows_max(mx));
+        const float m_ref = m_new == -INFINITY ? 0.f : m_new;
+        const float corr = expf(m - m_ref);
+        float sum = 0.f;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                st[u][i] = expf(st[u][i] - m_ref);
+                sum += st[u][i];
+            }
+        l = l * corr + rows_sum(sum);
+        m = m_new;
+#pragma unroll
+        for (int j = 0; j < DT; ++j) {
+            acc[j] *= corr;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[u][j][i], st[u][i], acc[j], 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < DT; ++j) part[wave][j][lane] = acc[j];
+    if (g == 0) {
+        part_m[wave][n] = m;
+        part_l[wave][n] = l;
+    }
+    __syncthreads();
+    float top = -INFINITY, f[NW], total = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) top = fmaxf(top, part_m[w][n]);
+    if (top == -INFINITY) top = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+        f[w] = expf(part_m[w][n] - top);
+        total += part_l[w][n] * f[w];
+    }
+    if (!head_ok) return;
+    const float inv = 1.0f / total;
+    for (int j = wave; j < DT; j += NW) {
+        ffloatx4_t o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) o += part[w][j][lane] * f[w];
+        // lane (head n, g): the head's features 16 j + 4 g .. + 3
+        *(ffloatx4_t*)(out + ((long)t * nh + head) * HD + 16 * j + 4 * g) = o * inv;
+    }
+}
+
+template <int DT>
+static bool attention_f32_launch(const float* q, float* out, const float* kpool, const float* vpool, PagedView pv,
+                                 const int* positions, const int* tok_slot, int n, int nh, int nkv, float scale,
+                                 const int* sel_blocks, const int* sel_count, int max_sel, int block_size,
+                                 const float* head_slopes, int hd, hipStream_t stream) {
+    if (hd != 16 * DT) {
+        if constexpr (DT < 8)
+            return attention_f32_launch<DT + 1>(q, out, kpool, vpool, pv, positions, tok_slot, n, nh, nkv, scale, sel_blocks,
+                                                sel_count, max_sel, block_size, head_slopes, hd, stream);
+        return false;
+    }
+    const dim3 grid(n, nkv * ((nh / nkv + 15) / 16));
+    attention_f32_mfma_kernel<DT><<<grid, ATT_F32_WAVES * 64, 0, stream>>>(q, out, kpool, vpool, pv, positions, tok_slot, nh,
+                                                                          nkv, scale, sel_blocks, sel_count, max_sel,
+                                                                          block_size, head_slopes);
+    return true;
+}
+
 extern "C" const char* cpmcu_attention_plain(const void* q, void* out, int dtype, int n, int nh, int nkv, int hd,
                                              float scale, const void* kpool, const void* vpool,
                                              const int* page_table, int table_width, int page_size,
@@ -105,7 +260,12 @@ extern "C" const char* cpmcu_attention_plain(const void* q, void* out, int dtype
     CPMCU_REQUIRE(!sel_count || (sel_blocks && max_sel > 0 && block_size > 0), "attention: block list incomplete");
     PagedView pv{page_table, table_width, page_size};
     dim3 grid(n, nh);
-    if (dtype == CPMCU_F32)
+    const bool aligned = (((uintptr_t)q | (uintptr_t)out | (uintptr_t)kpool | (uintptr_t)vpool) & 15) == 0;
+    if (dtype == CPMCU_F32 && aligned && page_size % 32 == 0 && (!sel_count || block_size % 32 == 0) &&
+        attention_f32_launch<1>((const float*)q, (float*)out, (const float*)kpool, (const float*)vpool, pv, positions, tok_slot,
+                                n, nh, nkv, scale, sel_blocks, sel_count, max_sel, block_size, head_slopes, hd, stream)) {
+        // head sizes 16, 32, ... 128 on the matrix cores
+    } else if (dtype == CPMCU_F32)
         attention_paged_kernel<float><<<grid, 64, 0, stream>>>((const float*)q, (float*)out, (const float*)kpool,
                                                                (const float*)vpool, pv, positions, tok_slot, nh, nkv,
                                                                hd, scale, sel_blocks, sel_count, max_sel, block_size,
