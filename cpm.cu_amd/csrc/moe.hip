@@ -24,6 +24,8 @@
 // aligned), so an expert's weights stream once for every token that chose it: the form for steps of few tokens.
 #include "common.h"
 
+#include <type_traits>
+
 #define MOE_MAX_EXPERTS 1024
 enum { MOE_SCORE_SOFTMAX = 0, MOE_SCORE_SIGMOID = 1, MOE_SCORE_LOGIT = 2 };
 enum { MOE_GROUP_MAX = 0, MOE_GROUP_TOP2_SUM = 1 };
@@ -469,185 +471,221 @@ extern "C" const char* cpmcu_moe_down(const void* act, int dtype, const void* wd
 
 // ===========================================================================
 // The same experts for steps of many tokens, bf16 on the matrix cores (v_mfma_f32_16x16x32_bf16): the (token,
-// chosen expert) pairs are grouped by expert into tiles of 64 rows, and every tile is a product with its
-// expert's weights.
+// chosen expert) pairs are grouped by expert into tiles of up to MOE_TILE or 2 MOE_TILE rows, and every tile is a
+// product with its expert's weights.
 //
-//  * moe_group_kernel (one workgroup): counts the pairs of every expert, gives every expert whole tiles of 64 rows
-//    (rows[tile * 64 + i] = pair, -1 in a tile's unused rows), tile_expert[tile] and the number of tiles.  Which row
-//    of its expert's tiles a pair gets depends on timing; its result does not (a row's sums are its own).
-//  * moe_gated_mfma_kernel: act[pair] = silu(Wg_e h_t) * (Wu_e h_t); a wavefront owns the 64 rows of a tile and 32
-//    features (two tiles of gate rows, two of up rows): 16 matrix instructions for 8 operand loads, operands
-//    straight from memory (the 4 wavefronts of a workgroup read the same rows of h, which meet in the CU's cache).
-//    Without a gate (GATED false; wgu then holds up rows only) it owns 64 features: act[pair] = act(Wu_e h_t).
-//  * moe_down_mfma_kernel: y[pair] = Wd_e act[pair] (bf16); a wavefront owns the 64 rows and 64 columns.
+//  * moe_group_kernel (one workgroup): counts the pairs of every expert and lists them expert by expert: rows[offs[e] ..
+//    offs[e + 1]) are expert e's pairs, tile_expert[tile] = e + 1024 * (the tile's number among its expert's), offs[E + 1]
+//    the number of tiles; n_tiles is what tiles of MOE_TILE rows would need, the rest of whose rows hold -1.  Which row of its expert's tiles a pair gets depends on timing; its result does not (a row's sums
+//    are its own).
+//  * moe_tile_kernel: GATED act[pair] = act(Wg_e h_t) * (Wu_e h_t), PLAIN act[pair] = act(Wu_e h_t), DOWN y[pair] =
+//    Wd_e act[pair] (bf16).
 //  * moe_combine_kernel: out[t] = sum_k w[t, k] y[t, k] (h_t where the chosen expert is an identity expert) (+ sg[t] * shared[t]) in float, k in order.
 // ===========================================================================
 typedef __bf16 mbf16x8_t __attribute__((ext_vector_type(8)));
 typedef float mfloatx4_t __attribute__((ext_vector_type(4)));
+typedef unsigned mu32x4_t __attribute__((ext_vector_type(4)));
 
 #define MOE_TILE 64
+enum { MOE_GATED = 0, MOE_PLAIN = 1, MOE_DOWN = 2 };
 
-__global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__ idx, int n_pairs, int E,
-                                                         int* __restrict__ rows, int* __restrict__ tile_expert,
-                                                         int* __restrict__ n_tiles_out, int max_tiles) {
+// tile_rows: rows a tile at most; an expert's pairs are spread evenly over as few tiles as hold them (moe_tile_kernel)
+__global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__ idx, int n_pairs, int E, int tile_rows,
+                                                         int* __restrict__ rows, int* __restrict__ offs, int behind,
+                                                         int* __restrict__ tile_expert, int* __restrict__ n_tiles_out) {
     __shared__ int counts[MOE_MAX_EXPERTS];
-    __shared__ int offs[MOE_MAX_EXPERTS];
-    for (int e = threadIdx.x; e < E; e += 1024) counts[e] = 0;
-    for (int i = threadIdx.x; i < max_tiles * MOE_TILE; i += 1024) rows[i] = -1;
+    __shared__ int pair_sum[16], tile_sum[16], whole, placed;
+    const int e = threadIdx.x, lane = e & 63, wave = e >> 6;
+    counts[e] = 0;
+    if (e == 0) whole = 0;
     __syncthreads();
     for (int p = threadIdx.x; p < n_pairs; p += 1024)
         if (idx[p] < E) atomicAdd(&counts[idx[p]], 1);              // identity experts have no tiles
     __syncthreads();
-    if (threadIdx.x == 0) {
-        int t = 0;
-        for (int e = 0; e < E; ++e) {
-            offs[e] = t * MOE_TILE;
-            const int nt = (counts[e] + MOE_TILE - 1) / MOE_TILE;
-            for (int i = 0; i < nt; ++i) tile_expert[t + i] = e;
-            t += nt;
+    // running sums of pairs and tiles over the experts, one expert a thread
+    const int c = counts[e], nt = (c + tile_rows - 1) / tile_rows;
+    int pairs = c, tiles = nt;
+    if (c) atomicAdd(&whole, (c + MOE_TILE - 1) / MOE_TILE);
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+        const int a = __shfl_up(pairs, d, 64), b = __shfl_up(tiles, d, 64);
+        if (lane >= d) {
+            pairs += a;
+            tiles += b;
         }
-        *n_tiles_out = t;
+    }
+    if (lane == 63) {
+        pair_sum[wave] = pairs;
+        tile_sum[wave] = tiles;
     }
     __syncthreads();
-    for (int e = threadIdx.x; e < E; e += 1024) counts[e] = 0;
+    for (int w = 0; w < wave; ++w) {
+        pairs += pair_sum[w];
+        tiles += tile_sum[w];
+    }
+    if (e < E) {
+        offs[e] = pairs - c;
+        if (e == E - 1) {
+            offs[E] = pairs;
+            offs[E + 1] = tiles;
+        }
+        for (int i = 0; i < nt; ++i) tile_expert[tiles - nt + i] = e + 1024 * i;
+    }
+    if (e == 0) *n_tiles_out = whole;
+    counts[e] = pairs - c;
+    if (e == E - 1) placed = pairs;
     __syncthreads();
+    for (int i = placed + threadIdx.x; i < min(whole * MOE_TILE, behind); i += 1024) rows[i] = -1;
     for (int p = threadIdx.x; p < n_pairs; p += 1024) {
-        const int e = idx[p];
-        if (e >= E) continue;
-        rows[offs[e] + atomicAdd(&counts[e], 1)] = p;
+        const int x = idx[p];
+        if (x < E) rows[atomicAdd(&counts[x], 1)] = p;
     }
 }
 
-// grid (ceil(F / 128), or ceil(F / 256) without a gate, max_tiles), 256 threads: a wavefront takes all 64 rows of the tile
-// and 32 features (64 without a gate)
-template <bool GATED>
-__global__ __launch_bounds__(256) void moe_gated_mfma_kernel(const bf16_t* __restrict__ h, long ldh,
-                                                             const bf16_t* __restrict__ wgu, const int* __restrict__ rows,
-                                                             const int* __restrict__ tile_expert,
-                                                             const int* __restrict__ n_tiles, bf16_t* __restrict__ act,
-                                                             int H, int F, int top, int act_fn, float act_limit) {
-    const int tile = blockIdx.y;
-    if (tile >= *n_tiles) return;
+// Workgroups of 4 wavefronts; a tile of up to 16 RT rows against 128 weight rows (GATED: 64 features, gate and up row of
+// each), a wavefront all rows and 32 weight rows (GATED: 16 features).  Pieces of 64 columns of both go through LDS in
+// two buffers, the next piece on its way to registers meanwhile (with both operands straight from memory every wavefront
+// fetched all of the rows for itself, 16 bytes of a row an access, and the address unit, not HBM or the matrix cores,
+// was the bound).  A piece's row is 8 chunks of 16 bytes, chunk c of row r at place c ^ (r % 8): 8 neighbouring lanes
+// then read all banks.  The tile's rows beyond the last 16 in use are neither loaded nor multiplied.
+// K is the rows' width, N the number of features; in: h rows by token (GATED, PLAIN: pair / top) or act rows by pair.
+// Measured (64 experts, width 4,096, 6 a token; us, before -> now): gated experts of 1,408, 2,048 tokens 1,250 -> 464
+// and 612 -> 278 (down), 24 tokens 303 -> 222 and 169 -> 116 (their 58 experts' matrices at 6 TB/s); 8 tokens 129 + 67.
+// Two pieces on their way at once: one made no difference beyond 300 tokens, at 24 it took 234 + 122 us.
+// The grid is dealt to the 8 XCDs in turn; each takes one run of the tasks, ordered expert by expert and within an expert
+// weight rows by weight rows, so that the tiles that share weights meet in one L2.
+template <int KIND, int RT>
+__global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restrict__ in, long ldi,
+                                                          const bf16_t* __restrict__ w, const int* __restrict__ rows,
+                                                          const int* __restrict__ offs, const int* __restrict__ tile_expert,
+                                                          int E, bf16_t* __restrict__ out, int K, int N, int top, int act_fn,
+                                                          float act_limit) {
+    constexpr int BM = 16 * RT, FEATURES = KIND == MOE_GATED ? 64 : 128;
+    __shared__ mu32x4_t lds[2][(BM + 128) * 8];
+    const int nts = (N + FEATURES - 1) / FEATURES;
+    const int tasks = offs[E + 1] * nts, per = (tasks + 7) / 8;
+    const int task = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || task >= tasks) return;
+    const int q = task / nts, te = tile_expert[q], e = te & 1023;
+    const int start = offs[e], cnt = offs[e + 1] - start;
+    const int m = (cnt + BM - 1) / BM, rpt = ((cnt + m - 1) / m + 15) & ~15;
+    const int local = task - (q - (te >> 10)) * nts, mt = local % m, f0 = local / m * FEATURES;
+    const int row0 = start + mt * rpt, n_rows = min(rpt, cnt - mt * rpt);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const int e = tile_expert[tile];
-    const int f0 = GATED ? blockIdx.x * 128 + wave * 32 : blockIdx.x * 256 + wave * 64;
-    if (f0 >= F) return;
-    const bf16_t* xp[4];
+    const int chunk = threadIdx.x & 7, lrow = threadIdx.x >> 3;       // what this thread brings: chunk of rows lrow + 32 i
+    const bf16_t* wp[4];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-        const int pair = rows[tile * MOE_TILE + rt * 16 + r];
-        xp[rt] = h + (long)(pair >= 0 ? pair / top : 0) * ldh + g * 8;
+    for (int i = 0; i < 4; ++i) {
+        // weight row 32 w + 16 j + x of the tile: GATED feature f0 + 16 w + x, gate (j = 0) or up (j = 1)
+        const int row = lrow + 32 * i;
+        const int f = min(f0 + (KIND == MOE_GATED ? (row >> 5) * 16 + (row & 15) : row), N - 1);
+        wp[i] = w + ((long)e * (KIND == MOE_GATED ? 2 : 1) * N + (KIND == MOE_GATED && (row & 16) ? N : 0) + f) * K + chunk * 8;
     }
-    const bf16_t* wp = wgu + (long)e * (GATED ? 2 : 1) * F * H + g * 8;
-    mfloatx4_t acc[4][4];
+    const int place = lrow * 8 + (chunk ^ (lrow & 7));                // rows 32 apart have the same place in their 256
+
+    auto product = [&](auto groups) {
+        constexpr int NRT = decltype(groups)::value, AP = (NRT + 1) / 2;
+        const bf16_t* ap[AP];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[rt][j] = mfloatx4_t{0.f, 0.f, 0.f, 0.f};
-    long wrow[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {                 // j = 0, 1: gate rows f0 + 16 j + r; j = 2, 3: their up rows
-        const int f = min(f0 + 16 * (GATED ? (j & 1) : j) + r, F - 1);
-        wrow[j] = (long)((GATED ? (j >> 1) * F : 0) + f) * H;
-    }
-    for (int k0 = 0; k0 < H; k0 += 32) {
-        const bool k_ok = k0 + g * 8 < H;
-        const int kk = k_ok ? k0 : k0 - g * 8;       // a lane beyond the row's end reads the step's first columns (in range) and is zeroed
-        mbf16x8_t a[4], b[4];
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) a[rt] = *(const mbf16x8_t*)(xp[rt] + kk);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = *(const mbf16x8_t*)(wp + wrow[j] + kk);
-        if (!k_ok) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) a[j] = b[j] = mbf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        for (int i = 0; i < AP; ++i) {
+            const int pair = rows[row0 + min(lrow + 32 * i, n_rows - 1)];
+            ap[i] = in + (long)(KIND == MOE_DOWN ? pair : pair / top) * ldi + chunk * 8;
         }
+        struct Piece { mu32x4_t a[AP], w[4]; } p0, p1;                // on their way: this piece and the next
+        auto fetch = [&](Piece& p, int k0) {
+            const int k = min(k0, K - 8 - chunk * 8);                 // beyond the row's end: its last columns, zeroed below
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+            for (int i = 0; i < 4; ++i) p.w[i] = *(const mu32x4_t*)(wp[i] + k);
 #pragma unroll
-            for (int j = 0; j < 4; ++j) acc[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], b[j], acc[rt][j], 0, 0, 0);
-    }
-    // lane (feature column r, g): acc[rt][j][i] belongs to the tile's row rt * 16 + 4 g + i
+            for (int i = 0; i < AP; ++i) p.a[i] = *(const mu32x4_t*)(ap[i] + k);
+        };
+        mfloatx4_t acc[NRT][2];
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
+        for (int rt = 0; rt < NRT; ++rt) acc[rt][0] = acc[rt][1] = mfloatx4_t{0.f, 0.f, 0.f, 0.f};
+        auto step = [&](Piece& p, int k0, int buf, auto last) {
+            // (only behind the loop: a branch here would make every step wait for all loads in flight)
+            if (decltype(last)::value && k0 + chunk * 8 >= K) {       // K % 8 == 0: the whole chunk lies beyond the end
+                const mu32x4_t zero = {0u, 0u, 0u, 0u};
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int p = rows[tile * MOE_TILE + rt * 16 + 4 * g + i];
-            if (p < 0) continue;
+                for (int i = 0; i < 4; ++i) p.w[i] = zero;
 #pragma unroll
-            for (int j = 0; j < (GATED ? 2 : 4); ++j) {
-                const int f = f0 + 16 * j + r;
-                if (f < F) {
-                    if (GATED) {
-                        float gt = acc[rt][j][i], up = acc[rt][(2 + j) & 3][i];
-                        gate_prepare(gt, up, act_fn, act_limit);
-                        act[(long)p * F + f] = f32_to_bf16(gate_act(gt, act_fn) * up);
-                    } else {
-                        act[(long)p * F + f] = f32_to_bf16(plain_act(acc[rt][j][i], act_fn));
+                for (int i = 0; i < AP; ++i) p.a[i] = zero;
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) lds[buf][BM * 8 + 256 * i + place] = p.w[i];
+#pragma unroll
+            for (int i = 0; i < AP; ++i)
+                if (NRT > 1 || lrow < 16) lds[buf][256 * i + place] = p.a[i];
+            if (!decltype(last)::value) fetch(p, k0 + 128);
+            __syncthreads();
+            mbf16x8_t a[2][NRT], b[2][2];
+            auto read = [&](int kk) {
+                const int at = (kk * 4 + g) ^ (r & 7);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) b[kk][j] = *(const mbf16x8_t*)&lds[buf][(BM + wave * 32 + j * 16 + r) * 8 + at];
+#pragma unroll
+                for (int rt = 0; rt < NRT; ++rt) a[kk][rt] = *(const mbf16x8_t*)&lds[buf][(rt * 16 + r) * 8 + at];
+            };
+            read(0);
+            read(1);
+#pragma unroll
+            for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+                for (int rt = 0; rt < NRT; ++rt)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][rt], b[kk][j], acc[rt][j], 0, 0, 0);
+            if constexpr (NRT > 4) {
+                // the order to keep: the first half's operands, then the second half's one by one between the first half's
+                // matrix instructions; left alone, the scheduler reads each operand just before its use (2,048 tokens: 495
+                // against 464 us).  With few rows, where memory is the bound, it is left alone.
+                __builtin_amdgcn_sched_group_barrier(0x100, NRT + 4, 0);
+#pragma unroll
+                for (int rt = 0; rt < NRT; ++rt) {
+                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
+                }
+                __builtin_amdgcn_sched_group_barrier(0x008, 2 * NRT, 0);
+            }
+        };
+        fetch(p0, 0);
+        fetch(p1, 64);
+        int k0 = 0;
+        for (; k0 + 128 <= K; k0 += 128) {
+            step(p0, k0, 0, std::false_type());
+            step(p1, k0 + 64, 1, std::false_type());
+        }
+        if (k0 < K) step(p0, k0, 0, std::true_type());
+        if (k0 + 64 < K) step(p1, k0 + 64, 1, std::true_type());
+        // lane (weight row r, g): acc[rt][j][i] belongs to the tile's row rt * 16 + 4 g + i
+#pragma unroll
+        for (int rt = 0; rt < NRT; ++rt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = rt * 16 + 4 * g + i;
+                if (row >= n_rows) continue;
+                bf16_t* to = out + (long)rows[row0 + row] * N;
+                if (KIND == MOE_GATED) {
+                    const int f = f0 + wave * 16 + r;
+                    float gt = acc[rt][0][i], up = acc[rt][1][i];
+                    gate_prepare(gt, up, act_fn, act_limit);
+                    if (f < N) to[f] = f32_to_bf16(gate_act(gt, act_fn) * up);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const int f = f0 + wave * 32 + j * 16 + r;
+                        if (f < N) to[f] = f32_to_bf16(KIND == MOE_PLAIN ? plain_act(acc[rt][j][i], act_fn) : acc[rt][j][i]);
                     }
                 }
             }
-        }
-}
-
-// grid (ceil(H / 256), max_tiles), 256 threads: a wavefront takes all 64 rows of the tile and 64 columns
-__global__ __launch_bounds__(256) void moe_down_mfma_kernel(const bf16_t* __restrict__ act, const bf16_t* __restrict__ wd,
-                                                            const int* __restrict__ rows,
-                                                            const int* __restrict__ tile_expert,
-                                                            const int* __restrict__ n_tiles, bf16_t* __restrict__ y,
-                                                            int H, int F) {
-    const int tile = blockIdx.y;
-    if (tile >= *n_tiles) return;
-    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const int e = tile_expert[tile];
-    const int c0 = blockIdx.x * 256 + wave * 64;
-    if (c0 >= H) return;
-    const bf16_t* xp[4];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt) {
-        const int pair = rows[tile * MOE_TILE + rt * 16 + r];
-        xp[rt] = act + (long)(pair >= 0 ? pair : 0) * F + g * 8;
+    };
+    if constexpr (RT > 4) {
+        if (n_rows > 96) { product(std::integral_constant<int, 8>()); return; }
+        if (n_rows > 64) { product(std::integral_constant<int, 6>()); return; }
     }
-    const bf16_t* wp = wd + (long)e * H * F + g * 8;
-    mfloatx4_t acc[4][4];
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[rt][j] = mfloatx4_t{0.f, 0.f, 0.f, 0.f};
-    long wrow[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) wrow[j] = (long)min(c0 + 16 * j + r, H - 1) * F;
-    for (int k0 = 0; k0 < F; k0 += 32) {
-        const bool k_ok = k0 + g * 8 < F;
-        const int kk = k_ok ? k0 : k0 - g * 8;
-        mbf16x8_t a[4], b[4];
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) a[rt] = *(const mbf16x8_t*)(xp[rt] + kk);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) b[j] = *(const mbf16x8_t*)(wp + wrow[j] + kk);
-        if (!k_ok) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) a[j] = b[j] = mbf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
-        }
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[rt], b[j], acc[rt][j], 0, 0, 0);
-    }
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int p = rows[tile * MOE_TILE + rt * 16 + 4 * g + i];
-            if (p < 0) continue;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int c = c0 + 16 * j + r;
-                if (c < H) y[(long)p * H + c] = f32_to_bf16(acc[rt][j][i]);
-            }
-        }
+    if (n_rows > 32) product(std::integral_constant<int, 4>());
+    else if (n_rows > 16) product(std::integral_constant<int, 2>());
+    else product(std::integral_constant<int, 1>());
 }
 
 // V neighbouring columns a thread (4: 8-byte loads of a pair's row)
@@ -701,7 +739,7 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16_t* __restri
     }
 }
 
-// scratch: rows int [max_tiles * 64], tile_expert int [max_tiles], n_tiles int [1], y bf16 [n * top, H];
+// scratch: rows int [max_tiles * 64] (the pairs by expert; at its end the experts' offsets), tile_expert int [max_tiles], n_tiles int [1], y bf16 [n * top, H];
 // max_tiles = ceil(n * top / 64) + E
 extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const void* wgu, const void* wd, const int* idx,
                                               const float* w, const void* shared, int shared_dtype, int shared_parts,
@@ -721,18 +759,33 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     const long pairs = (long)n * top;
     CPMCU_REQUIRE(max_tiles >= (pairs + MOE_TILE - 1) / MOE_TILE + E && max_tiles <= 65535,
                   "moe_experts_mfma: %d tiles of scratch for %ld pairs of %d experts (at most 65535)", max_tiles, pairs, E);
-    moe_group_kernel<<<1, 1024, 0, stream>>>(idx, (int)pairs, E, rows, tile_expert, n_tiles, max_tiles);
+    // Tiles of 128 rows where experts have many; the scratch is sized for tiles of 64: it holds the pairs without gaps and,
+    // at its end, the experts' offsets.
+    const bool wide = pairs >= 48L * E;
+    const int tile_rows = wide ? 2 * MOE_TILE : MOE_TILE;
+    const long tiles = (pairs + tile_rows - 1) / tile_rows + E;
+    const long behind = (long)max_tiles * MOE_TILE - (E + 2);         // pairs <= behind: max_tiles covers 64 E rows more
+    int* offs = rows + behind;
+    CPMCU_REQUIRE(pairs <= behind && (long)max_tiles * MOE_TILE < (1L << 31), "moe_experts_mfma: scratch of %d tiles for %ld pairs", max_tiles, pairs);
+    moe_group_kernel<<<1, 1024, 0, stream>>>(idx, (int)pairs, E, tile_rows, rows, offs, (int)behind, tile_expert, n_tiles);
     CPMCU_LAUNCH_CHECK("moe_group");
-    if (gated)
-        moe_gated_mfma_kernel<true><<<dim3((F + 127) / 128, max_tiles), 256, 0, stream>>>(
-            (const bf16_t*)h, ldh, (const bf16_t*)wgu, rows, tile_expert, n_tiles, (bf16_t*)act, H, F, top, act_fn, act_limit);
-    else
-        moe_gated_mfma_kernel<false><<<dim3((F + 255) / 256, max_tiles), 256, 0, stream>>>(
-            (const bf16_t*)h, ldh, (const bf16_t*)wgu, rows, tile_expert, n_tiles, (bf16_t*)act, H, F, top, act_fn, act_limit);
-    CPMCU_LAUNCH_CHECK("moe_gated_mfma");
-    moe_down_mfma_kernel<<<dim3((H + 255) / 256, max_tiles), 256, 0, stream>>>((const bf16_t*)act, (const bf16_t*)wd, rows,
-                                                                           tile_expert, n_tiles, (bf16_t*)y, H, F);
-    CPMCU_LAUNCH_CHECK("moe_down_mfma");
+#define TILES(KIND, in, ldi, w, out, K, N, act, limit)                                                                    \
+    do {                                                                                                                      \
+        const long blocks = (tiles * (((N) + (KIND == MOE_GATED ? 63 : 127)) / (KIND == MOE_GATED ? 64 : 128)) + 7) / 8 * 8;   \
+        CPMCU_REQUIRE(blocks < (1L << 31), "moe_experts_mfma: %ld workgroups exceed the launch grid", blocks);                 \
+        if (wide)                                                                                                             \
+            moe_tile_kernel<KIND, 8><<<(unsigned)blocks, 256, 0, stream>>>(in, ldi, (const bf16_t*)(w), rows, offs, tile_expert, \
+                                                                               E, (bf16_t*)(out), K, N, top, act, limit);         \
+        else                                                                                                                  \
+            moe_tile_kernel<KIND, 4><<<(unsigned)blocks, 256, 0, stream>>>(in, ldi, (const bf16_t*)(w), rows, offs, tile_expert, \
+                                                                               E, (bf16_t*)(out), K, N, top, act, limit);         \
+    } while (0)
+    if (gated) TILES(MOE_GATED, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
+    else TILES(MOE_PLAIN, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
+    CPMCU_LAUNCH_CHECK("moe_up_tiles");
+    TILES(MOE_DOWN, (const bf16_t*)act, (long)F, wd, y, F, H, 0, 0.f);
+    CPMCU_LAUNCH_CHECK("moe_down_tiles");
+#undef TILES
     const long total = (long)n * H;
     const bool vec = H % 4 == 0 && ldh % 4 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)(x ? x : out) % 16 == 0;
     const long work = vec ? total / 4 : total;

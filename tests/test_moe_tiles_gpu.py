@@ -1,0 +1,48 @@
+"""Experts grouped into tiles: row counts at the edges of tiles, of 16 rows and of the rule for wide tiles; widths that end
+inside a piece of 64 columns or a tile of features (GPU)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+# rows: how many pairs each expert gets (the last one none); `top` 1 makes that exact
+@pytest.mark.parametrize("rows", [[1], [16, 17], [32, 33, 1], [64, 65], [128, 129, 96, 97], [257, 5], [1030, 3, 0, 500]])
+@pytest.mark.parametrize("H,F", [(8, 8), (72, 136), (200, 56)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_tiles_of_every_fill(rows, H, F, gated):
+    from cpmcu_amd import ops
+    E, n = len(rows) + 1, sum(rows)
+    g = torch.Generator(device=DEV).manual_seed(n + H + F)
+    idx = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(rows)])
+    idx = idx[torch.randperm(n, generator=torch.Generator().manual_seed(n))].to(DEV)[:, None].contiguous()
+    h = torch.randn(n, H, generator=g, device=DEV).to(torch.bfloat16)
+    up = torch.randn(E, F * (2 if gated else 1), H, generator=g, device=DEV).to(torch.bfloat16)
+    down = torch.randn(E, H, F, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.rand(n, 1, generator=g, device=DEV)
+    tiles = ops.moe_tiles(n, 1, E)
+    i32 = lambda k: torch.empty(k, dtype=torch.int32, device=DEV)
+    act = torch.full((n, 1, F), float("nan"), dtype=torch.bfloat16, device=DEV)
+    y = torch.full((n, 1, H), float("nan"), dtype=torch.bfloat16, device=DEV)
+    out = torch.full((n, H), float("nan"), device=DEV)
+    ops.moe_experts_mfma(h, up, down, idx, w, out, act, y, i32(tiles * ops.MOE_TILE), i32(tiles), i32(1), gated=gated,
+                         activation="silu" if gated else "relu_squared")
+    e = idx[:, 0].long()
+    half, sums = 2.0 ** -8, 2.0 ** -23
+    z = torch.einsum("nk,nfk->nf", h.double(), up.double()[e])
+    mag = torch.einsum("nk,nfk->nf", h.double().abs(), up.double().abs()[e])
+    off = H * sums * mag                                             # float sums in any order
+    if gated:
+        a, u = z[:, :F], z[:, F:]
+        want = torch.nn.functional.silu(a) * u
+        off = 1.1 * off[:, :F] * u.abs() + (a.abs() + off[:, :F]) * off[:, F:]      # |silu'| <= 1.1
+    else:
+        want = torch.relu(z) ** 2
+        off = 2 * z.abs() * off + off ** 2
+    assert bool(((act[:, 0].double() - want).abs() <= off + (half + 8 * sums) * want.abs() + 1e-30).all())
+    got = act[:, 0].double()                                         # the second product of what the first one wrote
+    ref = torch.einsum("nf,nhf->nh", got, down.double()[e])
+    off = F * sums * torch.einsum("nf,nhf->nh", got.abs(), down.double().abs()[e])
+    off = off + half * (ref.abs() + off)
+    assert bool(((out.double() - w.double() * ref).abs() <= w.double() * off + 2 * sums * ref.abs() + 1e-30).all())
