@@ -609,6 +609,252 @@ extern "C" const char* cpmcu_attention_general_mfma(const void* q, void* out, in
 }
 
 // ===========================================================================
+// The same attention for prompts whose values have more than 128 features (latent attention's 576 and 512, two score
+// maps over values of 256): a workgroup of 8 wavefronts owns 64 columns, the heads of 64 / G consecutive tokens of one
+// sequence (G query heads a kv head), and visits their keys 64 at a time.
+//   S^T = K . Q^T     the 64 keys stand in LDS; wavefront (kh, ct) multiplies the 32 keys of half kh by the 16 columns of
+//                     tile ct, whose Q it keeps in registers
+//   P^T               a wavefront turns its own scores into weights; the columns' maxima of both halves meet in LDS first,
+//                     the weights go there as the operand that
+//   O^T += V^T . P^T  takes: a wavefront owns DTW tiles of 16 value features for all 64 columns, its values come straight
+//                     from the page
+// The next keys are on their way to registers meanwhile; two barriers a round.  attention_general_mfma_kernel reads every
+// key and value once for 16 columns, whose bytes from L2 were the bound (14 TB/s).  Measured, that kernel -> this one: 2,048
+// tokens, 32 heads over a latent of 512 + 64 700 -> 269 us (585 TFLOP/s; the LDS reads of the keys are next), 1,500 tokens,
+// 32 maps on 8 keys of 128 and 4 values of 256 205 -> 81 us.  The running maximum follows only when a column's has moved up by more than 8 (in powers of two):
+// weights then reach 2^8 at most, which float sums and bf16 weights take as well as 1.
+// PK: up to 64 PK key features (EXACT: so many); DTW: up to 128 DTW value features.
+// ===========================================================================
+typedef unsigned gu32x4_t __attribute__((ext_vector_type(4)));
+
+template <int PK, int DTW, bool EXACT>
+__global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
+    const bf16_t* __restrict__ q, void* __restrict__ out, int out_f32, const bf16_t* __restrict__ kpool,
+    const bf16_t* __restrict__ vtpool, PagedView pv, const int* __restrict__ positions, const int* __restrict__ tok_slot,
+    int nh, int nkv, int hdk, int hdv, int pool_hdk, int pool_hdv, float scale_log2e, int chunk, int window, int keep_first,
+    const float* __restrict__ sink, const int* __restrict__ tiles, int v_share, const bf16_t* __restrict__ gate, long ld_gate,
+    float cap_in, float cap_out) {
+    constexpr int KS = 2 * PK;
+    __shared__ gu32x4_t keys_s[512 * PK];                         // [half][tile of 16 keys][32 features][lane]
+    __shared__ gbf16x8_t p_s[4][2][64];                            // weights [column tile][half][lane]
+    __shared__ float top_s[2][64], sum_s[2][64];                   // a column's largest score of a half; at the end its sums
+    const int tile = gridDim.x - 1 - blockIdx.x;                   // later tiles of a prompt see more keys: they start first
+    const int kvh = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int ct = wave & 3, kh = wave >> 2;
+    const int G = nh / nkv, pk = EXACT ? PK : pool_hdk >> 6, dtn = pool_hdv >> 4;
+    const int t0 = tiles[2 * tile], n_tok = tiles[2 * tile + 1], slot = tok_slot[t0];
+    const int pos_min = positions[t0], pos_max = pos_min + n_tok - 1;
+    auto token_of = [&](int c) { const int k = (c * 16 + n) / G; return k < n_tok ? k : 0; };    // of column tile c
+    auto head_of = [&](int c) { return kvh * G + (c * 16 + n) % G; };
+    const int pos = pos_min + token_of(ct);                        // a tile's tokens are consecutive
+    const int first_key = chunk > 0 ? pos - pos % chunk : (window > 0 ? max(pos - window + 1, 0) : 0);
+    const int first_min = chunk > 0 ? pos_min - pos_min % chunk : (window > 0 ? max(pos_min - window + 1, 0) : 0);
+    const int first_max = chunk > 0 ? pos_max - pos_max % chunk : (window > 0 ? max(pos_max - window + 1, 0) : 0);
+    const int cfirst = first_min >> 5, ckeep = min((keep_first + 31) >> 5, cfirst);
+    const int total = ckeep + (pos_max >> 5) + 1 - cfirst, rounds = (total + 1) / 2;
+
+    gbf16x8_t qf[KS];
+    {
+        const bf16_t* qr = q + ((long)(t0 + token_of(ct)) * nh + head_of(ct)) * hdk;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int d = ks * 32 + g * 8;
+            const gbf16x8_t v = *(const gbf16x8_t*)(qr + min(d, hdk - 8));
+            qf[ks] = d < hdk ? v : gbf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        }
+    }
+    // chunk c of 32 keys: its first key, and where it lies (a number beyond the last chunk: the last one, masked below)
+    auto key0_of = [&](int c) { return (c < ckeep ? c : cfirst + (c - ckeep)) << 5; };
+    auto place_of = [&](int c) { return (int)(paged_row(pv, slot, key0_of(min(c, total - 1))) >> 5); };
+    // What a thread brings of 64 keys: pk pieces of 16 bytes of its half's 32 keys, which lie in a row in the page and
+    // in LDS (two tiles of 16 keys each, a tile [features / 8][key][8]).
+    const long kchunk = 32L * pool_hdk, vchunk = 32L * pool_hdv;
+    const int piece = threadIdx.x & 255, half0 = kh * 256 * pk;
+    gu32x4_t kr[PK];
+    auto fetch_keys = [&](int place) {
+        const gu32x4_t* from = (const gu32x4_t*)(kpool + ((long)place * nkv + kvh) * kchunk) + piece;
+#pragma unroll
+        for (int i = 0; i < PK; ++i)
+            if (EXACT || i < pk) kr[i] = from[256 * i];
+    };
+    auto store_keys = [&]() {
+#pragma unroll
+        for (int i = 0; i < PK; ++i)
+            if (EXACT || i < pk) keys_s[half0 + piece + 256 * i] = kr[i];
+    };
+    gfloatx4_t acc[DTW][4];
+    float m[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY}, l = 0.f;        // of all four column tiles; of the own keys
+#pragma unroll
+    for (int d = 0; d < DTW; ++d)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[d][c] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    int p0 = place_of(0), p1 = place_of(1), n0 = place_of(2), n1 = place_of(3);
+    fetch_keys(kh ? p1 : p0);
+    store_keys();
+    __syncthreads();
+    for (int it = 0; it < rounds; ++it) {
+        gbf16x8_t vf[2][DTW];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const bf16_t* vp = vtpool + ((long)(h ? p1 : p0) * (nkv / v_share) + kvh / v_share) * vchunk + (g * 16 + n) * 8;
+#pragma unroll
+            for (int d = 0; d < DTW; ++d) vf[h][d] = *(const gbf16x8_t*)(vp + min(wave * DTW + d, dtn - 1) * 512);
+        }
+        fetch_keys(kh ? n1 : n0);
+        p0 = n0;
+        p1 = n1;
+        n0 = place_of(2 * it + 4);
+        n1 = place_of(2 * it + 5);
+        gfloatx4_t st[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+            if (EXACT || ks < 2 * pk) {
+#pragma unroll
+                for (int u = 0; u < 2; ++u) {
+                    const gbf16x8_t kf = *(const gbf16x8_t*)&keys_s[half0 + (u * 2 * pk + ks) * 64 + lane];
+                    st[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[ks], st[u], 0, 0, 0);
+                }
+            }
+        // lane (column n, g): st[u][e] is key key0 + 8 g + 4 u + e
+        if (cap_out > 0.f) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) st[u][e] = cap_out * tanhf(st[u][e] * cap_in);
+        }
+        const int c = 2 * it + kh, key0 = key0_of(min(c, total - 1));
+        if (c >= total || key0 + 31 > pos_min || (key0 < first_max && key0 + 31 >= keep_first)) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int key = key0 + 8 * g + 4 * u + e;
+                    if (c >= total || key > pos || (key < first_key && key >= keep_first)) st[u][e] = -INFINITY;
+                }
+        }
+        float mx = fmaxf(fmaxf(fmaxf(st[0][0], st[0][1]), fmaxf(st[0][2], st[0][3])),
+                         fmaxf(fmaxf(st[1][0], st[1][1]), fmaxf(st[1][2], st[1][3])));
+        mx = rows_max(mx);
+        if (g == 0) top_s[kh][ct * 16 + n] = mx;
+        __syncthreads();
+        float corr[4];
+        bool moved = false;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const float to_m = fmaxf(m[k], fmaxf(top_s[0][k * 16 + n], top_s[1][k * 16 + n]) * scale_log2e);
+            const bool up = to_m > m[k] + 8.0f;
+            corr[k] = up ? __builtin_amdgcn_exp2f(m[k] - to_m) : 1.0f;           // (m = -inf: 0)
+            m[k] = up ? to_m : m[k];
+            moved |= up;
+        }
+        const float m_own = ct == 0 ? m[0] : (ct == 1 ? m[1] : (ct == 2 ? m[2] : m[3]));
+        const float corr_own = ct == 0 ? corr[0] : (ct == 1 ? corr[1] : (ct == 2 ? corr[2] : corr[3]));
+        const float ref = m_own == -INFINITY ? 0.f : m_own;                      // nothing seen yet: all weights 0
+        float rs = 0.f;
+        gbf16x8_t pb;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[u][e], scale_log2e, -ref));
+                rs += p;
+                pb[u * 4 + e] = (__bf16)p;
+            }
+        l = l * corr_own + rows_sum(rs);
+        p_s[ct][kh][lane] = pb;
+        store_keys();
+        __syncthreads();
+        if (__builtin_amdgcn_ballot_w64(moved)) {
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int d = 0; d < DTW; ++d) acc[d][k] *= corr[k];
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const gbf16x8_t pf = p_s[k][h][lane];
+#pragma unroll
+                for (int d = 0; d < DTW; ++d) acc[d][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[h][d], pf, acc[d][k], 0, 0, 0);
+            }
+    }
+    if (g == 0) sum_s[kh][ct * 16 + n] = l;
+    __syncthreads();
+    // lane (column n of tile k, g): acc[d][k][i] is value feature (wave * DTW + d) * 16 + 4 g + i
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if ((k * 16 + n) / G >= n_tok) continue;
+        const long t = t0 + token_of(k);
+        const int head = head_of(k);
+        float total_l = sum_s[0][k * 16 + n] + sum_s[1][k * 16 + n];
+        if (sink) total_l += exp2f(sink[head] * 1.4426950408889634f - m[k]);
+        const float inv = 1.0f / total_l;
+#pragma unroll
+        for (int d = 0; d < DTW; ++d) {
+            const int f = (wave * DTW + d) * 16 + 4 * g;
+            if (f >= hdv) continue;
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                v[i] = acc[d][k][i] * inv;
+                if (gate) v[i] /= 1.0f + expf(-to_f32(gate[t * ld_gate + (long)head * hdv + f + i]));
+            }
+            const long at = (t * nh + head) * hdv + f;
+            if (out_f32) store4((float*)out + at, v[0], v[1], v[2], v[3]);
+            else store4((bf16_t*)out + at, v[0], v[1], v[2], v[3]);
+        }
+    }
+}
+
+// tiles: runs of at most 64 * nkv / nh consecutive tokens of one sequence, int [n_tiles][2] (first packed token, tokens)
+extern "C" const char* cpmcu_attention_wide_prefill(const void* q, void* out, int out_f32, int nh, int nkv, int hdk, int hdv,
+                                                    int pool_hdk, int pool_hdv, float scale, int chunk, int window,
+                                                    int keep_first, const float* sink, const void* kpool, const void* vtpool,
+                                                    const int* page_table, int table_width, int page_size,
+                                                    const int* positions, const int* tok_slot, const int* tiles, int n_tiles,
+                                                    int v_share, const void* gate, long ld_gate, float softcap,
+                                                    hipStream_t stream) {
+    CPMCU_REQUIRE(nh > 0 && nkv > 0 && nh % nkv == 0 && 64 % (nh / nkv) == 0 && nkv <= 65535,
+                  "attention_wide_prefill: %d heads in %d groups (1, 2, 4 ... 64 heads a group are taken)", nh, nkv);
+    CPMCU_REQUIRE(hdk >= 8 && hdk % 8 == 0 && pool_hdk >= hdk && pool_hdk % 64 == 0 && pool_hdk <= 576,
+                  "attention_wide_prefill: %d key features cached as %d (multiples of 64 up to 576 are taken)", hdk, pool_hdk);
+    CPMCU_REQUIRE(hdv >= 4 && hdv % 4 == 0 && pool_hdv >= hdv && pool_hdv % 16 == 0 && pool_hdv <= 512,
+                  "attention_wide_prefill: %d value features cached as %d (multiples of 4, cached up to 512)", hdv, pool_hdv);
+    CPMCU_REQUIRE(n_tiles > 0 && page_size % 32 == 0 && v_share >= 1 && nkv % v_share == 0, "attention_wide_prefill: bad shape");
+    CPMCU_REQUIRE(chunk >= 0 && window >= 0 && keep_first >= 0 && (chunk == 0 || window == 0) && (window > 0 || keep_first == 0),
+                  "attention_wide_prefill: mask chunk %d, window %d, kept first tokens %d", chunk, window, keep_first);
+    CPMCU_REQUIRE(!gate || ld_gate >= (long)nh * hdv, "attention_wide_prefill: gate rows of %ld elements for %d heads of %d", ld_gate, nh, hdv);
+    CPMCU_REQUIRE((((uintptr_t)q | (uintptr_t)out | (uintptr_t)kpool | (uintptr_t)vtpool) & 15) == 0,
+                  "attention_wide_prefill: operands must start on 16-byte borders");
+    PagedView pv{page_table, table_width, page_size};
+    const float sl = softcap > 0.f ? 1.0f : scale * 1.4426950408889634f;
+    const float cap_in = softcap > 0.f ? scale / softcap : 0.f, cap_out = softcap > 0.f ? softcap * 1.4426950408889634f : 0.f;
+    const dim3 grid(n_tiles, nkv);
+#define LAUNCH(PKv, DTWv, EXACTv)                                                                                       \
+    attention_wide_prefill_kernel<PKv, DTWv, EXACTv><<<grid, 512, 0, stream>>>(                                                 \
+        (const bf16_t*)q, out, out_f32, (const bf16_t*)kpool, (const bf16_t*)vtpool, pv, positions, tok_slot, nh, nkv,  \
+        hdk, hdv, pool_hdk, pool_hdv, sl, chunk, window, keep_first, sink, tiles, v_share, (const bf16_t*)gate, ld_gate, \
+        cap_in, cap_out)
+#define BY_VALUES(PKv)                                                    \
+    do {                                                                  \
+        if (pool_hdk == 64 * PKv && pool_hdv <= 256) LAUNCH(PKv, 2, true); \
+        else if (pool_hdk == 64 * PKv) LAUNCH(PKv, 4, true);              \
+        else if (pool_hdv <= 256) LAUNCH(PKv, 2, false);                  \
+        else LAUNCH(PKv, 4, false);                                       \
+    } while (0)
+    if (pool_hdk <= 128) BY_VALUES(2);
+    else if (pool_hdk <= 256) BY_VALUES(4);
+    else BY_VALUES(9);
+#undef BY_VALUES
+#undef LAUNCH
+    CPMCU_LAUNCH_CHECK("attention_wide_prefill");
+    return nullptr;
+}
+
+// ===========================================================================
 // Fused forms of the steps between a mixer's input projection and its attention.
 // ===========================================================================
 template <typename IT, typename OT>

@@ -2127,6 +2127,54 @@ def attention_general_mfma(q: torch.Tensor, out: torch.Tensor, nh: int, nkv: int
         c_long(ld_head), _stream()))
 
 
+ATTENTION_WIDE_COLUMNS = 64
+
+
+def attention_wide_prefill_ok(q: torch.Tensor, nh: int, nkv: int, hdk: int, hdv: int, pool_hdk: int, pool_hdv: int,
+                              page_size: int) -> bool:
+    """Whether attention_wide_prefill takes these sizes: values of more than 128 features (up to 128 a wavefront keeps a
+    whole output row, and attention_general_mfma serves), keys cached in multiples of 64 up to 576, heads a kv head that
+    divide 64."""
+    return (q.dtype == torch.bfloat16 and ATTENTION_WIDE_COLUMNS % (nh // nkv) == 0 and hdk % 8 == 0 and pool_hdk % 64 == 0
+            and pool_hdk <= 576 and hdv % 4 == 0 and 128 < pool_hdv <= 512 and page_size % 32 == 0)
+
+
+def attention_wide_prefill(q: torch.Tensor, out: torch.Tensor, tiles: torch.Tensor, nh: int, nkv: int, hdk: int, hdv: int,
+                           scale: float, kpool: torch.Tensor, vpool: torch.Tensor, page_table: torch.Tensor, page_size: int,
+                           positions: torch.Tensor, tok_slot: torch.Tensor, chunk: int = 0, window: int = 0,
+                           keep_first: int = 0, sink: Optional[torch.Tensor] = None, v_share: int = 1,
+                           gate: Optional[torch.Tensor] = None, softcap: float = 0.0):
+    """attention_general_mfma for prompts with wide values (attention_wide_prefill_ok): tiles int32 [T, 2] = (first packed
+    token, tokens), each a run of at most 64 * nkv / nh consecutive tokens of one sequence."""
+    _need(q, "attention q", torch.bfloat16, (None, nh * hdk))
+    n = q.shape[0]
+    if out.dtype not in (torch.bfloat16, torch.float32):
+        raise KernelError(f"attention out: dtype {out.dtype} (bfloat16 or float32)")
+    _need(out, "attention out", out.dtype, (n, nh * hdv))
+    _need(tiles, "attention tiles", torch.int32, (None, 2))
+    _need(kpool, "attention key pool", torch.bfloat16, (None, page_size, None))
+    _need(vpool, "attention value pool", torch.bfloat16, (kpool.shape[0], page_size, None))
+    nvh = _value_heads(nkv, v_share)
+    if kpool.shape[2] % nkv or vpool.shape[2] % nvh:
+        raise KernelError(f"attention_wide_prefill: pools of {kpool.shape[2]} / {vpool.shape[2]} features do not hold {nkv} / {nvh} heads")
+    _need(page_table, "attention page table", torch.int32, (None, None))
+    _need(positions, "attention positions", torch.int32, (n,))
+    _need(tok_slot, "attention token slots", torch.int32, (n,))
+    if sink is not None:
+        _need(sink, "attention sink", torch.float32, (nh,))
+    ld_gate = 0
+    if gate is not None:
+        ld_gate = _ld(gate, "attention gate")
+        if gate.dtype != torch.bfloat16 or tuple(gate.shape) != (n, nh * hdv):
+            raise KernelError(f"attention gate: {gate.dtype} {tuple(gate.shape)}, expected bfloat16 {(n, nh * hdv)}")
+    _check(_fn("attention_general", "cpmcu_attention_wide_prefill")(
+        _p(q), _p(out), c_int(1 if out.dtype == torch.float32 else 0), c_int(nh), c_int(nkv), c_int(hdk), c_int(hdv),
+        c_int(kpool.shape[2] // nkv), c_int(vpool.shape[2] // nvh), c_float(scale), c_int(chunk), c_int(window),
+        c_int(keep_first), _p(sink), _p(kpool), _p(vpool), _p(page_table), c_int(page_table.shape[1]), c_int(page_size),
+        _p(positions), _p(tok_slot), _p(tiles), c_int(tiles.shape[0]), c_int(v_share), _p(gate), c_long(ld_gate),
+        c_float(softcap or 0.0), _stream()))
+
+
 def attention_general_tokens_per_tile(n_tokens: int, nh: int, nkv: int, pool_hdv: int) -> int:
     """Tokens that share a matrix-core tile in attention_general_mfma: prompts of more than 256 tokens whose
     kv heads serve fewer than 16 query heads fill the tile's 16 columns with the heads of several consecutive
@@ -2172,6 +2220,15 @@ def attention_any(q, out, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, pa
             and kpool.shape[2] == nkv * hdk and v_share == 1 and not softcap and out.dtype == q.dtype):
         attention(q, out, nh, nkv, hdk, scale, kpool, vpool, page_table, page_size, ctx)
         return False
+    if not ctx.single_token and attention_wide_prefill_ok(q, nh, nkv, hdk, hdv, kpool.shape[2] // nkv, pool_hdv, page_size):
+        per = ATTENTION_WIDE_COLUMNS * nkv // nh
+        key = ("prefill_tiles", per)
+        tiles = ctx.extras.get(key)
+        if tiles is None:
+            tiles = ctx.extras[key] = prefill_tiles(ctx.q_lens, per, q.device)
+        attention_wide_prefill(q, out, tiles, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, page_size, ctx.positions,
+                               ctx.tok_slot, chunk, window, keep_first, sink, v_share, gate, softcap)
+        return gate is not None
     if attention_general_mfma_ok(q, hdk, hdv, page_size):
         n = q.shape[0]
         keys = ctx.max_pos + 1

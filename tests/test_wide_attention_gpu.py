@@ -1,0 +1,90 @@
+"""Prompt attention with wide values against a plain computation in double: heads a group, key and value sizes at and beside
+the built ones, masks, sinks, caps, gates, shared values, page sizes, tiles that end early, a history in the cache (GPU)."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def element_order(tokens, heads, hd, keys):
+    """Where element [token, head, feature] of a run of pages lies (pages one behind the other)."""
+    t, h, d = torch.arange(tokens)[:, None, None], torch.arange(heads)[None, :, None], torch.arange(hd)[None, None]
+    base, i = ((t // 32) * heads + h) * 32 * hd, t % 32
+    if keys:
+        return base + ((i // 4) % 2) * hd * 16 + ((i // 8) * 4 + i % 4) * 8 + (d // 8) * 128 + d % 8
+    return base + (i // 8) * 128 + i % 8 + (d // 16) * 512 + (d % 16) * 8
+
+
+CASES = [
+    # heads, kv heads, key features, cached as, value features, v_share, options
+    (32, 1, 576, 576, 512, 1, {}),
+    (32, 1, 576, 576, 512, 1, {"window": 37, "sink": True, "gate": True}),
+    (32, 8, 128, 128, 256, 2, {"out": torch.float32}),
+    (4, 4, 120, 128, 144, 1, {"chunk": 48}),
+    (64, 1, 192, 192, 512, 1, {"softcap": 3.0}),
+    (6, 3, 64, 64, 260, 3, {"window": 20, "keep_first": 5, "page": 32}),
+    (16, 2, 320, 320, 132, 1, {"page": 96, "sink": True}),
+]
+
+
+@pytest.mark.parametrize("nh,nkv,hdk,pool_hdk,hdv,v_share,opt", CASES)
+def test_wide_prompt_attention(nh, nkv, hdk, pool_hdk, hdv, v_share, opt):
+    from cpmcu_amd import ops
+    page, pool_hdv, nvh = opt.get("page", 64), -(-hdv // 16) * 16, nkv // v_share
+    g = torch.Generator().manual_seed(hdk + hdv)
+    spans = [(0, 131), (70, 96), (5, 6), (33, 64)]                 # (first new token, length) of every sequence
+    pages = [-(-b // page) for _, b in spans]
+    place = torch.randperm(sum(pages), generator=g)
+    table = torch.zeros(len(spans), max(pages), dtype=torch.int32)
+    kpool = torch.zeros(sum(pages), page, nkv * pool_hdk, dtype=torch.bfloat16)
+    vpool = torch.zeros(sum(pages), page, nvh * pool_hdv, dtype=torch.bfloat16)
+    ks, vs, at = [], [], 0
+    for s, (_, length) in enumerate(spans):
+        k = torch.randn(length, nkv, hdk, generator=g).to(torch.bfloat16)
+        v = torch.randn(length, nvh, hdv, generator=g).to(torch.bfloat16)
+        ks.append(k.double())
+        vs.append(v.double())
+        mine = place[at:at + pages[s]]
+        at += pages[s]
+        table[s, :pages[s]] = mine.int()
+        for pool, x, heads, hd, is_key in ((kpool, k, nkv, pool_hdk, True), (vpool, v, nvh, pool_hdv, False)):
+            flat = torch.zeros(pages[s] * page * heads * hd, dtype=torch.bfloat16)
+            order = element_order(length, heads, hd, is_key)[..., :x.shape[-1]]
+            flat[order.flatten()] = x.flatten()
+            pool[mine] = flat.view(pages[s], page, heads * hd)
+    pos = torch.cat([torch.arange(a, b) for a, b in spans]).int()
+    slot = torch.cat([torch.full((b - a,), s) for s, (a, b) in enumerate(spans)]).int()
+    n = pos.numel()
+    q = torch.randn(n, nh, hdk, generator=g).to(torch.bfloat16)
+    sink = torch.randn(nh, generator=g) if opt.get("sink") else None
+    gate = torch.randn(n, nh * hdv, generator=g).to(torch.bfloat16) if opt.get("gate") else None
+    scale, cap = 1.3 * hdk ** -0.5, opt.get("softcap", 0.0)
+    chunk, window, keep = opt.get("chunk", 0), opt.get("window", 0), opt.get("keep_first", 0)
+    dev = lambda t: None if t is None else t.to(DEV)
+    tiles = ops.prefill_tiles([b - a for a, b in spans], 64 * nkv // nh, DEV)
+    out = torch.full((n, nh * hdv), float("nan"), dtype=opt.get("out", torch.bfloat16), device=DEV)
+    assert ops.attention_wide_prefill_ok(dev(q), nh, nkv, hdk, hdv, pool_hdk, pool_hdv, page)
+    ops.attention_wide_prefill(dev(q.view(n, -1)), out, tiles, nh, nkv, hdk, hdv, scale, dev(kpool), dev(vpool), dev(table), page,
+                               dev(pos), dev(slot), chunk, window, keep, dev(sink), v_share, dev(gate), cap)
+    got = out.double().cpu().view(n, nh, hdv)
+    rep = nh // nkv
+    for t in range(n):
+        p, s = int(pos[t]), int(slot[t])
+        k, v = ks[s][:p + 1].repeat_interleave(rep, 1), vs[s][:p + 1].repeat_interleave(rep * v_share, 1)
+        sc = torch.einsum("hd,jhd->hj", q[t].double(), k) * scale
+        sc = cap * torch.tanh(sc / cap) if cap else sc
+        j = torch.arange(p + 1)
+        hidden = (j // chunk != p // chunk) if chunk else ((p - j >= window) & (j >= keep)) if window else torch.zeros(p + 1, dtype=torch.bool)
+        sc = sc.masked_fill(hidden, -math.inf)
+        if sink is not None:
+            sc = torch.cat([sc, sink.double()[:, None]], 1)
+        w = torch.softmax(sc, -1)[:, :p + 1]
+        want, size = torch.einsum("hj,jhd->hd", w, v), torch.einsum("hj,jhd->hd", w, v.abs())
+        if gate is not None:
+            s_g = torch.sigmoid(gate[t].double().view(nh, hdv))
+            want, size = want * s_g, size * s_g
+        # weights rounded to bf16 (half an ulp each) against values of that size, and the output's own rounding
+        assert bool(((got[t] - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-5).all()), (t, p, s)
