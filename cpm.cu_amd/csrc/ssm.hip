@@ -331,10 +331,192 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const float* __restrict__
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same recurrence for prompts, 64 tokens at a time on the matrix cores' float instruction (v_mfma_f32_16x16x4_f32:
+// operands as they are, sums in float).  With la_t = the sum of -A d_s over the chunk's tokens up to t, every term of
+//     y_t = exp(la_t) C_t . S + sum_(s <= t) (C_t . B_s) exp(la_t - la_s) d_s x_s + D x_t
+//     S  <- exp(la_63) S + sum_s exp(la_63 - la_s) d_s x_s B_s^T
+// is a product over the chunk, and every exponent is <= 0; la is summed in double, so that a difference of two large sums
+// is as good as the walk's product of factors.  A workgroup owns one (sequence, head, 32 columns of P); its state stays in
+// the accumulators' registers and passes through LDS as an operand.  The walk's cost is one dependent chain a token (0.35
+// us); a chunk takes 7.5 us: 128 heads of 64, state 128, 2,048 tokens 719 -> 241 us.
+// A lane's 16 bytes serve four instructions: instruction j of a block takes index 4 g + j of the 16 in both operands.
+// ---------------------------------------------------------------------------
+typedef float sfloatx4_t __attribute__((ext_vector_type(4)));
+#define CHUNK_T 64        // tokens a chunk
+#define CHUNK_N 128       // state values a column, at most
+#define CHUNK_LN 132      // LDS rows of CHUNK_N: rows 4 banks apart, so that 8 rows' 16 bytes read all banks
+#define CHUNK_LT 68       // LDS rows of CHUNK_T
+#define CHUNK_MIN 64      // tokens a sequence from which chunks are taken
+
+template <int NB, typename DT>
+__global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict__ xbc, long ldx,
+                                                        const DT* __restrict__ dt, long lddt,
+                                                        const float* __restrict__ dt_bias,
+                                                        const float* __restrict__ A_log, const float* __restrict__ Dskip,
+                                                        float* __restrict__ state, float* __restrict__ y,
+                                                        const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
+                                                        int heads, int P, int N, int groups, int write_state) {
+    __shared__ __align__(16) float Cs[CHUNK_T * CHUNK_LN], Bs[CHUNK_T * CHUNK_LN];
+    __shared__ __align__(16) float Ss[SCAN_PB * CHUNK_LN];             // the state before the chunk, [p][n]
+    __shared__ __align__(16) float Gs[CHUNK_T * CHUNK_LT];             // (C_t . B_s) exp(la_t - la_s) d_s
+    __shared__ __align__(16) float xT[SCAN_PB * CHUNK_LT];             // [p][t]
+    __shared__ __align__(16) float ds[CHUNK_T], left_s[CHUNK_T], from_s[CHUNK_T];   // d; exp(la_63 - la_t) d; exp(la_t)
+    __shared__ double la_s[CHUNK_T];
+    const int b = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * SCAN_PB;
+    const int start = cu_q[b], q = cu_q[b + 1] - start;
+    if (q <= 0) return;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int inner = heads * P;
+    const long b_col = inner + (long)(h / (heads / groups)) * N, c_col = b_col + (long)groups * N;
+    float* sp = state + (((long)seq_slot[b] * heads + h) * P + p0) * N;
+    // the state as the accumulators hold it: st[i][e] is column p = 16 i + 4 g + e, value n = 16 wave + r
+    const int n_own = 16 * wave + r;
+    sfloatx4_t st[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int p = 16 * i + 4 * g + e;
+            st[i][e] = (p0 + p < P && n_own < N) ? sp[(long)p * N + n_own] : 0.f;
+        }
+    const float A = expf(A_log[h]), bias = dt_bias[h], Dh = Dskip[h];
+    const sfloatx4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    sfloatx4_t rb[4], rc[4], rx;
+    float rdt = 0.f;
+    auto fetch = [&](int t0) {
+        const int tn = min(CHUNK_T, q - t0);
+        const float* base = xbc + (long)(start + t0) * ldx;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = threadIdx.x + 512 * i, n = (e & 31) * 4;
+            const float* row = base + (long)min(e >> 5, tn - 1) * ldx + min(n, N - 4);
+            rb[i] = *(const sfloatx4_t*)(row + b_col);
+            rc[i] = *(const sfloatx4_t*)(row + c_col);
+            if (n >= N) rb[i] = rc[i] = zero4;
+        }
+        const int p = p0 + (threadIdx.x & 7) * 4;
+        rx = *(const sfloatx4_t*)(base + (long)min((int)threadIdx.x >> 3, tn - 1) * ldx + (long)h * P + min(p, P - 4));
+        if (p >= P) rx = zero4;
+        if (wave == 0) rdt = to_f32(dt[(long)(start + t0 + min(lane, tn - 1)) * lddt + h]);
+    };
+    auto state_to_lds = [&]() {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Ss[(16 * i + 4 * g + e) * CHUNK_LN + n_own] = st[i][e];
+    };
+    fetch(0);
+    for (int t0 = 0; t0 < q; t0 += CHUNK_T) {
+        const int tn = min(CHUNK_T, q - t0);
+        state_to_lds();
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = threadIdx.x + 512 * i, at = (e >> 5) * CHUNK_LN + (e & 31) * 4;
+            *(sfloatx4_t*)&Bs[at] = rb[i];
+            *(sfloatx4_t*)&Cs[at] = rc[i];
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) xT[((threadIdx.x & 7) * 4 + j) * CHUNK_LT + (threadIdx.x >> 3)] = rx[j];
+        if (wave == 0) {
+            // a token beyond the end has d = 0: it neither writes nor forgets
+            const float d = lane < tn ? softplus_f(rdt + bias) : 0.f;
+            double la = -(double)A * (double)d;
+#pragma unroll
+            for (int k = 1; k < 64; k <<= 1) {
+                const double up = __shfl_up(la, k, 64);
+                if (lane >= k) la += up;
+            }
+            const double all = __shfl(la, 63, 64);
+            ds[lane] = d;
+            la_s[lane] = la;
+            left_s[lane] = expf((float)(all - la)) * d;
+            from_s[lane] = expf((float)la);
+        }
+        __syncthreads();
+        if (t0 + CHUNK_T < q) fetch(t0 + CHUNK_T);
+        // G, the tiles on and below the diagonal, dealt to the wavefronts
+        for (int k = wave; k < 10; k += 8) {
+            const int i = k < 1 ? 0 : (k < 3 ? 1 : (k < 6 ? 2 : 3)), j = k - i * (i + 1) / 2;
+            sfloatx4_t a = zero4;
+#pragma unroll
+            for (int kb = 0; kb < NB; ++kb) {
+                const sfloatx4_t c4 = *(const sfloatx4_t*)&Cs[(16 * i + r) * CHUNK_LN + 16 * kb + 4 * g];
+                const sfloatx4_t b4 = *(const sfloatx4_t*)&Bs[(16 * j + r) * CHUNK_LN + 16 * kb + 4 * g];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) a = __builtin_amdgcn_mfma_f32_16x16x4f32(c4[e], b4[e], a, 0, 0, 0);
+            }
+            const int s = 16 * j + r;
+            const double la = la_s[s];
+            const float d = ds[s];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * i + 4 * g + e;
+                Gs[t * CHUNK_LT + s] = s <= t ? a[e] * expf((float)(la_s[t] - la)) * d : 0.f;
+            }
+        }
+        // tokens 16 tt .. + 15, columns 16 pt .. + 15: what the state before the chunk gives them
+        const int tt = wave >> 1, pt = wave & 1;
+        sfloatx4_t yt = zero4;
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb) {
+            const sfloatx4_t c4 = *(const sfloatx4_t*)&Cs[(16 * tt + r) * CHUNK_LN + 16 * kb + 4 * g];
+            const sfloatx4_t s4 = *(const sfloatx4_t*)&Ss[(16 * pt + r) * CHUNK_LN + 16 * kb + 4 * g];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) yt = __builtin_amdgcn_mfma_f32_16x16x4f32(c4[e], s4[e], yt, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) yt[e] *= from_s[16 * tt + 4 * g + e];
+        __syncthreads();
+        // ... and what the chunk's own tokens give them
+        for (int kb = 0; kb <= tt; ++kb) {
+            const sfloatx4_t g4 = *(const sfloatx4_t*)&Gs[(16 * tt + r) * CHUNK_LT + 16 * kb + 4 * g];
+            const sfloatx4_t x4 = *(const sfloatx4_t*)&xT[(16 * pt + r) * CHUNK_LT + 16 * kb + 4 * g];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) yt = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[e], x4[e], yt, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 16 * tt + 4 * g + e, p = 16 * pt + r;
+            if (t < tn && p0 + p < P)
+                y[(long)(start + t0 + t) * inner + (long)h * P + p0 + p] = yt[e] + Dh * xT[p * CHUNK_LT + t];
+        }
+        // the state behind the chunk
+        const float keep = from_s[CHUNK_T - 1];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) st[i] *= keep;
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            const sfloatx4_t w4 = *(const sfloatx4_t*)&left_s[16 * kb + 4 * g];
+            sfloatx4_t x4[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) x4[i] = *(const sfloatx4_t*)&xT[(16 * i + r) * CHUNK_LT + 16 * kb + 4 * g] * w4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float bv = Bs[(16 * kb + 4 * g + e) * CHUNK_LN + n_own];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) st[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x4[i][e], bv, st[i], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+    if (write_state) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int p = 16 * i + 4 * g + e;
+                if (p0 + p < P && n_own < N) sp[(long)p * N + n_own] = st[i][e];
+            }
+    }
+}
+
+// max_q: the longest run of tokens a sequence brings (0: not known, the walk)
 extern "C" const char* cpmcu_ssm_scan(const float* xbc, long ldx, const void* dt, long lddt, int dt_dtype,
                                       const float* dt_bias, const float* A_log, const float* Dskip, float* state,
                                       float* y, const int* cu_q, const int* seq_slot, int n_seqs, int heads, int P,
-                                      int N, int groups, int write_state, hipStream_t stream) {
+                                      int N, int groups, int write_state, int max_q, hipStream_t stream) {
     CPMCU_REQUIRE(n_seqs > 0 && heads > 0 && P > 0 && N > 0 && groups > 0, "ssm_scan: empty shape");
     CPMCU_REQUIRE(heads % groups == 0, "ssm_scan: %d heads are not a multiple of %d groups", heads, groups);
     CPMCU_REQUIRE(N <= 256, "ssm_scan: a state of %d values a column is not supported (at most 256)", N);
@@ -342,6 +524,25 @@ extern "C" const char* cpmcu_ssm_scan(const float* xbc, long ldx, const void* dt
     const int pb = (P + SCAN_PB - 1) / SCAN_PB;
     CPMCU_REQUIRE(heads <= 65535 && pb <= 65535, "ssm_scan: shape exceeds the launch grid");
     dim3 grid(n_seqs, heads, pb);
+    // A chunk costs the same whatever it holds, and its LDS leaves a CU one workgroup: from 64 tokens a sequence on it is
+    // the cheaper one at any number of sequences (us, walk / chunks: 1 x 64 tokens 29 / 18, 32 x 64 363 / 295, 8 x 32
+    // 55 / 71, 32 x 16 114 / 269).
+    if (max_q >= CHUNK_MIN && N <= CHUNK_N && N % 4 == 0 && P % 4 == 0 && ldx % 4 == 0 && (uintptr_t)xbc % 16 == 0 &&
+        (dt_dtype == CPMCU_F32 || dt_dtype == CPMCU_BF16)) {
+#define CHUNKS(NBv, DTv)                                                                                           \
+    ssm_chunk_kernel<NBv, DTv><<<grid, 512, 0, stream>>>(xbc, ldx, (const DTv*)dt, lddt, dt_bias, A_log, Dskip, state, y, \
+                                                         cu_q, seq_slot, heads, P, N, groups, write_state)
+        if (dt_dtype == CPMCU_F32) {
+            if (N <= 64) CHUNKS(4, float);
+            else CHUNKS(8, float);
+        } else {
+            if (N <= 64) CHUNKS(4, bf16_t);
+            else CHUNKS(8, bf16_t);
+        }
+#undef CHUNKS
+        CPMCU_LAUNCH_CHECK("ssm_chunk");
+        return nullptr;
+    }
     const int need = (N + SCAN_L - 1) / SCAN_L;
 #define LAUNCH(NRv, TTv, DTv)                                                                                    \
     ssm_scan_kernel<NRv, TTv, DTv><<<grid, 256, 0, stream>>>(xbc, ldx, (const DTv*)dt, lddt, dt_bias, A_log, Dskip, \

@@ -616,8 +616,9 @@ def conv_silu(u: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
 
 def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor,
              state: torch.Tensor, y: torch.Tensor, cu_q: torch.Tensor, seq_slot: torch.Tensor, heads: int, P: int,
-             N: int, groups: int, write_state: bool = True):
-    """The state-space recurrence over each sequence's tokens, in float: per head h (group h // (heads/groups)),
+             N: int, groups: int, write_state: bool = True, max_q: int = 0):
+    """The state-space recurrence over each sequence's tokens, in float (max_q, the longest run of tokens a sequence brings,
+    lets prompts be taken 64 tokens at a time; 0: walked token by token): per head h (group h // (heads/groups)),
     d = softplus(dt + dt_bias[h]); S <- exp(-exp(A_log[h]) d) S + d B x^T; y = S^T C + D[h] x.
     xbc float32 [n, heads*P + 2*groups*N] = [x | B | C]; dt [n, heads] (may be a column slice);
     state float32 [slots, heads, P, N]; y float32 [n, heads*P]."""
@@ -636,7 +637,7 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A_log: 
     _check(_fn("ssm", "cpmcu_ssm_scan")(_p(xbc), c_long(xbc.shape[1]), _p(dt), c_long(lddt), c_int(_code(dt)),
                                         _p(dt_bias), _p(A_log), _p(D), _p(state), _p(y), _p(cu_q), _p(seq_slot),
                                         c_int(B), c_int(heads), c_int(P), c_int(N), c_int(groups),
-                                        c_int(1 if write_state else 0), _stream()))
+                                        c_int(1 if write_state else 0), c_int(max_q), _stream()))
 
 
 ROTATE_TO_ROWS, ROTATE_TO_KEYS, ROTATE_TO_VALUES = 0, 1, 2

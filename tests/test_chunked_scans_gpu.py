@@ -1,0 +1,54 @@
+"""Recurrences taken 64 tokens at a time against a walk in double: runs that end inside, at and behind a chunk, several
+sequences, a state that is carried on, sizes that do not fill a tile (GPU)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def i32(x):
+    return torch.tensor(x, dtype=torch.int32, device=DEV)
+
+
+def off(got, want):
+    return float((got.double().cpu() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("H,P,N,G,scale", [(4, 64, 128, 2, 1.0), (3, 36, 20, 1, 1.0), (2, 8, 64, 2, 6.0), (1, 4, 4, 1, 0.05)])
+def test_state_space_chunks(H, P, N, G, scale):
+    """`scale` stretches the step sizes: strong decays within a chunk, and nearly none."""
+    from cpmcu_amd import ops
+    g = torch.Generator().manual_seed(P + N)
+    first, second = [17, 64, 65, 200], [64, 1, 130, 16]
+    width = H * P + 2 * G * N
+    A_log, bias, D = torch.log(0.05 + 3 * torch.rand(H, generator=g)), torch.randn(H, generator=g), torch.randn(H, generator=g)
+    state = torch.zeros(6, H, P, N, device=DEV)
+    walked = state.clone()
+    S = [torch.zeros(H, P, N, dtype=torch.float64) for _ in first]
+    slots = [4, 0, 5, 2]
+    for lens in (first, second):
+        n = sum(lens)
+        cu = [0]
+        for q in lens:
+            cu.append(cu[-1] + q)
+        xbc, dt = torch.randn(n, width, generator=g), torch.randn(n, H, generator=g) * scale
+        want = torch.empty(n, H, P, dtype=torch.float64)
+        d = torch.nn.functional.softplus(dt.double() + bias.double())
+        x = xbc[:, :H * P].double().view(n, H, P)
+        B, C = (xbc[:, H * P + k * G * N:H * P + (k + 1) * G * N].double().view(n, G, N).repeat_interleave(H // G, 1) for k in (0, 1))
+        for s, q in enumerate(lens):
+            for t in range(cu[s], cu[s] + q):
+                S[s] = torch.exp(-torch.exp(A_log.double()) * d[t])[:, None, None] * S[s] + (d[t][:, None] * x[t])[:, :, None] * B[t][:, None]
+                want[t] = (S[s] * C[t][:, None]).sum(-1) + D.double()[:, None] * x[t]
+        outs = []
+        for st, most in ((state, max(lens)), (walked, 0)):
+            y = torch.full((n, H * P), float("nan"), device=DEV)
+            ops.ssm_scan(xbc.to(DEV), dt.to(DEV), bias.to(DEV), A_log.to(DEV), D.to(DEV), st, y, i32(cu), i32(slots), H, P, N, G, max_q=most)
+            outs.append(off(y.view(n, H, P), want))
+        final = torch.stack(S)
+        here, walk = (off(st[slots], final) for st in (state, walked))
+        # float sums of up to 64 + N terms, every factor an exponential good to an ulp or two
+        assert outs[0] <= 2e-6 and here <= 2e-6, (outs, here, walk)
+        assert outs[0] <= 1.5 * outs[1] + 2e-7 and here <= 1.5 * walk + 2e-7, (outs, here, walk)
+    assert float(state[[1, 3]].abs().max()) == 0.0
