@@ -189,11 +189,269 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
     }
 }
 
+// ---------------------------------------------------------------------------
+// The delta rule with a decay a head (RULE_DELTA) for prompts, 64 tokens at a time on the matrix cores' float instruction
+// (v_mfma_f32_16x16x4_f32: operands as they are, sums in float).  With la_t = the sum of ln g over the chunk's tokens up to
+// t (in double, so that a difference of two sums is as good as the walk's product of factors; no exponent is positive) and
+// S the state before the chunk, the walk's u_t are the solution of a triangular system, and the rest are products:
+//     u_t + sum_(s < t) A[t, s] u_s = beta_t (v_t - exp(la_t) S^T k_t),    A[t, s] = beta_t exp(la_t - la_s) k_t . k_s
+//     o_t = exp(la_t) S^T q_t + sum_(s <= t) exp(la_t - la_s) (q_t . k_s) u_s
+//     S  <- exp(la_63) S + sum_s exp(la_63 - la_s) k_s u_s^T
+// (k, q the unit vectors: their factors are multiplied in where a product's results leave the accumulators.)  The system is
+// solved 16 rows at a time: the diagonal blocks of I + A are inverted by one wavefront, a lane a column; then a wavefront
+// owns 16 columns of u and needs nobody else's.  A workgroup owns one (sequence, head, 16 PT columns of dv), its state stays
+// in the accumulators' registers and passes through LDS as an operand.  The walk's cost is one dependent chain a token (0.35
+// us), a chunk takes 11 us: 32 heads of 128 by 128, 1,500 tokens 528 -> 262 us (298 with 32 columns a workgroup).
+// A lane's 16 bytes serve four instructions: instruction j of a block takes index 4 g + j of the 16 in both operands.
+// ---------------------------------------------------------------------------
+typedef float dfloatx4_t __attribute__((ext_vector_type(4)));
+#define DCHUNK_T 64       // tokens a chunk
+#define DCHUNK_N 128      // key features, at most
+#define DCHUNK_LN 132     // LDS rows of DCHUNK_N: rows 4 banks apart, so that 8 rows' 16 bytes read all banks
+#define DCHUNK_LT 68      // LDS rows of DCHUNK_T
+#define DCHUNK_MIN 64     // tokens a sequence from which chunks are taken
+
+template <int NB, int PT, typename GT>
+__global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restrict__ qkv, long ld,
+                                                          const GT* __restrict__ gates, long ldg, long a_off, long b_off,
+                                                          const float* __restrict__ dt_bias, const float* __restrict__ A_log,
+                                                          float* __restrict__ state, float* __restrict__ y,
+                                                          const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
+                                                          int heads, int kv_heads, int dk, int dv, float q_scale,
+                                                          int write_state) {
+    constexpr int PB = 16 * PT;                                         // columns of dv a workgroup
+    __shared__ __align__(16) float Ks[DCHUNK_T * DCHUNK_LN], Qs[DCHUNK_T * DCHUNK_LN];
+    __shared__ __align__(16) float Ss[PB * DCHUNK_LN];            // the state before the chunk, [p][n]
+    __shared__ __align__(16) float As[DCHUNK_T * DCHUNK_LT];            // -A
+    __shared__ __align__(16) float Gs[DCHUNK_T * DCHUNK_LT];            // exp(la_t - la_s) q_t . k_s
+    __shared__ __align__(16) float uT[PB * DCHUNK_LT];            // v, then the right-hand side, then u: [p][t]
+    __shared__ __align__(16) float inv_s[4 * 16 * 20];                  // inverses of the diagonal blocks
+    __shared__ __align__(16) float fk_s[DCHUNK_T], fq_s[DCHUNK_T], beta_s[DCHUNK_T], left_s[DCHUNK_T], from_s[DCHUNK_T];
+    __shared__ double la_s[DCHUNK_T];
+    const int b = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * PB;
+    const int start = cu_q[b], q = cu_q[b + 1] - start;
+    if (q <= 0) return;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int kvh = h / (heads / kv_heads);
+    const long q_col = (long)kvh * dk, k_col = q_col + (long)kv_heads * dk, v_col = 2L * kv_heads * dk + (long)h * dv;
+    float* sp = state + (((long)seq_slot[b] * heads + h) * dv + p0) * dk;
+    // the state as the accumulators hold it: st[i][e] is column p = 16 i + 4 g + e, key feature n = 16 wave + r
+    const int n_own = 16 * wave + r;
+    dfloatx4_t st[PT];
+#pragma unroll
+    for (int i = 0; i < PT; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int p = 16 * i + 4 * g + e;
+            st[i][e] = (p0 + p < dv && n_own < dk) ? sp[(long)p * dk + n_own] : 0.f;
+        }
+    const float A = expf(A_log[h]), bias = dt_bias[h];
+    const dfloatx4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    const int vrow = threadIdx.x / (PB / 4), vcol = threadIdx.x % (PB / 4) * 4;      // (with 16 columns half of the threads)
+    dfloatx4_t rq[4], rk[4], rv;
+    float ra = 0.f, rb = 0.f;
+    auto fetch = [&](int t0) {
+        const int tn = min(DCHUNK_T, q - t0);
+        const float* base = qkv + (long)(start + t0) * ld;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = threadIdx.x + 512 * i, n = (e & 31) * 4;
+            const float* row = base + (long)min(e >> 5, tn - 1) * ld + min(n, dk - 4);
+            rq[i] = *(const dfloatx4_t*)(row + q_col);
+            rk[i] = *(const dfloatx4_t*)(row + k_col);
+            if (n >= dk) rq[i] = rk[i] = zero4;
+        }
+        const int p = p0 + vcol;
+        rv = *(const dfloatx4_t*)(base + (long)min(vrow, tn - 1) * ld + v_col + min(p, dv - 4));
+        if (p >= dv) rv = zero4;
+        if (wave == 0) {
+            const GT* gr = gates + (long)(start + t0 + min(lane, tn - 1)) * ldg + h;
+            ra = to_f32(gr[a_off]);
+            rb = to_f32(gr[b_off]);
+        }
+    };
+    // one 16 x 16 tile of rows[i] . cols[j] over the key features
+    auto dot_tile = [&](const float* rows, int i, const float* cols, int j) {
+        dfloatx4_t a = zero4;
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb) {
+            const dfloatx4_t x = *(const dfloatx4_t*)&rows[(16 * i + r) * DCHUNK_LN + 16 * kb + 4 * g];
+            const dfloatx4_t z = *(const dfloatx4_t*)&cols[(16 * j + r) * DCHUNK_LN + 16 * kb + 4 * g];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], z[e], a, 0, 0, 0);
+        }
+        return a;
+    };
+    // this wavefront's tokens 16 tt .. and columns 16 pt .. (with 16 columns only the first four have any)
+    const int tt = PT == 2 ? wave >> 1 : wave & 3, pt = PT == 2 ? wave & 1 : 0;
+    const bool owns = PT == 2 || wave < 4;
+    fetch(0);
+    for (int t0 = 0; t0 < q; t0 += DCHUNK_T) {
+        const int tn = min(DCHUNK_T, q - t0);
+#pragma unroll
+        for (int i = 0; i < PT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) Ss[(16 * i + 4 * g + e) * DCHUNK_LN + n_own] = st[i][e];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = threadIdx.x + 512 * i, t = e >> 5, at = t * DCHUNK_LN + (e & 31) * 4;
+            *(dfloatx4_t*)&Ks[at] = rk[i];
+            *(dfloatx4_t*)&Qs[at] = rq[i];
+            // a row's 128 features lie in 32 neighbouring lanes
+            float sk = row16_sum(rk[i][0] * rk[i][0] + rk[i][1] * rk[i][1] + rk[i][2] * rk[i][2] + rk[i][3] * rk[i][3]);
+            float sq = row16_sum(rq[i][0] * rq[i][0] + rq[i][1] * rq[i][1] + rq[i][2] * rq[i][2] + rq[i][3] * rq[i][3]);
+            sk += __shfl_xor(sk, 16, 64);
+            sq += __shfl_xor(sq, 16, 64);
+            if ((lane & 31) == 0) {
+                fk_s[t] = 1.0f / sqrtf(sk + 1e-6f);
+                fq_s[t] = q_scale / sqrtf(sq + 1e-6f);
+            }
+        }
+        if (vrow < DCHUNK_T) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) uT[(vcol + j) * DCHUNK_LT + vrow] = rv[j];
+        }
+        if (wave == 0) {
+            // a token beyond the end has beta = 0 and g = 1: it neither writes nor forgets
+            double la = lane < tn ? -(double)A * (double)delta_softplus(ra + bias) : 0.0;
+#pragma unroll
+            for (int k = 1; k < 64; k <<= 1) {
+                const double up = __shfl_up(la, k, 64);
+                if (lane >= k) la += up;
+            }
+            const double all = __shfl(la, 63, 64);
+            beta_s[lane] = lane < tn ? 1.0f / (1.0f + expf(-rb)) : 0.f;
+            la_s[lane] = la;
+            left_s[lane] = expf((float)(all - la));
+            from_s[lane] = expf((float)la);
+        }
+        __syncthreads();
+        if (t0 + DCHUNK_T < q) fetch(t0 + DCHUNK_T);
+        // -A: the tiles on and below the diagonal, dealt to the wavefronts, first to those without a tile of their own
+        for (int k = (wave + 4) & 7; k < 10; k += 8) {
+            const int i = k < 1 ? 0 : (k < 3 ? 1 : (k < 6 ? 2 : 3)), j = k - i * (i + 1) / 2, s = 16 * j + r;
+            const dfloatx4_t a = dot_tile(Ks, i, Ks, j);
+            const double la = la_s[s];
+            const float f = fk_s[s];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * i + 4 * g + e;
+                As[t * DCHUNK_LT + s] = s < t ? -beta_s[t] * fk_s[t] * f * a[e] * expf((float)(la_s[t] - la)) : 0.f;
+            }
+        }
+        if (owns) {   // the right-hand side, in place of v
+            const dfloatx4_t a = dot_tile(Ks, tt, Ss, pt);
+            dfloatx4_t* at = (dfloatx4_t*)&uT[(16 * pt + r) * DCHUNK_LT + 16 * tt + 4 * g];
+            dfloatx4_t v = *at;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * tt + 4 * g + e;
+                v[e] = beta_s[t] * (v[e] - from_s[t] * fk_s[t] * a[e]);
+            }
+            *at = v;
+        }
+        __syncthreads();
+        if (wave == 7) {
+            // lane (block g, column r) of the inverse of I + A: x_t = [t == r] - sum_(s < t) A[t, s] x_s
+            float x[16];
+#pragma unroll
+            for (int t = 0; t < 16; ++t) {
+                float v = t == r ? 1.f : 0.f;
+#pragma unroll
+                for (int s = 0; s < t; ++s) v += As[(16 * g + t) * DCHUNK_LT + 16 * g + s] * x[s];
+                x[t] = v;
+            }
+#pragma unroll
+            for (int t = 0; t < 16; ++t) inv_s[(16 * g + t) * 20 + r] = x[t];
+        }
+        // what the state before the chunk gives this wavefront's tokens
+        dfloatx4_t yt = zero4;
+        if (owns) yt = dot_tile(Qs, tt, Ss, pt);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) yt[e] *= from_s[16 * tt + 4 * g + e] * fq_s[16 * tt + 4 * g + e];
+        __syncthreads();
+        if (wave < PT) {
+            // u of columns 16 wave .. + 15, 16 tokens after 16 tokens
+            float* u = uT + (16 * wave + r) * DCHUNK_LT + 4 * g;
+            for (int i = 0; i < 4; ++i) {
+                dfloatx4_t rhs = *(const dfloatx4_t*)(u + 16 * i);
+                for (int j = 0; j < i; ++j) {
+                    const dfloatx4_t a = *(const dfloatx4_t*)&As[(16 * i + r) * DCHUNK_LT + 16 * j + 4 * g];
+                    const dfloatx4_t x = *(const dfloatx4_t*)(u + 16 * j);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) rhs = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], x[e], rhs, 0, 0, 0);
+                }
+                // the accumulators (row 4 g + e, column r) lie where the operand (column r, index 4 g + e) is read
+                const dfloatx4_t d = *(const dfloatx4_t*)&inv_s[(16 * i + r) * 20 + 4 * g];
+                dfloatx4_t x = zero4;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x = __builtin_amdgcn_mfma_f32_16x16x4f32(d[e], rhs[e], x, 0, 0, 0);
+                *(dfloatx4_t*)(u + 16 * i) = x;
+                __builtin_amdgcn_wave_barrier();
+            }
+        } else {
+            for (int k = wave - PT; k < 10; k += 8 - PT) {
+                const int i = k < 1 ? 0 : (k < 3 ? 1 : (k < 6 ? 2 : 3)), j = k - i * (i + 1) / 2, s = 16 * j + r;
+                const dfloatx4_t a = dot_tile(Qs, i, Ks, j);
+                const double la = la_s[s];
+                const float f = fk_s[s];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = 16 * i + 4 * g + e;
+                    Gs[t * DCHUNK_LT + s] = s <= t ? fq_s[t] * f * a[e] * expf((float)(la_s[t] - la)) : 0.f;
+                }
+            }
+        }
+        __syncthreads();
+        // ... and what the chunk's own tokens give them
+        for (int kb = 0; owns && kb <= tt; ++kb) {
+            const dfloatx4_t a = *(const dfloatx4_t*)&Gs[(16 * tt + r) * DCHUNK_LT + 16 * kb + 4 * g];
+            const dfloatx4_t u = *(const dfloatx4_t*)&uT[(16 * pt + r) * DCHUNK_LT + 16 * kb + 4 * g];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) yt = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], u[e], yt, 0, 0, 0);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int t = 16 * tt + 4 * g + e, p = 16 * pt + r;
+            if (owns && t < tn && p0 + p < dv) y[(long)(start + t0 + t) * heads * dv + (long)h * dv + p0 + p] = yt[e];
+        }
+        // the state behind the chunk
+        const float keep = from_s[DCHUNK_T - 1];
+#pragma unroll
+        for (int i = 0; i < PT; ++i) st[i] *= keep;
+#pragma unroll
+        for (int kb = 0; kb < 4; ++kb) {
+            const dfloatx4_t w4 = *(const dfloatx4_t*)&left_s[16 * kb + 4 * g] * *(const dfloatx4_t*)&fk_s[16 * kb + 4 * g];
+            dfloatx4_t u4[PT];
+#pragma unroll
+            for (int i = 0; i < PT; ++i) u4[i] = *(const dfloatx4_t*)&uT[(16 * i + r) * DCHUNK_LT + 16 * kb + 4 * g] * w4;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float kv = Ks[(16 * kb + 4 * g + e) * DCHUNK_LN + n_own];
+#pragma unroll
+                for (int i = 0; i < PT; ++i) st[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(u4[i][e], kv, st[i], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+    if (write_state) {
+#pragma unroll
+        for (int i = 0; i < PT; ++i)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int p = 16 * i + 4 * g + e;
+                if (p0 + p < dv && n_own < dk) sp[(long)p * dk + n_own] = st[i][e];
+            }
+    }
+}
+
+// max_q: the longest run of tokens a sequence brings (0: not known, the walk)
 extern "C" const char* cpmcu_delta_scan(const float* qkv, long ld, const void* gates, long ldg, int gate_dtype,
                                         long a_off, long b_off, const float* chan_a, long ld_a, const float* dt_bias,
                                         const float* A_log, float* state, float* y, const int* cu_q,
                                         const int* seq_slot, int n_seqs, int heads, int kv_heads, int dk, int dv,
-                                        float q_scale, int write_state, int lanes, int rule, hipStream_t stream) {
+                                        float q_scale, int write_state, int lanes, int rule, int max_q, hipStream_t stream) {
     CPMCU_REQUIRE(rule == RULE_DELTA || rule == RULE_CHANNEL || rule == RULE_DECAY, "delta_scan: unknown rule %d", rule);
     CPMCU_REQUIRE(n_seqs > 0 && heads > 0 && kv_heads > 0 && dk > 0 && dv > 0, "delta_scan: empty shape");
     CPMCU_REQUIRE(heads % kv_heads == 0, "delta_scan: %d heads are not a multiple of %d key heads", heads, kv_heads);
@@ -204,6 +462,36 @@ extern "C" const char* cpmcu_delta_scan(const float* qkv, long ld, const void* g
     CPMCU_REQUIRE(rule != RULE_CHANNEL || (chan_a && ld_a >= (long)heads * dk), "delta_scan: channel decay rows too short");
     CPMCU_REQUIRE(A_log && (rule == RULE_DECAY || dt_bias), "delta_scan: decay constants missing");
     CPMCU_REQUIRE(lanes == 0 || lanes == 8 || lanes == 16, "delta_scan: %d lanes a column (0: chosen here, 8 or 16)", lanes);
+    if (rule == RULE_DELTA && lanes == 0 && max_q >= DCHUNK_MIN && dk <= DCHUNK_N && dk % 4 == 0 && dv % 4 == 0 && ld % 4 == 0 &&
+        (uintptr_t)qkv % 16 == 0 && (gate_dtype == CPMCU_F32 || gate_dtype == CPMCU_BF16)) {
+        // From 64 tokens a sequence on chunks are the cheaper form at any number of sequences (us, walk / chunks: 1 x 64
+        // tokens 29 / 18, 8 x 64 75 / 60, 32 x 64 245 / 237; 8 x 32 42 / 58).
+        // 32 columns a workgroup share the products among keys and queries; 16 where 32 would leave CUs without one (a
+        // workgroup's LDS leaves a CU one at a time)
+        const bool narrow = (long)n_seqs * heads * ((dv + 31) / 32) < 256;
+        const dim3 grid(n_seqs, heads, narrow ? (dv + 15) / 16 : (dv + 31) / 32);
+        CPMCU_REQUIRE(heads <= 65535 && grid.z <= 65535, "delta_scan: shape exceeds the launch grid");
+#define CHUNKS(NBv, GTv)                                       \
+    do {                                                       \
+        if (narrow) CHUNKS_OF(NBv, 1, GTv);                    \
+        else CHUNKS_OF(NBv, 2, GTv);                           \
+    } while (0)
+#define CHUNKS_OF(NBv, PTv, GTv)                                                                                               \
+    delta_chunk_kernel<NBv, PTv, GTv><<<grid, 512, 0, stream>>>(qkv, ld, (const GTv*)gates, ldg, a_off, b_off, dt_bias, A_log, \
+                                                           state, y, cu_q, seq_slot, heads, kv_heads, dk, dv, q_scale,    \
+                                                           write_state)
+        if (gate_dtype == CPMCU_F32) {
+            if (dk <= 64) CHUNKS(4, float);
+            else CHUNKS(8, float);
+        } else {
+            if (dk <= 64) CHUNKS(4, bf16_t);
+            else CHUNKS(8, bf16_t);
+        }
+#undef CHUNKS
+#undef CHUNKS_OF
+        CPMCU_LAUNCH_CHECK("delta_chunk");
+        return nullptr;
+    }
     // 16 lanes a column where 8 would leave fewer than two workgroups a compute unit and a column is long enough
     if (lanes == 0) lanes = ((long)n_seqs * heads * ((dv + 31) / 32) < 512 && dk > 16 && dv > 16) ? 16 : 8;
     const int cols = 256 / lanes;

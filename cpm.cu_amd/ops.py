@@ -1185,8 +1185,9 @@ def softcap(logits: torch.Tensor, cap: float):
 def delta_scan(qkv: torch.Tensor, gates: Optional[torch.Tensor], a_off: int, b_off: int, dt_bias: Optional[torch.Tensor],
                A_log: torch.Tensor, state: torch.Tensor, y: torch.Tensor, cu_q: torch.Tensor, seq_slot: torch.Tensor,
                heads: int, kv_heads: int, dk: int, dv: int, q_scale: float, write_state: bool = True, lanes: int = 0,
-               rule: str = "delta", channel_decay: Optional[torch.Tensor] = None):
-    """The gated delta rule over each sequence's tokens, in float.  qkv float32 [n, 2*kv_heads*dk + heads*dv] =
+               rule: str = "delta", channel_decay: Optional[torch.Tensor] = None, max_q: int = 0):
+    """The gated delta rule over each sequence's tokens, in float (max_q, the longest run of tokens a sequence brings, lets
+    rule 'delta' take prompts 64 tokens at a time; 0: walked token by token).  qkv float32 [n, 2*kv_heads*dk + heads*dv] =
     [q | k | v]; gates [n, W] holds the raw decay projection at columns a_off.. and the raw beta projection at
     b_off.. (heads each).  Per head (its q, k from head h // (heads/kv_heads)): q, k made unit vectors
     (x / sqrt(sum x^2 + 1e-6)), q times q_scale; beta = sigmoid(b); g = exp(-exp(A_log) softplus(a + dt_bias));
@@ -1225,7 +1226,7 @@ def delta_scan(qkv: torch.Tensor, gates: Optional[torch.Tensor], a_off: int, b_o
                                             _p(channel_decay), c_long(ld_a), _p(dt_bias), _p(A_log), _p(state), _p(y),
                                             _p(cu_q), _p(seq_slot), c_int(B), c_int(heads), c_int(kv_heads), c_int(dk),
                                             c_int(dv), c_float(q_scale), c_int(1 if write_state else 0), c_int(lanes),
-                                            c_int(DELTA_RULES[rule]), _stream()))
+                                            c_int(DELTA_RULES[rule]), c_int(max_q), _stream()))
 
 
 DELTA_RULES = {"delta": 0, "channel": 1, "decay": 2}

@@ -52,3 +52,46 @@ def test_state_space_chunks(H, P, N, G, scale):
         assert outs[0] <= 2e-6 and here <= 2e-6, (outs, here, walk)
         assert outs[0] <= 1.5 * outs[1] + 2e-7 and here <= 1.5 * walk + 2e-7, (outs, here, walk)
     assert float(state[[1, 3]].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("H,G,dk,dv,scale", [(4, 2, 128, 128, 1.0), (3, 3, 36, 20, 1.0), (2, 1, 64, 40, 8.0), (2, 2, 4, 4, 0.05)])
+def test_delta_rule_chunks(H, G, dk, dv, scale):
+    """`scale` stretches decay and write rates.  Keys share a direction, so that the triangular system is far from the
+    identity."""
+    from cpmcu_amd import ops
+    g = torch.Generator().manual_seed(dk + dv)
+    first, second = [17, 64, 65, 200], [64, 1, 130, 16]
+    A_log, bias = torch.log(0.05 + 3 * torch.rand(H, generator=g)), torch.randn(H, generator=g)
+    state = torch.zeros(6, H, dv, dk, device=DEV)
+    walked = state.clone()
+    S = torch.zeros(4, H, dv, dk, dtype=torch.float64)
+    slots, rep = [4, 0, 5, 2], H // G
+    for lens in (first, second):
+        n, cu = sum(lens), [0]
+        for q in lens:
+            cu.append(cu[-1] + q)
+        qkv, gates = torch.randn(n, 2 * G * dk + H * dv, generator=g), torch.randn(n, 2 * H + 1, generator=g) * scale
+        qkv[:, G * dk:2 * G * dk] += 1.0
+        unit = lambda x: x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)
+        Q = unit(qkv[:, :G * dk].double().view(n, G, dk)).repeat_interleave(rep, 1) * dk ** -0.5
+        K = unit(qkv[:, G * dk:2 * G * dk].double().view(n, G, dk)).repeat_interleave(rep, 1)
+        V = qkv[:, 2 * G * dk:].double().view(n, H, dv)
+        keep = torch.exp(-torch.exp(A_log.double()) * torch.nn.functional.softplus(gates[:, 1:1 + H].double() + bias.double()))
+        beta = torch.sigmoid(gates[:, 1 + H:].double())
+        want = torch.empty(n, H, dv, dtype=torch.float64)
+        for s in range(4):
+            for t in range(cu[s], cu[s + 1]):
+                S[s] *= keep[t][:, None, None]
+                u = beta[t][:, None] * (V[t] - (S[s] * K[t][:, None]).sum(-1))
+                S[s] += u[:, :, None] * K[t][:, None]
+                want[t] = (S[s] * Q[t][:, None]).sum(-1)
+        outs = []
+        for st, most in ((state, max(lens)), (walked, 0)):
+            y = torch.full((n, H * dv), float("nan"), device=DEV)
+            ops.delta_scan(qkv.to(DEV), gates.to(DEV), 1, 1 + H, bias.to(DEV), A_log.to(DEV), st, y, i32(cu), i32(slots), H, G, dk, dv,
+                           dk ** -0.5, max_q=most)
+            outs.append(off(y.view(n, H, dv), want))
+        here, walk = (off(st[slots], S) for st in (state, walked))
+        assert outs[0] <= 5e-6 and here <= 5e-6, (outs, here, walk)
+        assert outs[0] <= 1.5 * outs[1] + 2e-7 and here <= 1.5 * walk + 2e-7, (outs, here, walk)
+    assert float(state[[1, 3]].abs().max()) == 0.0
