@@ -388,6 +388,103 @@ __global__ __launch_bounds__(256) void gemm_heads_mfma_kernel(const bf16_t* __re
     }
 }
 
+// The same for many rows: 128 rows x 128 columns of a head a workgroup, a wavefront 64 x 64, pieces of 64 columns of both
+// operands through two LDS buffers with the next piece on its way to registers.  With operands straight from memory every
+// wavefront fetched rows and weights for itself, 16 bytes of a row an access, and the address unit was the bound (105
+// TFLOP/s): 2,048 rows, 32 heads, 128 features to 512 columns 88 -> 63 us, 512 to 128 88 -> 31 us.  A piece's row is 8 chunks of 16 bytes,
+// chunk c of row r at place c ^ (r % 8), so that 8 neighbouring lanes read all banks.  W takes the first operand's place: a
+// lane then holds 4 neighbouring columns of a row of Y and writes them together.
+typedef unsigned hu32x4_t __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(256) void gemm_heads_tile_kernel(const bf16_t* __restrict__ X, long ldx, long hsx,
+                                                              const bf16_t* __restrict__ W, bf16_t* __restrict__ Y,
+                                                              long ldy, long hsy, const bf16_t* __restrict__ gate,
+                                                              long ldg, int gate_wide, int M, int N, int K, int pairs) {
+    __shared__ hu32x4_t lds[2][256 * 8];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int h = blockIdx.z, m0 = blockIdx.y * 128, n0 = blockIdx.x * 128;
+    const int chunk = threadIdx.x & 7, lrow = threadIdx.x >> 3;
+    const int place = lrow * 8 + (chunk ^ (lrow & 7));
+    const bf16_t *xp[4], *wp[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        xp[i] = X + (long)h * hsx + (long)min(m0 + lrow + 32 * i, M - 1) * ldx + chunk * 8;
+        wp[i] = W + ((long)h * N + min(n0 + lrow + 32 * i, N - 1)) * K + chunk * 8;
+    }
+    hu32x4_t nx[4], nw[4];
+    auto fetch = [&](int k0) {
+        const int k = min(k0, K - 8 - chunk * 8);                  // beyond the row's end: its last columns, zeroed below
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            nx[i] = *(const hu32x4_t*)(xp[i] + k);
+            nw[i] = *(const hu32x4_t*)(wp[i] + k);
+        }
+    };
+    hfloatx4_t acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = hfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    const int mw = (wave & 1) * 64, nw0 = (wave >> 1) * 64;
+    fetch(0);
+    int buf = 0;
+    for (int k0 = 0; k0 < K; k0 += 64, buf ^= 1) {
+        if (k0 + chunk * 8 >= K) {                                 // K % 8 == 0: the whole chunk lies beyond the end
+#pragma unroll
+            for (int i = 0; i < 4; ++i) nx[i] = nw[i] = hu32x4_t{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            lds[buf][256 * i + place] = nx[i];
+            lds[buf][1024 + 256 * i + place] = nw[i];
+        }
+        __syncthreads();
+        if (k0 + 64 < K) fetch(k0 + 64);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const int at = (kk * 4 + g) ^ (r & 7);
+            hbf16x8_t x[4], w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                x[i] = *(const hbf16x8_t*)&lds[buf][(mw + 16 * i + r) * 8 + at];
+                w[i] = *(const hbf16x8_t*)&lds[buf][1024 + (nw0 + 16 * i + r) * 8 + at];
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j], x[i], acc[i][j], 0, 0, 0);
+        }
+    }
+    // lane (row r, g): acc[i][j][e] is row m0 + mw + 16 i + r, column n0 + nw0 + 16 j + 4 g + e
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = m0 + mw + 16 * i + r;
+        if (m >= M) continue;
+        const float one = gate && !gate_wide ? to_f32(gate[(long)m * ldg + h]) : 0.f;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int n = n0 + nw0 + 16 * j + 4 * g;
+            if (n >= N) continue;
+            bf16_t o[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float v = acc[i][j][e];
+                if (gate) v /= 1.0f + expf(-(gate_wide ? to_f32(gate[(long)m * ldg + (long)h * N + min(n + e, N - 1)]) : one));
+                o[e] = f32_to_bf16(v);
+            }
+            bf16_t* to = Y + (long)h * hsy + (long)m * ldy + n;
+            if (pairs && n + 4 <= N) {                             // rows and heads of Y start on 8-byte borders
+                *(uint2*)to = make_uint2((uint32_t)o[0].v | (uint32_t)o[1].v << 16, (uint32_t)o[2].v | (uint32_t)o[3].v << 16);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) to[e] = o[e];
+            }
+        }
+    }
+}
+
 extern "C" const char* cpmcu_gemm_nt_heads_mfma(const void* X, long ldx, long hsx, const void* W, void* Y, long ldy,
                                                 long hsy, const void* gate, long ldg, int gate_wide, int M, int H, int N,
                                                 int K, hipStream_t stream) {
@@ -402,7 +499,14 @@ extern "C" const char* cpmcu_gemm_nt_heads_mfma(const void* X, long ldx, long hs
         dim3 grid((N + 63) / 64, 1, H);
         gemm_heads_mfma_kernel<1, 1><<<grid, 256, 0, stream>>>((const bf16_t*)X, ldx, hsx, (const bf16_t*)W, (bf16_t*)Y, ldy,
                                                                hsy, (const bf16_t*)gate, ldg, gate && gate_wide, M, N, K);
+    } else if ((long)((M + 127) / 128) * ((N + 127) / 128) * H >= 256) {
+        dim3 grid((N + 127) / 128, (M + 127) / 128, H);
+        CPMCU_REQUIRE(grid.y <= 65535, "gemm_heads_mfma: M=%d too large for one launch", M);
+        const int pairs = ldy % 4 == 0 && hsy % 4 == 0 && (uintptr_t)Y % 8 == 0;
+        gemm_heads_tile_kernel<<<grid, 256, 0, stream>>>((const bf16_t*)X, ldx, hsx, (const bf16_t*)W, (bf16_t*)Y, ldy, hsy,
+                                                         (const bf16_t*)gate, ldg, gate && gate_wide, M, N, K, pairs);
     } else {
+        // fewer tiles of 128 than CUs: tiles of 64, four times as many
         dim3 grid((N + 63) / 64, (M + 63) / 64, H);
         CPMCU_REQUIRE(grid.y <= 65535, "gemm_heads_mfma: M=%d too large for one launch", M);
         gemm_heads_mfma_kernel<4, 4><<<grid, 256, 0, stream>>>((const bf16_t*)X, ldx, hsx, (const bf16_t*)W, (bf16_t*)Y, ldy,
