@@ -12,6 +12,7 @@
 // the head norm that follows divides.  S, n and m live per cache slot and are carried from step to
 // step, so a step of any number of tokens continues where the last one ended.
 #include "common.h"
+#include "vec4.h"
 
 // A workgroup of 256 threads walks ML_PB = 256 / ML_L columns; a column's d state values lie over ML_L neighbouring
 // lanes (8 or 32: key index c = l + ML_L i), which sum their shares inside the vector unit.  Keys beyond 128
@@ -201,17 +202,249 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const T* __restrict__ p
     }
 }
 
+// ---------------------------------------------------------------------------
+// The same recurrence for prompts, 32 tokens at a time on the matrix cores' float instruction (v_mfma_f32_16x16x4_f32:
+// operands as they are, sums in float).  With F_t = the sum of b over the chunk's tokens up to t, w_s = a_s - F_s and
+// M_t = max(m before the chunk, w_s for s <= t), all three in double, m_t = F_t + M_t and
+//     y_t = exp(m - M_t) S^T q_t + sum_(s <= t) exp(w_s - M_t) (q_t . k_s) v_s
+//     S  <- exp(m - M_31) S + sum_s exp(w_s - M_31) k_s v_s^T
+// where no exponent is positive; the normaliser is column dv, whose value is always 1, as in the walk.  A workgroup owns
+// one (sequence, head, 32 columns); its state stays in the accumulators' registers and passes through LDS as an operand.
+// 8 heads of 256 by 512, prompts of 613, 479, 211, 345 and 400 tokens in one pass: 870 -> 311 us.
+// A lane's 16 bytes serve four instructions: instruction j of a block takes index 4 g + j of the 16 in both operands.
+// ---------------------------------------------------------------------------
+typedef float mlfloatx4_t __attribute__((ext_vector_type(4)));
+#define MCHUNK_T 32       // tokens a chunk
+#define MCHUNK_P 32       // columns a workgroup
+#define MCHUNK_LT 36      // LDS rows of MCHUNK_T: rows 4 banks apart, so that 8 rows' 16 bytes read all banks
+#define MCHUNK_MIN 32     // tokens a sequence from which chunks are taken: 8 sequences of 32, 101 -> 55 us; of 16, 58 -> 53 us, as little as a walk
+
+// NB: blocks of 16 key features, a multiple of 8
+template <int NB, typename T>
+__global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ proj, long ld, long q_off, long k_off,
+                                                          long v_off, long i_off, long f_off,
+                                                          const float* __restrict__ i_bias, const float* __restrict__ f_bias,
+                                                          float cap, float q_scale, float* __restrict__ S_state,
+                                                          float* __restrict__ n_state, float* __restrict__ m_state,
+                                                          float* __restrict__ y, float* __restrict__ den,
+                                                          const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
+                                                          int heads, int d, int dv, int write_state) {
+    constexpr int LN = 16 * NB + 4, NJ = NB / 8, C4 = 4 * NB, QK = MCHUNK_T * C4 / 512;
+    __shared__ __align__(16) float Qs[MCHUNK_T * LN], Ks[MCHUNK_T * LN];
+    __shared__ __align__(16) float Ss[MCHUNK_P * LN];                  // the state before the chunk, [p][c]
+    __shared__ __align__(16) float Gs[MCHUNK_T * MCHUNK_LT];            // exp(w_s - M_t) q_t . k_s
+    __shared__ __align__(16) float vT[MCHUNK_P * MCHUNK_LT];            // [p][t]
+    __shared__ __align__(16) float left_s[MCHUNK_T], from_s[MCHUNK_T], floor_s[MCHUNK_T];
+    __shared__ double w_s[MCHUNK_T], M_s[MCHUNK_T];
+    const int b = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * MCHUNK_P;
+    const int start = cu_q[b], q = cu_q[b + 1] - start, slot = seq_slot[b];
+    if (q <= 0) return;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    auto state_row = [&](int p) {
+        return p == dv ? n_state + ((long)slot * heads + h) * d : S_state + (((long)slot * heads + h) * dv + min(p, dv - 1)) * d;
+    };
+    // the state as the accumulators hold it: st[i][j][e] is column p = 16 i + 4 g + e, key feature c = 16 (NJ wave + j) + r
+    mlfloatx4_t st[2][NJ];
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int p = p0 + 16 * i + 4 * g + e, c = 16 * (NJ * wave + j) + r;
+                st[i][j][e] = (p <= dv && c < d) ? state_row(p)[c] : 0.f;
+            }
+    double m = (double)m_state[(long)slot * heads + h];                // wavefront 0 carries it on
+    const float bi = i_bias[h], bf = f_bias[h], inv_cap = 1.0f / cap;
+    const mlfloatx4_t zero4 = {0.f, 0.f, 0.f, 0.f};
+    const int vrow = threadIdx.x >> 3, vcol = (threadIdx.x & 7) * 4;   // (256 threads bring values)
+    float4 rq[QK], rk[QK], rv = make_float4(0.f, 0.f, 0.f, 0.f);
+    float ri = 0.f, rf = 0.f;
+    auto fetch = [&](int t0) {
+        const int tn = min(MCHUNK_T, q - t0);
+        const T* base = proj + (long)(start + t0) * ld;
+#pragma unroll
+        for (int i = 0; i < QK; ++i) {
+            const int e = threadIdx.x + 512 * i, c = (e % C4) * 4;
+            const T* row = base + (long)min(e / C4, tn - 1) * ld + (long)h * d + min(c, d - 4);
+            rq[i] = load4(row + q_off);
+            rk[i] = load4(row + k_off);
+            if (c >= d) rq[i] = rk[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        const int p = p0 + vcol;
+        rv = load4(base + (long)min(vrow, tn - 1) * ld + v_off + (long)h * dv + min(p, dv - 4));
+        if (p >= dv) rv = make_float4(p == dv ? 1.f : 0.f, 0.f, 0.f, 0.f);
+        if (wave == 0) {
+            const T* row = base + (long)min(lane, tn - 1) * ld + h;
+            ri = to_f32(row[i_off]);
+            rf = to_f32(row[f_off]);
+        }
+    };
+    // one 16 x 16 tile of rows[i] . cols[j] over the key features
+    auto dot_tile = [&](const float* rows, int i, const float* cols, int j) {
+        mlfloatx4_t a = zero4;
+#pragma unroll
+        for (int kb = 0; kb < NB; ++kb) {
+            const mlfloatx4_t x = *(const mlfloatx4_t*)&rows[(16 * i + r) * LN + 16 * kb + 4 * g];
+            const mlfloatx4_t z = *(const mlfloatx4_t*)&cols[(16 * j + r) * LN + 16 * kb + 4 * g];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], z[e], a, 0, 0, 0);
+        }
+        return a;
+    };
+    fetch(0);
+    for (int t0 = 0; t0 < q; t0 += MCHUNK_T) {
+        const int tn = min(MCHUNK_T, q - t0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) Ss[(16 * i + 4 * g + e) * LN + 16 * (NJ * wave + j) + r] = st[i][j][e];
+#pragma unroll
+        for (int i = 0; i < QK; ++i) {
+            const int e = threadIdx.x + 512 * i, at = (e / C4) * LN + (e % C4) * 4;
+            store4(&Qs[at], rq[i].x * q_scale, rq[i].y * q_scale, rq[i].z * q_scale, rq[i].w * q_scale);
+            store4(&Ks[at], rk[i].x, rk[i].y, rk[i].z, rk[i].w);
+        }
+        if (vrow < MCHUNK_T) {
+            vT[vcol * MCHUNK_LT + vrow] = rv.x;
+            vT[(vcol + 1) * MCHUNK_LT + vrow] = rv.y;
+            vT[(vcol + 2) * MCHUNK_LT + vrow] = rv.z;
+            vT[(vcol + 3) * MCHUNK_LT + vrow] = rv.w;
+        }
+        if (wave == 0) {
+            // a token beyond the end neither writes (w = -inf) nor forgets (b = 0); lanes 32 .. 63 are such tokens too
+            const bool in = lane < tn;
+            double F = in ? (double)log_sigmoid_f(cap * tanhf((rf + bf) * inv_cap)) : 0.0;
+#pragma unroll
+            for (int k = 1; k < 64; k <<= 1) {
+                const double up = __shfl_up(F, k, 64);
+                if (lane >= k) F += up;
+            }
+            const double w = in ? (double)(cap * tanhf((ri + bi) * inv_cap)) - F : -INFINITY;
+            double M = fmax(m, w);
+#pragma unroll
+            for (int k = 1; k < 64; k <<= 1) {
+                const double up = __shfl_up(M, k, 64);
+                if (lane >= k) M = fmax(M, up);
+            }
+            const double M_end = __shfl(M, 63, 64);
+            if (lane < MCHUNK_T) {
+                w_s[lane] = w;
+                M_s[lane] = M;
+                left_s[lane] = expf((float)(w - M_end));
+                from_s[lane] = expf((float)(m - M));
+                floor_s[lane] = expf((float)(-(F + M)));
+            }
+            m = __shfl(F, 63, 64) + M_end;
+        }
+        __syncthreads();
+        if (t0 + MCHUNK_T < q) fetch(t0 + MCHUNK_T);
+        // wavefronts 0 to 2: the tiles of G on and below the diagonal; 3 to 6: what the state before the chunk gives tokens
+        // 16 tt .. + 15 in columns 16 pt .. + 15
+        const int tt = wave < 3 ? (wave + 1) / 2 : ((wave - 3) >> 1) & 1, pt = (wave - 3) & 1;
+        mlfloatx4_t yt = zero4;
+        if (wave < 3) {
+            const int j = wave == 2 ? 1 : 0, s = 16 * j + r;
+            const mlfloatx4_t a = dot_tile(Qs, tt, Ks, j);
+            const double w = w_s[s];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * tt + 4 * g + e;
+                Gs[t * MCHUNK_LT + s] = s <= t ? a[e] * expf((float)(w - M_s[t])) : 0.f;
+            }
+        } else if (wave < 7) {
+            yt = dot_tile(Qs, tt, Ss, pt);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) yt[e] *= from_s[16 * tt + 4 * g + e];
+        }
+        __syncthreads();
+        if (wave >= 3 && wave < 7) {
+            // ... and what the chunk's own tokens give them
+            for (int kb = 0; kb <= tt; ++kb) {
+                const mlfloatx4_t a = *(const mlfloatx4_t*)&Gs[(16 * tt + r) * MCHUNK_LT + 16 * kb + 4 * g];
+                const mlfloatx4_t v = *(const mlfloatx4_t*)&vT[(16 * pt + r) * MCHUNK_LT + 16 * kb + 4 * g];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) yt = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], v[e], yt, 0, 0, 0);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * tt + 4 * g + e, p = p0 + 16 * pt + r;
+                if (t >= tn) continue;
+                if (p < dv) y[(long)(start + t0 + t) * heads * dv + (long)h * dv + p] = yt[e];
+                else if (p == dv) den[(long)(start + t0 + t) * heads + h] = fmaxf(fabsf(yt[e]), floor_s[t]) + 1e-6f;
+            }
+        }
+        // the state behind the chunk
+        const float keep = from_s[MCHUNK_T - 1];
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) st[i][j] *= keep;
+#pragma unroll
+        for (int kb = 0; kb < MCHUNK_T / 16; ++kb) {
+            const mlfloatx4_t w4 = *(const mlfloatx4_t*)&left_s[16 * kb + 4 * g];
+            mlfloatx4_t v4[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) v4[i] = *(const mlfloatx4_t*)&vT[(16 * i + r) * MCHUNK_LT + 16 * kb + 4 * g] * w4;
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float kv = Ks[(16 * kb + 4 * g + e) * LN + 16 * (NJ * wave + j) + r];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) st[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[i][e], kv, st[i][j], 0, 0, 0);
+                }
+        }
+        __syncthreads();
+    }
+    if (write_state) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int p = p0 + 16 * i + 4 * g + e, c = 16 * (NJ * wave + j) + r;
+                    if (p <= dv && c < d) state_row(p)[c] = st[i][j][e];
+                }
+        if (blockIdx.z == 0 && threadIdx.x == 0) m_state[(long)slot * heads + h] = (float)m;
+    }
+}
+
+// max_q: the longest run of tokens a sequence brings (0: not known, the walk)
 extern "C" const char* cpmcu_mlstm_scan(const void* proj, long ld, int dtype, long q_off, long k_off, long v_off,
                                         long i_off, long f_off, const float* i_bias, const float* f_bias, float cap,
                                         float q_scale, float* S_state, float* n_state, float* m_state, float* y,
                                         float* den, const int* cu_q, const int* seq_slot, int n_seqs, int heads, int d, int dv,
-                                        int write_state, hipStream_t stream) {
+                                        int write_state, int max_q, hipStream_t stream) {
     CPMCU_REQUIRE(n_seqs > 0 && heads > 0 && d > 0 && dv > 0, "mlstm_scan: empty shape");
     CPMCU_REQUIRE(d <= 1024, "mlstm_scan: a key size of %d is not supported (at most 1024)", d);
     CPMCU_REQUIRE(cap > 0.f, "mlstm_scan: gate cap %g", cap);
     CPMCU_REQUIRE(q_off >= 0 && k_off >= 0 && v_off >= 0 && i_off >= 0 && f_off >= 0 && q_off + (long)heads * d <= ld &&
                   k_off + (long)heads * d <= ld && v_off + (long)heads * dv <= ld && i_off + heads <= ld && f_off + heads <= ld,
                   "mlstm_scan: columns beyond rows of %ld", ld);
+    if (max_q >= MCHUNK_MIN && d <= 256 && d % 4 == 0 && dv % 4 == 0 && ld % 4 == 0 && q_off % 4 == 0 && k_off % 4 == 0 &&
+        v_off % 4 == 0 && (uintptr_t)proj % 16 == 0 && (dtype == CPMCU_F32 || dtype == CPMCU_BF16)) {
+        const dim3 grid(n_seqs, heads, (dv + 1 + MCHUNK_P - 1) / MCHUNK_P);
+        CPMCU_REQUIRE(heads <= 65535 && grid.z <= 65535, "mlstm_scan: shape exceeds the launch grid");
+#define CHUNKS(NBv, Tv)                                                                                             \
+    mlstm_chunk_kernel<NBv, Tv><<<grid, 512, 0, stream>>>((const Tv*)proj, ld, q_off, k_off, v_off, i_off, f_off,   \
+                                                          i_bias, f_bias, cap, q_scale, S_state, n_state, m_state, y, \
+                                                          den, cu_q, seq_slot, heads, d, dv, write_state)
+        if (dtype == CPMCU_F32) {
+            if (d <= 128) CHUNKS(8, float);
+            else CHUNKS(16, float);
+        } else {
+            if (d <= 128) CHUNKS(8, bf16_t);
+            else CHUNKS(16, bf16_t);
+        }
+#undef CHUNKS
+        CPMCU_LAUNCH_CHECK("mlstm_chunk");
+        return nullptr;
+    }
     const int lanes = d > 128 ? 32 : 8, cols = 256 / lanes;
     const int pb = (dv + 1 + cols - 1) / cols;       // the normaliser is walked as column dv
     CPMCU_REQUIRE(heads <= 65535 && pb <= 65535, "mlstm_scan: shape exceeds the launch grid");

@@ -913,8 +913,9 @@ def bigram_add(table: torch.Tensor, ids: torch.Tensor, positions: torch.Tensor, 
 def mlstm_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, i_off: int, f_off: int, i_bias: torch.Tensor,
                f_bias: torch.Tensor, cap: float, q_scale: float, S: torch.Tensor, n_state: torch.Tensor,
                m_state: torch.Tensor, y: torch.Tensor, den: torch.Tensor, cu_q: torch.Tensor, seq_slot: torch.Tensor,
-               heads: int, d: int, dv: int, write_state: bool = True):
-    """The matrix-memory recurrence over each sequence's tokens, in float.  proj [n, W] holds, from the given
+               heads: int, d: int, dv: int, write_state: bool = True, max_q: int = 0):
+    """The matrix-memory recurrence over each sequence's tokens, in float (max_q, the longest run of tokens a sequence
+    brings, lets prompts be taken 32 tokens at a time; 0: walked token by token).  proj [n, W] holds, from the given
     columns on, q and k (heads * d each), v (heads * dv) and the raw input and forget gates (heads each); per head
     a = cap tanh((i + i_bias)/cap), b = logsigmoid(cap tanh((f + f_bias)/cap)), m' = max(b + m, a),
     S' = exp(b + m - m') S + exp(a - m') k v^T, n' likewise with k, q multiplied by q_scale.  It leaves the output
@@ -940,7 +941,7 @@ def mlstm_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, i_off: in
                                             c_long(v_off), c_long(i_off), c_long(f_off), _p(i_bias), _p(f_bias),
                                             c_float(cap), c_float(q_scale), _p(S), _p(n_state), _p(m_state), _p(y),
                                             _p(den), _p(cu_q), _p(seq_slot), c_int(B), c_int(heads), c_int(d), c_int(dv),
-                                            c_int(1 if write_state else 0), _stream()))
+                                            c_int(1 if write_state else 0), c_int(max_q), _stream()))
 
 
 def streams_fill(x: torch.Tensor, streams: torch.Tensor):

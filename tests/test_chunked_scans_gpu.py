@@ -95,3 +95,46 @@ def test_delta_rule_chunks(H, G, dk, dv, scale):
         assert outs[0] <= 5e-6 and here <= 5e-6, (outs, here, walk)
         assert outs[0] <= 1.5 * outs[1] + 2e-7 and here <= 1.5 * walk + 2e-7, (outs, here, walk)
     assert float(state[[1, 3]].abs().max()) == 0.0
+
+
+@pytest.mark.parametrize("H,d,dv,scale", [(2, 256, 64, 1.0), (3, 128, 32, 8.0), (2, 36, 20, 1.0), (1, 4, 4, 0.05)])
+def test_mlstm_chunks(H, d, dv, scale):
+    """`scale` stretches the gates: the running maximum then jumps within a chunk, or hardly moves."""
+    from cpmcu_amd import ops
+    g = torch.Generator().manual_seed(d + dv)
+    first, second, cap = [17, 32, 33, 150], [64, 1, 65, 16], 15.0
+    ib, fb = torch.randn(H, generator=g), torch.randn(H, generator=g) + 2.0
+    zeros = lambda *s: torch.zeros(*s, device=DEV)
+    states = [(zeros(6, H, dv, d), zeros(6, H, d), zeros(6, H)) for _ in range(2)]
+    S, N, M = (torch.zeros(4, *s, dtype=torch.float64) for s in ((H, dv, d), (H, d), (H,)))
+    slots, ko, vo, io, fo = [4, 0, 5, 2], H * d, 2 * H * d, 2 * H * d + H * dv, 2 * H * d + H * dv + H
+    for lens in (first, second):
+        n, cu = sum(lens), [0]
+        for q in lens:
+            cu.append(cu[-1] + q)
+        proj = torch.randn(n, -(-(fo + H) // 4) * 4, generator=g)
+        proj[:, io:fo + H] *= scale
+        Q, K = (proj[:, o:o + H * d].double().view(n, H, d) for o in (0, ko))
+        V = proj[:, vo:vo + H * dv].double().view(n, H, dv)
+        a = cap * torch.tanh((proj[:, io:io + H].double() + ib.double()) / cap)
+        b = torch.nn.functional.logsigmoid(cap * torch.tanh((proj[:, fo:fo + H].double() + fb.double()) / cap))
+        want = torch.empty(n, H, dv, dtype=torch.float64)
+        for s in range(4):
+            for t in range(cu[s], cu[s + 1]):
+                new = torch.maximum(b[t] + M[s], a[t])
+                keep, take = torch.exp(b[t] + M[s] - new)[:, None], torch.exp(a[t] - new)[:, None] * K[t]
+                S[s], N[s], M[s] = keep[..., None] * S[s] + V[t][:, :, None] * take[:, None], keep * N[s] + take, new
+                qt = Q[t] * d ** -0.5
+                low = torch.maximum((N[s] * qt).sum(-1).abs(), torch.exp(-new)) + 1e-6
+                want[t] = (S[s] * qt[:, None]).sum(-1) / low[:, None]
+        errs = []
+        for (st, ns, ms), most in zip(states, (max(lens), 0)):
+            y, den = torch.full((n, H * dv), float("nan"), device=DEV), torch.full((n, H), float("nan"), device=DEV)
+            ops.mlstm_scan(proj.to(DEV), 0, ko, vo, io, fo, ib.to(DEV), fb.to(DEV), cap, d ** -0.5, st, ns, ms, y, den, i32(cu),
+                           i32(slots), H, d, dv, max_q=most)
+            scale_out = torch.exp(ms[slots].double().cpu() - M)            # a maximum a rounding away scales S and n alike
+            errs.append([off(y.view(n, H, dv) / den[..., None], want), off(st[slots].double().cpu() * scale_out[..., None, None], S),
+                         off(ns[slots].double().cpu() * scale_out[..., None], N), float((ms[slots].double().cpu() - M).abs().max())])
+        assert all(h <= 1.5 * w + 5e-7 for h, w in zip(*errs)), errs
+        assert errs[0][1] <= 2e-6 and errs[0][2] <= 2e-6, errs
+    assert all(float(t[[1, 3]].abs().max()) == 0.0 for t in states[0])
