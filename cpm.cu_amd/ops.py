@@ -414,7 +414,7 @@ def compute_units() -> int:
     return _cu_count
 
 
-def attention_splits(n_tokens: int, nkv: int, group: int, max_keys: int) -> int:
+def attention_splits(n_tokens: int, nkv: int, group: int, max_keys: int, hd: int = 0) -> int:
     """Shares of a token's keys for steps of few tokens.  Measured on the MI355X (head size 128, 2 kv heads,
     workgroups of 4 wavefronts, graph replay over keys that come from memory, attention + merge, in us for
     1/2/4/8/16/32 shares):
@@ -428,7 +428,13 @@ def attention_splits(n_tokens: int, nkv: int, group: int, max_keys: int) -> int:
     least 128 keys, at most 32 shares (beyond 32 the merge kernel no longer holds every share's output in
     registers: one sequence at 32,000 keys, whole step, 3.89 ms with 64 shares against 3.60 with 32).  A step
     that has 128 workgroups or more by itself takes two shares from 4,096 keys on (they even out the
-    workgroups' ends) and one below (no merge kernel: 64 sequences of the 0.5B shape)."""
+    workgroups' ends) and one below (no merge kernel: 64 sequences of the 0.5B shape).
+    With the head size given, few keys stay one share, whose 4 wavefronts finish them sooner than a merge kernel
+    starts (one sequence, 2 kv heads, keys from the caches, attention + merge in us for one share / the shares above):
+      head size 64 at 300 keys 4.4/5.9, 512 4.8/5.6, 768 5.7/5.7, 1,024 6.3/5.7; 32 sequences 5.0/6.8, 5.4/7.1, 7.7/8.0, 9.3/8.8;
+      head size 128 at 300 keys 5.9/6.8, 384 6.2/6.4, 512 6.7/6.4, 768 7.9/6.5; 32 sequences 7.5/8.7, 8.6/9.0, 10.0/9.8, 13.0/11.6."""
+    if hd and max_keys < (768 if hd <= 64 else 512):
+        return 1
     cus = compute_units()
     if n_tokens > cus:
         return 1
@@ -2043,7 +2049,7 @@ def attention(q, out, nh, nkv, hd, scale, kpool, vpool, page_table, page_size, c
         keys = ctx.max_pos + 1
         if sel_count is not None:
             keys = min(keys, sel_blocks.shape[2] * block_size)
-        splits = attention_splits(n, nkv, nh // nkv, keys)
+        splits = attention_splits(n, nkv, nh // nkv, keys, hd)
         part_o = part_ml = None
         if splits > 1:
             part_o = ctx.ws.get("attn.part_o", (n, nh, splits, hd), torch.float32)
