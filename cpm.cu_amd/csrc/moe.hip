@@ -651,6 +651,8 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
 // K is the rows' width, N the number of features; in: h rows by token (GATED, PLAIN: pair / top) or act rows by pair.
 // Measured (64 experts, width 4,096, 6 a token; us, before -> now): gated experts of 1,408, 2,048 tokens 1,250 -> 464
 // and 612 -> 278 (down), 24 tokens 303 -> 222 and 169 -> 116 (their 58 experts' matrices at 6 TB/s); 8 tokens 129 + 67.
+// With up to 64 rows a tile, where most weights are read once, they are streamed past the caches: both products of 24
+// tokens 338 -> 321 us, of 300 tokens 433 -> 403; with more tokens tiles share weights.
 // Two pieces on their way at once: one made no difference beyond 300 tokens, at 24 it took 234 + 122 us.
 // The grid is dealt to the 8 XCDs in turn; each takes one run of the tasks, ordered expert by expert and within an expert
 // weight rows by weight rows, so that the tiles that share weights meet in one L2.
@@ -696,7 +698,10 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
         auto fetch = [&](Piece& p, int k0) {
             const int k = min(k0, K - 8 - chunk * 8);                 // beyond the row's end: its last columns, zeroed below
 #pragma unroll
-            for (int i = 0; i < 4; ++i) p.w[i] = *(const mu32x4_t*)(wp[i] + k);
+            for (int i = 0; i < 4; ++i) {
+                if (RT == 4) p.w[i] = __builtin_nontemporal_load((const mu32x4_t*)(wp[i] + k));
+                else p.w[i] = *(const mu32x4_t*)(wp[i] + k);
+            }
 #pragma unroll
             for (int i = 0; i < AP; ++i) p.a[i] = *(const mu32x4_t*)(ap[i] + k);
         };
