@@ -652,7 +652,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
 // Measured (64 experts, width 4,096, 6 a token; us, before -> now): gated experts of 1,408, 2,048 tokens 1,250 -> 464
 // and 612 -> 278 (down), 24 tokens 303 -> 222 and 169 -> 116 (their 58 experts' matrices at 6 TB/s); 8 tokens 129 + 67.
 // With up to 64 rows a tile, where most weights are read once, they are streamed past the caches: both products of 24
-// tokens 338 -> 321 us, of 300 tokens 433 -> 403; with more tokens tiles share weights.
+// tokens 338 -> 322 us, of 300 tokens 433 -> 403; with more tokens tiles share weights.
 // Two pieces on their way at once: one made no difference beyond 300 tokens, at 24 it took 234 + 122 us.
 // The grid is dealt to the 8 XCDs in turn; each takes one run of the tasks, ordered expert by expert and within an expert
 // weight rows by weight rows, so that the tiles that share weights meet in one L2.
