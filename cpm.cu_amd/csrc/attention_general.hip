@@ -620,9 +620,11 @@ extern "C" const char* cpmcu_attention_general_mfma(const void* q, void* out, in
 //                     from the page
 // The next keys are on their way to registers meanwhile; two barriers a round.  attention_general_mfma_kernel reads every
 // key and value once for 16 columns, whose bytes from L2 were the bound (14 TB/s).  Measured, that kernel -> this one: 2,048
-// tokens, 32 heads over a latent of 512 + 64 700 -> 269 us (585 TFLOP/s; the LDS reads of the keys are next), 1,500 tokens,
-// 32 maps on 8 keys of 128 and 4 values of 256 205 -> 81 us.  The running maximum follows only when a column's has moved up by more than 8 (in powers of two):
-// weights then reach 2^8 at most, which float sums and bf16 weights take as well as 1.
+// tokens, 32 heads over a latent of 512 + 64 700 -> 267 us (545 TFLOP/s; the LDS reads of the keys are next), 1,500 tokens,
+// 32 maps on 8 keys of 128 and 4 values of 256 205 -> 84 us.
+// The running maximum follows every move, so that a column's largest weight is 1, which 16 bits hold, and the sum is that of
+// the rounded weights; a maximum that only follows moves by more than 8 powers of two saves 10 us of the first and has up to
+// 2.3 times the error where few keys hold most of the weight.
 // PK: up to 64 PK key features (EXACT: so many); DTW: up to 128 DTW value features.
 // ===========================================================================
 typedef unsigned gu32x4_t __attribute__((ext_vector_type(4)));
@@ -744,7 +746,7 @@ __global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const float to_m = fmaxf(m[k], fmaxf(top_s[0][k * 16 + n], top_s[1][k * 16 + n]) * scale_log2e);
-            const bool up = to_m > m[k] + 8.0f;
+            const bool up = to_m > m[k];
             corr[k] = up ? __builtin_amdgcn_exp2f(m[k] - to_m) : 1.0f;           // (m = -inf: 0)
             m[k] = up ? to_m : m[k];
             moved |= up;
@@ -759,8 +761,8 @@ __global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[u][e], scale_log2e, -ref));
-                rs += p;
                 pb[u * 4 + e] = (__bf16)p;
+                rs += (float)pb[u * 4 + e];                                      // the weights as the products take them
             }
         l = l * corr_own + rows_sum(rs);
         p_s[ct][kh][lane] = pb;

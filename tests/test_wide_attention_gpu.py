@@ -88,3 +88,30 @@ def test_wide_prompt_attention(nh, nkv, hdk, pool_hdk, hdv, v_share, opt):
             want, size = want * s_g, size * s_g
         # weights rounded to bf16 (half an ulp each) against values of that size, and the output's own rounding
         assert bool(((got[t] - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-5).all()), (t, p, s)
+
+
+@pytest.mark.parametrize("spread", [1.0, 3.0])
+def test_weights_round_no_worse_than_token_by_token(spread):
+    """Few keys that hold most of a softmax, and many that share it: the error of the kernel for wide values is at most that
+    of the general kernel, which keeps a token's largest weight at 1 (5% for other orders of summing)."""
+    from cpmcu_amd import ops
+    L, nh, hdk, hdv, page = 512, 16, 576, 512, 64
+    g = torch.Generator().manual_seed(int(spread))
+    k, q = torch.randn(L, 1, hdk, generator=g).to(torch.bfloat16), (spread * torch.randn(L, nh, hdk, generator=g)).to(torch.bfloat16)
+    v = k[..., :hdv].contiguous()
+    pools = []
+    for x, keys in ((k, True), (v, False)):
+        pool = torch.zeros(x.numel(), dtype=torch.bfloat16)
+        pool[element_order(L, 1, x.shape[-1], keys).flatten()] = x.flatten()
+        pools.append(pool.view(L // page, page, -1).to(DEV))
+    pos, table = torch.arange(L, dtype=torch.int32, device=DEV), torch.arange(L // page, dtype=torch.int32, device=DEV)[None]
+    slot, rows = torch.zeros_like(pos), q.view(L, -1).to(DEV)
+    wide, general = (torch.empty(L, nh * hdv, device=DEV) for _ in range(2))
+    shape = (nh, 1, hdk, hdv, hdk ** -0.5, *pools, table, page, pos, slot)
+    ops.attention_wide_prefill(rows, wide, ops.prefill_tiles([L], 64 // nh, DEV), *shape, 0, 0, 0, None, 1, None, 0.0)
+    ops.attention_general_mfma(rows, general, *shape)
+    s = torch.einsum("thd,jd->htj", q.double(), k[:, 0].double()) * hdk ** -0.5
+    s.masked_fill_(torch.ones(L, L, dtype=torch.bool).triu(1), float("-inf"))
+    want = torch.matmul(torch.softmax(s, -1), v[:, 0].double()).transpose(0, 1).reshape(L, -1)
+    off = [float((x.double().cpu() - want).norm()) for x in (wide, general)]
+    assert off[0] <= 1.05 * off[1], off
