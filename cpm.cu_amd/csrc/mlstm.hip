@@ -25,6 +25,10 @@ __device__ inline float log_sigmoid_f(float v) { return fminf(v, 0.f) - log1pf(e
 // k_off + h * d, v at v_off + h * dv, raw gates at i_off + h and f_off + h.  S: [slots][heads][dv][d],
 // nst: [slots][heads][d], mst: [slots][heads].
 //
+// Every workgroup of a (sequence, head) starts from its slot's maximum, and a launch may have more of them than run at a
+// time: none may write it.  The maximum behind the step goes to m_next [sequences][heads], which mlstm_maximum_kernel, a
+// launch of its own, moves to the slots.
+//
 // The normaliser n obeys the recurrence of a column of S whose value is always 1, so it is walked as column dv:
 // columns 0 .. dv - 1 give the unnormalised y = S^T q (float [n, heads * dv]) and column dv gives n . q, from which
 // den[t, h] = max(|n . q|, exp(-m)) + 1e-6 (float [n, heads]); whoever reads y divides by den (the head norm does).
@@ -37,7 +41,8 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const T* __restrict__ p
                                                          const float* __restrict__ i_bias,
                                                          const float* __restrict__ f_bias, float cap, float q_scale,
                                                          float* __restrict__ S_state, float* __restrict__ n_state,
-                                                         float* __restrict__ m_state, float* __restrict__ y,
+                                                         const float* __restrict__ m_state, float* __restrict__ m_next,
+                                                         float* __restrict__ y,
                                                          float* __restrict__ den, const int* __restrict__ cu_q,
                                                          const int* __restrict__ seq_slot, int heads, int d, int dv,
                                                          int write_state) {
@@ -198,8 +203,18 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const T* __restrict__ p
             const int c = l + ML_L * i;
             if (p_ok && c < d) sp[c] = S[i];
         }
-        if (blockIdx.z == 0 && threadIdx.x == 0) m_state[(long)slot * heads + h] = m_carry;
+        if (blockIdx.z == 0 && threadIdx.x == 0) m_next[(long)b * heads + h] = m_carry;
     }
+}
+
+// the slots' maxima behind a step: a launch behind the one whose workgroups all read those before it
+__global__ __launch_bounds__(256) void mlstm_maximum_kernel(const float* __restrict__ m_next, float* __restrict__ m_state,
+                                                            const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
+                                                            int n_seqs, int heads) {
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (long)n_seqs * heads) return;
+    const int b = (int)(i / heads);
+    if (cu_q[b + 1] > cu_q[b]) m_state[(long)seq_slot[b] * heads + i % heads] = m_next[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -225,7 +240,8 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
                                                           long v_off, long i_off, long f_off,
                                                           const float* __restrict__ i_bias, const float* __restrict__ f_bias,
                                                           float cap, float q_scale, float* __restrict__ S_state,
-                                                          float* __restrict__ n_state, float* __restrict__ m_state,
+                                                          float* __restrict__ n_state, const float* __restrict__ m_state,
+                                                          float* __restrict__ m_next,
                                                           float* __restrict__ y, float* __restrict__ den,
                                                           const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
                                                           int heads, int d, int dv, int write_state) {
@@ -255,7 +271,7 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
                 const int p = p0 + 16 * i + 4 * g + e, c = 16 * (NJ * wave + j) + r;
                 st[i][j][e] = (p <= dv && c < d) ? state_row(p)[c] : 0.f;
             }
-    double m = (double)m_state[(long)slot * heads + h];                // wavefront 0 carries it on
+    double m = (double)m_state[(long)slot * heads + h];                // wavefront 0 carries it on (m_next: see the walk)
     const float bi = i_bias[h], bf = f_bias[h], inv_cap = 1.0f / cap;
     const mlfloatx4_t zero4 = {0.f, 0.f, 0.f, 0.f};
     const int vrow = threadIdx.x >> 3, vcol = (threadIdx.x & 7) * 4;   // (256 threads bring values)
@@ -410,30 +426,36 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
                     const int p = p0 + 16 * i + 4 * g + e, c = 16 * (NJ * wave + j) + r;
                     if (p <= dv && c < d) state_row(p)[c] = st[i][j][e];
                 }
-        if (blockIdx.z == 0 && threadIdx.x == 0) m_state[(long)slot * heads + h] = (float)m;
+        if (blockIdx.z == 0 && threadIdx.x == 0) m_next[(long)b * heads + h] = (float)m;
     }
 }
 
-// max_q: the longest run of tokens a sequence brings (0: not known, the walk)
+// max_q: the longest run of tokens a sequence brings (0: not known, the walk); m_next: float [n_seqs * heads], scratch
 extern "C" const char* cpmcu_mlstm_scan(const void* proj, long ld, int dtype, long q_off, long k_off, long v_off,
                                         long i_off, long f_off, const float* i_bias, const float* f_bias, float cap,
-                                        float q_scale, float* S_state, float* n_state, float* m_state, float* y,
-                                        float* den, const int* cu_q, const int* seq_slot, int n_seqs, int heads, int d, int dv,
-                                        int write_state, int max_q, hipStream_t stream) {
+                                        float q_scale, float* S_state, float* n_state, float* m_state, float* m_next,
+                                        float* y, float* den, const int* cu_q, const int* seq_slot, int n_seqs, int heads,
+                                        int d, int dv, int write_state, int max_q, hipStream_t stream) {
     CPMCU_REQUIRE(n_seqs > 0 && heads > 0 && d > 0 && dv > 0, "mlstm_scan: empty shape");
     CPMCU_REQUIRE(d <= 1024, "mlstm_scan: a key size of %d is not supported (at most 1024)", d);
     CPMCU_REQUIRE(cap > 0.f, "mlstm_scan: gate cap %g", cap);
     CPMCU_REQUIRE(q_off >= 0 && k_off >= 0 && v_off >= 0 && i_off >= 0 && f_off >= 0 && q_off + (long)heads * d <= ld &&
                   k_off + (long)heads * d <= ld && v_off + (long)heads * dv <= ld && i_off + heads <= ld && f_off + heads <= ld,
                   "mlstm_scan: columns beyond rows of %ld", ld);
+    CPMCU_REQUIRE(!write_state || m_next, "mlstm_scan: scratch for the maxima is missing");
+    const auto move_maxima = [&]() {
+        if (write_state)
+            mlstm_maximum_kernel<<<(unsigned)(((long)n_seqs * heads + 255) / 256), 256, 0, stream>>>(m_next, m_state, cu_q,
+                                                                                                    seq_slot, n_seqs, heads);
+    };
     if (max_q >= MCHUNK_MIN && d <= 256 && d % 4 == 0 && dv % 4 == 0 && ld % 4 == 0 && q_off % 4 == 0 && k_off % 4 == 0 &&
         v_off % 4 == 0 && (uintptr_t)proj % 16 == 0 && (dtype == CPMCU_F32 || dtype == CPMCU_BF16)) {
         const dim3 grid(n_seqs, heads, (dv + 1 + MCHUNK_P - 1) / MCHUNK_P);
         CPMCU_REQUIRE(heads <= 65535 && grid.z <= 65535, "mlstm_scan: shape exceeds the launch grid");
 #define CHUNKS(NBv, Tv)                                                                                             \
     mlstm_chunk_kernel<NBv, Tv><<<grid, 512, 0, stream>>>((const Tv*)proj, ld, q_off, k_off, v_off, i_off, f_off,   \
-                                                          i_bias, f_bias, cap, q_scale, S_state, n_state, m_state, y, \
-                                                          den, cu_q, seq_slot, heads, d, dv, write_state)
+                                                          i_bias, f_bias, cap, q_scale, S_state, n_state, m_state,  \
+                                                          m_next, y, den, cu_q, seq_slot, heads, d, dv, write_state)
         if (dtype == CPMCU_F32) {
             if (d <= 128) CHUNKS(8, float);
             else CHUNKS(16, float);
@@ -443,6 +465,8 @@ extern "C" const char* cpmcu_mlstm_scan(const void* proj, long ld, int dtype, lo
         }
 #undef CHUNKS
         CPMCU_LAUNCH_CHECK("mlstm_chunk");
+        move_maxima();
+        CPMCU_LAUNCH_CHECK("mlstm_maximum");
         return nullptr;
     }
     const int lanes = d > 128 ? 32 : 8, cols = 256 / lanes;
@@ -453,8 +477,8 @@ extern "C" const char* cpmcu_mlstm_scan(const void* proj, long ld, int dtype, lo
 #define LAUNCH(NRv, Lv, TTv, Tv)                                                                                     \
     mlstm_scan_kernel<NRv, Lv, TTv, Tv><<<grid, 256, 0, stream>>>((const Tv*)proj, ld, q_off, k_off, v_off, i_off,   \
                                                                   f_off, i_bias, f_bias, cap, q_scale, S_state,      \
-                                                                  n_state, m_state, y, den, cu_q, seq_slot, heads,   \
-                                                                  d, dv, write_state)
+                                                                  n_state, m_state, m_next, y, den, cu_q, seq_slot,  \
+                                                                  heads, d, dv, write_state)
 #define BY_NR(Tv)                                  \
     do {                                           \
         if (lanes == 32 && need <= 8) LAUNCH(8, 32, 16, Tv);        \
@@ -471,5 +495,7 @@ extern "C" const char* cpmcu_mlstm_scan(const void* proj, long ld, int dtype, lo
 #undef BY_NR
 #undef LAUNCH
     CPMCU_LAUNCH_CHECK("mlstm_scan");
+    move_maxima();
+    CPMCU_LAUNCH_CHECK("mlstm_maximum");
     return nullptr;
 }

@@ -919,7 +919,8 @@ def bigram_add(table: torch.Tensor, ids: torch.Tensor, positions: torch.Tensor, 
 def mlstm_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, i_off: int, f_off: int, i_bias: torch.Tensor,
                f_bias: torch.Tensor, cap: float, q_scale: float, S: torch.Tensor, n_state: torch.Tensor,
                m_state: torch.Tensor, y: torch.Tensor, den: torch.Tensor, cu_q: torch.Tensor, seq_slot: torch.Tensor,
-               heads: int, d: int, dv: int, write_state: bool = True, max_q: int = 0):
+               heads: int, d: int, dv: int, write_state: bool = True, max_q: int = 0,
+               m_next: Optional[torch.Tensor] = None):
     """The matrix-memory recurrence over each sequence's tokens, in float (max_q, the longest run of tokens a sequence
     brings, lets prompts be taken 32 tokens at a time; 0: walked token by token).  proj [n, W] holds, from the given
     columns on, q and k (heads * d each), v (heads * dv) and the raw input and forget gates (heads each); per head
@@ -927,7 +928,8 @@ def mlstm_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, i_off: in
     S' = exp(b + m - m') S + exp(a - m') k v^T, n' likewise with k, q multiplied by q_scale.  It leaves the output
     in two pieces: y = S'^T q (float32 [n, heads * dv]) and den = max(|n'.q|, exp(-m')) + 1e-6 (float32 [n, heads]);
     the design's output is y / den head by head (rms_norm_groups takes den as its divisor).
-    S float32 [slots, heads, dv, d], n_state [slots, heads, d], m_state [slots, heads]."""
+    S float32 [slots, heads, dv, d], n_state [slots, heads, d], m_state [slots, heads]; m_next float32 [sequences, heads] is
+    scratch (the workgroups of a launch read a slot's maximum as they start, so a second launch moves it on)."""
     ld = _ld(proj, "mlstm projection")
     n = proj.shape[0]
     for off, w in ((q_off, heads * d), (k_off, heads * d), (v_off, heads * dv), (i_off, heads), (f_off, heads)):
@@ -943,11 +945,15 @@ def mlstm_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, i_off: in
     _need(cu_q, "mlstm sequence starts", torch.int32, (None,))
     B = cu_q.shape[0] - 1
     _need(seq_slot, "mlstm sequence slots", torch.int32, (B,))
+    if write_state:
+        m_next = torch.empty(B, heads, dtype=torch.float32, device=proj.device) if m_next is None else m_next
+        _need(m_next, "mlstm maxima behind the step", torch.float32, (B, heads))
     _check(_fn("mlstm", "cpmcu_mlstm_scan")(_p(proj), c_long(ld), c_int(_code(proj)), c_long(q_off), c_long(k_off),
                                             c_long(v_off), c_long(i_off), c_long(f_off), _p(i_bias), _p(f_bias),
-                                            c_float(cap), c_float(q_scale), _p(S), _p(n_state), _p(m_state), _p(y),
-                                            _p(den), _p(cu_q), _p(seq_slot), c_int(B), c_int(heads), c_int(d), c_int(dv),
-                                            c_int(1 if write_state else 0), c_int(max_q), _stream()))
+                                            c_float(cap), c_float(q_scale), _p(S), _p(n_state), _p(m_state),
+                                            _p(m_next if write_state else None), _p(y), _p(den), _p(cu_q), _p(seq_slot),
+                                            c_int(B), c_int(heads), c_int(d), c_int(dv), c_int(1 if write_state else 0),
+                                            c_int(max_q), _stream()))
 
 
 def streams_fill(x: torch.Tensor, streams: torch.Tensor):

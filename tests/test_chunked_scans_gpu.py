@@ -138,3 +138,53 @@ def test_mlstm_chunks(H, d, dv, scale):
         assert all(h <= 1.5 * w + 5e-7 for h, w in zip(*errs)), errs
         assert errs[0][1] <= 2e-6 and errs[0][2] <= 2e-6, errs
     assert all(float(t[[1, 3]].abs().max()) == 0.0 for t in states[0])
+
+
+@pytest.mark.parametrize("lens,chunks", [([33, 32, 40, 37, 64], True), ([33, 32, 40, 37, 64], False), ([1] * 8, False)])
+def test_mlstm_of_more_workgroups_than_run_at_a_time(lens, chunks):
+    """A carried state whose maxima differ from slot to slot and from those behind the step: every workgroup of a launch, the
+    last ones too, starts from the maximum before the step.  (680 workgroups of which 256 run at a time, a walk's 2,600 and
+    4,160 of which 1,024 do.)"""
+    from cpmcu_amd import ops
+    H, d, dv, cap = 8, 256, 512, 15.0
+    g = torch.Generator(device=DEV).manual_seed(sum(lens))
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    B, n, cu = len(lens), sum(lens), [0]
+    for q in lens:
+        cu.append(cu[-1] + q)
+    slots = [(3 * i + 1) % (B + 2) for i in range(B)]
+    st, ns, ms = 0.3 * rnd(B + 2, H, dv, d), 0.3 * rnd(B + 2, H, d), 4.0 * rnd(B + 2, H)
+    keep, ko, vo, io, fo = [t.clone() for t in (st, ns, ms)], H * d, 2 * H * d, 2 * H * d + H * dv, 2 * H * d + H * dv + H
+    proj, ib, fb = rnd(n, fo + H), rnd(H), rnd(H)
+    proj[:, io:] *= 4.0
+    Q, K = (proj[:, o:o + H * d].double().view(n, H, d) for o in (0, ko))
+    V = proj[:, vo:vo + H * dv].double().view(n, H, dv)
+    a = cap * torch.tanh((proj[:, io:io + H].double() + ib.double()) / cap)
+    b = torch.nn.functional.logsigmoid(cap * torch.tanh((proj[:, fo:fo + H].double() + fb.double()) / cap))
+    S, N, M = (t[slots].double() for t in (st, ns, ms))
+    want, low, mag = (torch.empty(n, H, *w, dtype=torch.float64, device=DEV) for w in ((dv,), (), ()))
+    for s in range(B):
+        for t in range(cu[s], cu[s + 1]):
+            new = torch.maximum(b[t] + M[s], a[t])
+            left, take = torch.exp(b[t] + M[s] - new)[:, None], torch.exp(a[t] - new)[:, None] * K[t]
+            S[s], N[s], M[s] = left[..., None] * S[s] + V[t][:, :, None] * take[:, None], left * N[s] + take, new
+            qt = Q[t] * d ** -0.5
+            want[t], low[t] = (S[s] * qt[:, None]).sum(-1), torch.maximum((N[s] * qt).sum(-1).abs(), torch.exp(-new)) + 1e-6
+            mag[t] = (N[s] * qt).abs().sum(-1) + torch.exp(-new)
+    y, den = torch.full((n, H * dv), float("nan"), device=DEV), torch.full((n, H), float("nan"), device=DEV)
+    args = (proj, 0, ko, vo, io, fo, ib, fb, cap, d ** -0.5, st, ns, ms, y, den, i32(cu), i32(slots), H, d, dv)
+    ops.mlstm_scan(*args, write_state=False, max_q=max(lens) if chunks else 0)
+    assert all(torch.equal(x, k) for x, k in zip((st, ns, ms), keep))
+    ops.mlstm_scan(*args, max_q=max(lens) if chunks else 0)
+    # sums of a few hundred float products and exponentials of float sums: a few 1e-6 (y and den carry the scale of a float
+    # maximum, which a walk sums up token by token); with another step's maximum a scale is off by the exponential of a
+    # difference of about 4
+    assert float((ms[slots].double() - M).abs().max()) <= 2e-5
+    scale_out = torch.exp(ms[slots].double() - M)
+    errs = [float((x - w).norm() / w.norm()) for x, w in ((st[slots].double() * scale_out[..., None, None], S),
+                                                          (ns[slots].double() * scale_out[..., None], N))]
+    assert max(errs) <= 1e-5, errs
+    off = (y.view(n, H, dv).double() - want).norm(dim=-1) / want.norm(dim=-1)
+    assert float(off.max()) <= 1e-4 and bool(((den.double() - low).abs() <= 1e-4 * mag).all()), (float(off.max()), errs)
+    others = [i for i in range(B + 2) if i not in slots]
+    assert all(torch.equal(x[others], k[others]) for x, k in zip((st, ns, ms), keep))
