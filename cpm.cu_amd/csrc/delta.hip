@@ -24,6 +24,7 @@
 //     S <- d_h S + k v^T;  o = S^T q = d_h (S_old^T q) + (k . q) v, with q and k taken as they come (no unit
 //     norm, no beta, no gates); `A_log` then holds the decays d_h themselves.
 #include "common.h"
+#include "runs.h"
 
 enum { RULE_DELTA = 0, RULE_CHANNEL = 1, RULE_DECAY = 2 };
 
@@ -34,6 +35,8 @@ __device__ inline float delta_softplus(float v) { return fmaxf(v, 0.f) + log1pf(
 // state: float [slots][heads][dv][dk]; y: float [n, heads*dv].
 // chan_a (RULE_CHANNEL): float [n, ld_a], the raw decay projection of head h and key channel i at column h*dk + i;
 // dt_bias then has heads*dk numbers.
+// grid (sequences x heads, blocks of DELTA_PB columns): a sequence's workgroups are dealt to all XCDs, also where one
+// sequence of a step is much longer than the others.  The launch takes the sequences of lo <= tokens < hi (runs.h).
 template <int NR, int TT, int DELTA_L, typename GT, int RULE>
 __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict__ qkv, long ld,
                                                          const GT* __restrict__ gates, long ldg, long a_off, long b_off,
@@ -42,7 +45,8 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
                                                          const float* __restrict__ A_log, float* __restrict__ state,
                                                          float* __restrict__ y, const int* __restrict__ cu_q,
                                                          const int* __restrict__ seq_slot, int heads, int kv_heads,
-                                                         int dk, int dv, float q_scale, int write_state) {
+                                                         int dk, int dv, float q_scale, int write_state, int n_seqs,
+                                                         int lo, int hi) {
     constexpr int DELTA_PB = 256 / DELTA_L;         // columns of dv a workgroup
     constexpr int NS = NR * DELTA_L;                // state values a column, padded
     constexpr int QK = TT * NS / 256;               // q (and k) values a thread brings a tile
@@ -54,7 +58,9 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
     __shared__ float vs[TT][DELTA_PB];
     __shared__ float betas[TT], gs[TT], kqs[TT];
     __shared__ float gcs[RULE == RULE_CHANNEL ? TT : 1][RULE == RULE_CHANNEL ? NS : 1];   // a decay a channel
-    const int b = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * DELTA_PB;
+    const int b = nth_run(cu_q, n_seqs, blockIdx.x / heads, lo, hi), p0 = blockIdx.y * DELTA_PB;
+    const int h = grouped_head(blockIdx.x % heads, heads, kv_heads);
+    if (b < 0) return;
     const int start = cu_q[b], n_q = cu_q[b + 1] - start;
     const int slot = seq_slot[b];
     const int kvh = h / (heads / kv_heads);
@@ -209,7 +215,6 @@ typedef float dfloatx4_t __attribute__((ext_vector_type(4)));
 #define DCHUNK_N 128      // key features, at most
 #define DCHUNK_LN 132     // LDS rows of DCHUNK_N: rows 4 banks apart, so that 8 rows' 16 bytes read all banks
 #define DCHUNK_LT 68      // LDS rows of DCHUNK_T
-#define DCHUNK_MIN 64     // tokens a sequence from which chunks are taken
 
 template <int NB, int PT, typename GT>
 __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restrict__ qkv, long ld,
@@ -218,7 +223,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
                                                           float* __restrict__ state, float* __restrict__ y,
                                                           const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
                                                           int heads, int kv_heads, int dk, int dv, float q_scale,
-                                                          int write_state) {
+                                                          int write_state, int n_seqs, int lo, int hi) {
     constexpr int PB = 16 * PT;                                         // columns of dv a workgroup
     __shared__ __align__(16) float Ks[DCHUNK_T * DCHUNK_LN], Qs[DCHUNK_T * DCHUNK_LN];
     __shared__ __align__(16) float Ss[PB * DCHUNK_LN];            // the state before the chunk, [p][n]
@@ -228,7 +233,9 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
     __shared__ __align__(16) float inv_s[4 * 16 * 20];                  // inverses of the diagonal blocks
     __shared__ __align__(16) float fk_s[DCHUNK_T], fq_s[DCHUNK_T], beta_s[DCHUNK_T], left_s[DCHUNK_T], from_s[DCHUNK_T];
     __shared__ double la_s[DCHUNK_T];
-    const int b = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * PB;
+    const int b = nth_run(cu_q, n_seqs, blockIdx.x / heads, lo, hi), p0 = blockIdx.y * PB;
+    const int h = grouped_head(blockIdx.x % heads, heads, kv_heads);
+    if (b < 0) return;
     const int start = cu_q[b], q = cu_q[b + 1] - start;
     if (q <= 0) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -446,12 +453,14 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
     }
 }
 
-// max_q: the longest run of tokens a sequence brings (0: not known, the walk)
+// The n_chunked sequences that bring at least chunk_from tokens are taken in chunks, the others are walked: two launches
+// where there are both.  (0, 0: all are walked, as they are under the rules and sizes that the chunks' kernel does not take.)
 extern "C" const char* cpmcu_delta_scan(const float* qkv, long ld, const void* gates, long ldg, int gate_dtype,
                                         long a_off, long b_off, const float* chan_a, long ld_a, const float* dt_bias,
                                         const float* A_log, float* state, float* y, const int* cu_q,
                                         const int* seq_slot, int n_seqs, int heads, int kv_heads, int dk, int dv,
-                                        float q_scale, int write_state, int lanes, int rule, int max_q, hipStream_t stream) {
+                                        float q_scale, int write_state, int lanes, int rule, int chunk_from,
+                                        int n_chunked, hipStream_t stream) {
     CPMCU_REQUIRE(rule == RULE_DELTA || rule == RULE_CHANNEL || rule == RULE_DECAY, "delta_scan: unknown rule %d", rule);
     CPMCU_REQUIRE(n_seqs > 0 && heads > 0 && kv_heads > 0 && dk > 0 && dv > 0, "delta_scan: empty shape");
     CPMCU_REQUIRE(heads % kv_heads == 0, "delta_scan: %d heads are not a multiple of %d key heads", heads, kv_heads);
@@ -462,15 +471,18 @@ extern "C" const char* cpmcu_delta_scan(const float* qkv, long ld, const void* g
     CPMCU_REQUIRE(rule != RULE_CHANNEL || (chan_a && ld_a >= (long)heads * dk), "delta_scan: channel decay rows too short");
     CPMCU_REQUIRE(A_log && (rule == RULE_DECAY || dt_bias), "delta_scan: decay constants missing");
     CPMCU_REQUIRE(lanes == 0 || lanes == 8 || lanes == 16, "delta_scan: %d lanes a column (0: chosen here, 8 or 16)", lanes);
-    if (rule == RULE_DELTA && lanes == 0 && max_q >= DCHUNK_MIN && dk <= DCHUNK_N && dk % 4 == 0 && dv % 4 == 0 && ld % 4 == 0 &&
-        (uintptr_t)qkv % 16 == 0 && (gate_dtype == CPMCU_F32 || gate_dtype == CPMCU_BF16)) {
-        // From 64 tokens a sequence on chunks are the cheaper form at any number of sequences (us, walk / chunks: 1 x 64
-        // tokens 29 / 18, 8 x 64 75 / 60, 32 x 64 245 / 237; 8 x 32 42 / 58).
+    CPMCU_REQUIRE(chunk_from >= 0 && n_chunked >= 0 && n_chunked <= n_seqs, "delta_scan: %d sequences of %d in chunks", n_chunked, n_seqs);
+    CPMCU_REQUIRE((long)n_seqs * heads < (1L << 31), "delta_scan: shape exceeds the launch grid");
+    if (!(rule == RULE_DELTA && lanes == 0 && dk <= DCHUNK_N && dk % 4 == 0 && dv % 4 == 0 && ld % 4 == 0 &&
+          (uintptr_t)qkv % 16 == 0 && (gate_dtype == CPMCU_F32 || gate_dtype == CPMCU_BF16)))
+        n_chunked = 0;
+    if (n_chunked > 0) {
         // 32 columns a workgroup share the products among keys and queries; 16 where 32 would leave CUs without one (a
         // workgroup's LDS leaves a CU one at a time)
-        const bool narrow = (long)n_seqs * heads * ((dv + 31) / 32) < 256;
-        const dim3 grid(n_seqs, heads, narrow ? (dv + 15) / 16 : (dv + 31) / 32);
-        CPMCU_REQUIRE(heads <= 65535 && grid.z <= 65535, "delta_scan: shape exceeds the launch grid");
+        const bool narrow = (long)n_chunked * heads * ((dv + 31) / 32) < 256;
+        const dim3 grid(heads * n_chunked, narrow ? (dv + 15) / 16 : (dv + 31) / 32);
+        const int hi = n_chunked < n_seqs ? 0x7fffffff : 0;
+        CPMCU_REQUIRE(grid.y <= 65535, "delta_scan: shape exceeds the launch grid");
 #define CHUNKS(NBv, GTv)                                       \
     do {                                                       \
         if (narrow) CHUNKS_OF(NBv, 1, GTv);                    \
@@ -479,7 +491,7 @@ extern "C" const char* cpmcu_delta_scan(const float* qkv, long ld, const void* g
 #define CHUNKS_OF(NBv, PTv, GTv)                                                                                               \
     delta_chunk_kernel<NBv, PTv, GTv><<<grid, 512, 0, stream>>>(qkv, ld, (const GTv*)gates, ldg, a_off, b_off, dt_bias, A_log, \
                                                            state, y, cu_q, seq_slot, heads, kv_heads, dk, dv, q_scale,    \
-                                                           write_state)
+                                                           write_state, n_seqs, chunk_from, hi)
         if (gate_dtype == CPMCU_F32) {
             if (dk <= 64) CHUNKS(4, float);
             else CHUNKS(8, float);
@@ -490,20 +502,21 @@ extern "C" const char* cpmcu_delta_scan(const float* qkv, long ld, const void* g
 #undef CHUNKS
 #undef CHUNKS_OF
         CPMCU_LAUNCH_CHECK("delta_chunk");
-        return nullptr;
+        if (n_chunked == n_seqs) return nullptr;
     }
+    const int n_walked = n_seqs - n_chunked, lo = 0, hi = n_chunked > 0 ? chunk_from : 0;
     // 16 lanes a column where 8 would leave fewer than two workgroups a compute unit and a column is long enough
-    if (lanes == 0) lanes = ((long)n_seqs * heads * ((dv + 31) / 32) < 512 && dk > 16 && dv > 16) ? 16 : 8;
+    if (lanes == 0) lanes = ((long)n_walked * heads * ((dv + 31) / 32) < 512 && dk > 16 && dv > 16) ? 16 : 8;
     const int cols = 256 / lanes;
     const int pb = (dv + cols - 1) / cols;
-    CPMCU_REQUIRE(heads <= 65535 && pb <= 65535, "delta_scan: shape exceeds the launch grid");
-    dim3 grid(n_seqs, heads, pb);
+    CPMCU_REQUIRE(pb <= 65535, "delta_scan: shape exceeds the launch grid");
+    dim3 grid(heads * n_walked, pb);
     const int need = (dk + lanes - 1) / lanes;
 #define LAUNCH(NRv, TTv, Lv, GTv, Rv)                                                                                \
     delta_scan_kernel<NRv, TTv, Lv, GTv, Rv><<<grid, 256, 0, stream>>>(qkv, ld, (const GTv*)gates, ldg, a_off, b_off, \
                                                                        chan_a, ld_a, dt_bias, A_log, state, y, cu_q,  \
                                                                        seq_slot, heads, kv_heads, dk, dv, q_scale,    \
-                                                                       write_state)
+                                                                       write_state, n_seqs, lo, hi)
 #define BY_NR(GTv, Rv)                                        \
     do {                                                      \
         if (lanes == 16) {                                    \

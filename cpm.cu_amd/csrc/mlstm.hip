@@ -12,6 +12,7 @@
 // the head norm that follows divides.  S, n and m live per cache slot and are carried from step to
 // step, so a step of any number of tokens continues where the last one ended.
 #include "common.h"
+#include "runs.h"
 #include "vec4.h"
 
 // A workgroup of 256 threads walks ML_PB = 256 / ML_L columns; a column's d state values lie over ML_L neighbouring
@@ -21,7 +22,8 @@
 
 __device__ inline float log_sigmoid_f(float v) { return fminf(v, 0.f) - log1pf(expf(-fabsf(v))); }
 
-// grid (sequences, heads, ceil((dv + 1) / ML_PB)), 256 threads.  proj: [n, ld]; q at column q_off + h * d, k at
+// grid (sequences x heads, ceil((dv + 1) / ML_PB)), 256 threads: a sequence's workgroups are dealt to all XCDs, also where
+// one sequence of a step is much longer than the others.  The launch takes the sequences of lo <= tokens < hi (runs.h).  proj: [n, ld]; q at column q_off + h * d, k at
 // k_off + h * d, v at v_off + h * dv, raw gates at i_off + h and f_off + h.  S: [slots][heads][dv][d],
 // nst: [slots][heads][d], mst: [slots][heads].
 //
@@ -45,7 +47,7 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const T* __restrict__ p
                                                          float* __restrict__ y,
                                                          float* __restrict__ den, const int* __restrict__ cu_q,
                                                          const int* __restrict__ seq_slot, int heads, int d, int dv,
-                                                         int write_state) {
+                                                         int write_state, int n_seqs, int lo, int hi) {
     constexpr int ML_PB = 256 / ML_L;               // columns a workgroup
     constexpr int NS = NR * ML_L;                   // key features, padded
     constexpr int QK = ML_TT * NS / 256;            // q (and k) values a thread brings a tile
@@ -55,7 +57,8 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const T* __restrict__ p
     __shared__ float vs[ML_TT][ML_PB];
     __shared__ float keep_s[ML_TT], take_s[ML_TT], em_s[ML_TT];
     __shared__ float m_carry;
-    const int b = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * ML_PB;
+    const int b = nth_run(cu_q, n_seqs, blockIdx.x / heads, lo, hi), h = blockIdx.x % heads, p0 = blockIdx.y * ML_PB;
+    if (b < 0) return;
     const int start = cu_q[b], q = cu_q[b + 1] - start;
     const int slot = seq_slot[b];
     const int pl = threadIdx.x / ML_L, l = threadIdx.x % ML_L;
@@ -203,7 +206,7 @@ __global__ __launch_bounds__(256) void mlstm_scan_kernel(const T* __restrict__ p
             const int c = l + ML_L * i;
             if (p_ok && c < d) sp[c] = S[i];
         }
-        if (blockIdx.z == 0 && threadIdx.x == 0) m_next[(long)b * heads + h] = m_carry;
+        if (blockIdx.y == 0 && threadIdx.x == 0) m_next[(long)b * heads + h] = m_carry;
     }
 }
 
@@ -232,7 +235,6 @@ typedef float mlfloatx4_t __attribute__((ext_vector_type(4)));
 #define MCHUNK_T 32       // tokens a chunk
 #define MCHUNK_P 32       // columns a workgroup
 #define MCHUNK_LT 36      // LDS rows of MCHUNK_T: rows 4 banks apart, so that 8 rows' 16 bytes read all banks
-#define MCHUNK_MIN 32     // tokens a sequence from which chunks are taken: 8 sequences of 32, 101 -> 55 us; of 16, 58 -> 53 us, as little as a walk
 
 // NB: blocks of 16 key features, a multiple of 8
 template <int NB, typename T>
@@ -244,7 +246,8 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
                                                           float* __restrict__ m_next,
                                                           float* __restrict__ y, float* __restrict__ den,
                                                           const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
-                                                          int heads, int d, int dv, int write_state) {
+                                                          int heads, int d, int dv, int write_state, int n_seqs, int lo,
+                                                          int hi) {
     constexpr int LN = 16 * NB + 4, NJ = NB / 8, C4 = 4 * NB, QK = MCHUNK_T * C4 / 512;
     __shared__ __align__(16) float Qs[MCHUNK_T * LN], Ks[MCHUNK_T * LN];
     __shared__ __align__(16) float Ss[MCHUNK_P * LN];                  // the state before the chunk, [p][c]
@@ -252,7 +255,8 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
     __shared__ __align__(16) float vT[MCHUNK_P * MCHUNK_LT];            // [p][t]
     __shared__ __align__(16) float left_s[MCHUNK_T], from_s[MCHUNK_T], floor_s[MCHUNK_T];
     __shared__ double w_s[MCHUNK_T], M_s[MCHUNK_T];
-    const int b = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * MCHUNK_P;
+    const int b = nth_run(cu_q, n_seqs, blockIdx.x / heads, lo, hi), h = blockIdx.x % heads, p0 = blockIdx.y * MCHUNK_P;
+    if (b < 0) return;
     const int start = cu_q[b], q = cu_q[b + 1] - start, slot = seq_slot[b];
     if (q <= 0) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -426,16 +430,19 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
                     const int p = p0 + 16 * i + 4 * g + e, c = 16 * (NJ * wave + j) + r;
                     if (p <= dv && c < d) state_row(p)[c] = st[i][j][e];
                 }
-        if (blockIdx.z == 0 && threadIdx.x == 0) m_next[(long)b * heads + h] = (float)m;
+        if (blockIdx.y == 0 && threadIdx.x == 0) m_next[(long)b * heads + h] = (float)m;
     }
 }
 
-// max_q: the longest run of tokens a sequence brings (0: not known, the walk); m_next: float [n_seqs * heads], scratch
+// The n_chunked sequences that bring at least chunk_from tokens are taken in chunks, the others are walked: two launches
+// where there are both.  (0, 0: all are walked, as they are where the chunks' kernel does not take the sizes.)
+// m_next: float [n_seqs * heads], scratch.
 extern "C" const char* cpmcu_mlstm_scan(const void* proj, long ld, int dtype, long q_off, long k_off, long v_off,
                                         long i_off, long f_off, const float* i_bias, const float* f_bias, float cap,
                                         float q_scale, float* S_state, float* n_state, float* m_state, float* m_next,
                                         float* y, float* den, const int* cu_q, const int* seq_slot, int n_seqs, int heads,
-                                        int d, int dv, int write_state, int max_q, hipStream_t stream) {
+                                        int d, int dv, int write_state, int chunk_from, int n_chunked,
+                                        hipStream_t stream) {
     CPMCU_REQUIRE(n_seqs > 0 && heads > 0 && d > 0 && dv > 0, "mlstm_scan: empty shape");
     CPMCU_REQUIRE(d <= 1024, "mlstm_scan: a key size of %d is not supported (at most 1024)", d);
     CPMCU_REQUIRE(cap > 0.f, "mlstm_scan: gate cap %g", cap);
@@ -448,14 +455,20 @@ extern "C" const char* cpmcu_mlstm_scan(const void* proj, long ld, int dtype, lo
             mlstm_maximum_kernel<<<(unsigned)(((long)n_seqs * heads + 255) / 256), 256, 0, stream>>>(m_next, m_state, cu_q,
                                                                                                     seq_slot, n_seqs, heads);
     };
-    if (max_q >= MCHUNK_MIN && d <= 256 && d % 4 == 0 && dv % 4 == 0 && ld % 4 == 0 && q_off % 4 == 0 && k_off % 4 == 0 &&
-        v_off % 4 == 0 && (uintptr_t)proj % 16 == 0 && (dtype == CPMCU_F32 || dtype == CPMCU_BF16)) {
-        const dim3 grid(n_seqs, heads, (dv + 1 + MCHUNK_P - 1) / MCHUNK_P);
-        CPMCU_REQUIRE(heads <= 65535 && grid.z <= 65535, "mlstm_scan: shape exceeds the launch grid");
+    CPMCU_REQUIRE(chunk_from >= 0 && n_chunked >= 0 && n_chunked <= n_seqs, "mlstm_scan: %d sequences of %d in chunks", n_chunked, n_seqs);
+    CPMCU_REQUIRE((long)n_seqs * heads < (1L << 31), "mlstm_scan: shape exceeds the launch grid");
+    if (!(d <= 256 && d % 4 == 0 && dv % 4 == 0 && ld % 4 == 0 && q_off % 4 == 0 && k_off % 4 == 0 && v_off % 4 == 0 &&
+          (uintptr_t)proj % 16 == 0 && (dtype == CPMCU_F32 || dtype == CPMCU_BF16)))
+        n_chunked = 0;
+    if (n_chunked > 0) {
+        const dim3 grid(heads * n_chunked, (dv + 1 + MCHUNK_P - 1) / MCHUNK_P);
+        const int hi = n_chunked < n_seqs ? 0x7fffffff : 0;
+        CPMCU_REQUIRE(grid.y <= 65535, "mlstm_scan: shape exceeds the launch grid");
 #define CHUNKS(NBv, Tv)                                                                                             \
     mlstm_chunk_kernel<NBv, Tv><<<grid, 512, 0, stream>>>((const Tv*)proj, ld, q_off, k_off, v_off, i_off, f_off,   \
                                                           i_bias, f_bias, cap, q_scale, S_state, n_state, m_state,  \
-                                                          m_next, y, den, cu_q, seq_slot, heads, d, dv, write_state)
+                                                          m_next, y, den, cu_q, seq_slot, heads, d, dv, write_state, \
+                                                          n_seqs, chunk_from, hi)
         if (dtype == CPMCU_F32) {
             if (d <= 128) CHUNKS(8, float);
             else CHUNKS(16, float);
@@ -465,20 +478,23 @@ extern "C" const char* cpmcu_mlstm_scan(const void* proj, long ld, int dtype, lo
         }
 #undef CHUNKS
         CPMCU_LAUNCH_CHECK("mlstm_chunk");
-        move_maxima();
-        CPMCU_LAUNCH_CHECK("mlstm_maximum");
-        return nullptr;
+        if (n_chunked == n_seqs) {
+            move_maxima();
+            CPMCU_LAUNCH_CHECK("mlstm_maximum");
+            return nullptr;
+        }
     }
+    const int lo = 0, hi = n_chunked > 0 ? chunk_from : 0;
     const int lanes = d > 128 ? 32 : 8, cols = 256 / lanes;
     const int pb = (dv + 1 + cols - 1) / cols;       // the normaliser is walked as column dv
-    CPMCU_REQUIRE(heads <= 65535 && pb <= 65535, "mlstm_scan: shape exceeds the launch grid");
-    dim3 grid(n_seqs, heads, pb);
+    CPMCU_REQUIRE(pb <= 65535, "mlstm_scan: shape exceeds the launch grid");
+    dim3 grid(heads * (n_seqs - n_chunked), pb);
     const int need = (d + lanes - 1) / lanes;
 #define LAUNCH(NRv, Lv, TTv, Tv)                                                                                     \
     mlstm_scan_kernel<NRv, Lv, TTv, Tv><<<grid, 256, 0, stream>>>((const Tv*)proj, ld, q_off, k_off, v_off, i_off,   \
                                                                   f_off, i_bias, f_bias, cap, q_scale, S_state,      \
                                                                   n_state, m_state, m_next, y, den, cu_q, seq_slot,  \
-                                                                  heads, d, dv, write_state)
+                                                                  heads, d, dv, write_state, n_seqs, lo, hi)
 #define BY_NR(Tv)                                  \
     do {                                           \
         if (lanes == 32 && need <= 8) LAUNCH(8, 32, 16, Tv);        \

@@ -18,6 +18,7 @@
 // column's N state values are spread over 8 neighbouring lanes, and the tokens' B, C, x and dt pass through
 // LDS in tiles of 16 or 32 tokens, the next tile asked for while the current one is worked on.
 #include "common.h"
+#include "runs.h"
 #include "vec4.h"
 
 __device__ inline float silu_f(float z) { return z / (1.0f + expf(-z)); }
@@ -231,6 +232,8 @@ __device__ inline float softplus_f(float v) { return fmaxf(v, 0.f) + log1pf(expf
 // columns at the given pointer); state: float [slots][heads][P][N]; y: float [n, heads*P].
 // Tiles of TT tokens pass through LDS; while a tile is worked on, the next one's values are already asked for
 // (held in registers until the tile is done), so that the walk over a long prompt waits for memory once.
+// grid (sequences x heads, blocks of SCAN_PB columns): a sequence's workgroups are dealt to all XCDs, also where one
+// sequence of a step is much longer than the others.  The launch takes the sequences of lo <= tokens < hi (runs.h).
 template <int NR, int TT, typename DT>
 __global__ __launch_bounds__(256) void ssm_scan_kernel(const float* __restrict__ xbc, long ldx,
                                                        const DT* __restrict__ dt, long lddt,
@@ -238,7 +241,8 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const float* __restrict__
                                                        const float* __restrict__ A_log, const float* __restrict__ Dskip,
                                                        float* __restrict__ state, float* __restrict__ y,
                                                        const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
-                                                       int heads, int P, int N, int groups, int write_state) {
+                                                       int heads, int P, int N, int groups, int write_state, int n_seqs,
+                                                       int lo, int hi) {
     constexpr int NS = NR * SCAN_L;                 // state values a column, padded
     constexpr int BC = TT * NS / 256;               // B (and C) values a thread brings a tile
     constexpr int XV = (TT * SCAN_PB + 255) / 256;  // x values a thread brings a tile
@@ -247,7 +251,9 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const float* __restrict__
     __shared__ float Cs[TT][NS];
     __shared__ float xs[TT][SCAN_PB];
     __shared__ float dts[TT], das[TT];
-    const int b = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * SCAN_PB;
+    const int b = nth_run(cu_q, n_seqs, blockIdx.x / heads, lo, hi), p0 = blockIdx.y * SCAN_PB;
+    const int h = grouped_head(blockIdx.x % heads, heads, groups);
+    if (b < 0) return;
     const int start = cu_q[b], q = cu_q[b + 1] - start;
     const int slot = seq_slot[b];
     const int g = h / (heads / groups);
@@ -347,7 +353,6 @@ typedef float sfloatx4_t __attribute__((ext_vector_type(4)));
 #define CHUNK_N 128       // state values a column, at most
 #define CHUNK_LN 132      // LDS rows of CHUNK_N: rows 4 banks apart, so that 8 rows' 16 bytes read all banks
 #define CHUNK_LT 68       // LDS rows of CHUNK_T
-#define CHUNK_MIN 64      // tokens a sequence from which chunks are taken
 
 template <int NB, typename DT>
 __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict__ xbc, long ldx,
@@ -356,14 +361,17 @@ __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict_
                                                         const float* __restrict__ A_log, const float* __restrict__ Dskip,
                                                         float* __restrict__ state, float* __restrict__ y,
                                                         const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
-                                                        int heads, int P, int N, int groups, int write_state) {
+                                                        int heads, int P, int N, int groups, int write_state, int n_seqs,
+                                                        int lo, int hi) {
     __shared__ __align__(16) float Cs[CHUNK_T * CHUNK_LN], Bs[CHUNK_T * CHUNK_LN];
     __shared__ __align__(16) float Ss[SCAN_PB * CHUNK_LN];             // the state before the chunk, [p][n]
     __shared__ __align__(16) float Gs[CHUNK_T * CHUNK_LT];             // (C_t . B_s) exp(la_t - la_s) d_s
     __shared__ __align__(16) float xT[SCAN_PB * CHUNK_LT];             // [p][t]
     __shared__ __align__(16) float ds[CHUNK_T], left_s[CHUNK_T], from_s[CHUNK_T];   // d; exp(la_63 - la_t) d; exp(la_t)
     __shared__ double la_s[CHUNK_T];
-    const int b = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * SCAN_PB;
+    const int b = nth_run(cu_q, n_seqs, blockIdx.x / heads, lo, hi), p0 = blockIdx.y * SCAN_PB;
+    const int h = grouped_head(blockIdx.x % heads, heads, groups);
+    if (b < 0) return;
     const int start = cu_q[b], q = cu_q[b + 1] - start;
     if (q <= 0) return;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -512,26 +520,30 @@ __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict_
     }
 }
 
-// max_q: the longest run of tokens a sequence brings (0: not known, the walk)
+// The n_chunked sequences that bring at least chunk_from tokens are taken in chunks, the others are walked: two launches
+// where there are both.  (0, 0: all are walked, as they are where the chunks' kernel does not take the sizes.)
 extern "C" const char* cpmcu_ssm_scan(const float* xbc, long ldx, const void* dt, long lddt, int dt_dtype,
                                       const float* dt_bias, const float* A_log, const float* Dskip, float* state,
                                       float* y, const int* cu_q, const int* seq_slot, int n_seqs, int heads, int P,
-                                      int N, int groups, int write_state, int max_q, hipStream_t stream) {
+                                      int N, int groups, int write_state, int chunk_from, int n_chunked,
+                                      hipStream_t stream) {
     CPMCU_REQUIRE(n_seqs > 0 && heads > 0 && P > 0 && N > 0 && groups > 0, "ssm_scan: empty shape");
     CPMCU_REQUIRE(heads % groups == 0, "ssm_scan: %d heads are not a multiple of %d groups", heads, groups);
     CPMCU_REQUIRE(N <= 256, "ssm_scan: a state of %d values a column is not supported (at most 256)", N);
     CPMCU_REQUIRE(ldx >= (long)heads * P + 2L * groups * N && lddt >= heads, "ssm_scan: rows too short");
+    CPMCU_REQUIRE(chunk_from >= 0 && n_chunked >= 0 && n_chunked <= n_seqs, "ssm_scan: %d sequences of %d in chunks", n_chunked, n_seqs);
     const int pb = (P + SCAN_PB - 1) / SCAN_PB;
-    CPMCU_REQUIRE(heads <= 65535 && pb <= 65535, "ssm_scan: shape exceeds the launch grid");
-    dim3 grid(n_seqs, heads, pb);
-    // A chunk costs the same whatever it holds, and its LDS leaves a CU one workgroup: from 64 tokens a sequence on it is
-    // the cheaper one at any number of sequences (us, walk / chunks: 1 x 64 tokens 29 / 18, 32 x 64 363 / 295, 8 x 32
-    // 55 / 71, 32 x 16 114 / 269).
-    if (max_q >= CHUNK_MIN && N <= CHUNK_N && N % 4 == 0 && P % 4 == 0 && ldx % 4 == 0 && (uintptr_t)xbc % 16 == 0 &&
-        (dt_dtype == CPMCU_F32 || dt_dtype == CPMCU_BF16)) {
+    CPMCU_REQUIRE((long)n_seqs * heads < (1L << 31) && pb <= 65535, "ssm_scan: shape exceeds the launch grid");
+    if (!(N <= CHUNK_N && N % 4 == 0 && P % 4 == 0 && ldx % 4 == 0 && (uintptr_t)xbc % 16 == 0 &&
+          (dt_dtype == CPMCU_F32 || dt_dtype == CPMCU_BF16)))
+        n_chunked = 0;
+    if (n_chunked > 0) {
+        const dim3 grid(heads * n_chunked, pb);
+        const int hi = n_chunked < n_seqs ? 0x7fffffff : 0;
 #define CHUNKS(NBv, DTv)                                                                                           \
     ssm_chunk_kernel<NBv, DTv><<<grid, 512, 0, stream>>>(xbc, ldx, (const DTv*)dt, lddt, dt_bias, A_log, Dskip, state, y, \
-                                                         cu_q, seq_slot, heads, P, N, groups, write_state)
+                                                         cu_q, seq_slot, heads, P, N, groups, write_state, n_seqs,  \
+                                                         chunk_from, hi)
         if (dt_dtype == CPMCU_F32) {
             if (N <= 64) CHUNKS(4, float);
             else CHUNKS(8, float);
@@ -541,12 +553,15 @@ extern "C" const char* cpmcu_ssm_scan(const float* xbc, long ldx, const void* dt
         }
 #undef CHUNKS
         CPMCU_LAUNCH_CHECK("ssm_chunk");
-        return nullptr;
+        if (n_chunked == n_seqs) return nullptr;
     }
+    const dim3 grid(heads * (n_seqs - n_chunked), pb);
+    const int lo = 0, hi = n_chunked > 0 ? chunk_from : 0;
     const int need = (N + SCAN_L - 1) / SCAN_L;
 #define LAUNCH(NRv, TTv, DTv)                                                                                    \
     ssm_scan_kernel<NRv, TTv, DTv><<<grid, 256, 0, stream>>>(xbc, ldx, (const DTv*)dt, lddt, dt_bias, A_log, Dskip, \
-                                                             state, y, cu_q, seq_slot, heads, P, N, groups, write_state)
+                                                             state, y, cu_q, seq_slot, heads, P, N, groups, write_state, \
+                                                             n_seqs, lo, hi)
 #define BY_NR(DTv)                                \
     do {                                          \
         if (need <= 2) LAUNCH(2, 32, DTv);        \

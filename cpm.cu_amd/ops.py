@@ -10,7 +10,7 @@ from __future__ import annotations
 
 import ctypes
 from ctypes import c_char_p, c_float, c_int, c_long, c_ulonglong, c_void_p
-from typing import Optional, Sequence, Tuple
+from typing import NamedTuple, Optional, Sequence, Tuple
 
 import torch
 
@@ -620,11 +620,84 @@ def conv_silu(u: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
                                          c_int(0 if activation else 1), _stream()))
 
 
+class Recurrence(NamedTuple):
+    """What a recurrence costs in its two forms, in us, fitted to measurements on the MI355X (recurrence_chunks)."""
+    tokens: int             # tokens a chunk
+    least: int              # a step whose longest run is shorter is walked
+    chunk_launch: float
+    chunk_seq: float        # a sequence's state in and out, and
+    chunk: float            # a chunk, of as many workgroups as there are CUs (its LDS leaves a CU one at a time)
+    walk_launch: float
+    walk_step: float        # one dependent step of the longest run
+    walk_seq: float         # a sequence's state, and
+    walk_token: float       # a token, of as many workgroups of 32 columns (mlstm: of the same columns) as there are CUs
+
+
+RECURRENCES = {"ssm": Recurrence(64, 64, 4.0, 1.4, 7.7, 6.0, 0.353, 1.6, 0.155),
+               "delta": Recurrence(64, 64, 3.0, 1.8, 12.7, 6.0, 0.345, 2.4, 0.22),
+               "mlstm": Recurrence(32, 32, 6.0, 4.2, 7.1, 8.0, 0.575, 4.5, 0.68)}
+
+
+def recurrence_chunks(kind: str, q_lens: Sequence[int], workgroups: int) -> Tuple[int, int]:
+    """(chunk_from, n): the n sequences that bring at least chunk_from tokens go through a recurrence's chunks, the others
+    through its walk; (0, 0): all are walked.  ``workgroups``: workgroups of 32 columns a sequence has.
+    A chunk costs the same whatever it holds, a walk one dependent step a token: chunks win where sequences are few or fill
+    them, the walk where many sequences bring few tokens or end soon behind a chunk's border.  Measured (us, walk / chunks;
+    128 heads of 64 with 128 state values, 32 heads of 128 by 128, 8 heads of 256 by 512):
+      ssm    1 x 64 tokens 28/12, 1 x 600 218/79, 8 x 64 96/74, 8 x 96 138/128, 32 x 64 361/293, 32 x 96 523/527, 64 x 96 1,007/1,058;
+      delta  1 x 64 27/15, 1 x 600 212/114, 8 x 96 107/108, 8 x 256 278/215, 32 x 64 244/236, 32 x 96 350/432, 32 x 200 729/857, 64 x 96 683/891;
+      mlstm  1 x 32 26/14, 8 x 32 101/56, 32 x 48 500/282, 16 x 256 1,533/525, 32 x 1 80/168.
+    Every split by length is priced with the costs above, which meet the measured times within about 10%.  One prompt of 64
+    (300) tokens beside 31 (7) sequences of one token, all in chunks / split: ssm 267/71 (103/60), delta 228/73 (113/77), mlstm
+    183/106; 4 of 100 beside 20 of 10: ssm 231/131, delta 199/113 (walked)."""
+    r = RECURRENCES[kind]
+    lens = sorted(q_lens, reverse=True)
+    n, longest, share = len(lens), lens[0], workgroups / compute_units()
+    if longest < r.least:
+        return 0, 0
+
+    def walk(longest, n, tokens):
+        chain, work = r.walk_step * longest, share * (r.walk_seq * n + r.walk_token * tokens)
+        return r.walk_launch + max(chain, work) + 0.35 * min(chain, work)
+
+    rest, done = sum(lens), 0
+    least, best = walk(longest, n, rest), (0, 0)
+    first = r.chunk_seq + r.chunk * -(-longest // r.tokens)
+    for i, q in enumerate(lens):
+        done += -(-q // r.tokens)
+        rest -= q
+        if i + 1 < n and lens[i + 1] == q:
+            continue
+        cost = r.chunk_launch + max(first, share * (r.chunk_seq * (i + 1) + r.chunk * done))
+        if i + 1 < n:
+            cost += walk(lens[i + 1], n - i - 1, rest)
+        if cost < least:
+            least, best = cost, (q, i + 1)
+    return best
+
+
+def step_recurrence_chunks(ctx, kind: str, workgroups: int) -> Tuple[int, int]:
+    """recurrence_chunks of a step, worked out once a step."""
+    if ctx.single_token:
+        return 0, 0
+    key = ("recurrence_chunks", kind, workgroups)
+    if key not in ctx.extras:
+        ctx.extras[key] = recurrence_chunks(kind, ctx.q_lens, workgroups)
+    return ctx.extras[key]
+
+
+def _chunk_args(kind: str, chunks: Optional[Tuple[int, int]], max_q: int, n_seqs: int):
+    if chunks is None:
+        chunks = (1, n_seqs) if max_q >= RECURRENCES[kind].least else (0, 0)
+    return c_int(chunks[0]), c_int(chunks[1])
+
+
 def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A_log: torch.Tensor, D: torch.Tensor,
              state: torch.Tensor, y: torch.Tensor, cu_q: torch.Tensor, seq_slot: torch.Tensor, heads: int, P: int,
-             N: int, groups: int, write_state: bool = True, max_q: int = 0):
-    """The state-space recurrence over each sequence's tokens, in float (max_q, the longest run of tokens a sequence brings,
-    lets prompts be taken 64 tokens at a time; 0: walked token by token): per head h (group h // (heads/groups)),
+             N: int, groups: int, write_state: bool = True, max_q: int = 0, chunks: Optional[Tuple[int, int]] = None):
+    """The state-space recurrence over each sequence's tokens, in float (``chunks`` says which sequences are taken 64 tokens
+    at a time, see recurrence_chunks; without it all are where max_q, the longest run of tokens a sequence brings, is 64 or
+    more; the others are walked token by token): per head h (group h // (heads/groups)),
     d = softplus(dt + dt_bias[h]); S <- exp(-exp(A_log[h]) d) S + d B x^T; y = S^T C + D[h] x.
     xbc float32 [n, heads*P + 2*groups*N] = [x | B | C]; dt [n, heads] (may be a column slice);
     state float32 [slots, heads, P, N]; y float32 [n, heads*P]."""
@@ -643,7 +716,8 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias: torch.Tensor, A_log: 
     _check(_fn("ssm", "cpmcu_ssm_scan")(_p(xbc), c_long(xbc.shape[1]), _p(dt), c_long(lddt), c_int(_code(dt)),
                                         _p(dt_bias), _p(A_log), _p(D), _p(state), _p(y), _p(cu_q), _p(seq_slot),
                                         c_int(B), c_int(heads), c_int(P), c_int(N), c_int(groups),
-                                        c_int(1 if write_state else 0), c_int(max_q), _stream()))
+                                        c_int(1 if write_state else 0),
+                                        *_chunk_args("ssm", chunks, max_q, B), _stream()))
 
 
 ROTATE_TO_ROWS, ROTATE_TO_KEYS, ROTATE_TO_VALUES = 0, 1, 2
@@ -920,9 +994,10 @@ def mlstm_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, i_off: in
                f_bias: torch.Tensor, cap: float, q_scale: float, S: torch.Tensor, n_state: torch.Tensor,
                m_state: torch.Tensor, y: torch.Tensor, den: torch.Tensor, cu_q: torch.Tensor, seq_slot: torch.Tensor,
                heads: int, d: int, dv: int, write_state: bool = True, max_q: int = 0,
-               m_next: Optional[torch.Tensor] = None):
-    """The matrix-memory recurrence over each sequence's tokens, in float (max_q, the longest run of tokens a sequence
-    brings, lets prompts be taken 32 tokens at a time; 0: walked token by token).  proj [n, W] holds, from the given
+               m_next: Optional[torch.Tensor] = None, chunks: Optional[Tuple[int, int]] = None):
+    """The matrix-memory recurrence over each sequence's tokens, in float (``chunks`` says which sequences are taken 32
+    tokens at a time, see recurrence_chunks; without it all are where max_q, the longest run of tokens a sequence brings, is
+    32 or more; the others are walked token by token).  proj [n, W] holds, from the given
     columns on, q and k (heads * d each), v (heads * dv) and the raw input and forget gates (heads each); per head
     a = cap tanh((i + i_bias)/cap), b = logsigmoid(cap tanh((f + f_bias)/cap)), m' = max(b + m, a),
     S' = exp(b + m - m') S + exp(a - m') k v^T, n' likewise with k, q multiplied by q_scale.  It leaves the output
@@ -953,7 +1028,7 @@ def mlstm_scan(proj: torch.Tensor, q_off: int, k_off: int, v_off: int, i_off: in
                                             c_float(cap), c_float(q_scale), _p(S), _p(n_state), _p(m_state),
                                             _p(m_next if write_state else None), _p(y), _p(den), _p(cu_q), _p(seq_slot),
                                             c_int(B), c_int(heads), c_int(d), c_int(dv), c_int(1 if write_state else 0),
-                                            c_int(max_q), _stream()))
+                                            *_chunk_args("mlstm", chunks, max_q, B), _stream()))
 
 
 def streams_fill(x: torch.Tensor, streams: torch.Tensor):
@@ -1198,9 +1273,11 @@ def softcap(logits: torch.Tensor, cap: float):
 def delta_scan(qkv: torch.Tensor, gates: Optional[torch.Tensor], a_off: int, b_off: int, dt_bias: Optional[torch.Tensor],
                A_log: torch.Tensor, state: torch.Tensor, y: torch.Tensor, cu_q: torch.Tensor, seq_slot: torch.Tensor,
                heads: int, kv_heads: int, dk: int, dv: int, q_scale: float, write_state: bool = True, lanes: int = 0,
-               rule: str = "delta", channel_decay: Optional[torch.Tensor] = None, max_q: int = 0):
-    """The gated delta rule over each sequence's tokens, in float (max_q, the longest run of tokens a sequence brings, lets
-    rule 'delta' take prompts 64 tokens at a time; 0: walked token by token).  qkv float32 [n, 2*kv_heads*dk + heads*dv] =
+               rule: str = "delta", channel_decay: Optional[torch.Tensor] = None, max_q: int = 0,
+               chunks: Optional[Tuple[int, int]] = None):
+    """The gated delta rule over each sequence's tokens, in float (``chunks`` says which sequences rule 'delta' takes 64
+    tokens at a time, see recurrence_chunks; without it all where max_q, the longest run of tokens a sequence brings, is 64
+    or more; the others are walked token by token).  qkv float32 [n, 2*kv_heads*dk + heads*dv] =
     [q | k | v]; gates [n, W] holds the raw decay projection at columns a_off.. and the raw beta projection at
     b_off.. (heads each).  Per head (its q, k from head h // (heads/kv_heads)): q, k made unit vectors
     (x / sqrt(sum x^2 + 1e-6)), q times q_scale; beta = sigmoid(b); g = exp(-exp(A_log) softplus(a + dt_bias));
@@ -1239,7 +1316,7 @@ def delta_scan(qkv: torch.Tensor, gates: Optional[torch.Tensor], a_off: int, b_o
                                             _p(channel_decay), c_long(ld_a), _p(dt_bias), _p(A_log), _p(state), _p(y),
                                             _p(cu_q), _p(seq_slot), c_int(B), c_int(heads), c_int(kv_heads), c_int(dk),
                                             c_int(dv), c_float(q_scale), c_int(1 if write_state else 0), c_int(lanes),
-                                            c_int(DELTA_RULES[rule]), c_int(max_q), _stream()))
+                                            c_int(DELTA_RULES[rule]), *_chunk_args("delta", chunks, max_q, B), _stream()))
 
 
 DELTA_RULES = {"delta": 0, "channel": 1, "decay": 2}

@@ -159,7 +159,9 @@ class GatedDeltaMixer(Mixer):
             ops.delta_scan(qkv, u, self.a_off or 0, self.b_off, self.dt_bias, self.A_log, cache.state["delta"], y, ctx.cu_q,
                            ctx.seq_slot, self.heads, self.kv_heads, self.dk, self.dv, self.dk ** -0.5,
                            write_state=writes_cache, rule="channel" if self.decay_rank else "delta",
-                           channel_decay=decay, max_q=max(ctx.q_lens))
+                           channel_decay=decay,
+                           chunks=(0, 0) if self.decay_rank else ops.step_recurrence_chunks(
+                               ctx, "delta", self.heads * -(-self.dv // 32)))
         gated = ctx.ws.get("delta.gated", (n, hv), self.rt.dtype)
         with ctx.timed("delta_norm"):
             ops.rms_norm_groups(y, self.norm_w, self.eps, gated, groups=self.heads, gate=gate,

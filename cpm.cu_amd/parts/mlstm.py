@@ -81,7 +81,8 @@ class MLSTMMixer(Mixer):
             ops.mlstm_scan(u, self.q_off, self.k_off, self.v_off, self.i_off, self.f_off, self.i_bias, self.f_bias,
                            self.cap, self.dk ** -0.5, cache.state["memory"], cache.state["normaliser"],
                            cache.state["maximum"], y, den, ctx.cu_q, ctx.seq_slot, self.heads, self.dk, self.dv,
-                           write_state=writes_cache, max_q=max(ctx.q_lens), m_next=m_next)
+                           write_state=writes_cache, m_next=m_next,
+                           chunks=ops.step_recurrence_chunks(ctx, "mlstm", self.heads * -(-(self.dv + 1) // 32)))
         gated = ctx.ws.get("mlstm.gated", (n, hv), self.rt.dtype)
         with ctx.timed("mlstm_norm"):
             ops.rms_norm_groups(y, self.norm_w, self.eps, gated, groups=self.heads,

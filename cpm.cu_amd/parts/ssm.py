@@ -86,7 +86,8 @@ class Mamba2Mixer(Mixer):
         with ctx.timed("ssm_scan"):
             ops.ssm_scan(xbc, u[:, inner + self.channels:], self.dt_bias, self.A_log, self.D, cache.state["ssm"], y,
                          ctx.cu_q, ctx.seq_slot, self.heads, self.head_dim, self.state_size, self.groups,
-                         write_state=writes_cache, max_q=max(ctx.q_lens))
+                         write_state=writes_cache,
+                         chunks=ops.step_recurrence_chunks(ctx, "ssm", self.heads * -(-self.head_dim // 32)))
         gated = ctx.ws.get("ssm.gated", (n, inner), self.rt.dtype)
         with ctx.timed("ssm_norm"):
             ops.rms_norm_groups(y, self.norm_w, self.eps, gated, groups=self.norm_groups, gate=u[:, :inner])

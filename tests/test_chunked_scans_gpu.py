@@ -140,6 +140,52 @@ def test_mlstm_chunks(H, d, dv, scale):
     assert all(float(t[[1, 3]].abs().max()) == 0.0 for t in states[0])
 
 
+# 64 sequences a ballot: the last one chosen alone, on both sides of that border, all in turn; every one of them or none
+@pytest.mark.parametrize("kind", ["ssm", "delta", "mlstm"])
+@pytest.mark.parametrize("lens,chunk_from", [([64, 1, 17, 130, 3], 64), ([1] * 63 + [33, 70, 1, 40], 40), ([5, 70] * 34, 70), ([9, 40], 9),
+                                             ([66, 2], 67)])
+def test_runs_are_taken_by_their_length(kind, lens, chunk_from):
+    """Long runs in chunks, short ones walked, in one call: every run as in a call of its own form, bit by bit."""
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(sum(lens))
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    B, n, cu = len(lens), sum(lens), [0]
+    for q in lens:
+        cu.append(cu[-1] + q)
+    H, slots = 2, torch.randperm(B + 1, generator=torch.Generator().manual_seed(B))[:B].tolist()
+    if kind == "ssm":
+        P, N, states = 36, 20, [rnd(B + 1, H, 36, 20)]
+        xbc, dt, A, b, D = rnd(n, H * P + 2 * N), rnd(n, H), rnd(H), rnd(H), rnd(H)
+        call = lambda y, st, **k: ops.ssm_scan(xbc, dt, b, A, D, st[0], y[0], i32(cu), i32(slots), H, P, N, 1, **k)
+        outs = [(n, H * P)]
+    elif kind == "delta":
+        dk, dv, states = 36, 20, [rnd(B + 1, H, 20, 36)]
+        qkv, gates, A, b = rnd(n, 2 * H * dk + H * dv), rnd(n, 2 * H), rnd(H), rnd(H)
+        call = lambda y, st, **k: ops.delta_scan(qkv, gates, 0, H, b, A, st[0], y[0], i32(cu), i32(slots), H, H, dk, dv, dk ** -0.5, **k)
+        outs = [(n, H * dv)]
+    else:
+        d, dv, states = 36, 20, [rnd(B + 1, H, 20, 36), rnd(B + 1, H, 36), rnd(B + 1, H)]
+        w = 2 * H * d + H * dv
+        proj, b = rnd(n, w + 2 * H), rnd(H)
+        call = lambda y, st, **k: ops.mlstm_scan(proj, 0, H * d, 2 * H * d, w, w + H, b, b, 9.0, d ** -0.5, *st, *y, i32(cu), i32(slots),
+                                                 H, d, dv, **k)
+        outs = [(n, H * dv), (n, H)]
+    got = []
+    chosen = [q >= chunk_from for q in lens]
+    for k in (dict(chunks=(chunk_from, sum(chosen))), dict(chunks=(1, B)), dict(max_q=0)):
+        y, st = [torch.full(o, float("nan"), device=DEV) for o in outs], [s.clone() for s in states]
+        call(y, st, **k)
+        got.append((y, st))
+    both, chunked, walked = got
+    for s in range(B):
+        like = chunked if chosen[s] else walked
+        assert all(torch.equal(a[cu[s]:cu[s + 1]], b[cu[s]:cu[s + 1]]) for a, b in zip(both[0], like[0])), s
+        assert all(torch.equal(a[slots[s]], b[slots[s]]) for a, b in zip(both[1], like[1])), s
+    left = next(i for i in range(B + 1) if i not in slots)
+    assert all(torch.equal(a[left], b[left]) for a, b in zip(both[1], states))
+    assert all(bool(torch.isfinite(y).all()) for y in both[0])
+
+
 @pytest.mark.parametrize("lens,chunks", [([33, 32, 40, 37, 64], True), ([33, 32, 40, 37, 64], False), ([1] * 8, False)])
 def test_mlstm_of_more_workgroups_than_run_at_a_time(lens, chunks):
     """A carried state whose maxima differ from slot to slot and from those behind the step: every workgroup of a launch, the
