@@ -208,6 +208,8 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
 // owns 16 columns of u and needs nobody else's.  A workgroup owns one (sequence, head, 16 PT columns of dv), its state stays
 // in the accumulators' registers and passes through LDS as an operand.  The walk's cost is one dependent chain a token (0.35
 // us), a chunk takes 11 us: 32 heads of 128 by 128, 1,500 tokens 528 -> 262 us (298 with 32 columns a workgroup).
+// A token's infinities reach no earlier token: their factors are zero, but a zero does not silence an infinity in a product,
+// so u and outputs that are not all finite are worked out again term by term.
 // A lane's 16 bytes serve four instructions: instruction j of a block takes index 4 g + j of the 16 in both operands.
 // ---------------------------------------------------------------------------
 typedef float dfloatx4_t __attribute__((ext_vector_type(4)));
@@ -229,7 +231,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
     __shared__ __align__(16) float Ss[PB * DCHUNK_LN];            // the state before the chunk, [p][n]
     __shared__ __align__(16) float As[DCHUNK_T * DCHUNK_LT];            // -A
     __shared__ __align__(16) float Gs[DCHUNK_T * DCHUNK_LT];            // exp(la_t - la_s) q_t . k_s
-    __shared__ __align__(16) float uT[PB * DCHUNK_LT];            // v, then the right-hand side, then u: [p][t]
+    __shared__ __align__(16) float rT[PB * DCHUNK_LT], uT[PB * DCHUNK_LT];  // v, then the right-hand side; u: [p][t]
     __shared__ __align__(16) float inv_s[4 * 16 * 20];                  // inverses of the diagonal blocks
     __shared__ __align__(16) float fk_s[DCHUNK_T], fq_s[DCHUNK_T], beta_s[DCHUNK_T], left_s[DCHUNK_T], from_s[DCHUNK_T];
     __shared__ double la_s[DCHUNK_T];
@@ -253,7 +255,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
             const int p = 16 * i + 4 * g + e;
             st[i][e] = (p0 + p < dv && n_own < dk) ? sp[(long)p * dk + n_own] : 0.f;
         }
-    const float A = expf(A_log[h]), bias = dt_bias[h];
+    const float A = decay_rate(A_log[h]), bias = dt_bias[h];
     const dfloatx4_t zero4 = {0.f, 0.f, 0.f, 0.f};
     const int vrow = threadIdx.x / (PB / 4), vcol = threadIdx.x % (PB / 4) * 4;      // (with 16 columns half of the threads)
     dfloatx4_t rq[4], rk[4], rv;
@@ -300,6 +302,13 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
         for (int i = 0; i < PT; ++i)
 #pragma unroll
             for (int e = 0; e < 4; ++e) Ss[(16 * i + 4 * g + e) * DCHUNK_LN + n_own] = st[i][e];
+        if (tn < DCHUNK_T) {                                           // rows behind the run's end repeat its last token
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if ((int)(threadIdx.x + 512 * i) >> 5 >= tn) rk[i] = zero4;
+            if (vrow >= tn) rv = zero4;
+        }
+        float largest = 0.f, k2[4], q2[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int e = threadIdx.x + 512 * i, t = e >> 5, at = t * DCHUNK_LN + (e & 31) * 4;
@@ -314,14 +323,26 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
                 fk_s[t] = 1.0f / sqrtf(sk + 1e-6f);
                 fq_s[t] = q_scale / sqrtf(sq + 1e-6f);
             }
+            largest = fmaxf(largest, fmaxf(sk, sq));
+            k2[i] = sk;
+            q2[i] = sq;
+        }
+        if (__builtin_amdgcn_ballot_w64(largest == INFINITY)) {
+            // a row whose square overflows counts as zero (its factor is), before products of it overflow too
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int e = threadIdx.x + 512 * i, at = (e >> 5) * DCHUNK_LN + (e & 31) * 4;
+                if (k2[i] == INFINITY) *(dfloatx4_t*)&Ks[at] = rk[i] * 0.f;
+                if (q2[i] == INFINITY) *(dfloatx4_t*)&Qs[at] = rq[i] * 0.f;
+            }
         }
         if (vrow < DCHUNK_T) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j) uT[(vcol + j) * DCHUNK_LT + vrow] = rv[j];
+            for (int j = 0; j < 4; ++j) rT[(vcol + j) * DCHUNK_LT + vrow] = rv[j];
         }
         if (wave == 0) {
             // a token beyond the end has beta = 0 and g = 1: it neither writes nor forgets
-            double la = lane < tn ? -(double)A * (double)delta_softplus(ra + bias) : 0.0;
+            double la = lane < tn ? -(double)A * (double)decay_step(delta_softplus(ra + bias), A) : 0.0;
 #pragma unroll
             for (int k = 1; k < 64; k <<= 1) {
                 const double up = __shfl_up(la, k, 64);
@@ -349,7 +370,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
         }
         if (owns) {   // the right-hand side, in place of v
             const dfloatx4_t a = dot_tile(Ks, tt, Ss, pt);
-            dfloatx4_t* at = (dfloatx4_t*)&uT[(16 * pt + r) * DCHUNK_LT + 16 * tt + 4 * g];
+            dfloatx4_t* at = (dfloatx4_t*)&rT[(16 * pt + r) * DCHUNK_LT + 16 * tt + 4 * g];
             dfloatx4_t v = *at;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -373,19 +394,29 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
             for (int t = 0; t < 16; ++t) inv_s[(16 * g + t) * 20 + r] = x[t];
         }
         // what the state before the chunk gives this wavefront's tokens
+        auto write_y = [&](const dfloatx4_t& v) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * tt + 4 * g + e, p = 16 * pt + r;
+                if (owns && t < tn && p0 + p < dv) y[(long)(start + t0 + t) * heads * dv + (long)h * dv + p0 + p] = v[e];
+            }
+        };
         dfloatx4_t yt = zero4;
         if (owns) yt = dot_tile(Qs, tt, Ss, pt);
 #pragma unroll
         for (int e = 0; e < 4; ++e) yt[e] *= from_s[16 * tt + 4 * g + e] * fq_s[16 * tt + 4 * g + e];
+        const dfloatx4_t y0 = yt;
         __syncthreads();
         if (wave < PT) {
             // u of columns 16 wave .. + 15, 16 tokens after 16 tokens
-            float* u = uT + (16 * wave + r) * DCHUNK_LT + 4 * g;
+            const float* rhs_p = rT + (16 * wave + r) * DCHUNK_LT;
+            float* u_p = uT + (16 * wave + r) * DCHUNK_LT;
+            dfloatx4_t odd = zero4;
             for (int i = 0; i < 4; ++i) {
-                dfloatx4_t rhs = *(const dfloatx4_t*)(u + 16 * i);
+                dfloatx4_t rhs = *(const dfloatx4_t*)(rhs_p + 16 * i + 4 * g);
                 for (int j = 0; j < i; ++j) {
                     const dfloatx4_t a = *(const dfloatx4_t*)&As[(16 * i + r) * DCHUNK_LT + 16 * j + 4 * g];
-                    const dfloatx4_t x = *(const dfloatx4_t*)(u + 16 * j);
+                    const dfloatx4_t x = *(const dfloatx4_t*)(u_p + 16 * j + 4 * g);
 #pragma unroll
                     for (int e = 0; e < 4; ++e) rhs = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], x[e], rhs, 0, 0, 0);
                 }
@@ -394,8 +425,24 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
                 dfloatx4_t x = zero4;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) x = __builtin_amdgcn_mfma_f32_16x16x4f32(d[e], rhs[e], x, 0, 0, 0);
-                *(dfloatx4_t*)(u + 16 * i) = x;
+                *(dfloatx4_t*)(u_p + 16 * i + 4 * g) = x;
+                odd += x * 0.f;
                 __builtin_amdgcn_wave_barrier();
+            }
+            if (wave_odd(odd[0], odd[1], odd[2], odd[3])) {
+#pragma unroll 1
+                for (int t = 0; t < DCHUNK_T; ++t) {
+                    float sum = 0.f;
+#pragma unroll 1
+                    for (int s0 = 0; s0 < t; s0 += 4) {
+                        const float term = As[t * DCHUNK_LT + s0 + g] * u_p[s0 + g];
+                        sum += s0 + g < t ? term : 0.f;
+                    }
+                    sum += __shfl_xor(sum, 16, 64);
+                    sum += __shfl_xor(sum, 32, 64);
+                    if (g == 0) u_p[t] = rhs_p[t] + sum;
+                    __builtin_amdgcn_wave_barrier();
+                }
             }
         } else {
             for (int k = wave - PT; k < 10; k += 8 - PT) {
@@ -418,11 +465,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
 #pragma unroll
             for (int e = 0; e < 4; ++e) yt = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], u[e], yt, 0, 0, 0);
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int t = 16 * tt + 4 * g + e, p = 16 * pt + r;
-            if (owns && t < tn && p0 + p < dv) y[(long)(start + t0 + t) * heads * dv + (long)h * dv + p0 + p] = yt[e];
-        }
+        write_y(yt);
         // the state behind the chunk
         const float keep = from_s[DCHUNK_T - 1];
 #pragma unroll
@@ -439,6 +482,19 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
 #pragma unroll
                 for (int i = 0; i < PT; ++i) st[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(u4[i][e], kv, st[i], 0, 0, 0);
             }
+        }
+        if (wave_odd(yt[0], yt[1], yt[2], yt[3])) {
+            dfloatx4_t again = y0;
+#pragma unroll 1
+            for (int s = 0; s < DCHUNK_T; ++s) {
+                const float one = uT[(16 * pt + r) * DCHUNK_LT + s];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = 16 * tt + 4 * g + e;
+                    if (s <= t) again[e] += Gs[t * DCHUNK_LT + s] * one;
+                }
+            }
+            write_y(again);
         }
         __syncthreads();
     }

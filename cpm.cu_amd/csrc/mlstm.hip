@@ -229,6 +229,8 @@ __global__ __launch_bounds__(256) void mlstm_maximum_kernel(const float* __restr
 // where no exponent is positive; the normaliser is column dv, whose value is always 1, as in the walk.  A workgroup owns
 // one (sequence, head, 32 columns); its state stays in the accumulators' registers and passes through LDS as an operand.
 // 8 heads of 256 by 512, prompts of 613, 479, 211, 345 and 400 tokens in one pass: 870 -> 311 us.
+// A token's infinities reach no earlier token: their weights are zero, but a zero does not silence an infinity in a product,
+// so outputs that are not all finite are added up again term by term.
 // A lane's 16 bytes serve four instructions: instruction j of a block takes index 4 g + j of the 16 in both operands.
 // ---------------------------------------------------------------------------
 typedef float mlfloatx4_t __attribute__((ext_vector_type(4)));
@@ -322,6 +324,12 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
             for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) Ss[(16 * i + 4 * g + e) * LN + 16 * (NJ * wave + j) + r] = st[i][j][e];
+        if (tn < MCHUNK_T) {                                           // rows behind the run's end repeat its last token
+#pragma unroll
+            for (int i = 0; i < QK; ++i)
+                if ((int)(threadIdx.x + 512 * i) / C4 >= tn) rk[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (vrow >= tn) rv = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
 #pragma unroll
         for (int i = 0; i < QK; ++i) {
             const int e = threadIdx.x + 512 * i, at = (e / C4) * LN + (e % C4) * 4;
@@ -365,6 +373,16 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
         // wavefronts 0 to 2: the tiles of G on and below the diagonal; 3 to 6: what the state before the chunk gives tokens
         // 16 tt .. + 15 in columns 16 pt .. + 15
         const int tt = wave < 3 ? (wave + 1) / 2 : ((wave - 3) >> 1) & 1, pt = (wave - 3) & 1;
+        const bool owns = wave >= 3 && wave < 7;
+        auto write_y = [&](const mlfloatx4_t& v) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * tt + 4 * g + e, p = p0 + 16 * pt + r;
+                if (t >= tn) continue;
+                if (p < dv) y[(long)(start + t0 + t) * heads * dv + (long)h * dv + p] = v[e];
+                else if (p == dv) den[(long)(start + t0 + t) * heads + h] = fmaxf(fabsf(v[e]), floor_s[t]) + 1e-6f;
+            }
+        };
         mlfloatx4_t yt = zero4;
         if (wave < 3) {
             const int j = wave == 2 ? 1 : 0, s = 16 * j + r;
@@ -380,8 +398,9 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
 #pragma unroll
             for (int e = 0; e < 4; ++e) yt[e] *= from_s[16 * tt + 4 * g + e];
         }
+        const mlfloatx4_t y0 = yt;
         __syncthreads();
-        if (wave >= 3 && wave < 7) {
+        if (owns) {
             // ... and what the chunk's own tokens give them
             for (int kb = 0; kb <= tt; ++kb) {
                 const mlfloatx4_t a = *(const mlfloatx4_t*)&Gs[(16 * tt + r) * MCHUNK_LT + 16 * kb + 4 * g];
@@ -389,13 +408,7 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
 #pragma unroll
                 for (int e = 0; e < 4; ++e) yt = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], v[e], yt, 0, 0, 0);
             }
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int t = 16 * tt + 4 * g + e, p = p0 + 16 * pt + r;
-                if (t >= tn) continue;
-                if (p < dv) y[(long)(start + t0 + t) * heads * dv + (long)h * dv + p] = yt[e];
-                else if (p == dv) den[(long)(start + t0 + t) * heads + h] = fmaxf(fabsf(yt[e]), floor_s[t]) + 1e-6f;
-            }
+            write_y(yt);
         }
         // the state behind the chunk
         const float keep = from_s[MCHUNK_T - 1];
@@ -417,6 +430,19 @@ __global__ __launch_bounds__(512) void mlstm_chunk_kernel(const T* __restrict__ 
 #pragma unroll
                     for (int i = 0; i < 2; ++i) st[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(v4[i][e], kv, st[i][j], 0, 0, 0);
                 }
+        }
+        if (owns && wave_odd(yt[0], yt[1], yt[2], yt[3])) {
+            mlfloatx4_t again = y0;
+#pragma unroll 1
+            for (int s = 0; s < MCHUNK_T; ++s) {
+                const float one = vT[(16 * pt + r) * MCHUNK_LT + s];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = 16 * tt + 4 * g + e;
+                    if (s <= t) again[e] += Gs[t * MCHUNK_LT + s] * one;
+                }
+            }
+            write_y(again);
         }
         __syncthreads();
     }

@@ -346,6 +346,8 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(const float* __restrict__
 // is as good as the walk's product of factors.  A workgroup owns one (sequence, head, 32 columns of P); its state stays in
 // the accumulators' registers and passes through LDS as an operand.  The walk's cost is one dependent chain a token (0.35
 // us); a chunk takes 7.5 us: 128 heads of 64, state 128, 2,048 tokens 719 -> 241 us.
+// A token's infinities reach no earlier token: their weights in G are zero, but a zero does not silence an infinity in a
+// product, so outputs that are not all finite are added up again term by term.
 // A lane's 16 bytes serve four instructions: instruction j of a block takes index 4 g + j of the 16 in both operands.
 // ---------------------------------------------------------------------------
 typedef float sfloatx4_t __attribute__((ext_vector_type(4)));
@@ -389,7 +391,7 @@ __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict_
             const int p = 16 * i + 4 * g + e;
             st[i][e] = (p0 + p < P && n_own < N) ? sp[(long)p * N + n_own] : 0.f;
         }
-    const float A = expf(A_log[h]), bias = dt_bias[h], Dh = Dskip[h];
+    const float A = decay_rate(A_log[h]), bias = dt_bias[h], Dh = Dskip[h];
     const sfloatx4_t zero4 = {0.f, 0.f, 0.f, 0.f};
     sfloatx4_t rb[4], rc[4], rx;
     float rdt = 0.f;
@@ -419,6 +421,12 @@ __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict_
     for (int t0 = 0; t0 < q; t0 += CHUNK_T) {
         const int tn = min(CHUNK_T, q - t0);
         state_to_lds();
+        if (tn < CHUNK_T) {                                            // rows behind the run's end repeat its last token
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if ((int)(threadIdx.x + 512 * i) >> 5 >= tn) rb[i] = zero4;
+            if ((int)threadIdx.x >> 3 >= tn) rx = zero4;
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int e = threadIdx.x + 512 * i, at = (e >> 5) * CHUNK_LN + (e & 31) * 4;
@@ -430,7 +438,7 @@ __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict_
         if (wave == 0) {
             // a token beyond the end has d = 0: it neither writes nor forgets
             const float d = lane < tn ? softplus_f(rdt + bias) : 0.f;
-            double la = -(double)A * (double)d;
+            double la = -(double)A * (double)decay_step(d, A);
 #pragma unroll
             for (int k = 1; k < 64; k <<= 1) {
                 const double up = __shfl_up(la, k, 64);
@@ -466,6 +474,14 @@ __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict_
         }
         // tokens 16 tt .. + 15, columns 16 pt .. + 15: what the state before the chunk gives them
         const int tt = wave >> 1, pt = wave & 1;
+        auto write_y = [&](const sfloatx4_t& v) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * tt + 4 * g + e, p = 16 * pt + r;
+                if (t < tn && p0 + p < P)
+                    y[(long)(start + t0 + t) * inner + (long)h * P + p0 + p] = v[e] + Dh * xT[p * CHUNK_LT + t];
+            }
+        };
         sfloatx4_t yt = zero4;
 #pragma unroll
         for (int kb = 0; kb < NB; ++kb) {
@@ -476,6 +492,7 @@ __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict_
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) yt[e] *= from_s[16 * tt + 4 * g + e];
+        const sfloatx4_t y0 = yt;
         __syncthreads();
         // ... and what the chunk's own tokens give them
         for (int kb = 0; kb <= tt; ++kb) {
@@ -484,12 +501,7 @@ __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict_
 #pragma unroll
             for (int e = 0; e < 4; ++e) yt = __builtin_amdgcn_mfma_f32_16x16x4f32(g4[e], x4[e], yt, 0, 0, 0);
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int t = 16 * tt + 4 * g + e, p = 16 * pt + r;
-            if (t < tn && p0 + p < P)
-                y[(long)(start + t0 + t) * inner + (long)h * P + p0 + p] = yt[e] + Dh * xT[p * CHUNK_LT + t];
-        }
+        write_y(yt);
         // the state behind the chunk
         const float keep = from_s[CHUNK_T - 1];
 #pragma unroll
@@ -506,6 +518,19 @@ __global__ __launch_bounds__(512) void ssm_chunk_kernel(const float* __restrict_
 #pragma unroll
                 for (int i = 0; i < 2; ++i) st[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(x4[i][e], bv, st[i], 0, 0, 0);
             }
+        }
+        if (wave_odd(yt[0], yt[1], yt[2], yt[3])) {
+            sfloatx4_t again = y0;
+#pragma unroll 1
+            for (int s = 0; s < CHUNK_T; ++s) {
+                const float one = xT[(16 * pt + r) * CHUNK_LT + s];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = 16 * tt + 4 * g + e;
+                    if (s <= t) again[e] += Gs[t * CHUNK_LT + s] * one;
+                }
+            }
+            write_y(again);
         }
         __syncthreads();
     }

@@ -186,6 +186,93 @@ def test_runs_are_taken_by_their_length(kind, lens, chunk_from):
     assert all(bool(torch.isfinite(y).all()) for y in both[0])
 
 
+ODD = [("value", float("inf")), ("value", float("nan")), ("key", float("-inf")), ("key", float("nan")), ("query", float("inf")),
+       ("gate", float("nan")), ("gate", float("inf")), ("gate", float("-inf")), ("second gate", float("nan")), ("constant", 100.0),
+       ("constant", float("nan"))]
+
+
+@pytest.mark.parametrize("kind", ["ssm", "delta", "mlstm"])
+@pytest.mark.parametrize("what,odd", ODD)
+@pytest.mark.parametrize("at", [5, 77, 90, 130])
+def test_an_odd_token_reaches_what_the_walk_says(kind, what, odd, at):
+    """An infinity or a NaN (or a decay constant whose exponential is infinite) in one token of a prompt: the same outputs and
+    state values are finite as in the walk, and those have the walk's values; tokens before it see nothing of it, whether they
+    stand in its block of 16 tokens, in its chunk, or before; the last token among them, behind which a chunk's rest is empty."""
+    from cpmcu_amd import ops
+    n, H = 131, 2
+    g = torch.Generator(device=DEV).manual_seed(at)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    cu, slots = i32([0, n]), i32([1])
+    if kind == "ssm":
+        P, N, states = 36, 20, [rnd(2, H, 36, 20)]
+        xbc, dt, A, b, D = rnd(n, H * P + 2 * N), rnd(n, H), torch.log(0.05 + rnd(H).abs()), rnd(H), rnd(H)
+        place = {"value": (xbc, P + 3), "key": (xbc, H * P + 2), "query": (xbc, H * P + N + 7), "gate": (dt, 1)}
+        call = lambda y, st, m: ops.ssm_scan(xbc, dt, b, A, D, st[0], y[0], cu, slots, H, P, N, 1, max_q=m)
+        outs, constant = [(n, H, P)], A
+    elif kind == "delta":
+        dk, dv, states = 36, 20, [rnd(2, H, 20, 36)]
+        qkv, gates, A, b = rnd(n, 2 * H * dk + H * dv), rnd(n, 2 * H), torch.log(0.05 + rnd(H).abs()), rnd(H)
+        place = {"value": (qkv, 2 * H * dk + dv + 3), "key": (qkv, H * dk + dk + 2), "query": (qkv, dk + 7), "gate": (gates, 1),
+                 "second gate": (gates, H + 1)}
+        call = lambda y, st, m: ops.delta_scan(qkv, gates, 0, H, b, A, st[0], y[0], cu, slots, H, H, dk, dv, dk ** -0.5, max_q=m)
+        outs, constant = [(n, H, dv)], A
+    else:
+        d, dv, states = 36, 20, [rnd(2, H, 20, 36), rnd(2, H, 36), rnd(2, H)]
+        w = 2 * H * d + H * dv
+        proj, b = rnd(n, w + 2 * H), rnd(H)
+        place = {"value": (proj, 2 * H * d + dv + 3), "key": (proj, H * d + d + 2), "query": (proj, d + 7), "gate": (proj, w + 1),
+                 "second gate": (proj, w + H + 1)}
+        call = lambda y, st, m: ops.mlstm_scan(proj, 0, H * d, 2 * H * d, w, w + H, b, b, 9.0, d ** -0.5, *st, *y, cu, slots, H, d, dv, max_q=m)
+        outs, constant = [(n, H, dv), (n, H)], None
+    if what == "constant" and constant is None or what not in (*place, "constant"):
+        pytest.skip("this recurrence has none")
+
+    def both():
+        got = []
+        for m in (n, 0):
+            y, st = [torch.zeros(o, device=DEV) for o in outs], [s.clone() for s in states]
+            call([t.view(n, -1) for t in y], st, m)
+            got.append((y, st))
+        return got
+    clean = both()[0][0]
+    if what == "constant":
+        constant[1] = odd
+    else:
+        t, column = place[what]
+        t[at, column] = odd
+    (y, st), (walk_y, walk_st) = both()
+    if kind == "mlstm":                                              # its output is y / den
+        clean, y, walk_y = ([o[0] / o[1][..., None]] for o in (clean, y, walk_y))
+        st, walk_st = st[:2], walk_st[:2]
+    for a, b in [*zip(y, walk_y), *zip(st, walk_st)]:
+        assert bool((a.isfinite() == b.isfinite()).all())
+        # two float recurrences of sums of up to 131 tokens, keys of 36: 1e-4 of the largest value is far above their rounding
+        keep = b.isfinite()
+        assert float((a - b)[keep].abs().max()) <= 1e-4 * max(1.0, float(b[keep].abs().max()))
+    if what != "constant":
+        for a, b in zip(y, clean):
+            assert float((a[:at] - b[:at]).abs().max()) <= 1e-5 * max(1.0, float(b.abs().max()))
+
+
+@pytest.mark.parametrize("scale", [1e19, 1e25])
+def test_keys_whose_squares_overflow(scale):
+    """A key or query whose square overflows counts as zero in both forms of the delta rule."""
+    from cpmcu_amd import ops
+    n, H, dk, dv = 70, 2, 36, 20
+    g = torch.Generator(device=DEV).manual_seed(1)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    qkv, gates, A, b, state = rnd(n, 2 * H * dk + H * dv), rnd(n, 2 * H), rnd(H), rnd(H), rnd(1, H, dv, dk)
+    qkv[[3, 4, 66], H * dk:2 * H * dk] *= scale
+    qkv[[9, 67], :H * dk] *= scale
+    got = []
+    for m in (n, 0):
+        y, st = torch.full((n, H * dv), float("nan"), device=DEV), state.clone()
+        ops.delta_scan(qkv, gates, 0, H, b, A, st, y, i32([0, n]), i32([0]), H, H, dk, dv, dk ** -0.5, max_q=m)
+        got.append((y, st))
+    for a, w in zip(*got):
+        assert bool(w.isfinite().all()) and float((a - w).abs().max()) <= 1e-5 * float(w.abs().max())
+
+
 @pytest.mark.parametrize("lens,chunks", [([33, 32, 40, 37, 64], True), ([33, 32, 40, 37, 64], False), ([1] * 8, False)])
 def test_mlstm_of_more_workgroups_than_run_at_a_time(lens, chunks):
     """A carried state whose maxima differ from slot to slot and from those behind the step: every workgroup of a launch, the
