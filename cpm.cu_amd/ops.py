@@ -2231,6 +2231,20 @@ def attention_wide_prefill_ok(q: torch.Tensor, nh: int, nkv: int, hdk: int, hdv:
             and pool_hdk <= 576 and hdv % 4 == 0 and 128 < pool_hdv <= 512 and page_size % 32 == 0)
 
 
+def attention_wide_prefill_pays(n_tokens: int, nh: int, nkv: int, max_keys: int) -> bool:
+    """Whether a step is one where attention_wide_prefill is the faster kernel.  It is nearly everywhere; only few tokens of
+    few keys each (a short prompt alone), where attention_general_mfma's smaller workgroups are all in flight at once, have
+    less to wait for there.  Measured (us, general / wide; tokens + tokens of history):
+      32 heads on a latent of 576 / 512: 16 + 0 11.3/16.3, 64 + 0 13.9/16.6, 128 + 0 18.3/19.5, 256 + 0 33/26; 16 + 128 19.4/21.5, 128 + 64
+        22.6/22.1, 16 + 192 23.6/23.9, 16 + 256 28/27, 2 + 1,000 74/53, 16 + 8,000 752/357; 256 + 0 beside 7 x 1 + 4,000 405/182;
+      32 heads on 8 of 128 / 256: 16 + 0 7.4/9.9, 64 + 0 9.2/10.2, 128 + 0 16.9/11.5, 16 + 128 11.7/12.4, 16 + 1,000 44/31;
+      16 heads on 8: 32 + 0 8.3/9.6, 64 + 0 9.6/9.7, 2 + 128 12.1/10.2; 16 heads on 16: 16 + 0 7.9/7.4, 64 + 0 12.6/9.7, 2 + 0 7.7/8.4.
+    So the general kernel while its workgroups (16 heads of a token each) are at most two a CU and no token sees more than
+    160 keys; not for heads with keys of their own, whose workgroups there hold one head."""
+    group = nh // nkv
+    return group < 2 or n_tokens > 256 or n_tokens * nkv * -(-group // 16) > 512 or max_keys > 160
+
+
 def attention_wide_prefill(q: torch.Tensor, out: torch.Tensor, tiles: torch.Tensor, nh: int, nkv: int, hdk: int, hdv: int,
                            scale: float, kpool: torch.Tensor, vpool: torch.Tensor, page_table: torch.Tensor, page_size: int,
                            positions: torch.Tensor, tok_slot: torch.Tensor, chunk: int = 0, window: int = 0,
@@ -2312,7 +2326,8 @@ def attention_any(q, out, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, pa
             and kpool.shape[2] == nkv * hdk and v_share == 1 and not softcap and out.dtype == q.dtype):
         attention(q, out, nh, nkv, hdk, scale, kpool, vpool, page_table, page_size, ctx)
         return False
-    if not ctx.single_token and attention_wide_prefill_ok(q, nh, nkv, hdk, hdv, kpool.shape[2] // nkv, pool_hdv, page_size):
+    if (not ctx.single_token and attention_wide_prefill_ok(q, nh, nkv, hdk, hdv, kpool.shape[2] // nkv, pool_hdv, page_size)
+            and attention_wide_prefill_pays(q.shape[0], nh, nkv, min(ctx.max_pos + 1, chunk or window + keep_first or 1 << 30))):
         per = ATTENTION_WIDE_COLUMNS * nkv // nh
         key = ("prefill_tiles", per)
         tiles = ctx.extras.get(key)

@@ -115,3 +115,45 @@ def test_weights_round_no_worse_than_token_by_token(spread):
     want = torch.matmul(torch.softmax(s, -1), v[:, 0].double()).transpose(0, 1).reshape(L, -1)
     off = [float((x.double().cpu() - want).norm()) for x in (wide, general)]
     assert off[0] <= 1.05 * off[1], off
+
+
+@pytest.mark.parametrize("nh,nkv,spans,wide", [(32, 1, [(0, 160)], False), (32, 1, [(0, 161)], True), (32, 1, [(120, 160), (0, 1)], False),
+                                               (32, 1, [(130, 170), (0, 1)], True), (8, 2, [(0, 64)] * 4, False), (8, 2, [(0, 65)] * 4, True),
+                                               (32, 1, [(0, 100)] * 2 + [(0, 57)], True), (4, 4, [(0, 8)], True)])
+def test_few_tokens_of_few_keys_take_the_general_kernel(nh, nkv, spans, wide, monkeypatch):
+    """Both sides of the rule's borders (keys, workgroups, tokens, heads a kv head), each right."""
+    from types import SimpleNamespace
+    from cpmcu_amd import ops
+    hdk, hdv, page = 128, 256, 64
+    g = torch.Generator().manual_seed(sum(b for _, b in spans))
+    width = max(-(-b // page) for _, b in spans)
+    table = torch.arange(width * len(spans), dtype=torch.int32).view(len(spans), width)
+    pools, kept = [], []
+    for hd, keys in ((hdk, True), (hdv, False)):
+        pool = torch.zeros(len(spans), width * page * nkv * hd, dtype=torch.bfloat16)
+        rows = [torch.randn(b, nkv, hd, generator=g).to(torch.bfloat16) for _, b in spans]
+        for s, x in enumerate(rows):
+            pool[s, element_order(len(x), nkv, hd, keys).flatten()] = x.flatten()
+        pools.append(pool.view(-1, page, nkv * hd).to(DEV))
+        kept.append(rows)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    ctx = SimpleNamespace(single_token=False, max_pos=max(b for _, b in spans) - 1, q_lens=[b - a for a, b in spans], extras={},
+                          positions=i32([t for a, b in spans for t in range(a, b)]),
+                          tok_slot=i32([s for s, (a, b) in enumerate(spans) for _ in range(a, b)]))
+    n = sum(ctx.q_lens)
+    q, out = torch.randn(n, nh, hdk, generator=g).to(torch.bfloat16), torch.full((n, nh * hdv), float("nan"), device=DEV)
+    called = []
+    for name in ("attention_wide_prefill", "attention_general_mfma"):
+        monkeypatch.setattr(ops, name, lambda *a, _f=getattr(ops, name), _n=name, **k: (called.append(_n), _f(*a, **k)))
+    ops.attention_any(q.view(n, -1).to(DEV), out, nh, nkv, hdk, hdv, hdk ** -0.5, *pools, table.to(DEV), page, ctx)
+    assert called == ["attention_wide_prefill" if wide else "attention_general_mfma"]
+    at = 0
+    for s, (a, b) in enumerate(spans):
+        k, v = (x[s].double().repeat_interleave(nh // nkv, 1) for x in kept)
+        sc = torch.einsum("thd,jhd->htj", q[at:at + b - a].double(), k) * hdk ** -0.5
+        sc.masked_fill_(torch.arange(b)[None] > torch.arange(a, b)[:, None], -math.inf)
+        w = torch.softmax(sc, -1)
+        want, size = (torch.einsum("htj,jhd->thd", w, x) for x in (v, v.abs()))
+        got = out[at:at + b - a].double().cpu().view(b - a, nh, hdv)
+        assert bool(((got - want).abs() <= 2.0 ** -8 * size + 1e-5).all()), s          # weights rounded to 8 bits
+        at += b - a
