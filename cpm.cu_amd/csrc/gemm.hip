@@ -485,6 +485,24 @@ __global__ __launch_bounds__(256) void gemm_heads_tile_kernel(const bf16_t* __re
     }
 }
 
+// Whether tiles of 128 x 128 are the faster ones: where there is one for every CU, features enough to pay for the two
+// barriers a piece, and rows and columns that fill them.  What fills them is how many 64 x 64 tiles they replace, four
+// each at most.  Measured (us, tiles of 64 / of 128; heads, rows: columns x features):
+//   4       256, 128: 128 x 128 15.5/10.6   64, 512: 128 x 64 9.7/9.8   16, 2,048: 512 x 128 43/25   32, 2,048: 512 x 32 28/37
+//   3       256, 65: 192 x 256 30/15   64, 160: 512 x 128 20.6/14.5   128, 160: 256 x 64 13.2/11.2   256, 160: 512 x 64 34/39
+//           with 256 tiles: 32, 160: 512 x 128 10.2/10.6   128, 65: 136 x 128 8.1/9.9   128, 128: 192 x 256 20/13
+//   2, 1.5  256, 64: 128 x 512 24/17   256, 65: 64 x 512 23/15   256, 64: 192 x 256 20/15   256, 24: 192 x 256 11.2/11.0
+//           256, 17: 192 x 256 10.6/10.9   256, 64: 128 x 128 9.0/9.8   128, 136: 136 x 128 14/13
+//   1       256, 64: 64 x 512 13.5/14.7   256, 17: 8 x 8 3.7/4.3
+static bool heads_in_tiles(int M, int H, int N, int K) {
+    const auto up = [](int a, int b) { return (long)((a + b - 1) / b); };
+    const long tiles = up(M, 128) * up(N, 128) * H, small = up(M, 64) * up(N, 64) * H;
+    if (tiles < 256 || M < 24 || N < 64 || K < 64) return false;
+    if (small == 4 * tiles) return true;
+    if (K >= 256) return 2 * small >= 3 * tiles;
+    return small >= 3 * tiles && tiles >= 512 && (K >= 128 || tiles < 1024);
+}
+
 extern "C" const char* cpmcu_gemm_nt_heads_mfma(const void* X, long ldx, long hsx, const void* W, void* Y, long ldy,
                                                 long hsy, const void* gate, long ldg, int gate_wide, int M, int H, int N,
                                                 int K, hipStream_t stream) {
@@ -499,14 +517,13 @@ extern "C" const char* cpmcu_gemm_nt_heads_mfma(const void* X, long ldx, long hs
         dim3 grid((N + 63) / 64, 1, H);
         gemm_heads_mfma_kernel<1, 1><<<grid, 256, 0, stream>>>((const bf16_t*)X, ldx, hsx, (const bf16_t*)W, (bf16_t*)Y, ldy,
                                                                hsy, (const bf16_t*)gate, ldg, gate && gate_wide, M, N, K);
-    } else if ((long)((M + 127) / 128) * ((N + 127) / 128) * H >= 256) {
+    } else if (heads_in_tiles(M, H, N, K)) {
         dim3 grid((N + 127) / 128, (M + 127) / 128, H);
         CPMCU_REQUIRE(grid.y <= 65535, "gemm_heads_mfma: M=%d too large for one launch", M);
         const int pairs = ldy % 4 == 0 && hsy % 4 == 0 && (uintptr_t)Y % 8 == 0;
         gemm_heads_tile_kernel<<<grid, 256, 0, stream>>>((const bf16_t*)X, ldx, hsx, (const bf16_t*)W, (bf16_t*)Y, ldy, hsy,
                                                          (const bf16_t*)gate, ldg, gate && gate_wide, M, N, K, pairs);
     } else {
-        // fewer tiles of 128 than CUs: tiles of 64, four times as many
         dim3 grid((N + 63) / 64, (M + 63) / 64, H);
         CPMCU_REQUIRE(grid.y <= 65535, "gemm_heads_mfma: M=%d too large for one launch", M);
         gemm_heads_mfma_kernel<4, 4><<<grid, 256, 0, stream>>>((const bf16_t*)X, ldx, hsx, (const bf16_t*)W, (bf16_t*)Y, ldy,

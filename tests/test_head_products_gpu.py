@@ -7,7 +7,12 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-@pytest.mark.parametrize("H,M,N,K", [(256, 17, 8, 8), (64, 130, 129, 72), (128, 129, 6, 128), (32, 1024, 132, 64), (256, 128, 127, 200)])
+@pytest.mark.parametrize("H,M,N,K", [(256, 17, 8, 8), (64, 130, 129, 72), (128, 129, 6, 128), (32, 1024, 132, 64), (256, 128, 127, 200),
+                                     # in tiles of 128: full ones, whose last columns or features end inside a piece ...
+                                     (256, 65, 72, 72), (16, 2000, 127, 64), (128, 128, 250, 136),
+                                     # ... three quarters, half and fewer, and beside each what stays in tiles of 64
+                                     (64, 130, 510, 128), (32, 130, 510, 128), (64, 300, 131, 280), (128, 129, 67, 264), (256, 24, 128, 256),
+                                     (256, 23, 128, 256), (256, 64, 64, 256)])
 @pytest.mark.parametrize("gate", [None, "head", "feature"])
 @pytest.mark.parametrize("odd", [False, True])
 def test_head_products_at_tile_edges(H, M, N, K, gate, odd):
