@@ -625,9 +625,21 @@ extern "C" const char* cpmcu_attention_general_mfma(const void* q, void* out, in
 // The running maximum follows every move, so that a column's largest weight is 1, which 16 bits hold, and the sum is that of
 // the rounded weights; a maximum that only follows moves by more than 8 powers of two saves 10 us of the first and has up to
 // 2.3 times the error where few keys hold most of the weight.
+// A round's values are multiplied for all columns, with weights of zero where a column does not see the key; a zero does not
+// silence an infinity or NaN there, so a column that is not finite though its weights' sum is finite is added up again over
+// the keys it sees.
 // PK: up to 64 PK key features (EXACT: so many); DTW: up to 128 DTW value features.
 // ===========================================================================
 typedef unsigned gu32x4_t __attribute__((ext_vector_type(4)));
+
+// What only the sums over again need: kept in LDS, since scalar registers that live across the loop would spill there
+// (2,048 tokens, 32 heads over a latent: 230 us, 283 from registers; 229 without these sums).
+struct WideLate {
+    const bf16_t *q, *kpool, *vtpool;
+    PagedView pv;
+    int hdk, pool_hdk, pool_hdv, nkv, v_share, chunk, window, keep_first, slot, ckeep, cfirst, total;
+    float scale_log2e, cap_in, cap_out;
+};
 
 template <int PK, int DTW, bool EXACT>
 __global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
@@ -640,6 +652,7 @@ __global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
     __shared__ gu32x4_t keys_s[512 * PK];                         // [half][tile of 16 keys][32 features][lane]
     __shared__ gbf16x8_t p_s[4][2][64];                            // weights [column tile][half][lane]
     __shared__ float top_s[2][64], sum_s[2][64];                   // a column's largest score of a half; at the end its sums
+    __shared__ WideLate late_s;
     const int tile = gridDim.x - 1 - blockIdx.x;                   // later tiles of a prompt see more keys: they start first
     const int kvh = blockIdx.y;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -656,6 +669,9 @@ __global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
     const int first_max = chunk > 0 ? pos_max - pos_max % chunk : (window > 0 ? max(pos_max - window + 1, 0) : 0);
     const int cfirst = first_min >> 5, ckeep = min((keep_first + 31) >> 5, cfirst);
     const int total = ckeep + (pos_max >> 5) + 1 - cfirst, rounds = (total + 1) / 2;
+    if (threadIdx.x == 0)
+        late_s = {q, kpool, vtpool, pv, hdk, pool_hdk, pool_hdv, nkv, v_share, chunk, window, keep_first, slot, ckeep, cfirst, total,
+                  scale_log2e, cap_in, cap_out};
 
     gbf16x8_t qf[KS];
     {
@@ -786,14 +802,22 @@ __global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
     if (g == 0) sum_s[kh][ct * 16 + n] = l;
     __syncthreads();
     // lane (column n of tile k, g): acc[d][k][i] is value feature (wave * DTW + d) * 16 + 4 g + i
+    unsigned long long again = 0;                                  // bit c: column c is to be added up again
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
-        if ((k * 16 + n) / G >= n_tok) continue;
+        const bool live = (k * 16 + n) / G < n_tok;
         const long t = t0 + token_of(k);
         const int head = head_of(k);
         float total_l = sum_s[0][k * 16 + n] + sum_s[1][k * 16 + n];
         if (sink) total_l += exp2f(sink[head] * 1.4426950408889634f - m[k]);
         const float inv = 1.0f / total_l;
+        float odd = 0.f;
+#pragma unroll
+        for (int d = 0; d < DTW; ++d) odd += acc[d][k][0] * 0.f + acc[d][k][1] * 0.f + acc[d][k][2] * 0.f + acc[d][k][3] * 0.f;
+        unsigned long long bad = __builtin_amdgcn_ballot_w64(live && odd != 0.f && total_l * 0.f == 0.f);
+        bad |= bad >> 32;
+        again |= ((bad | bad >> 16) & 0xffff) << (16 * k);
+        if (!live) continue;
 #pragma unroll
         for (int d = 0; d < DTW; ++d) {
             const int f = (wave * DTW + d) * 16 + 4 * g;
@@ -808,6 +832,44 @@ __global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
             if (out_f32) store4((float*)out + at, v[0], v[1], v[2], v[3]);
             else store4((bf16_t*)out + at, v[0], v[1], v[2], v[3]);
         }
+    }
+    if (!again) return;
+    __builtin_amdgcn_s_waitcnt(0);                                 // what is stored below comes behind the stores above
+    const WideLate a = late_s;
+    for (; again; again &= again - 1) {
+        const int col = (int)__builtin_ctzll(again);
+        const long t1 = t0 + col / G;
+        const int pos1 = pos_min + col / G, head1 = kvh * G + col % G;
+        const int first1 = a.chunk > 0 ? pos1 - pos1 % a.chunk : (a.window > 0 ? max(pos1 - a.window + 1, 0) : 0);
+        const float m_of = col < 16 ? m[0] : (col < 32 ? m[1] : (col < 48 ? m[2] : m[3]));
+        const float m1 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(m_of), col & 15));
+        float l1 = sum_s[0][col] + sum_s[1][col];
+        if (sink) l1 += exp2f(sink[head1] * 1.4426950408889634f - m1);
+        const int f = wave * DTW * 16 + lane;                       // this lane's feature
+        const bool mine = lane < DTW * 16 && f < hdv;
+        const bf16_t* q1 = a.q + (t1 * nh + head1) * a.hdk;
+        float o = 0.f;
+        for (int c = 0; c < a.total; ++c) {
+            const int key0 = (c < a.ckeep ? c : a.cfirst + (c - a.ckeep)) << 5;
+            const long row0 = paged_row(a.pv, a.slot, key0);
+            for (int i = 0; i < 32; ++i) {
+                const int key = key0 + i;
+                if (key > pos1 || (key < first1 && key >= a.keep_first)) continue;
+                const bf16_t* k1 = a.kpool + key_index(row0 + i, kvh, a.nkv, a.pool_hdk);
+                float s = 0.f;
+                for (int d = lane; d < a.hdk; d += 64) s += to_f32(q1[d]) * to_f32(k1[key_d_offset(d)]);
+                s = wave_sum(s);
+                if (a.cap_out > 0.f) s = a.cap_out * tanhf(s * a.cap_in);
+                const float p = to_f32(f32_to_bf16(__builtin_amdgcn_exp2f(__builtin_fmaf(s, a.scale_log2e, -m1))));
+                if (mine) o += p * to_f32(a.vtpool[value_index(row0 + i, kvh / a.v_share, a.nkv / a.v_share, a.pool_hdv) + value_d_offset(f)]);
+            }
+        }
+        if (!mine) continue;
+        o /= l1;
+        if (gate) o /= 1.0f + expf(-to_f32(gate[t1 * ld_gate + (long)head1 * hdv + f]));
+        const long at = (t1 * nh + head1) * hdv + f;
+        if (out_f32) ((float*)out)[at] = o;
+        else ((bf16_t*)out)[at] = f32_to_bf16(o);
     }
 }
 

@@ -157,3 +157,49 @@ def test_few_tokens_of_few_keys_take_the_general_kernel(nh, nkv, spans, wide, mo
         got = out[at:at + b - a].double().cpu().view(b - a, nh, hdv)
         assert bool(((got - want).abs() <= 2.0 ** -8 * size + 1e-5).all()), s          # weights rounded to 8 bits
         at += b - a
+
+
+@pytest.mark.parametrize("nh,nkv,hdk,hdv,opt", [(32, 1, 576, 512, {}), (8, 2, 128, 256, {"window": 40, "keep_first": 3, "gate": True}),
+                                                (4, 4, 72, 132, {"sink": True, "softcap": 4.0}), (2, 1, 192, 512, {"chunk": 48, "out": torch.bfloat16})])
+def test_infinities_reach_only_tokens_that_see_them(nh, nkv, hdk, hdv, opt):
+    """Infinities and NaNs among the values of some tokens: tokens before them, or behind their window or chunk, have the
+    results that they have without; the others what the sum over the keys that they see gives."""
+    from cpmcu_amd import ops
+    L, page, G = 203, 64, nh // nkv
+    pool_hdk, pool_hdv, pages = -(-hdk // 64) * 64, -(-hdv // 16) * 16, 4
+    g = torch.Generator().manual_seed(hdk)
+    k, v = (torch.randn(L, nkv, hd, generator=g).to(torch.bfloat16) for hd in (hdk, hdv))
+    for t, f, value in ((37, 5, math.inf), (38, 5, -math.inf), (90, hdv - 1, -math.inf), (91, 64, math.nan), (202, 0, math.inf)):
+        v[t, t % nkv, f] = value
+    q = torch.randn(L, nh, hdk, generator=g).to(torch.bfloat16)
+    pools = []
+    for x, hd, keys in ((k, pool_hdk, True), (v, pool_hdv, False)):
+        flat = torch.full((pages * page * nkv * hd,), 0.0, dtype=torch.bfloat16)
+        flat[element_order(L, nkv, hd, keys)[..., :x.shape[-1]].flatten()] = x.flatten()
+        pools.append(flat.view(pages, page, -1).to(DEV))
+    dev = lambda t: None if t is None else t.to(DEV)
+    sink = torch.randn(nh, generator=g) if opt.get("sink") else None
+    gate = torch.randn(L, nh * hdv, generator=g).to(torch.bfloat16) if opt.get("gate") else None
+    chunk, window, keep, cap = (opt.get(t, 0) for t in ("chunk", "window", "keep_first", "softcap"))
+    pos = torch.arange(L, dtype=torch.int32)
+    out = torch.full((L, nh * hdv), 7.0, dtype=opt.get("out", torch.float32), device=DEV)
+    ops.attention_wide_prefill(dev(q.view(L, -1)), out, ops.prefill_tiles([L], 64 // G, DEV), nh, nkv, hdk, hdv, hdk ** -0.5, *pools,
+                               torch.arange(pages, dtype=torch.int32, device=DEV)[None], page, dev(pos), dev(torch.zeros_like(pos)),
+                               chunk, window, keep, dev(sink), 1, dev(gate), float(cap))
+    got = out.double().cpu().view(L, nh, hdv)
+    kd, vd, j = k.double().repeat_interleave(G, 1), v.double().repeat_interleave(G, 1), torch.arange(L)
+    for t in range(L):
+        sees = (j <= t) & ((j // chunk == t // chunk) if chunk else ((t - j < window) | (j < keep)) if window else True)
+        sc = torch.einsum("hd,jhd->hj", q[t].double(), kd[sees]) * hdk ** -0.5
+        sc = cap * torch.tanh(sc / cap) if cap else sc
+        if sink is not None:
+            sc = torch.cat([sc, sink.double()[:, None]], 1)
+        w = torch.softmax(sc, -1)[:, :int(sees.sum()), None]
+        terms = w * vd[sees].transpose(0, 1)
+        want, size = terms.sum(1), terms.abs().sum(1)
+        if gate is not None:
+            s_g = torch.sigmoid(gate[t].double().view(nh, hdv))
+            want, size = want * s_g, size * s_g
+        fine = torch.isfinite(want)
+        assert torch.equal(got[t].isnan(), want.isnan()) and torch.equal(got[t][~fine].nan_to_num(0.0), want[~fine].nan_to_num(0.0)), t
+        assert bool(((got[t] - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-5)[fine].all()), t
