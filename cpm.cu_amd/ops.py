@@ -2326,7 +2326,9 @@ def attention_any(q, out, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, pa
             and kpool.shape[2] == nkv * hdk and v_share == 1 and not softcap and out.dtype == q.dtype):
         attention(q, out, nh, nkv, hdk, scale, kpool, vpool, page_table, page_size, ctx)
         return False
+    # (operands off 16-byte borders, which the kernel for wide values refuses, are the general kernel's)
     if (not ctx.single_token and attention_wide_prefill_ok(q, nh, nkv, hdk, hdv, kpool.shape[2] // nkv, pool_hdv, page_size)
+            and (q.data_ptr() | out.data_ptr() | kpool.data_ptr() | vpool.data_ptr()) % 16 == 0
             and attention_wide_prefill_pays(q.shape[0], nh, nkv, min(ctx.max_pos + 1, chunk or window + keep_first or 1 << 30))):
         per = ATTENTION_WIDE_COLUMNS * nkv // nh
         key = ("prefill_tiles", per)

@@ -203,3 +203,26 @@ def test_infinities_reach_only_tokens_that_see_them(nh, nkv, hdk, hdv, opt):
         fine = torch.isfinite(want)
         assert torch.equal(got[t].isnan(), want.isnan()) and torch.equal(got[t][~fine].nan_to_num(0.0), want[~fine].nan_to_num(0.0)), t
         assert bool(((got[t] - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-5)[fine].all()), t
+
+
+def test_outputs_off_16_byte_borders_take_the_general_kernel():
+    from types import SimpleNamespace
+    from cpmcu_amd import ops
+    L, hdk, hdv, page = 200, 64, 132, 64
+    g = torch.Generator().manual_seed(5)
+    k, v, q = (torch.randn(L, 1, hd, generator=g).to(torch.bfloat16) for hd in (hdk, hdv, hdk))
+    pools = []
+    for x, hd, keys in ((k, hdk, True), (v, 144, False)):
+        flat = torch.zeros(4 * page * hd, dtype=torch.bfloat16)
+        flat[element_order(L, 1, hd, keys)[..., :x.shape[-1]].flatten()] = x.flatten()
+        pools.append(flat.view(4, page, -1).to(DEV))
+    pos = torch.arange(L, dtype=torch.int32, device=DEV)
+    ctx = SimpleNamespace(single_token=False, max_pos=L - 1, q_lens=[L], extras={}, positions=pos, tok_slot=torch.zeros_like(pos))
+    out = torch.zeros(L + 1, hdv, dtype=torch.bfloat16, device=DEV)[1:]                 # 264 bytes on
+    ops.attention_any(q.view(L, -1).to(DEV), out, 1, 1, hdk, hdv, 0.1, *pools, torch.arange(4, dtype=torch.int32, device=DEV)[None],
+                      page, ctx)
+    s = 0.1 * q[:, 0].double() @ k[:, 0].double().T
+    w = torch.softmax(s.masked_fill(torch.ones(L, L, dtype=torch.bool).triu(1), -math.inf), -1)
+    want, size = w @ v[:, 0].double(), w @ v[:, 0].double().abs()
+    # weights rounded to bf16 against values of that size, and the output's own rounding
+    assert bool(((out.double().cpu() - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-5).all())
