@@ -575,8 +575,8 @@ extern "C" const char* cpmcu_moe_down(const void* act, int dtype, const void* wd
 // product with its expert's weights.
 //
 //  * moe_group_kernel (one workgroup): counts the pairs of every expert and lists them expert by expert: rows[offs[e] ..
-//    offs[e + 1]) are expert e's pairs, tile_expert[tile] = e + 1024 * (the tile's number among its expert's), offs[E + 1]
-//    the number of tiles; n_tiles is what tiles of MOE_TILE rows would need, the rest of whose rows hold -1.  Which row of its expert's tiles a pair gets depends on timing; its result does not (a row's sums
+//    offs[e + 1]) are expert e's pairs, tile_expert[tile] = e + 1024 * (the tile's number among its expert's), n_tiles the
+//    number of tiles.  Which row of its expert's tiles a pair gets depends on timing; its result does not (a row's sums
 //    are its own).
 //  * moe_tile_kernel: GATED act[pair] = act(Wg_e h_t) * (Wu_e h_t), PLAIN act[pair] = act(Wu_e h_t), DOWN y[pair] =
 //    Wd_e act[pair] (bf16).
@@ -591,13 +591,12 @@ enum { MOE_GATED = 0, MOE_PLAIN = 1, MOE_DOWN = 2 };
 
 // tile_rows: rows a tile at most; an expert's pairs are spread evenly over as few tiles as hold them (moe_tile_kernel)
 __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__ idx, int n_pairs, int E, int tile_rows,
-                                                         int* __restrict__ rows, int* __restrict__ offs, int behind,
-                                                         int* __restrict__ tile_expert, int* __restrict__ n_tiles_out) {
+                                                         int* __restrict__ rows, int* __restrict__ offs,
+                                                         int* __restrict__ tile_expert, int* __restrict__ n_tiles) {
     __shared__ int counts[MOE_MAX_EXPERTS];
-    __shared__ int pair_sum[16], tile_sum[16], whole, placed;
+    __shared__ int pair_sum[16], tile_sum[16];
     const int e = threadIdx.x, lane = e & 63, wave = e >> 6;
     counts[e] = 0;
-    if (e == 0) whole = 0;
     __syncthreads();
     for (int p = threadIdx.x; p < n_pairs; p += 1024)
         if (idx[p] < E) atomicAdd(&counts[idx[p]], 1);              // identity experts have no tiles
@@ -605,7 +604,6 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
     // running sums of pairs and tiles over the experts, one expert a thread
     const int c = counts[e], nt = (c + tile_rows - 1) / tile_rows;
     int pairs = c, tiles = nt;
-    if (c) atomicAdd(&whole, (c + MOE_TILE - 1) / MOE_TILE);
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
         const int a = __shfl_up(pairs, d, 64), b = __shfl_up(tiles, d, 64);
@@ -627,15 +625,12 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
         offs[e] = pairs - c;
         if (e == E - 1) {
             offs[E] = pairs;
-            offs[E + 1] = tiles;
+            *n_tiles = tiles;
         }
         for (int i = 0; i < nt; ++i) tile_expert[tiles - nt + i] = e + 1024 * i;
     }
-    if (e == 0) *n_tiles_out = whole;
     counts[e] = pairs - c;
-    if (e == E - 1) placed = pairs;
     __syncthreads();
-    for (int i = placed + threadIdx.x; i < min(whole * MOE_TILE, behind); i += 1024) rows[i] = -1;
     for (int p = threadIdx.x; p < n_pairs; p += 1024) {
         const int x = idx[p];
         if (x < E) rows[atomicAdd(&counts[x], 1)] = p;
@@ -660,12 +655,12 @@ template <int KIND, int RT>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restrict__ in, long ldi,
                                                           const bf16_t* __restrict__ w, const int* __restrict__ rows,
                                                           const int* __restrict__ offs, const int* __restrict__ tile_expert,
-                                                          int E, bf16_t* __restrict__ out, int K, int N, int top, int act_fn,
+                                                          const int* __restrict__ n_tiles, bf16_t* __restrict__ out, int K, int N, int top, int act_fn,
                                                           float act_limit) {
     constexpr int BM = 16 * RT, FEATURES = KIND == MOE_GATED ? 64 : 128;
     __shared__ mu32x4_t lds[2][(BM + 128) * 8];
     const int nts = (N + FEATURES - 1) / FEATURES;
-    const int tasks = offs[E + 1] * nts, per = (tasks + 7) / 8;
+    const int tasks = *n_tiles * nts, per = (tasks + 7) / 8;
     const int task = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
     if ((int)(blockIdx.x >> 3) >= per || task >= tasks) return;
     const int q = task / nts, te = tile_expert[q], e = te & 1023;
@@ -844,7 +839,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16_t* __restri
     }
 }
 
-// scratch: rows int [max_tiles * 64] (the pairs by expert; at its end the experts' offsets), tile_expert int [max_tiles], n_tiles int [1], y bf16 [n * top, H];
+// scratch: rows int [max_tiles * 64] (the pairs by expert; its last E + 1 words are the experts' offsets), tile_expert int
+// [max_tiles], n_tiles int [1], y bf16 [n * top, H];
 // max_tiles = ceil(n * top / 64) + E
 extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const void* wgu, const void* wd, const int* idx,
                                               const float* w, const void* shared, int shared_dtype, int shared_parts,
@@ -864,15 +860,20 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     const long pairs = (long)n * top;
     CPMCU_REQUIRE(max_tiles >= (pairs + MOE_TILE - 1) / MOE_TILE + E && max_tiles <= 65535,
                   "moe_experts_mfma: %d tiles of scratch for %ld pairs of %d experts (at most 65535)", max_tiles, pairs, E);
-    // Tiles of 128 rows where experts have many; the scratch is sized for tiles of 64: it holds the pairs without gaps and,
-    // at its end, the experts' offsets.
+    // Tiles of 128 rows where experts have many: from 56 pairs an expert on most have more than one tile of 64, whose weights
+    // come twice.  Both products and the sum in us, tiles of 64 / 128 at 32, 48, 56, 64, 96, 192 pairs an expert:
+    //   64 experts of 1,408 at width 4,096  401/446  432/452  479/470  573/482  782/541  1,257/765
+    //   64 experts of 2,112 at width 4,096  567/624  615/649  633/658  858/678  1,137/749  1,856/1,096
+    //   16 experts of 512 at width 1,024    32/30  35/32  35/35  36/38  36/43  49/47
+    // The line lies where an uneven choice of experts, as routers make it, has crossed over.
+    // The scratch is sized for tiles of 64: it holds the pairs without gaps and, at its end, the experts' offsets.
     const bool wide = pairs >= 48L * E;
     const int tile_rows = wide ? 2 * MOE_TILE : MOE_TILE;
     const long tiles = (pairs + tile_rows - 1) / tile_rows + E;
-    const long behind = (long)max_tiles * MOE_TILE - (E + 2);         // pairs <= behind: max_tiles covers 64 E rows more
+    const long behind = (long)max_tiles * MOE_TILE - (E + 1);         // pairs <= behind: max_tiles covers 64 E rows more
     int* offs = rows + behind;
     CPMCU_REQUIRE(pairs <= behind && (long)max_tiles * MOE_TILE < (1L << 31), "moe_experts_mfma: scratch of %d tiles for %ld pairs", max_tiles, pairs);
-    moe_group_kernel<<<1, 1024, 0, stream>>>(idx, (int)pairs, E, tile_rows, rows, offs, (int)behind, tile_expert, n_tiles);
+    moe_group_kernel<<<1, 1024, 0, stream>>>(idx, (int)pairs, E, tile_rows, rows, offs, tile_expert, n_tiles);
     CPMCU_LAUNCH_CHECK("moe_group");
 #define TILES(KIND, in, ldi, w, out, K, N, act, limit)                                                                    \
     do {                                                                                                                      \
@@ -880,10 +881,10 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
         CPMCU_REQUIRE(blocks < (1L << 31), "moe_experts_mfma: %ld workgroups exceed the launch grid", blocks);                 \
         if (wide)                                                                                                             \
             moe_tile_kernel<KIND, 8><<<(unsigned)blocks, 256, 0, stream>>>(in, ldi, (const bf16_t*)(w), rows, offs, tile_expert, \
-                                                                               E, (bf16_t*)(out), K, N, top, act, limit);         \
+                                                                               n_tiles, (bf16_t*)(out), K, N, top, act, limit);         \
         else                                                                                                                  \
             moe_tile_kernel<KIND, 4><<<(unsigned)blocks, 256, 0, stream>>>(in, ldi, (const bf16_t*)(w), rows, offs, tile_expert, \
-                                                                               E, (bf16_t*)(out), K, N, top, act, limit);         \
+                                                                               n_tiles, (bf16_t*)(out), K, N, top, act, limit);         \
     } while (0)
     if (gated) TILES(MOE_GATED, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
     else TILES(MOE_PLAIN, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);

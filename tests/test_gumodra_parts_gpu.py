@@ -368,7 +368,7 @@ def test_experts(dtype, shape):
 @pytest.mark.parametrize("shape", [(96, 40, 8, 3, 300), (104, 24, 6, 2, 65), (64, 24, 5, 1, 700), (128, 72, 12, 4, 1000),
                                    (256, 136, 40, 6, 129)])
 def test_experts_of_many_tokens_on_the_matrix_cores(shape):
-    """Pairs grouped by expert in tiles of 64 rows: equal to the few-token kernels pair by pair, whatever row of a
+    """Pairs grouped by expert in tiles of 64 or 128 rows: equal to the few-token kernels pair by pair, whatever row of a
     tile a pair lands in; experts that nobody chose, experts with more than a tile of tokens, a last tile partly
     empty."""
     from cpmcu_amd import ops
@@ -403,10 +403,16 @@ def test_experts_of_many_tokens_on_the_matrix_cores(shape):
         ops.moe_experts_mfma(hd, gud, dnd, idxd, wd, out, act2, y, rows, te, nt, dev(shared), dev(sgate))
         close(act2, act.float().cpu(), "bfloat16")
         close(out, want.cpu(), "bfloat16")
-    counts = torch.bincount(idx.flatten().long(), minlength=E)
-    assert int(nt) == int(((counts + 63) // 64).sum())
-    placed = rows[:int(nt) * 64].cpu()
-    assert sorted(placed[placed >= 0].tolist()) == list(range(n * top))
+    # the grouping that the products ran on: the experts' runs of pairs, their borders in the scratch's last words, the tiles
+    flat, size = idx.flatten().long(), 128 if n * top >= 48 * E else 64
+    counts = torch.bincount(flat, minlength=E)
+    runs, offs = rows.cpu().long(), rows[-E - 1:].tolist()
+    assert offs == [0] + counts.cumsum(0).tolist()
+    for e in range(E):
+        assert sorted(runs[offs[e]:offs[e + 1]].tolist()) == (flat == e).nonzero().flatten().tolist()
+    tiles_of = [-(-c // size) for c in counts.tolist()]
+    assert int(nt) == sum(tiles_of)
+    assert te[:int(nt)].tolist() == [e + 1024 * i for e in range(E) for i in range(tiles_of[e])]
 
 
 @pytest.mark.parametrize("dtype", ["float32", "bfloat16"])
