@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const XT* __restrict__ 
 // ---------------------------------------------------------------------------
 // The 32-bit product on the matrix cores: v_mfma_f32_16x16x4_f32 takes float operands as they are and adds in float,
 // so nothing is reduced; a lane's FMAs of the scalar kernel had the vector units and their LDS reads as bound (13
-// TFLOP/s), this instruction does 64 multiply-adds a cycle and SIMD (157 TFLOP/s on the chip).
+// TFLOP/s), this instruction does 32 multiply-adds a cycle and SIMD (157 TFLOP/s on the chip).
 //
 // gemm_f32_mfma_kernel: 256 threads, 2 x 2 wavefronts of 16 TM x 16 TN outputs each; BK columns of both operands go
 // through LDS in two buffers, the next ones on their way to registers meanwhile, one barrier a piece.  A row of a piece

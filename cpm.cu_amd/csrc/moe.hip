@@ -860,12 +860,15 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     const long pairs = (long)n * top;
     CPMCU_REQUIRE(max_tiles >= (pairs + MOE_TILE - 1) / MOE_TILE + E && max_tiles <= 65535,
                   "moe_experts_mfma: %d tiles of scratch for %ld pairs of %d experts (at most 65535)", max_tiles, pairs, E);
-    // Tiles of 128 rows where experts have many: from 56 pairs an expert on most have more than one tile of 64, whose weights
-    // come twice.  Both products and the sum in us, tiles of 64 / 128 at 32, 48, 56, 64, 96, 192 pairs an expert:
-    //   64 experts of 1,408 at width 4,096  401/446  432/452  479/470  573/482  782/541  1,257/765
-    //   64 experts of 2,112 at width 4,096  567/624  615/649  633/658  858/678  1,137/749  1,856/1,096
-    //   16 experts of 512 at width 1,024    32/30  35/32  35/35  36/38  36/43  49/47
-    // The line lies where an uneven choice of experts, as routers make it, has crossed over.
+    // Tiles of 128 rows where experts have many: once most have more than 64 pairs, tiles of 64 read their weights twice.  Both
+    // products and the sum in us, tiles of 64 / 128 rows, at 32, 40, 48, 56, 64, 96 pairs an expert; experts chosen evenly, and
+    // unevenly (logits with a normal bias of 0.5 an expert), as routers do, for which the line lies where it does:
+    //   64 experts of 1,408 at width 4,096  even    401/446  415/451  432/452  479/470  573/482  782/541
+    //                                       uneven  410/443  448/457  490/473  531/480  578/498  771/555
+    //   64 experts of 2,112 at width 4,096  even    567/624  588/637  615/649  633/658  858/678  1,137/749
+    //                                       uneven  593/633  652/659  706/669  762/698  863/712  1,087/802
+    //   16 experts of 512 at width 1,024    even    32/30    33/31    35/32    35/35    36/38    36/43
+    //                                       uneven  32/36    34/35    34/42    34/36    35/42    44/43
     // The scratch is sized for tiles of 64: it holds the pairs without gaps and, at its end, the experts' offsets.
     const bool wide = pairs >= 48L * E;
     const int tile_rows = wide ? 2 * MOE_TILE : MOE_TILE;

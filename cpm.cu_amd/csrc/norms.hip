@@ -297,6 +297,8 @@ __global__ __launch_bounds__(1024) void poly_norm_reg_kernel(const ZT* __restric
 // The same for 16-bit rows of whole 16-byte pieces (a prompt's): PIECES pieces a thread stay in registers as they came, and
 // the three sums cross the workgroup together, behind one barrier.  Memory bounds it; with 2-byte accesses a row's 1,024
 // threads waited for the address unit and at six barriers.  2,048 rows of 11,008: 48 -> 21 us; 4,096 wide 22 -> 12; 8 rows the same.
+// Built for 1, 3 and 4 pieces; widths of 4,097 to 8,192 take three, the last of them empty, and gain as the others do (2,048
+// rows that stay in the caches, us: 4,096 18 -> 11, 4,608 24 -> 14, 6,144 27 -> 15, 8,192 31 -> 15, 11,008 35 -> 16).
 #define POLY_WIDE_THREADS 512
 template <int PIECES>
 __global__ __launch_bounds__(POLY_WIDE_THREADS) void poly_norm_wide_kernel(const bf16_t* __restrict__ z,

@@ -432,7 +432,10 @@ def attention_splits(n_tokens: int, nkv: int, group: int, max_keys: int, hd: int
     With the head size given, few keys stay one share, whose 4 wavefronts finish them sooner than a merge kernel
     starts (one sequence, 2 kv heads, keys from the caches, attention + merge in us for one share / the shares above):
       head size 64 at 300 keys 4.4/5.9, 512 4.8/5.6, 768 5.7/5.7, 1,024 6.3/5.7; 32 sequences 5.0/6.8, 5.4/7.1, 7.7/8.0, 9.3/8.8;
-      head size 128 at 300 keys 5.9/6.8, 384 6.2/6.4, 512 6.7/6.4, 768 7.9/6.5; 32 sequences 7.5/8.7, 8.6/9.0, 10.0/9.8, 13.0/11.6."""
+      head size 128 at 300 keys 5.9/6.8, 384 6.2/6.4, 512 6.7/6.4, 768 7.9/6.5; 32 sequences 7.5/8.7, 8.6/9.0, 10.0/9.8, 13.0/11.6.
+    max_keys is the step's bound: a decode step captured in a graph is sized for a power of two of keys (256 at least), so
+    there one share serves sequences of up to 512 keys at head sizes up to 64 and of up to 256 above; the borders between act
+    in steps that are not captured.  Head sizes 16 to 48 take the border of 64, 80 to 112 that of 128."""
     if hd and max_keys < (768 if hd <= 64 else 512):
         return 1
     cus = compute_units()
