@@ -768,12 +768,21 @@ extern "C" const char* cpmcu_attention_mfma_static(const void* q, void* out, int
 // row, and a tile is skipped for chunks that lie behind all of its rows.
 // `tiles` holds, per wavefront, the first packed token and the number of tokens.
 // ===========================================================================
-template <int HD, int R, int NW>
+// GEN: with a mask that cuts off old keys (`chunk`: a token sees the keys of its own run of that many positions; `window`:
+// its last so many), a sink in the denominator, an output gate (times sigmoid, heads side by side) or float output.
+// Chunks of keys that no row sees are not visited; a tile takes no part in a chunk that none of its own rows sees.
+struct PromptExtras {
+    const float* sink;
+    const bf16_t* gate;
+    long ld_gate;
+    int out_f32, chunk, window;
+};
+template <int HD, int R, int NW, bool GEN>
 __global__ __launch_bounds__(NW * 64) void attention_prefill_mfma_kernel(
-    const bf16_t* __restrict__ q, bf16_t* __restrict__ out, const bf16_t* __restrict__ kpool,
+    const bf16_t* __restrict__ q, void* __restrict__ out, const bf16_t* __restrict__ kpool,
     const bf16_t* __restrict__ vtpool, PagedView pv, const int* __restrict__ tiles,
     const int* __restrict__ positions, const int* __restrict__ tok_slot, int nh, int nkv, float scale_log2e,
-    int rows_per_token, int tokens_per_tile) {
+    int rows_per_token, int tokens_per_tile, PromptExtras extras) {
     constexpr int KSTEPS = (HD + 31) / 32;
     constexpr int DT = HD / 16;
     const int tile_id = gridDim.x - 1 - blockIdx.x;      // later tiles of a prompt see more keys: start them first
@@ -814,6 +823,21 @@ __global__ __launch_bounds__(NW * 64) void attention_prefill_mfma_kernel(
     const int n_tiles_used = (n_tok + tokens_per_tile - 1) / tokens_per_tile;
     const int last_pos = pos0 + n_tok - 1;
     const int total_chunks = last_pos / 32 + 1;
+    // the first key that the query at position p sees (GEN): it never falls as p grows
+    auto first_seen = [&](int p) {
+        return !GEN ? 0 : extras.chunk > 0 ? p - p % extras.chunk : extras.window > 0 ? max(p - extras.window + 1, 0) : 0;
+    };
+    int row_first[R], tile_first_key[R], tile_all_from[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        row_first[r] = first_seen(row_pos[r]);
+        tile_first_key[r] = first_seen(tile_first_pos[r]);
+        tile_all_from[r] = first_seen(tile_last_pos[r]);
+    }
+    const int first_chunk = first_seen(pos0) / 32;
+    auto sees = [&](int r, int key0) {
+        return r < n_tiles_used && key0 <= tile_last_pos[r] && key0 + 31 >= tile_first_key[r];
+    };
 
     afloatx4_t acc[R][DT];
     float m[R], l[R];
@@ -847,7 +871,7 @@ __global__ __launch_bounds__(NW * 64) void attention_prefill_mfma_kernel(
     };
     // the wavefront's chunks in turn: page number and chunk inside the page advance without a division
     const int cpp = pv.page_size / 32;
-    int pg_i = wave / cpp, in_pg = wave % cpp;
+    int pg_i = (first_chunk + wave) / cpp, in_pg = (first_chunk + wave) % cpp;
     const int pg_step = NW / cpp, in_step = NW % cpp;      // (without a branch: the loop's code stays one stretch)
     auto next_pchunk = [&]() {
         in_pg += in_step;
@@ -860,7 +884,7 @@ __global__ __launch_bounds__(NW * 64) void attention_prefill_mfma_kernel(
     // scores are issued, its values as soon as the last tile's P.V is, so both arrive behind other work
     // with NW wavefronts a workgroup the chunks are dealt to them in turn and merged at the end
     abf16x8_t kf[2][KSTEPS], vf[DT];
-    if (wave < total_chunks) {
+    if (first_chunk + wave < total_chunks) {
         const int pchunk = ptab[pg_i] * cpp + in_pg;
         load_k(pchunk, kf);
         load_v(pchunk, vf);
@@ -885,31 +909,36 @@ __global__ __launch_bounds__(NW * 64) void attention_prefill_mfma_kernel(
         for (int u = 0; u < 2; ++u)
 #pragma unroll
             for (int i = 0; i < 4; ++i) sc[u * 4 + i] = st[u][i];
-        if (masked && key0 + 31 > tile_first_pos[r]) {
+        if (masked && (key0 + 31 > tile_first_pos[r] || (GEN && key0 < tile_all_from[r]))) {
 #pragma unroll
             for (int u = 0; u < 2; ++u)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-                    if (key0 + 8 * g + 4 * u + i > row_pos[r]) sc[u * 4 + i] = -INFINITY;
+                    if (key0 + 8 * g + 4 * u + i > row_pos[r] || (GEN && key0 + 8 * g + 4 * u + i < row_first[r])) sc[u * 4 + i] = -INFINITY;
         }
         float mx = fmaxf(fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3])),
                          fmaxf(fmaxf(sc[4], sc[5]), fmaxf(sc[6], sc[7])));
         mx = rows_max(mx);
         // running maximum in units of scaled scores (scale > 0); a row whose position lies before
         // this chunk sees none of its keys: nothing changes for it
-        // the reference follows the maximum only past a move of more than 8 (see attention_mfma_kernel)
+        // the reference follows the maximum only past a move of more than 8 (see attention_mfma_kernel); with GEN it follows
+        // every move, as in the general kernel that took these calls before: a token's largest weight is 1, exact in 16 bits
         const float m_top = fmaxf(m[r], mx * scale_log2e);
-        moved = __builtin_amdgcn_ballot_w64(m_top > m[r] + 8.0f) != 0;
+        moved = __builtin_amdgcn_ballot_w64(m_top > (GEN ? m[r] : m[r] + 8.0f)) != 0;
         const float m_new = moved ? m_top : m[r];
         const float m_use = m_new == -INFINITY ? 0.f : m_new;
         corr = fast_exp2(m[r] - m_use);
-        float rs = 0.f;
+        float rs = 0.f, p[8];
         abf16x8_t pb;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            const float p = fast_exp2(fmaf(sc[j], scale_log2e, -m_use));
-            rs += p;
-            pb[j] = (__bf16)p;
+            p[j] = fast_exp2(fmaf(sc[j], scale_log2e, -m_use));
+            if (!GEN) rs += p[j];
+            pb[j] = (__bf16)p[j];
+        }
+        if (GEN) {                     // the general kernel's order of the sum: with one wavefront the results are its own
+#pragma unroll
+            for (int j = 0; j < 4; ++j) rs += p[j] + p[4 + j];
         }
         rs = rows_sum(rs);
         l[r] = l[r] * corr + rs;
@@ -940,16 +969,51 @@ __global__ __launch_bounds__(NW * 64) void attention_prefill_mfma_kernel(
         // values' products of one tile run under the other tile's vector work (a wavefront issues in order, and
         // a matrix instruction holds only its own pipe).  A tile that does not see a chunk (the first tile at
         // the last chunk of the second, an unused tile) is computed all the same: the mask leaves it weights of 0.
-        if (wave < total_chunks) {
+        if (first_chunk + wave < total_chunks) {
             afloatx4_t s0[2], s1[2];
             scores(0, s0);
             scores(1, s1);
             int pchunk_v = 0;                                  // the chunk whose keys kf holds or awaits
-            if (wave + NW < total_chunks) {
+            if (first_chunk + wave + NW < total_chunks) {
                 pchunk_v = next_pchunk();
                 load_k(pchunk_v, kf);
             }
-            int c = wave;
+            int c = first_chunk + wave;
+            // a chunk that the mask may cut into, or one of the last
+            auto masked_step = [&]() {
+                const int key0 = c * 32;
+                const bool more = c + NW < total_chunks;
+                afloatx4_t n0[2], n1[2];
+                const int pchunk_next = pchunk_v;
+                if (more) {
+                    scores(0, n0);
+                    scores(1, n1);
+                    if (c + 2 * NW < total_chunks) {
+                        pchunk_v = next_pchunk();
+                        load_k(pchunk_v, kf);
+                    }
+                }
+                if (!GEN || sees(0, key0)) {
+                    const abf16x8_t p0 = weights(0, key0, s0);
+                    values(0, p0);
+                }
+                if (!GEN || sees(1, key0)) {
+                    const abf16x8_t p1 = weights(1, key0, s1);
+                    values(1, p1);
+                }
+                if (more) {
+                    load_v(pchunk_next, vf);
+#pragma unroll
+                    for (int u = 0; u < 2; ++u) {
+                        s0[u] = n0[u];
+                        s1[u] = n1[u];
+                    }
+                }
+            };
+            if (GEN) {
+                const int cut_end = min(total_chunks, (first_seen(last_pos) + 31) / 32);
+                for (; c < cut_end; c += NW) masked_step();
+            }
             // The chunks that lie before both tiles' rows and have two more behind them: no mask, no test
             // for the end, so that the matrix instructions and the vector work stand in one stretch of code
             // and are issued in turn (the order is said below: a wavefront issues in order, and a matrix
@@ -988,42 +1052,17 @@ __global__ __launch_bounds__(NW * 64) void attention_prefill_mfma_kernel(
                     s1[u] = n1[u];
                 }
             }
-            for (; c < total_chunks; c += NW) {
-                const int key0 = c * 32;
-                const bool more = c + NW < total_chunks;
-                afloatx4_t n0[2], n1[2];
-                const int pchunk_next = pchunk_v;
-                if (more) {
-                    scores(0, n0);
-                    scores(1, n1);
-                    if (c + 2 * NW < total_chunks) {
-                        pchunk_v = next_pchunk();
-                        load_k(pchunk_v, kf);
-                    }
-                }
-                const abf16x8_t p0 = weights(0, key0, s0);
-                values(0, p0);
-                const abf16x8_t p1 = weights(1, key0, s1);
-                values(1, p1);
-                if (more) {
-                    load_v(pchunk_next, vf);
-#pragma unroll
-                    for (int u = 0; u < 2; ++u) {
-                        s0[u] = n0[u];
-                        s1[u] = n1[u];
-                    }
-                }
-            }
+            for (; c < total_chunks; c += NW) masked_step();
         }
     } else {
-        for (int c = wave; c < total_chunks; c += NW) {
+        for (int c = first_chunk + wave; c < total_chunks; c += NW) {
             const int key0 = c * 32;
             const bool more = c + NW < total_chunks;
             int pchunkn = 0;
             if (more) pchunkn = next_pchunk();
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                const bool active = r < n_tiles_used && key0 <= tile_last_pos[r];
+                const bool active = sees(r, key0);
                 afloatx4_t st[2];
                 if (active) scores(r, st);
                 if (r == R - 1 && more) load_k(pchunkn, kf);      // the last tile's scores are issued: keys are free
@@ -1076,12 +1115,19 @@ __global__ __launch_bounds__(NW * 64) void attention_prefill_mfma_kernel(
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         if (!row_ok[r]) continue;
+        if (GEN && extras.sink) l[r] += exp2f(extras.sink[row_head[r]] * 1.4426950408889634f - m[r]);
         const float inv = 1.0f / l[r];
-        bf16_t* o = out + ((long)row_tok[r] * nh + row_head[r]) * HD;
+        const long at = ((long)row_tok[r] * nh + row_head[r]) * HD + 4 * g;
+        const bf16_t* gate = GEN && extras.gate ? extras.gate + (long)row_tok[r] * extras.ld_gate + row_head[r] * HD + 4 * g : nullptr;
 #pragma unroll
         for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) o[dt * 16 + 4 * g + i] = f32_to_bf16(acc[r][dt][i] * inv);
+            for (int i = 0; i < 4; ++i) {
+                float v = acc[r][dt][i] * inv;
+                if (GEN && gate) v /= 1.0f + expf(-to_f32(gate[dt * 16 + i]));
+                if (GEN && extras.out_f32) ((float*)out)[at + dt * 16 + i] = v;
+                else ((bf16_t*)out)[at + dt * 16 + i] = f32_to_bf16(v);
+            }
     }
 }
 
@@ -1098,7 +1144,10 @@ extern "C" const char* cpmcu_attention_prefill_mfma(const void* q, void* out, in
                                                     int nkv, int hd, float scale, const void* kpool,
                                                     const void* vtpool, const int* page_table, int table_width,
                                                     int page_size, const int* positions, const int* tok_slot,
-                                                    hipStream_t stream) {
+                                                    int out_f32, int chunk, int window, const float* sink,
+                                                    const void* gate, long ld_gate, int general, hipStream_t stream) {
+    CPMCU_REQUIRE(chunk >= 0 && window >= 0 && (chunk == 0 || window == 0), "attention_prefill: mask chunk %d, window %d (one of them)", chunk, window);
+    CPMCU_REQUIRE(!gate || ld_gate >= (long)nh * hd, "attention_prefill: gate rows of %ld elements for %d heads of %d", ld_gate, nh, hd);
     CPMCU_REQUIRE(n_tiles > 0 && nh > 0 && nkv > 0 && nh % nkv == 0, "attention_prefill: bad shape tiles=%d heads=%d kv_heads=%d", n_tiles, nh, nkv);
     CPMCU_REQUIRE(hd >= 16 && hd <= 128 && hd % 16 == 0,
                   "attention_prefill: head_dim %d has no matrix-core kernel (16, 32, ... 128 have)", hd);
@@ -1114,18 +1163,24 @@ extern "C" const char* cpmcu_attention_prefill_mfma(const void* q, void* out, in
     CPMCU_REQUIRE(tiles_per_wave == 2 || tiles_per_wave == 4, "attention_prefill: %d tiles a wavefront (2 or 4 are built)", tiles_per_wave);
     CPMCU_REQUIRE(waves_per_group == 1 || waves_per_group == 2 || waves_per_group == 4,
                   "attention_prefill: %d wavefronts a workgroup (1, 2 or 4 are built)", waves_per_group);
-#define LAUNCH(HDv, Rv, NWv)                                                                                     \
-    attention_prefill_mfma_kernel<HDv, Rv, NWv><<<grid, NWv * 64, 0, stream>>>(                                  \
-        (const bf16_t*)q, (bf16_t*)out, (const bf16_t*)kpool, (const bf16_t*)vtpool, pv, tiles, positions,       \
-        tok_slot, nh, nkv, sl, rpt, tpt)
-#define BY_R(HDv)                                                               \
-    do {                                                                        \
-        if (tiles_per_wave == 4 && waves_per_group == 4) LAUNCH(HDv, 4, 4);     \
-        else if (tiles_per_wave == 4 && waves_per_group == 2) LAUNCH(HDv, 4, 2); \
-        else if (tiles_per_wave == 4) LAUNCH(HDv, 4, 1);                        \
-        else if (waves_per_group == 4) LAUNCH(HDv, 2, 4);                       \
-        else if (waves_per_group == 2) LAUNCH(HDv, 2, 2);                       \
-        else LAUNCH(HDv, 2, 1);                                                 \
+    const PromptExtras extras{sink, (const bf16_t*)gate, ld_gate, out_f32, chunk, window};
+    const bool gen = general || sink || gate || out_f32 || chunk || window;
+    CPMCU_REQUIRE(!gen || tiles_per_wave == 2, "attention_prefill: masks, sinks, gates and float output are built for 2 tiles a wavefront");
+#define LAUNCH(HDv, Rv, NWv, GENv)                                                                               \
+    attention_prefill_mfma_kernel<HDv, Rv, NWv, GENv><<<grid, NWv * 64, 0, stream>>>(                            \
+        (const bf16_t*)q, out, (const bf16_t*)kpool, (const bf16_t*)vtpool, pv, tiles, positions,                \
+        tok_slot, nh, nkv, sl, rpt, tpt, extras)
+#define BY_WAVES(HDv, Rv, GENv)                                  \
+    do {                                                         \
+        if (waves_per_group == 4) LAUNCH(HDv, Rv, 4, GENv);      \
+        else if (waves_per_group == 2) LAUNCH(HDv, Rv, 2, GENv); \
+        else LAUNCH(HDv, Rv, 1, GENv);                           \
+    } while (0)
+#define BY_R(HDv)                                         \
+    do {                                                  \
+        if (tiles_per_wave == 4) BY_WAVES(HDv, 4, false); \
+        else if (gen) BY_WAVES(HDv, 2, true);             \
+        else BY_WAVES(HDv, 2, false);                     \
     } while (0)
     switch (hd) {
         case 16: BY_R(16); break;
@@ -1138,6 +1193,7 @@ extern "C" const char* cpmcu_attention_prefill_mfma(const void* q, void* out, in
         default: BY_R(128); break;
     }
 #undef BY_R
+#undef BY_WAVES
 #undef LAUNCH
     CPMCU_LAUNCH_CHECK("attention_prefill_mfma");
     return nullptr;

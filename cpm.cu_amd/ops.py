@@ -370,12 +370,24 @@ def attention_prefill_shape(n_tokens: int, nh: int, nkv: int, hd: int):
 def attention_prefill_mfma(q: torch.Tensor, out: torch.Tensor, tiles: torch.Tensor, nh: int, nkv: int, hd: int,
                            scale: float, kpool: torch.Tensor, vpool: torch.Tensor, page_table: torch.Tensor,
                            page_size: int, positions: torch.Tensor, tok_slot: torch.Tensor, tiles_per_wave: int = 4,
-                           waves_per_group: int = 1):
-    """Dense causal bf16 attention for prompts: tiles int32 [T, 2] = (first packed token, tokens), each a run of
-    consecutive tokens of one sequence, at most attention_prefill_tokens_per_wave(nh, nkv, tiles_per_wave) long."""
+                           waves_per_group: int = 1, chunk: int = 0, window: int = 0, sink: Optional[torch.Tensor] = None,
+                           gate: Optional[torch.Tensor] = None, general: bool = False):
+    """Causal bf16 attention for prompts: tiles int32 [T, 2] = (first packed token, tokens), each a run of
+    consecutive tokens of one sequence, at most attention_prefill_tokens_per_wave(nh, nkv, tiles_per_wave) long.
+    With 2 tiles a wavefront also with a mask (chunks, or a sliding window), a softmax sink, an output gate [n, nh*hd]
+    (out * sigmoid(gate)) and a float32 ``out``, as in attention_general_mfma; ``general`` asks for that form without any."""
     _need(q, "attention q", torch.bfloat16, (None, nh * hd))
     n = q.shape[0]
-    _need(out, "attention out", torch.bfloat16, (n, nh * hd))
+    if out.dtype not in (torch.bfloat16, torch.float32):
+        raise KernelError(f"attention out: dtype {out.dtype} (bfloat16 or float32)")
+    _need(out, "attention out", out.dtype, (n, nh * hd))
+    if sink is not None:
+        _need(sink, "attention sink", torch.float32, (nh,))
+    ld_gate = 0
+    if gate is not None:
+        ld_gate = _ld(gate, "attention gate")
+        if gate.dtype != torch.bfloat16 or tuple(gate.shape) != (n, nh * hd):
+            raise KernelError(f"attention gate: {gate.dtype} {tuple(gate.shape)}, expected bfloat16 {(n, nh * hd)}")
     _need(tiles, "attention tiles", torch.int32, (None, 2))
     _need(kpool, "attention key pool", torch.bfloat16, (None, page_size, nkv * hd))
     _need(vpool, "attention value pool", torch.bfloat16, tuple(kpool.shape))
@@ -387,7 +399,8 @@ def attention_prefill_mfma(q: torch.Tensor, out: torch.Tensor, tiles: torch.Tens
         c_int(nkv), c_int(hd),
         c_float(scale),
         _p(kpool), _p(vpool), _p(page_table), c_int(page_table.shape[1]), c_int(page_size), _p(positions),
-        _p(tok_slot), _stream()))
+        _p(tok_slot), c_int(1 if out.dtype == torch.float32 else 0), c_int(chunk), c_int(window), _p(sink), _p(gate),
+        c_long(ld_gate), c_int(1 if general else 0), _stream()))
 
 
 def prefill_tiles(q_lens: Sequence[int], tokens_per_wave: int, device) -> torch.Tensor:
@@ -2114,6 +2127,19 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, alpha: float = 1
     gemm_nt_plain(x, w, out, alpha)
 
 
+def attention_prompt(q, out, nh, nkv, hd, scale, kpool, vpool, page_table, page_size, ctx, waves: int = 0, **extras):
+    """attention_prefill_mfma with the step's tiles and the shape that suits its tokens (waves: wavefronts that share a group
+    of tiles, 0 for the rule's)."""
+    r, nw = attention_prefill_shape(q.shape[0], nh, nkv, hd)
+    tpw = attention_prefill_tokens_per_wave(nh, nkv, r)
+    key = ("prefill_tiles", tpw)
+    tiles = ctx.extras.get(key)
+    if tiles is None:
+        tiles = ctx.extras[key] = prefill_tiles(ctx.q_lens, tpw, q.device)
+    attention_prefill_mfma(q, out, tiles, nh, nkv, hd, scale, kpool, vpool, page_table, page_size, ctx.positions, ctx.tok_slot,
+                           r, waves or nw, **extras)
+
+
 def attention(q, out, nh, nkv, hd, scale, kpool, vpool, page_table, page_size, ctx,
               sel_blocks=None, sel_count=None, block_size=0, window_blocks=0, head_slopes=None):
     """Attention of the step's queries over the cache, with the kernel that suits the step; writes ``out``.
@@ -2124,14 +2150,7 @@ def attention(q, out, nh, nkv, hd, scale, kpool, vpool, page_table, page_size, c
                         sel_blocks, sel_count, block_size, head_slopes)
         return
     if sel_count is None and not ctx.single_token and attention_mfma_ok(q, hd, page_size):
-        r, nw = attention_prefill_shape(q.shape[0], nh, nkv, hd)
-        tpw = attention_prefill_tokens_per_wave(nh, nkv, r)
-        key = ("prefill_tiles", tpw)
-        tiles = ctx.extras.get(key)
-        if tiles is None:
-            tiles = ctx.extras[key] = prefill_tiles(ctx.q_lens, tpw, q.device)
-        attention_prefill_mfma(q, out, tiles, nh, nkv, hd, scale, kpool, vpool, page_table, page_size,
-                               ctx.positions, ctx.tok_slot, r, nw)
+        attention_prompt(q, out, nh, nkv, hd, scale, kpool, vpool, page_table, page_size, ctx)
         return
     if attention_mfma_ok(q, hd, page_size, block_size if sel_count is not None else 0):
         n = q.shape[0]
@@ -2318,6 +2337,18 @@ class HeadFinish:
         self.out, self.inv_freq, self.gate, self.interleaved = out, inv_freq, gate, bool(interleaved)
 
 
+def attention_prompt_pays(n_tokens: int, max_pos: int) -> bool:
+    """Whether attention_any's prompts of heads up to 128 features go to the prompt kernel, whose wavefronts load the keys for
+    two tiles of 16 columns instead of one.  Measured (us, general kernel / the prompt kernel with 1, 2 wavefronts sharing a
+    group of tiles; 32 heads on 8 of 128; tokens + tokens of history):
+      2,048 + 0 214/98/88, 2,048 + 2,048 in a window of 2,048 311/185/124 and in chunks of 2,048 202/92/80, 1,500 + 0 114/54/54,
+      4 x 479 68/35/38, 8 x 200 40/27/28, 347 + 0 26/17/17, 300 + 0 beside 8 x 1 + 4,000 282/99/56;
+      12 heads on 4 of 64, 1,000 39/32/27; 32 heads of their own, 700 61/29/24.
+    Up to 256 tokens the two are level.  With one wavefront a group the results are the general kernel's to the last bit, and up to
+    2,048 positions that costs little."""
+    return n_tokens > 256
+
+
 def attention_any(q, out, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, page_size, ctx, chunk: int = 0,
                   window: int = 0, keep_first: int = 0, sink: Optional[torch.Tensor] = None, v_share: int = 1,
                   gate: Optional[torch.Tensor] = None, softcap: float = 0.0, finish: Optional["HeadFinish"] = None) -> bool:
@@ -2332,6 +2363,17 @@ def attention_any(q, out, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, pa
             and kpool.shape[2] == nkv * hdk and v_share == 1 and not softcap and out.dtype == q.dtype):
         attention(q, out, nh, nkv, hdk, scale, kpool, vpool, page_table, page_size, ctx)
         return False
+    if not ctx.single_token:
+        # a mask that cuts nothing off at the step's positions is none
+        if ctx.max_pos < chunk:
+            chunk = 0
+        if ctx.max_pos < window:
+            window = keep_first = 0
+        if (hdk == hdv and keep_first == 0 and not softcap and v_share == 1 and kpool.shape[2] == nkv * hdk
+                and vpool.shape[2] == nkv * hdv and attention_mfma_ok(q, hdk, page_size) and attention_prompt_pays(q.shape[0], ctx.max_pos)):
+            attention_prompt(q, out, nh, nkv, hdk, scale, kpool, vpool, page_table, page_size, ctx, chunk=chunk, window=window,
+                             sink=sink, gate=gate, general=True, waves=1 if ctx.max_pos < 2048 else 0)
+            return gate is not None
     # (operands off 16-byte borders, which the kernel for wide values refuses, are the general kernel's)
     if (not ctx.single_token and attention_wide_prefill_ok(q, nh, nkv, hdk, hdv, kpool.shape[2] // nkv, pool_hdv, page_size)
             and (q.data_ptr() | out.data_ptr() | kpool.data_ptr() | vpool.data_ptr()) % 16 == 0
