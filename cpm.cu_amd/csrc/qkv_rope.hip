@@ -136,7 +136,7 @@ __global__ __launch_bounds__(NW * 64) void qkv_rope_kernel(
                     rot_sn[t][T][j] = sinf(ang) * mscale;
                 }
             }
-    if (row_ss) row_scales<NW * 64, MT * 16>(row_ss, ss_slices, M, 1.0f / (float)K, eps, rs_s);
+    if (row_ss && wave < 4) row_scales<256, MT * 16>(row_ss, ss_slices, M, 1.0f / (float)K, eps, rs_s);
     int kb = kb0;
     for (; kb + 2 * PF <= kb1; kb += PF) {           // every block and every block asked for exists
 #pragma unroll
@@ -301,15 +301,20 @@ extern "C" const char* cpmcu_qkv_rope(const void* X, long ldx, const void* W, in
     PagedView pv{page_table, table_width, page_size};
     const int total_rows = (nh + 2 * nkv) * hd;
     const int wgs = (total_rows + R - 1) / R;
-#define LAUNCH(PFv, MTv, TLv)                                                                                    \
-    qkv_rope_kernel<PFv, 4, MTv, TLv><<<wgs, 256, 0, stream>>>((const bf16_t*)X, ldx, (const bf16_t*)W, M, K, R,  \
+#define LAUNCH(PFv, MTv, TLv) LAUNCH_OF(PFv, 4, MTv, TLv)
+#define LAUNCH_OF(PFv, NWv, MTv, TLv)                                                                                    \
+    qkv_rope_kernel<PFv, NWv, MTv, TLv><<<wgs, NWv * 64, 0, stream>>>((const bf16_t*)X, ldx, (const bf16_t*)W, M, K, R,  \
                                                            (bf16_t*)q_out,                                           \
                                                            nh, nkv, hd, positions, tok_slot, inv_freq, mscale,       \
                                                            (bf16_t*)kpool, (bf16_t*)vpool, pv, row_ss, ss_slices, eps, \
                                                            (bf16_t*)ckpool, ck_size, ck_stride)
     // more tokens hold more of x in registers for every block in flight: fewer blocks then
+    // K up to 1,024 has 8 blocks: one for each of 8 wavefronts, where 4 asked for 4 each and had 2 (1,280 x 1,024 in a chain of
+    // launches over weights that no cache holds, 1 / 8 / 32 tokens: 4.92/5.48/8.84 -> 4.28/4.56/6.74 us)
     if (R == 16) {
-        if (M <= 16) LAUNCH(4, 1, 1);
+        if (M <= 16 && K <= 1024) LAUNCH_OF(1, 8, 1, 1);
+        else if (M <= 32 && M > 16 && K <= 1024) LAUNCH_OF(1, 8, 2, 1);
+        else if (M <= 16) LAUNCH(4, 1, 1);
         else if (M <= 32) LAUNCH(4, 2, 1);
         else LAUNCH(2, 4, 1);
     } else {
@@ -317,6 +322,7 @@ extern "C" const char* cpmcu_qkv_rope(const void* X, long ldx, const void* W, in
         else if (M <= 32) LAUNCH(2, 2, 2);
         else LAUNCH(2, 4, 2);
     }
+#undef LAUNCH_OF
 #undef LAUNCH
     CPMCU_LAUNCH_CHECK("qkv_rope");
     return nullptr;

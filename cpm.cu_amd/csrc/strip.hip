@@ -137,13 +137,17 @@ extern "C" const char* cpmcu_proj_add_norm(const void* A, long lda, const void* 
 #define LAUNCH(PFv, NWv, MTv)                                                                                   \
     proj_add_norm_kernel<PFv, NWv, MTv><<<strips, NWv * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, M, N, \
                                                                         K, alpha, x, w_norm, (bf16_t*)out, row_ss, strips)
-    // 4 blocks in flight in each of 4 wavefronts measured best at K = 4,096 (8 wavefronts: the same; 8 blocks:
-    // slower; 16 wavefronts of 4 blocks spill)
+    // What a wavefront asks for before its first product should be all that it will multiply, and no more: with 4 blocks asked
+    // for where it has 2 (K = 1,024) it read its neighbours' too.  Measured in a chain of launches over weights that no cache
+    // holds (us at 1 / 8 tokens; blocks in flight x wavefronts 4 x 4, 2 x 4, 1 x 8, 2 x 8):
+    //   1,024 x 1,024   3.80/4.44  3.27/3.57  3.37/3.62  3.96/4.45     4,096 x 4,096   8.30/8.83  8.31/8.63  8.29/8.69  8.21/8.69
+    //   1,024 x 4,096   5.73/6.72  5.98/6.50  5.74/6.35  5.75/6.60     4,096 x 11,008  18.0/19.8  18.0/18.6  17.7/18.7  18.1/19.4
+    //   4,096 x 16,384  26.0/26.7 (2 x 8)  25.9/27.2  30.7/31.6
     // (more tokens hold more of a in registers for every block in flight: fewer blocks then)
-    // long rows (down: K = 16,384) in 8 wavefronts of 2 blocks in flight: 24.3 against 25.1 us at 8 tokens, 27.4
-    // against 29.6 at 16; at K = 4,096 the two are level
-    if (M <= 16 && K >= 8192) LAUNCH(2, 8, 1);
-    else if (M <= 16) LAUNCH(4, 4, 1);
+    if (M <= 16 && K <= 1024) LAUNCH(2, 4, 1);
+    else if (M <= 16 && K < 12288) LAUNCH(1, 8, 1);
+    else if (M <= 16) LAUNCH(2, 8, 1);
+    else if (M <= 32 && K <= 1024) LAUNCH(1, 8, 2);       // 1,024 x 1,024 at 32 tokens 7.3 -> 5.4 us
     else if (M <= 32) LAUNCH(4, 4, 2);
     else LAUNCH(2, 4, 4);
 #undef LAUNCH
@@ -152,13 +156,13 @@ extern "C" const char* cpmcu_proj_add_norm(const void* A, long lda, const void* 
 }
 
 // ===========================================================================
-// silu(a . Wg^T) * (a . Wu^T) for decode steps of at most 16 tokens, by strips: a workgroup owns a strip of 16
+// silu(a . Wg^T) * (a . Wu^T) for decode steps of at most 16 tokens (64 of up to 1,024 columns), by strips: a workgroup owns a strip of 16
 // gate rows and the strip of their up rows over all of K (W holds the gate rows, then the up rows; I gate rows,
 // a multiple of 16).  Its wavefronts take a quarter of K each, with a straight from global memory into the B
-// operand as above, add up through LDS, and the first one applies the norm's row factor (if a is the x * w of a
+// operand as above (or an eighth: see the launcher), add up through LDS, and the first one applies the norm's row factor (if a is the x * w of a
 // norm cut by columns), the gate's nonlinearity and writes 16 columns.  1,024 small workgroups at 16,384 gate
 // rows keep more loads in flight than the skinny product's 512 (gemm.hip), which stages a through LDS behind
-// barriers: 43.4 against 45.8 us at 8 tokens and 4,096 columns (6.2 TB/s of weights).
+// barriers: 43.4 against 45.8 us at 8 tokens and 4,096 columns, over one weight.
 // (reference: src/model/ffn.cuh:31-59, 77-84; src/model/activation.cuh:6-18)
 // ===========================================================================
 template <int PF, int NW, int MT>
@@ -207,7 +211,7 @@ __global__ __launch_bounds__(NW * 64) void gated_strip_kernel(
     };
 #pragma unroll
     for (int j = 0; j < PF; ++j) load_block(kb0 + j, wv[j], av[j]);
-    if (row_ss) row_scales<NW * 64, MT * 16>(row_ss, ss_slices, M, 1.0f / (float)K, eps, rs_s);
+    if (row_ss && wave < 4) row_scales<256, MT * 16>(row_ss, ss_slices, M, 1.0f / (float)K, eps, rs_s);
     int kb = kb0;
     for (; kb + 2 * PF <= kb1; kb += PF) {
 #pragma unroll
@@ -261,14 +265,26 @@ extern "C" const char* cpmcu_gated_strip(const void* A, long lda, const void* W,
                                          const float* row_ss, int ss_slices, float eps, int act, float act_limit,
                                          hipStream_t stream) {
     CPMCU_REQUIRE(CPMCU_ACT_KNOWN(act), "gated_strip: unknown nonlinearity %d", act);
-    CPMCU_REQUIRE(M > 0 && M <= 16, "gated_strip: %d tokens (1..16 are taken; more go through the skinny product)", M);
+    CPMCU_REQUIRE(M > 0 && (M <= 16 || (M <= 64 && K <= 1024)),
+                  "gated_strip: %d tokens of %d columns (1..16 are taken, up to 64 of 1,024; more go through the skinny product)", M, K);
     CPMCU_REQUIRE(I > 0 && I % 16 == 0 && K > 0 && K % 8 == 0 && lda % 8 == 0 && lda >= K,
                   "gated_strip: %d gate rows must be a multiple of 16, K=%d and the row stride %ld multiples of 8", I, K, lda);
     CPMCU_REQUIRE(A && W && out && (!row_ss || ss_slices > 0), "gated_strip: null pointer");
     CPMCU_REQUIRE(((uintptr_t)A % 16 == 0) && ((uintptr_t)W % 16 == 0) && ((uintptr_t)out % 8 == 0),
                   "gated_strip: operands must be 16-byte aligned");
-    gated_strip_kernel<4, 4, 1><<<I / 16, 256, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, M, I, K, (bf16_t*)out,
-                                                           row_ss, ss_slices, eps, act, act_limit);
+#define LAUNCH(PFv, NWv, MTv)                                                                                             \
+    gated_strip_kernel<PFv, NWv, MTv><<<I / 16, NWv * 64, 0, stream>>>((const bf16_t*)A, lda, (const bf16_t*)W, M, I, K,  \
+                                                                       (bf16_t*)out, row_ss, ss_slices, eps, act, act_limit)
+    // 8 wavefronts of a block in flight each, against 4 of 4 (us at 1 / 8 tokens, measured as above; gate rows x columns):
+    //   4,096 x 1,024 7.51/7.91 -> 5.57/5.78 (a wavefront of 4 has 2 blocks there and asked for 4), 16,384 x 4,096 47.9/47.3 ->
+    //   45.8/45.2 (5.9 TB/s); level between: 11,008 x 4,096 32.6/32.7 -> 31.8/32.7, 2,816 x 4,096 11.1/12.2 -> 11.3/12.4
+    // More than 16 tokens, where every workgroup reads up to four times as much of a: it pays while K is short and a wavefront
+    // has all of its blocks in flight (4,096 x 1,024, skinny product -> here: 32 tokens 9.3 -> 7.9 us, 64 tokens 15.4 -> 11.6).
+    if (M > 32) LAUNCH(2, 4, 4);
+    else if (M > 16) LAUNCH(2, 4, 2);
+    else if (K <= 1024 || I >= 16384) LAUNCH(1, 8, 1);
+    else LAUNCH(4, 4, 1);
+#undef LAUNCH
     CPMCU_LAUNCH_CHECK("gated_strip");
     return nullptr;
 }

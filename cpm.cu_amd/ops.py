@@ -2008,12 +2008,20 @@ def proj_add_norm(a: torch.Tensor, w: "TiledWeight", alpha: float, x: torch.Tens
                                              c_float(alpha), _p(x), _p(weight), _p(out), _p(sums), _stream()))
 
 
+def gated_strip_ok(n: int, K: int) -> bool:
+    """Whether gated_strip takes n tokens of K columns, and is the faster kernel for them (measured in csrc/strip.hip)."""
+    return n <= STRIP_ROWS or (n <= STRIP_MAX_ROWS and K <= 1024)
+
+
 def gated_strip(x: torch.Tensor, w: "TiledWeight", out: torch.Tensor, row_scale: Optional[RowScale] = None,
-                activation="silu"):
-    """out = act(x . Wg^T) * (x . Wu^T) (act as in silu_mul) for a step of at most 16 tokens, w tiled with the gate rows first (a
-    multiple of 16 of them); out bfloat16 [n, N/2].  With row_scale as in gemm_skinny."""
+                activation="silu", most: int = STRIP_ROWS):
+    """out = act(x . Wg^T) * (x . Wu^T) (act as in silu_mul) for a step of at most ``most`` tokens (16; up to 64 where
+    gated_strip_ok says so), w tiled with the gate rows first (a multiple of 16 of them); out bfloat16 [n, N/2].  With
+    row_scale as in gemm_skinny."""
     _need(x, "gated x", torch.bfloat16, (None, None))
     n, K = x.shape
+    if n > most:
+        raise KernelError(f"gated_strip: {n} tokens (1..{most} are taken; more go through the skinny product)")
     if not isinstance(w, TiledWeight) or w.K != K or w.N % 32:
         raise KernelError(f"gated_strip: the weight must be tiled for K = {K} with a multiple of 16 gate rows")
     _need(out, "gated out", torch.bfloat16, (n, w.N // 2))

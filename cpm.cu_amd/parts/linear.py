@@ -121,9 +121,9 @@ class Linear(Part):
         another of ops.GATE_ACTIVATIONS."""
         n, half = x.shape[0], self.out_features // 2
         act = ctx.ws.get(tag + ".act", (n, half), x.dtype)
-        if (n <= ops.STRIP_ROWS and x.dtype == torch.bfloat16 and self.tiled is not None and half % 16 == 0
+        if (ops.gated_strip_ok(n, self.in_features) and x.dtype == torch.bfloat16 and self.tiled is not None and half % 16 == 0
                 and self.in_features % 8 == 0):
-            ops.gated_strip(x, self.tiled, act, row_scale=row_scale, activation=activation)   # a strip of columns a workgroup
+            ops.gated_strip(x, self.tiled, act, row_scale=row_scale, activation=activation, most=n)   # a strip of columns a workgroup
         elif self._gated_skinny(n, x.dtype):
             ops.gemm_skinny(x, self.tiled if self.tiled is not None else self.weight, act, mode="gated",
                             row_scale=row_scale, activation=activation)

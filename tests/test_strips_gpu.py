@@ -1,0 +1,49 @@
+"""Products of decode steps by strips of output columns, at the borders of the rules that share their work out (GPU)."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def rnd(*shape, g, dtype=torch.float32, scale=1.0):
+    return (torch.randn(*shape, generator=g, device=DEV) * scale).to(dtype)
+
+
+@pytest.mark.parametrize("n,I,K", [(17, 16, 8), (32, 4096, 1024), (33, 48, 1000), (64, 1008, 136), (64, 16, 1024)])
+@pytest.mark.parametrize("scaled", [False, True])
+def test_gated_strips_of_up_to_64_tokens(n, I, K, scaled):
+    from cpmcu_amd import ops
+    assert ops.gated_strip_ok(n, K) and not ops.gated_strip_ok(n, 1032) and not ops.gated_strip_ok(65, 8)
+    g = torch.Generator(device=DEV).manual_seed(n + K)
+    x, w = rnd(n, K, g=g, dtype=torch.bfloat16), rnd(2 * I, K, g=g, dtype=torch.bfloat16, scale=2.0 * K ** -0.5)
+    rs, r = None, 1.0
+    if scaled:
+        rs = ops.RowScale(torch.rand(n, 5, generator=g, device=DEV) + 0.1, 1e-3)
+        r = torch.rsqrt(rs.sums.double().sum(1) / K + 1e-3).view(n, 1)
+    out = torch.full((n, I), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.gated_strip(x, ops.TiledWeight(w), out, row_scale=rs, most=64)
+    y = (x.double() @ w.double().T) * r
+    ref = F.silu(y[:, :I]) * y[:, I:]
+    # the output's rounding, and K float sums of terms of order one before the nonlinearity
+    assert bool(((out.double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4 * (1 + y[:, I:].abs())).all())
+    with pytest.raises(ops.KernelError):
+        ops.gated_strip(rnd(17, 1032, g=g, dtype=torch.bfloat16), ops.TiledWeight(rnd(32, 1032, g=g, dtype=torch.bfloat16)),
+                        torch.empty(17, 16, dtype=torch.bfloat16, device=DEV), most=64)
+
+
+@pytest.mark.parametrize("n", [1, 16, 20, 32])
+@pytest.mark.parametrize("K", [8, 1016, 1024, 1032, 12280, 12288])
+def test_residual_products_at_the_borders_of_the_wavefronts_shares(n, K):
+    """Up to 1,024 columns, up to 12,288 and beyond: blocks shared by 4 or 8 wavefronts, some of which have none."""
+    from cpmcu_amd import ops
+    N = 36
+    g = torch.Generator(device=DEV).manual_seed(n + K)
+    a, w = rnd(n, K, g=g, dtype=torch.bfloat16), rnd(N, K, g=g, dtype=torch.bfloat16, scale=K ** -0.5)
+    x0, nw = rnd(n, N, g=g), rnd(N, g=g)
+    x, xw, sums = x0.clone(), torch.empty(n, N, dtype=torch.bfloat16, device=DEV), torch.empty(n, 3, device=DEV)
+    ops.proj_add_norm(a, ops.TiledWeight(w), 0.6, x, nw, xw, sums)
+    want = x0.double() + 0.6 * (a.double() @ w.double().T)
+    assert float((x.double() - want).abs().max()) <= 1e-5 * float(want.abs().max())
+    assert float((sums.double().sum(1) - (want ** 2).sum(1)).abs().max()) <= 1e-5 * float((want ** 2).sum(1).max())
