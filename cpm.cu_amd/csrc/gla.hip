@@ -337,14 +337,14 @@ extern "C" const char* cpmcu_gla_scan(const void* rows, int dtype, long ld, long
 // grid (B, heads), NT threads: 16 lanes a column of the state.  rows: T [n, ld]; sequence b's one token is row cu_q[b];
 // up float [R][heads*dk]; out T [n, heads*dv].
 // out = rms(o) * norm_w (per head) * silu(gate), or * sigmoid(gate) with gate_sigmoid
-template <typename T>
+template <typename T, bool FULL>
 __global__ __launch_bounds__(1024) void gla_step_kernel(const T* __restrict__ rows, long ld, long q_off, long k_off,
                                                         long v_off, long g_off, long low_off, int R,
                                                         const float* __restrict__ up, const float* __restrict__ bias,
                                                         float inv_tau, const float* __restrict__ norm_w, float eps,
                                                         int gate_sigmoid, float* __restrict__ state, T* __restrict__ out,
                                                         const int* __restrict__ cu_q, const int* __restrict__ seq_slot,
-                                                        int heads, int dk, int dv, float q_scale) {
+                                                        int heads, int dk, int dv, float q_scale, int sum_nt) {
     extern __shared__ float sm[];                    // q, k, a: [dkp] each; then o: [dv]
     __shared__ float red[17];
     const int b = blockIdx.x, h = blockIdx.y, NT = blockDim.x;
@@ -354,26 +354,31 @@ __global__ __launch_bounds__(1024) void gla_step_kernel(const T* __restrict__ ro
     const T* row = rows + t * ld;
     float* sp = state + ((long)seq_slot[b] * heads + h) * (long)dv * dk;
     const int g = threadIdx.x >> 4, l = threadIdx.x & 15, G = NT >> 4;
-    // a column's share of a lane: pieces of 4 values, the first column asked for before the decays are formed
-    float S[16];
-    auto load = [&](int p) {
+    // a column's share of a lane: pieces of 4 values; the first two columns are asked for before the decays are formed, and
+    // every other two columns before its turn
+    float S0[16], S1[16];
+    auto load1s = [&](float (&S)[16], int p) {
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int n = ((i >> 2) * 16 + l) * 4 + (i & 3);
             S[i] = (p < dv && n < dk) ? sp[(long)p * dk + n] : 0.f;
         }
     };
-    auto load4s = [&](int p) {                       // dk a multiple of 4
+    auto load4s = [&](float (&S)[16], int p) {       // dk a multiple of 4; FULL: of 64, and no load stands in a branch
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const int n = (j * 16 + l) * 4;
-            const float4 v = (p < dv && n < dk) ? *(const float4*)(sp + (long)p * dk + n) : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float4 v = FULL ? *(const float4*)(sp + (long)min(p, dv - 1) * dk + min(n, dk - 4)) : (p < dv && n < dk) ? *(const float4*)(sp + (long)p * dk + n) : make_float4(0.f, 0.f, 0.f, 0.f);
             S[4 * j] = v.x; S[4 * j + 1] = v.y; S[4 * j + 2] = v.z; S[4 * j + 3] = v.w;
         }
     };
     const bool vec = dk % 4 == 0;
-    if (vec) load4s(g);
-    else load(g);
+    auto load = [&](float (&S)[16], int p) {
+        if (FULL || vec) load4s(S, p);
+        else load1s(S, p);
+    };
+    load(S0, g);
+    load(S1, g + G);
     // decays: 4 neighbouring lanes a channel
     for (int c0 = 0; c0 < dkp; c0 += NT / 4) {
         const int c = c0 + (threadIdx.x >> 2), part = threadIdx.x & 3;
@@ -388,8 +393,7 @@ __global__ __launch_bounds__(1024) void gla_step_kernel(const T* __restrict__ ro
         ks[c] = c < dk ? to_f32(row[k_off + (long)h * dk + c]) : 0.f;
     }
     __syncthreads();
-    float ss = 0.f;
-    for (int p = g; p < dv; p += G) {
+    auto column = [&](float (&S)[16], int p) {
         const float v = to_f32(row[v_off + (long)h * dv + p]);
         float o = 0.f;
 #pragma unroll
@@ -402,23 +406,36 @@ __global__ __launch_bounds__(1024) void gla_step_kernel(const T* __restrict__ ro
             S[4 * j + 2] = fmaf(a4.z, S[4 * j + 2], k4.z * v);
             S[4 * j + 3] = fmaf(a4.w, S[4 * j + 3], k4.w * v);
             o += (S[4 * j] * q4.x + S[4 * j + 1] * q4.y) + (S[4 * j + 2] * q4.z + S[4 * j + 3] * q4.w);
-            if (vec) {
-                if (n < dk) *(float4*)(sp + (long)p * dk + n) = make_float4(S[4 * j], S[4 * j + 1], S[4 * j + 2], S[4 * j + 3]);
+            if (FULL || vec) {
+                if (FULL || n < dk) *(float4*)(sp + (long)p * dk + n) = make_float4(S[4 * j], S[4 * j + 1], S[4 * j + 2], S[4 * j + 3]);
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if (n + e < dk) sp[(long)p * dk + n + e] = S[4 * j + e];
             }
         }
-        if (vec) load4s(p + G);
-        else load(p + G);
+        load(S, p + 2 * G);
         o = row16_sum(o);
-        if (l == 0) {
-            os[p] = o;
-            ss += o * o;
-        }
+        if (l == 0) os[p] = o;
+    };
+    for (int p = g; p < dv; p += 2 * G) {
+        column(S0, p);
+        if (p + G < dv) column(S1, p + G);
     }
-    const float r = 1.0f / sqrtf(block_sum(ss, red) / (float)dv + eps);     // (its barriers make os visible)
+    __syncthreads();
+    // the squares' sum, in one order whatever the number of threads: as 16 lanes a column add up in workgroups of sum_nt
+    const int sg = sum_nt >> 4;
+    for (int w = threadIdx.x >> 6; w < sum_nt >> 6; w += NT >> 6) {
+        float ss = 0.f;
+        if (l == 0)
+            for (int p = w * 4 + ((threadIdx.x & 63) >> 4); p < dv; p += sg) ss += os[p] * os[p];
+        ss = wave_sum(ss);
+        if ((threadIdx.x & 63) == 0) red[w] = ss;
+    }
+    __syncthreads();
+    float total = 0.f;
+    for (int w = 0; w < sum_nt >> 6; ++w) total += red[w];
+    const float r = 1.0f / sqrtf(total / (float)dv + eps);
     for (int p = threadIdx.x; p < dv; p += NT) {
         const float gt = to_f32(row[g_off + (long)h * dv + p]);
         const float s = 1.0f / (1.0f + expf(-gt));
@@ -439,17 +456,25 @@ extern "C" const char* cpmcu_gla_step(const void* rows, int dtype, long ld, long
                   ld >= low_off + R, "gla_step: rows of %ld too short", ld);
     CPMCU_REQUIRE(rows && up && bias && norm_w && state && out && cu_q && seq_slot, "gla_step: null pointer");
     CPMCU_REQUIRE(heads <= 65535, "gla_step: %d heads exceed the launch grid", heads);
-    int nt = 1024;
-    while (nt > 256 && nt / 16 > dv) nt /= 2;
+    // more workgroups than two of 1,024 threads a CU: four of 512, all in flight at once
+    int sum_nt = 1024;
+    while (sum_nt > 256 && sum_nt / 16 > dv) sum_nt /= 2;
+    const int nt = (long)n_seqs * heads > 512 && sum_nt > 512 ? 512 : sum_nt;
     const size_t lds = (3 * ((dk + 63) & ~63) + dv) * sizeof(float);
     const dim3 grid(n_seqs, heads);
-#define LAUNCH(Tv)                                                                                                      \
-    gla_step_kernel<Tv><<<grid, nt, lds, stream>>>((const Tv*)rows, ld, q_off, k_off, v_off, g_off, low_off, R, up, bias, \
-                                                   inv_tau, norm_w, eps, gate_sigmoid, state, (Tv*)out, cu_q, seq_slot, \
-                                                   heads, dk, dv, q_scale)
-    if (dtype == CPMCU_F32) LAUNCH(float);
-    else if (dtype == CPMCU_BF16) LAUNCH(bf16_t);
+#define LAUNCH(Tv, FULLv)                                                                                               \
+    gla_step_kernel<Tv, FULLv><<<grid, nt, lds, stream>>>((const Tv*)rows, ld, q_off, k_off, v_off, g_off, low_off, R, up, bias, \
+                                                          inv_tau, norm_w, eps, gate_sigmoid, state, (Tv*)out, cu_q, seq_slot, \
+                                                          heads, dk, dv, q_scale, sum_nt)
+#define BY_SIZE(Tv)                              \
+    do {                                         \
+        if (dk % 64 == 0) LAUNCH(Tv, true);      \
+        else LAUNCH(Tv, false);                  \
+    } while (0)
+    if (dtype == CPMCU_F32) BY_SIZE(float);
+    else if (dtype == CPMCU_BF16) BY_SIZE(bf16_t);
     else CPMCU_FAIL("gla_step: unknown dtype %d", dtype);
+#undef BY_SIZE
 #undef LAUNCH
     CPMCU_LAUNCH_CHECK("gla_step");
     return nullptr;
