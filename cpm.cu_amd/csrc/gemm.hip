@@ -3,8 +3,8 @@
 // src/model/linear.cuh:9-37 calls a library product with fp32 accumulation).
 //
 //  * gemm_tiled_kernel: LDS-tiled product with scalar float FMAs, any size: the plain twin of the bf16 products.
-//  * gemm_f32_mfma_kernel, gemm_f32_rows_kernel: the whole 32-bit engine's product, on the matrix cores' float
-//    instruction (true fp32: no reduced inputs), any size.
+//  * gemm_f32_split_kernel, gemm_f32_shares_kernel, gemm_f32_mfma_kernel, gemm_f32_rows_kernel: the whole 32-bit engine's
+//    product on the matrix cores, any size: with every float as the exact sum of three bf16, or on the float instruction.
 #include "common.h"
 
 #define GT_BM 64
@@ -58,19 +58,16 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const XT* __restrict__ 
 }
 
 // ---------------------------------------------------------------------------
-// The 32-bit product on the matrix cores: v_mfma_f32_16x16x4_f32 takes float operands as they are and adds in float,
-// so nothing is reduced; a lane's FMAs of the scalar kernel had the vector units and their LDS reads as bound (13
-// TFLOP/s), this instruction does 32 multiply-adds a cycle and SIMD (157 TFLOP/s on the chip).
+// The 32-bit product on the matrix cores.  v_mfma_f32_16x16x4_f32 takes float operands as they are and adds in float
+// (32 multiply-adds a cycle and SIMD, 157 TFLOP/s on the chip); v_mfma_f32_16x16x32_bf16 does 16 times as many, so that six
+// of its products, which a float as three bf16 asks for (below), still are 2.7 times as fast.
 //
-// gemm_f32_mfma_kernel: 256 threads, 2 x 2 wavefronts of 16 TM x 16 TN outputs each; BK columns of both operands go
-// through LDS in two buffers, the next ones on their way to registers meanwhile, one barrier a piece.  A row of a piece
-// is BK / 4 chunks of 16 bytes, chunk c of row r at place c ^ (r % 8), so that 8 neighbouring lanes (8 rows, one chunk)
-// read all banks.  A lane's 16 bytes serve four instructions: in instruction s, lane group g stands for column 4 g + s
-// of the 16, in both operands alike (a sum over columns may take them in any order).
-// Measured (us, scalar kernel -> this one; rows x outputs x columns): 523 x 8,192 x 1,024 246 -> 109 (56 at 157
-// TFLOP/s), 523 x 1,024 x 4,096 557 -> 75, 2,048 x 4,096 x 4,096 1,650 -> 540, 1 x 8,192 x 1,024 144 -> 11,
-// 16 x 73,448 x 1,024 267 -> 70; its distance from a product in double is the scalar kernel's (5.7e-7 at 1,024
-// columns, 1.1e-6 at 4,096) or, at up to 16 rows, a third of it.
+// gemm_f32_mfma_kernel: the float instruction, for few columns and for few rows of very many outputs.  256 threads, a
+// wavefront 16 x 16 of a 32 x 32 tile; 64 columns of both operands go through LDS in two buffers, the next ones on their way
+// to registers meanwhile, one barrier a piece.  A row of a piece is 16 chunks of 16 bytes, chunk c of row r at place
+// c ^ (r % 8), so that 8 neighbouring lanes (8 rows, one chunk) read all banks.  A lane's 16 bytes serve four instructions: in
+// instruction s, lane group g stands for column 4 g + s of the 16, in both operands alike (a sum over columns may take them
+// in any order).  16 x 73,448 x 1,024 takes 70 us; its distance from a product in double is a float sum's.
 // ---------------------------------------------------------------------------
 typedef float gfloatx4_t __attribute__((ext_vector_type(4)));
 
@@ -89,11 +86,11 @@ __device__ inline gfloatx4_t f32_piece(const float* __restrict__ row, int k, int
     return v;
 }
 
-template <int TM, int TN, int BK, bool VEC>
+template <bool VEC>
 __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ X, long ldx,
                                                             const float* __restrict__ W, long ldw, float* __restrict__ Y,
                                                             long ldy, int M, int N, int K, float alpha) {
-    constexpr int BM = 32 * TM, BN = 32 * TN, CH = BK / 4, PIECES = (BM + BN) * CH / 256;
+    constexpr int BM = 32, BN = 32, BK = 64, CH = BK / 4, PIECES = (BM + BN) * CH / 256;
     __shared__ float lds[2][(BM + BN) * BK];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
@@ -110,12 +107,8 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
     gfloatx4_t next[PIECES];
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) next[i] = f32_piece<VEC>(src[i], chunk * 4, K);
-    gfloatx4_t acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
-    const int row_a = (wave & 1) * 16 * TM + r, row_b = BM + (wave >> 1) * 16 * TN + r;
+    gfloatx4_t acc = {0.f, 0.f, 0.f, 0.f};
+    const int row_a = (wave & 1) * 16 + r, row_b = BM + (wave >> 1) * 16 + r;
     int buf = 0;
     for (int k0 = 0; k0 < K; k0 += BK, buf ^= 1) {
 #pragma unroll
@@ -128,33 +121,281 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 #pragma unroll
         for (int kb = 0; kb < BK / 16; ++kb) {
             const int at = ((kb * 4 + g) ^ (r & 7)) << 2;
-            gfloatx4_t a[TM], b[TN];
+            const gfloatx4_t a = *(const gfloatx4_t*)&lds[buf][row_a * BK + at], b = *(const gfloatx4_t*)&lds[buf][row_b * BK + at];
 #pragma unroll
-            for (int i = 0; i < TM; ++i) a[i] = *(const gfloatx4_t*)&lds[buf][(row_a + 16 * i) * BK + at];
-#pragma unroll
-            for (int j = 0; j < TN; ++j) b[j] = *(const gfloatx4_t*)&lds[buf][(row_b + 16 * j) * BK + at];
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][s], b[j][s], acc[i][j], 0, 0, 0);
+            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc, 0, 0, 0);
         }
     }
-    // lane (column r, g): acc[i][j][e] is row 4 g + e of its 16 x 16 outputs
+    // lane (column r, g): acc[e] is row 4 g + e of its 16 x 16 outputs
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int m = m0 + (wave & 1) * 16 + 4 * g + e, n = n0 + (wave >> 1) * 16 + r;
+        if (m < M && n < N) Y[(long)m * ldy + n] = alpha * acc[e];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// The same product with every float as the sum of three bf16, x = h + m + l: the upper 8 bits, the upper 8 of what is left
+// and the rest, exact for all that a float holds (down to 2^-110, where the last part ends below the smallest bf16).  Six of
+// the nine products, hh, hm, mh, mm, hl, lh, go through v_mfma_f32_16x16x32_bf16, whose sums are float, the small ones first;
+// the other three are below 2^-21 of a product at most and 2^-24 of it on average.  With a sum every 32 columns instead of
+// every 4 the result is nearer to a product in double than the float instruction's (relative error, before -> now: 1,024
+// columns 5.7e-7 -> 4.9e-7 and, with the columns shared out, 1.7e-7; 4,096 columns 1.15e-6 -> 1.0e-6 and 3.5e-7).
+// Infinities, NaNs and results so small that the parts' own limit may show are worked out on the float instruction
+// (f32_finish_tile).
+//
+// gemm_f32_split_kernel: 64 rows against 64 TN outputs a workgroup.  X's piece of 32 columns is split once and its parts go
+// through LDS in two buffers; a wavefront splits its own 16 TN rows of W in registers, which nobody else needs.  Two pieces on
+// their way to registers.
+// gemm_f32_shares_kernel: for outputs that give too few such workgroups: every one of 8 wavefronts has the whole tile of
+// 16 TM x 16 TN outputs and every eighth piece of the columns, no barrier until their sums meet in LDS.  Pieces are brought
+// whole lines a row (8 lanes each) and turned into operands through the wavefront's own LDS: loads straight into the operand's
+// order, where 64 neighbouring lanes ask for 64 rows, pass one lane a cycle (523 x 1,024 x 4,096: 59.5 -> 46.2 us).
+// What bounds both: a piece's conversions (352 vector instructions for 64 x 64 outputs) take about as long as its 96 matrix
+// instructions, and the two overlap little; then grids that 256 CUs do not divide.
+// Measured (us, tiles on the float instruction -> here; rows x outputs x columns): 523 x 8,192 x 1,024 113 -> 73 (121 TFLOP/s),
+// 523 x 1,024 x 4,096 80 -> 46, 523 x 1,024 x 1,024 22.4 -> 15.7, 523 x 1,280 x 1,024 22.9 -> 16.1, 700 x 8,192 x 1,024 126 -> 76,
+// 2,048 x 4,096 x 4,096 552 -> 367, 130 x 8,192 x 1,024 41 -> 32, 130 x 1,024 x 4,096 43 -> 24, 40 x 8,192 x 1,024 16.4 -> 13.2,
+// 17 x 1,024 x 4,096 42 -> 22, 300 x 1,000 x 1,001 29.7 -> 24.9.
+// ---------------------------------------------------------------------------
+typedef __bf16 gbf16x8_t __attribute__((ext_vector_type(8)));
+struct Split8 {      // eight floats as three bf16 each
+    gbf16x8_t h, m, l;
+};
+// the upper halves of two floats, a's first
+__device__ inline uint32_t f32_upper(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
+__device__ inline Split8 f32_split(const gfloatx4_t& x, const gfloatx4_t& y) {
+    union { uint32_t u[4]; gbf16x8_t v; } part[3];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        uint32_t a = __float_as_uint(i < 2 ? x[2 * i] : y[2 * i - 4]), b = __float_as_uint(i < 2 ? x[2 * i + 1] : y[2 * i - 3]);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            part[p].u[i] = f32_upper(a, b);
+            if (p < 2) {
+                a = __float_as_uint(__uint_as_float(a) - __uint_as_float(a & 0xffff0000u));
+                b = __float_as_uint(__uint_as_float(b) - __uint_as_float(b & 0xffff0000u));
+            }
+        }
+    }
+    return {part[0].v, part[1].v, part[2].v};
+}
+
+// One 16 x 16 tile of a split product as it is stored.  A sum that is no finite number may stand for an infinity (whose parts
+// are an infinity and no numbers), and one below 2^-64 for inputs whose last parts fall below the smallest bf16: those tiles
+// are worked out again on the float instruction.
+template <bool VEC>
+__device__ inline void f32_finish_tile(gfloatx4_t sum, const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw,
+                                       float* __restrict__ Y, long ldy, int M, int N, int K, float alpha, int m0, int n0) {
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    bool odd = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) odd |= !(fabsf(sum[e]) < __builtin_inff()) || (fabsf(sum[e]) < 0x1p-64f && sum[e] != 0.f);
+    if (__any(odd)) {
+        const float* xr = X + (long)min(m0 + r, M - 1) * ldx;
+        const float* wr = W + (long)min(n0 + r, N - 1) * ldw;
+        sum = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < K; k += 16) {
+            const gfloatx4_t a = f32_piece<VEC>(xr, k + 4 * g, K), b = f32_piece<VEC>(wr, k + 4 * g, K);
+#pragma unroll
+            for (int s = 0; s < 4; ++s) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], sum, 0, 0, 0);
+        }
+    }
+    // lane (column r, g): sum[e] is row 4 g + e
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int m = m0 + 4 * g + e, n = n0 + r;
+        if (m < M && n < N) Y[(long)m * ldy + n] = alpha * sum[e];
+    }
+}
+
+// Which tile a workgroup takes: workgroups go to the 8 XCDs in turn, and neighbouring tiles (same outputs, other rows) to
+// one XCD, whose L2 then reads their weights once.
+__device__ inline int tile_of_workgroup(int wg, int tiles) {
+    const int per = tiles / 8, more = tiles % 8, x = wg % 8;
+    return x * per + min(x, more) + wg / 8;
+}
+
+template <int TM, int TN, bool VEC>
+__global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
+    const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, float* __restrict__ Y, long ldy, int M, int N,
+    int K, float alpha, int m_tiles, int tiles) {
+    constexpr int TASKS = TM / 4, PLANE = TM * 16 * 64, BUF = 3 * PLANE;
+    __shared__ __attribute__((aligned(16))) char lds[2 * BUF];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int t = tile_of_workgroup(blockIdx.x, tiles);
+    const int m0 = t % m_tiles * 16 * TM, n0 = (t / m_tiles * 4 + wave) * 16 * TN;
+    const float *xr[TASKS], *wr[TN];
+    int place[TASKS];
+    const int chunk = threadIdx.x & 3;
+#pragma unroll
+    for (int i = 0; i < TASKS; ++i) {
+        const int row = (threadIdx.x >> 2) + 64 * i;
+        xr[i] = X + (long)min(m0 + row, M - 1) * ldx;
+        place[i] = row * 64 + ((chunk ^ ((row >> 1) & 3)) << 4);
+    }
+#pragma unroll
+    for (int j = 0; j < TN; ++j) wr[j] = W + (long)min(n0 + 16 * j + r, N - 1) * ldw;
+    struct Piece { gfloatx4_t x[TASKS][2], w[TN][2]; } p0, p1;
+    const auto fetch = [&](const float* row, int k, gfloatx4_t (&v)[2]) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            if (VEC) v[c] = *(const gfloatx4_t*)(row + min(k + 16 * c, K - 4));
+            else v[c] = f32_piece<false>(row, k + 16 * c, K);
+        }
+    };
+    const auto clear = [&](int k, gfloatx4_t (&v)[2]) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+            if (VEC && k + 16 * c >= K) v[c] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    };
+    const auto fetch_x = [&](Piece& p, int k) {
+#pragma unroll
+        for (int i = 0; i < TASKS; ++i) fetch(xr[i], k + 4 * chunk, p.x[i]);
+    };
+    const auto fetch_w = [&](Piece& p, int k) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fetch(wr[j], k + 4 * g, p.w[j]);
+    };
+    const auto stage = [&](Piece& p, int k, int buf) {
+#pragma unroll
+        for (int i = 0; i < TASKS; ++i) {
+            if (k + 32 > K) clear(k + 4 * chunk, p.x[i]);
+            const Split8 x = f32_split(p.x[i][0], p.x[i][1]);
+            *(gbf16x8_t*)(lds + buf + place[i]) = x.h;
+            *(gbf16x8_t*)(lds + buf + PLANE + place[i]) = x.m;
+            *(gbf16x8_t*)(lds + buf + 2 * PLANE + place[i]) = x.l;
+        }
+    };
+    gfloatx4_t acc[TM][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int m = m0 + (wave & 1) * 16 * TM + 16 * i + 4 * g + e;
-            if (m >= M) continue;
+        for (int j = 0; j < TN; ++j) acc[i][j] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    const int at = r * 64 + ((g ^ ((r >> 1) & 3)) << 4);
+    // p: piece k (its rows of X in lds[buf]); q: piece k + 32, whose rows go to the other buffer
+    const auto step = [&](Piece& p, Piece& q, int k, int buf) {
+        __syncthreads();
+        gbf16x8_t x[3][TM];
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int n = n0 + (wave >> 1) * 16 * TN + 16 * j + r;
-                if (n < N) Y[(long)m * ldy + n] = alpha * acc[i][j][e];
-            }
+        for (int c = 0; c < 3; ++c)
+#pragma unroll
+            for (int i = 0; i < TM; ++i) x[c][i] = *(const gbf16x8_t*)(lds + buf + c * PLANE + at + i * 1024);
+        fetch_x(p, k + 64);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            if (k + 32 > K) clear(k + 4 * g, p.w[j]);
+            const Split8 w = f32_split(p.w[j][0], p.w[j][1]);
+            fetch(wr[j], k + 64 + 4 * g, p.w[j]);
+#define TERM(P, Q)                                                                                   \
+    _Pragma("unroll") for (int i = 0; i < TM; ++i) acc[i][j] =                                       \
+        __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[P][i], w.Q, acc[i][j], 0, 0, 0)
+            TERM(2, h);
+            TERM(0, l);
+            TERM(1, m);
+            TERM(1, h);
+            TERM(0, m);
+            TERM(0, h);
+#undef TERM
         }
+        stage(q, k + 32, BUF - buf);
+    };
+    fetch_x(p0, 0);
+    fetch_w(p0, 0);
+    fetch_x(p1, 32);
+    fetch_w(p1, 32);
+    stage(p0, 0, 0);
+    int k = 0;
+    for (; k + 32 < K; k += 64) {
+        step(p0, p1, k, 0);
+        step(p1, p0, k + 32, BUF);
+    }
+    if (k < K) step(p0, p1, k, 0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) f32_finish_tile<VEC>(acc[i][j], X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j);
+}
+
+template <int TM, int TN, int NW, bool VEC>
+__global__ __launch_bounds__(NW * 64, 2) void gemm_f32_shares_kernel(
+    const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, float* __restrict__ Y, long ldy, int M, int N,
+    int K, float alpha, int m_tiles, int tiles) {
+    constexpr int PER = (TM * TN + NW - 1) / NW, ROWS = 16 * (TM + TN), LOADS = ROWS / 8;
+    constexpr int REGION = (TM + TN) * 2 > TM * TN ? (TM + TN) * 128 : TM * TN * 64;       // a wavefront's, in 16 bytes
+    __shared__ gfloatx4_t lds[NW * REGION];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    gfloatx4_t* own = lds + wave * REGION;
+    const int t = tile_of_workgroup(blockIdx.x, tiles);
+    const int m0 = t % m_tiles * 16 * TM, n0 = t / m_tiles * 16 * TN;
+    // a piece: 32 columns of the tile's rows, X's before W's; a load brings 8 rows, 8 lanes a row
+    const int chunk = lane & 7, row8 = lane >> 3;
+    const float *xb = X + (long)m0 * ldx, *wb = W + (long)n0 * ldw;
+    uint32_t off[LOADS];                                                                   // floats from there
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = 8 * i + row8;
+        off[i] = i < 2 * TM ? min(row, M - 1 - m0) * (uint32_t)ldx : min(row - 16 * TM, N - 1 - n0) * (uint32_t)ldw;
+    }
+    gfloatx4_t next[LOADS];
+    const auto fetch = [&](int k0) {
+        const int k = VEC ? min(k0 + 4 * chunk, K - 4) : k0 + 4 * chunk;                   // beyond the end: cleared below
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const float* base = i < 2 * TM ? xb : wb;
+            if (VEC) next[i] = *(const gfloatx4_t*)(base + (off[i] + (uint32_t)k));
+            else next[i] = f32_piece<false>(base + off[i], k, K);
+        }
+    };
+    gfloatx4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    const int place = row8 * 8 + (chunk ^ row8), at0 = r * 8 + (g ^ (r & 7)), at1 = at0 ^ 4;
+    fetch(wave * 32);
+    for (int k = wave * 32; k < K; k += NW * 32) {
+        if (VEC && k + 32 > K && k + 4 * chunk >= K) {
+#pragma unroll
+            for (int i = 0; i < LOADS; ++i) next[i] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+        }
+        // (a wavefront's LDS accesses keep their order: no barrier)
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) own[64 * i + place] = next[i];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        fetch(k + NW * 32);
+        Split8 x[TM];
+#pragma unroll
+        for (int i = 0; i < TM; ++i) x[i] = f32_split(own[128 * i + at0], own[128 * i + at1]);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const Split8 w = f32_split(own[128 * (TM + j) + at0], own[128 * (TM + j) + at1]);
+#define TERM(P, Q)                                                                                   \
+    _Pragma("unroll") for (int i = 0; i < TM; ++i) acc[i][j] =                                       \
+        __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i].P, w.Q, acc[i][j], 0, 0, 0)
+            TERM(l, h);
+            TERM(h, l);
+            TERM(m, m);
+            TERM(m, h);
+            TERM(h, m);
+            TERM(h, h);
+#undef TERM
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) own[(i * TN + j) * 64 + lane] = acc[i][j];
+    __syncthreads();
+#pragma unroll
+    for (int f = 0; f < PER; ++f) {
+        const int tile = wave * PER + f, i = tile / TN, j = tile % TN;
+        if (tile >= TM * TN) break;
+        gfloatx4_t sum = lds[tile * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < NW; ++w) sum += lds[w * REGION + tile * 64 + lane];
+        f32_finish_tile<VEC>(sum, X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j);
+    }
 }
 
 // The same for at most 16 rows (decode steps), where the weight's bytes are the bound: a workgroup owns 16 outputs a row
@@ -200,15 +441,37 @@ static void gemm_f32_launch(const float* X, long ldx, const float* W, long ldw, 
         gemm_f32_rows_kernel<16, VEC><<<up(N, 16), 1024, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
         return;
     }
-    // The largest tile that the rows fill and that still gives every CU two workgroups (whose waits then overlap):
-    // 2,048 x 4,096 x 4,096 540 us in tiles of 128 against 595 (64) and 776 (32), 2,048 x 1,024 x 4,096 289 / 153 / 191,
-    // 523 x 1,024 x 4,096 291 / 95 / 75.
-#define TILES(TM, TN, BK)                                                                                        \
-    gemm_f32_mfma_kernel<TM, TN, BK, VEC><<<dim3(up(N, 32 * TN), up(M, 32 * TM)), 256, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha)
-    if (M > 64 && (long)up(M, 128) * up(N, 128) >= 512) TILES(4, 4, 32);
-    else if (M > 32 && (long)up(M, 64) * up(N, 64) >= 512) TILES(2, 2, 32);
-    else TILES(1, 1, 64);
-#undef TILES
+    // (few columns: the parts that a split leaves out would show beside so few roundings)
+    if ((K < 64 && up(M, 32) <= 65535) || (M <= 32 && N > 32768)) {
+        gemm_f32_mfma_kernel<VEC><<<dim3(up(N, 32), up(M, 32)), 256, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
+        return;
+    }
+    // Columns shared out while the tiles are at most one a CU: the smallest tile for which that holds (its wavefronts' pieces cost
+    // the least).  Beyond, 64 rows by as many outputs as still leave one and a half workgroups a CU, which then overlap (tiles of
+    // 64 / 128 / 192 / 256 outputs: 523 x 8,192 x 1,024 76/77/73/86, 700 x 8,192 x 1,024 87/75/74/88, 2,048 x 4,096 x 4,096 480/423/427/378).
+#define SHARES(TM, TN)                                                                                                   \
+    if (up(M, 16 * TM) * (long)up(N, 16 * TN) <= 256) {                                                                  \
+        const int tiles = up(M, 16 * TM) * up(N, 16 * TN);                                                               \
+        gemm_f32_shares_kernel<TM, TN, 8, VEC><<<tiles, 512, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha, up(M, 16 * TM), tiles); \
+        return;                                                                                                          \
+    }
+    SHARES(2, 2);
+    SHARES(2, 4);
+    SHARES(5, 2);
+    SHARES(3, 4);
+    SHARES(4, 4);
+#undef SHARES
+#define SPLIT(TN)                                                                                                        \
+    if (TN == 1 || up(M, 64) * (long)up(N, 64 * TN) >= 384) {                                                            \
+        const int tiles = up(M, 64) * up(N, 64 * TN);                                                                    \
+        gemm_f32_split_kernel<4, TN, VEC><<<tiles, 256, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha, up(M, 64), tiles); \
+        return;                                                                                                          \
+    }
+    SPLIT(4);
+    SPLIT(3);
+    SPLIT(2);
+    SPLIT(1);
+#undef SPLIT
 }
 
 extern "C" const char* cpmcu_gemm_nt_plain(const void* X, long ldx, const void* W, long ldw, void* Y, long ldy,

@@ -22,6 +22,50 @@ def test_float_product_at_tile_edges(M, N, K):
     assert bool(((out.double() - ref).abs() <= bound).all())
 
 
+# every tile that the rule chooses (its workgroups up to 256: 32 x 32, 32 x 64, 80 x 32, 48 x 64, 64 x 64 with the columns shared
+# out; beyond: 64 rows by 64, 128, 192 and 256), columns that end inside a piece of 32, rows on and off 16-byte borders
+SPLITS = [(17, 40, 64), (130, 1000, 100), (260, 1100, 72), (523, 1024, 96), (523, 1023, 65), (700, 1020, 68), (1000, 1000, 257),
+          (1030, 1100, 131), (2000, 1500, 64), (2000, 2300, 97), (1999, 3101, 164)]
+
+
+@pytest.mark.parametrize("M,N,K", SPLITS)
+def test_float_product_in_three_parts(M, N, K):
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    x *= 2.0 ** torch.randint(-40, 40, (M, 1), generator=g, device=DEV)                # rows of all sizes
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops.gemm_nt_plain(x, w, out, 1.5)
+    ref, mag = (1.5 * (a @ b.T) for a, b in ((x.double(), w.double()), (x.double().abs(), w.double().abs())))
+    # sums as above, and the left out products of middle and last parts: below 2^-21 of a product
+    assert bool(((out.double() - ref).abs() <= ((K + 2) * 2.0 ** -24 + 2.0 ** -21) * mag).all())
+    # the error on the whole: no larger than that of a float sum with a rounding every 4 columns
+    assert float((out.double() - ref).norm() / ref.norm()) <= 2.0 ** -24 * (K / 4) ** 0.5
+
+
+@pytest.mark.parametrize("M,N,K", [(70, 130, 96), (1030, 1100, 131)])
+def test_float_product_of_odd_values(M, N, K):
+    """Infinities, NaNs, the largest floats and floats whose last parts no bf16 holds: the float instruction's results."""
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(K)
+    x, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    for t, (row, value) in enumerate([(0, float("inf")), (17, float("-inf")), (33, float("nan")), (34, 3.4e38), (69, -torch.finfo(torch.float32).max)]):
+        x[row, 7 * t] = value
+    w[5, 3], w[100, K - 1] = float("inf"), float("nan")
+    x[40] *= 2.0 ** -122
+    x[41] *= 2.0 ** -100
+    out = torch.full((M, N), 7.0, device=DEV)
+    ops.gemm_nt_plain(x, w, out, 1.0)
+    ref = x.double() @ w.double().T
+    mag = x.double().abs() @ w.double().abs().T
+    fine = torch.isfinite(ref) & (mag < 1e38)
+    assert torch.equal(out.isnan(), ref.isnan())
+    assert bool((out.double() == ref)[torch.isinf(ref)].all())
+    # (denormal products may be flushed one by one)
+    assert bool(((out.double() - ref).abs() <= ((K + 2) * 2.0 ** -24 + 2.0 ** -21) * mag + K * 2.0 ** -126)[fine].all())
+    assert bool(((out[40].double() - ref[40]).abs() <= (K + 2) * 2.0 ** -24 * mag[40] + K * 2.0 ** -126)[fine[40]].all())
+
+
 @pytest.mark.parametrize("nh,nkv,hd", [(17, 1, 16), (6, 2, 128), (4, 4, 80)])
 def test_float_attention_ignores_what_lies_behind_the_token(nh, nkv, hd):
     """A token's page may hold anything behind it, infinities too; 1, 2, 4, 5 and 9 chunks of 32 keys for 4 wavefronts."""
