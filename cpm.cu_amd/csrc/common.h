@@ -152,11 +152,9 @@ __device__ inline float lanes_sum(float v) {
     if (TPR >= 16) v += CPMCU_DPP(v, 0x140);    // row_mirror
     return v;
 }
-template <int NT, int ROWS>
-__device__ inline void row_scales(const float* __restrict__ row_ss, int n_slices, int n_rows, float inv_width,
-                                  float eps, float* rs_out) {
-    constexpr int TPR = NT / ROWS;
-    const int row = threadIdx.x / TPR, part = threadIdx.x % TPR;
+template <int TPR>
+__device__ inline void row_scale(const float* __restrict__ row_ss, int n_slices, int n_rows, float inv_width, float eps,
+                                 int row, int part, float* rs_out) {
     const float* src = row_ss + (long)min(row, n_rows - 1) * n_slices;
     const int per = ((n_slices + TPR - 1) / TPR + 3) & ~3;
     const int i0 = part * per, i1 = min(i0 + per, n_slices);
@@ -172,6 +170,12 @@ __device__ inline void row_scales(const float* __restrict__ row_ss, int n_slices
     }
     s = lanes_sum<TPR>(s);
     if (part == 0) rs_out[row] = 1.0f / sqrtf(s * inv_width + eps);
+}
+template <int NT, int ROWS>
+__device__ inline void row_scales(const float* __restrict__ row_ss, int n_slices, int n_rows, float inv_width,
+                                  float eps, float* rs_out) {
+    constexpr int TPR = NT / ROWS;
+    row_scale<TPR>(row_ss, n_slices, n_rows, inv_width, eps, threadIdx.x / TPR, threadIdx.x % TPR, rs_out);
 }
 
 // ---- error convention ----

@@ -1034,6 +1034,69 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
     }
 }
 
+// The same for at most 16 rows of X and a tiled weight, a wavefront a workgroup: 16 rows of W over all of K, x straight from L2
+// into the operand, PF blocks of 128 columns asked for ahead.  The sums are the kernel's above, in its order, to the last bit.
+// Four times the workgroups of the kernel above, which has 96 of them for 6,144 weight rows on 256 CUs, and no barriers.
+// Measured in a chain of launches over weights that no cache holds (us at 1 / 8 / 16 rows, above -> here):
+//   4,096 x 4,096 13.4/13.9/14.3 -> 8.0/8.4/9.7     6,144 x 4,096 16.3/16.6/17.0 -> 11.0/12.1/14.4     9,280 x 4,096 17.2/18.0/19.0 -> 16.5/17.0/18.8
+//   16,384 x 4,096 25.9/26.2/26.7 -> 24.5/24.5/27.5 73,448 x 4,096 101/102/105 -> 92.6/100/122         4,096 x 16,384 45.8/47.1/49.2 -> 24.2/25.3/29.7
+// K is a multiple of 128 (nothing is padded).  ACT: Y (bf16) = act(alpha * product).
+template <int PF, typename OT, bool ACT>
+__global__ __launch_bounds__(64) void gemm_strip_kernel(const bf16_t* __restrict__ X, long ldx, const bf16_t* __restrict__ W,
+                                                        OT* __restrict__ Y, long ldy, int M, int N, int K, float alpha,
+                                                        const float* __restrict__ row_ss, int ss_slices, float eps, int act) {
+    __shared__ float rs_s[16];
+    const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
+    const int nkb = K / 128;
+    const bf16_t* wp = W + (long)blockIdx.x * nkb * 2048 + lane * 8;
+    const bf16_t* xp = X + (long)min(r, M - 1) * ldx + g * 8;             // rows beyond the step repeat its last one
+    bf16x8_t w[PF][4], x[PF][4];
+    auto load = [&](int kb, bf16x8_t (&wd)[4], bf16x8_t (&xd)[4]) {       // no branch around a load: the last block again
+        const int at = min(kb, nkb - 1);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) wd[i] = __builtin_nontemporal_load((const bf16x8_t*)(wp + ((long)at * 4 + i) * 512));
+#pragma unroll
+        for (int i = 0; i < 4; ++i) xd[i] = *(const bf16x8_t*)(xp + at * 128 + i * 32);
+    };
+    floatx4_t acc = {0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](bf16x8_t (&wd)[4], bf16x8_t (&xd)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wd[i], xd[i], acc, 0, 0, 0);
+    };
+#pragma unroll
+    for (int j = 0; j < PF; ++j) load(j, w[j], x[j]);
+    if (row_ss) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p)                                       // 16 lanes a row, as 256 threads share 16 rows
+            row_scale<16>(row_ss, ss_slices, M, 1.0f / (float)K, eps, 4 * p + (lane >> 4), lane & 15, rs_s);
+        __syncthreads();
+    }
+    int kb = 0;
+    for (; kb + 2 * PF <= nkb; kb += PF) {
+#pragma unroll
+        for (int j = 0; j < PF; ++j) {
+            multiply(w[j], x[j]);
+            load(kb + j + PF, w[j], x[j]);
+        }
+    }
+    for (; kb < nkb; kb += PF) {
+#pragma unroll
+        for (int j = 0; j < PF; ++j) {
+            if (kb + j < nkb) multiply(w[j], x[j]);
+            if (kb + j + PF < nkb) load(kb + j + PF, w[j], x[j]);
+        }
+    }
+    // lane (row r of X, g): acc[e] is row 4 g + e of the strip
+    if (r >= M) return;
+    const float rs = row_ss ? rs_s[r] : 1.0f;
+    OT* y = Y + (long)r * ldy + blockIdx.x * 16 + 4 * g;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float v = alpha * rs * acc[e];
+        if (blockIdx.x * 16 + 4 * g + e < N) y[e] = from_f32<OT>(ACT ? plain_act(v, act) : v);
+    }
+}
+
 // out_mode: 0 = Y[m,N] in out_dtype; 1 = float partial sums Y[ksplit][m][N]; 2 = gated (N = 2*I rows of W, Y[m,I] bf16);
 // 3 = Y[m,N] bf16 with a nonlinearity without a gate
 // row_ss (or null): X is x * w of a norm cut by columns, whose sums of squares [M][ss_slices] these are (a
@@ -1064,6 +1127,27 @@ extern "C" const char* cpmcu_gemm_skinny(const void* X, long ldx, const void* W,
     const int MT = (M + 15) / 16 == 3 ? 4 : (M + 15) / 16;
     const int I = N / 2;
     const long part_stride = (long)M * ldy;
+    // One wavefront a strip where that is the faster one: up to 8 rows everywhere, up to 16 where the kernel below leaves CUs
+    // without a workgroup of 64 weight rows (beyond, every strip's own copy of x costs more).  Blocks in flight: 8 where a CU has few
+    // strips, and where so many weights are streamed that only memory counts.
+    if (tiled && M <= (N <= 8192 ? 16 : 8) && (out_mode == 0 || out_mode == 3) && K % 128 == 0 &&
+        (out_mode == 3 || out_dtype == CPMCU_F32 || out_dtype == CPMCU_BF16)) {
+#define STRIPS(PFv, OT, ACTv)                                                                                        \
+    gemm_strip_kernel<PFv, OT, ACTv><<<(N + 15) / 16, 64, 0, stream>>>((const bf16_t*)X, ldx, (const bf16_t*)W, (OT*)Y, ldy, M, \
+                                                                       N, K, alpha, row_ss, ss_slices, eps, act)
+#define BY_SIZE(OT, ACTv)                                       \
+    do {                                                        \
+        if (N <= 4096 || N > 32768) STRIPS(8, OT, ACTv);        \
+        else STRIPS(4, OT, ACTv);                               \
+    } while (0)
+        if (out_mode == 3) BY_SIZE(bf16_t, true);
+        else if (out_dtype == CPMCU_F32) BY_SIZE(float, false);
+        else BY_SIZE(bf16_t, false);
+#undef BY_SIZE
+#undef STRIPS
+        CPMCU_LAUNCH_CHECK("gemm_strips");
+        return nullptr;
+    }
 #define LAUNCH(MTv, MODEv, OT, SPW, NW)                                                                           \
     do {                                                                                                          \
         const int rows_wg = (MODEv == 2) ? NW * 16 : NW * SPW * 16;                                               \

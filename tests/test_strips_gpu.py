@@ -47,3 +47,19 @@ def test_residual_products_at_the_borders_of_the_wavefronts_shares(n, K):
     want = x0.double() + 0.6 * (a.double() @ w.double().T)
     assert float((x.double() - want).abs().max()) <= 1e-5 * float(want.abs().max())
     assert float((sums.double().sum(1) - (want ** 2).sum(1)).abs().max()) <= 1e-5 * float((want ** 2).sum(1).max())
+
+
+@pytest.mark.parametrize("n,N,K", [(1, 16, 128), (8, 100, 1152), (16, 8192, 256), (9, 2000, 384), (3, 9000, 640), (8, 33000, 128), (16, 40, 4096)])
+@pytest.mark.parametrize("mode,dtype", [("plain", torch.float32), ("plain", torch.bfloat16), ("act", torch.bfloat16)])
+def test_products_of_one_wavefront_a_strip(n, N, K, mode, dtype):
+    """Fewer blocks than are asked for ahead, one more, many; columns that end inside a strip: the results of the product that
+    stages its rows through LDS (which takes the weight as it stands in the checkpoint), to the last bit."""
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n + N)
+    x, w = rnd(n, K, g=g, dtype=torch.bfloat16), rnd(N, K, g=g, dtype=torch.bfloat16, scale=K ** -0.5)
+    for rs in (None, ops.RowScale(torch.rand(n, 21, generator=g, device=DEV) + 0.1, 1e-3)):
+        outs = [torch.full((n, N), float("nan"), dtype=dtype, device=DEV) for _ in range(2)]
+        for weight, out in zip((ops.TiledWeight(w), w), outs):
+            kw = {"activation": "relu_squared"} if mode == "act" else {}
+            ops.gemm_skinny(x, weight, out, 0.75, mode=mode, row_scale=rs, **kw)
+        assert torch.equal(*outs)
