@@ -256,12 +256,16 @@ extern "C" const char* cpmcu_moe_route(const void* h, long ldh, int dtype, const
 
 #define MOE_ROWS 4       // output rows a wavefront (moe_down_kernel names its four)
 
-// grid (tokens * top, ceil(F / 16)), 256 threads: wavefront w takes rows [16 y + 4 w, +4) of the expert's F, gate and up
+// grid (ceil(F / 16), tokens * top), 256 threads: wavefront w takes rows [16 x + 4 w, +4) of the expert's F, gate and up
 // rows together, for all pairs of its run of 128 that chose the expert, up to 4 at a time against the same weights; the
 // workgroups of the expert's other pairs in the run end at once.  The weights bound it: 8 tokens with 6 of 64 experts of
 // 1,408 at width 4,096 (48 pairs, 35 experts) 179 -> 151 us, 5.4 TB/s; 15 tokens 283 -> 192, one token 41 -> 31.  A
 // pair's sums do not depend on which others share its expert.
+// An expert's workgroups are neighbours in the grid and so are dealt to all 8 XCDs alike: with the pairs first, 48 of them
+// gave XCD i the experts of pairs i, i + 8, ..., of which only the first of each expert's
+// have work: 8 tokens 148 -> 127 us (6.5 TB/s), 16 tokens 252 -> 178, 4 tokens 80 -> 76, 2 tokens and 1 the same.
 #define MOE_RUN 128
+#define MOE_GRID_Y 32768
 
 template <typename T, int NT>
 __device__ inline void gated_rows(const T* __restrict__ h, long ldh, const T* __restrict__ wg, const long (&pair)[4],
@@ -329,13 +333,15 @@ __global__ __launch_bounds__(256) void moe_gated_kernel(const T* __restrict__ h,
                                                         const int* __restrict__ idx, T* __restrict__ act, int H, int F,
                                                         int top, int E, int n_pairs, int act_fn, float act_limit) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int run0 = blockIdx.x / MOE_RUN * MOE_RUN, own = blockIdx.x - run0;
+    const int p0 = blockIdx.z * MOE_GRID_Y + blockIdx.y;
+    if (p0 >= n_pairs) return;
+    const int run0 = p0 / MOE_RUN * MOE_RUN, own = p0 - run0;
     const int a = run0 + lane < n_pairs ? idx[run0 + lane] : -1, b = run0 + 64 + lane < n_pairs ? idx[run0 + 64 + lane] : -1;
     const int e = own < 64 ? __builtin_amdgcn_readlane(a, own & 63) : __builtin_amdgcn_readlane(b, own & 63);
     if (e >= E) return;                 // an identity expert
     unsigned long long first = __builtin_amdgcn_ballot_w64(a == e), second = __builtin_amdgcn_ballot_w64(b == e);
     if ((first ? __builtin_ctzll(first) : 64 + __builtin_ctzll(second)) != own) return;
-    const int j0 = blockIdx.y * 4 * MOE_ROWS + wave * MOE_ROWS;
+    const int j0 = blockIdx.x * 4 * MOE_ROWS + wave * MOE_ROWS;
     if (j0 >= F) return;
     const T* wg = wgu + (long)e * 2 * F * H;
     const bool vec = (H % 8 == 0) && (ldh % 8 == 0) && ((uintptr_t)h % 32 == 0) && ((uintptr_t)wgu % 32 == 0);
@@ -368,11 +374,13 @@ extern "C" const char* cpmcu_moe_gated(const void* h, long ldh, int dtype, const
     CPMCU_REQUIRE(CPMCU_ACT_KNOWN(act_fn), "moe_gated: unknown nonlinearity %d", act_fn);
     const int fy = (F + 4 * MOE_ROWS - 1) / (4 * MOE_ROWS);
     CPMCU_REQUIRE(fy <= 65535, "moe_gated: %d rows an expert exceed the launch grid", F);
-    dim3 grid((unsigned)((long)n * top), fy);
+    const long pairs = (long)n * top;
+    CPMCU_REQUIRE(pairs < (1L << 31), "moe_gated: %ld pairs", pairs);
+    const dim3 grid(fy, (unsigned)(pairs < MOE_GRID_Y ? pairs : MOE_GRID_Y), (unsigned)((pairs + MOE_GRID_Y - 1) / MOE_GRID_Y));
     if (dtype == CPMCU_F32)
-        moe_gated_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, ldh, (const float*)wgu, idx, (float*)act, H, F, top, E, (int)grid.x, act_fn, act_limit);
+        moe_gated_kernel<float><<<grid, 256, 0, stream>>>((const float*)h, ldh, (const float*)wgu, idx, (float*)act, H, F, top, E, (int)pairs, act_fn, act_limit);
     else if (dtype == CPMCU_BF16)
-        moe_gated_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)h, ldh, (const bf16_t*)wgu, idx, (bf16_t*)act, H, F, top, E, (int)grid.x, act_fn, act_limit);
+        moe_gated_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)h, ldh, (const bf16_t*)wgu, idx, (bf16_t*)act, H, F, top, E, (int)pairs, act_fn, act_limit);
     else
         CPMCU_FAIL("moe_gated: unknown dtype %d", dtype);
     CPMCU_LAUNCH_CHECK("moe_gated");
@@ -461,10 +469,19 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const T* __restrict__ act
                                                        long shared_stride, const float* __restrict__ sg,
                                                        const T* __restrict__ h, long ldh, int E,
                                                        float* __restrict__ out, int H, int F, int top, Join join) {
-    const long t = blockIdx.x;
+    // Workgroups are dealt to the 8 XCDs in turn: an XCD's take all tokens of a block of columns one behind the other, and tokens that
+    // share an expert find its rows in that L2 (the experts above: 16 tokens 152 -> 132 us, 12 117 -> 107, 8 83 -> 80).
+    long t = blockIdx.x;
+    int block = blockIdx.y;
+    const int n = gridDim.x, whole = gridDim.y / 8 * 8;
+    if (block < whole) {
+        const long lin = (long)block * n + t, i = lin / 8;
+        t = i % n;
+        block = (int)(i / n) * 8 + (int)(lin % 8);
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const bool vec = (F % 8 == 0) && ((uintptr_t)act % 32 == 0) && ((uintptr_t)wd % 32 == 0);
-    const int c0 = blockIdx.y * 4 * MOE_ROWS + wave * MOE_ROWS;
+    const int c0 = block * 4 * MOE_ROWS + wave * MOE_ROWS;
     if (c0 >= H) return;
     const int mine = c0 + (lane >> 4), p0 = lane & 15;               // this lane's column at the end, and its part
     const long at = t * H + min(mine, H - 1);
