@@ -666,6 +666,11 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
 // With up to 64 rows a tile, where most weights are read once, they are streamed past the caches: both products of 24
 // tokens 338 -> 322 us, of 300 tokens 433 -> 403; with more tokens tiles share weights.
 // Two pieces on their way at once: one made no difference beyond 300 tokens, at 24 it took 234 + 122 us.
+// Of 128-row tiles there is a form for every 16 rows, and results leave through LDS as whole lines (every lane stored its
+// 2 bytes): 2,048 tokens, both products and the sum, us: 64 experts of 1,408, 6 of 80 (16 identity) 791 -> 748, of 64 864
+// -> 802; of 2,112 without a gate 831 -> 774; 512 tokens 513 -> 496, 1,024 of 2,112 621 -> 588.
+// What bounds the wide tiles is the stream of pieces: products without stores or multiplications take 80% of the time, and
+// 256 rows or 256 weight rows a workgroup of 8 wavefronts, with half of the LDS reads, were no faster (449 to 540 us for 420).
 // The grid is dealt to the 8 XCDs in turn; each takes one run of the tasks, ordered expert by expert and within an expert
 // weight rows by weight rows, so that the tiles that share weights meet in one L2.
 template <int KIND, int RT>
@@ -698,6 +703,7 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
     }
     const int place = lrow * 8 + (chunk ^ (lrow & 7));                // rows 32 apart have the same place in their 256
 
+    const bool whole = (uintptr_t)out % 16 == 0;                      // (pair outputs may start anywhere)
     auto product = [&](auto groups) {
         constexpr int NRT = decltype(groups)::value, AP = (NRT + 1) / 2;
         const bf16_t* ap[AP];
@@ -733,7 +739,7 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
             for (int i = 0; i < 4; ++i) lds[buf][BM * 8 + 256 * i + place] = p.w[i];
 #pragma unroll
             for (int i = 0; i < AP; ++i)
-                if (NRT > 1 || lrow < 16) lds[buf][256 * i + place] = p.a[i];
+                if (NRT % 2 == 0 || i + 1 < AP || lrow < 16) lds[buf][256 * i + place] = p.a[i];
             if (!decltype(last)::value) fetch(p, k0 + 128);
             __syncthreads();
             mbf16x8_t a[2][NRT], b[2][2];
@@ -774,31 +780,46 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
         }
         if (k0 < K) step(p0, k0, 0, std::true_type());
         if (k0 + 64 < K) step(p1, k0 + 64, 1, std::true_type());
-        // lane (weight row r, g): acc[rt][j][i] belongs to the tile's row rt * 16 + 4 g + i
+        // lane (weight row r, g): acc[rt][j][i] belongs to the tile's row rt * 16 + 4 g + i.  The results pass through LDS, so
+        // that 8 or 16 neighbouring lanes write a row's 16-byte chunks
+        constexpr int LINE = FEATURES + 8;
+        bf16_t* stage = (bf16_t*)lds;
+        __syncthreads();
 #pragma unroll
         for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int row = rt * 16 + 4 * g + i;
-                if (row >= n_rows) continue;
-                bf16_t* to = out + (long)rows[row0 + row] * N;
+                bf16_t* to = stage + (rt * 16 + 4 * g + i) * LINE + wave * (FEATURES / 4) + r;
                 if (KIND == MOE_GATED) {
-                    const int f = f0 + wave * 16 + r;
                     float gt = acc[rt][0][i], up = acc[rt][1][i];
                     gate_prepare(gt, up, act_fn, act_limit);
-                    if (f < N) to[f] = f32_to_bf16(gate_act(gt, act_fn) * up);
+                    *to = f32_to_bf16(gate_act(gt, act_fn) * up);
                 } else {
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const int f = f0 + wave * 32 + j * 16 + r;
-                        if (f < N) to[f] = f32_to_bf16(KIND == MOE_PLAIN ? plain_act(acc[rt][j][i], act_fn) : acc[rt][j][i]);
-                    }
+                    for (int j = 0; j < 2; ++j)
+                        to[j * 16] = f32_to_bf16(KIND == MOE_PLAIN ? plain_act(acc[rt][j][i], act_fn) : acc[rt][j][i]);
+                }
+            }
+        __syncthreads();
+        constexpr int CHUNKS = FEATURES / 8;
+        const int c = threadIdx.x % CHUNKS * 8;
+        if (f0 + c < N)                                               // (N % 8 == 0: the whole chunk)
+            for (int row = threadIdx.x / CHUNKS; row < n_rows; row += 256 / CHUNKS) {
+                bf16_t* to = out + (long)rows[row0 + row] * N + f0 + c;
+                const bf16_t* from = stage + row * LINE + c;
+                if (whole) {
+                    *(mu32x4_t*)to = *(const mu32x4_t*)from;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) to[j] = from[j];
                 }
             }
     };
     if constexpr (RT > 4) {
-        if (n_rows > 96) { product(std::integral_constant<int, 8>()); return; }
-        if (n_rows > 64) { product(std::integral_constant<int, 6>()); return; }
+        if (n_rows > 112) { product(std::integral_constant<int, 8>()); return; }
+        if (n_rows > 96) { product(std::integral_constant<int, 7>()); return; }
+        if (n_rows > 80) { product(std::integral_constant<int, 6>()); return; }
+        if (n_rows > 64) { product(std::integral_constant<int, 5>()); return; }
     }
     if (n_rows > 32) product(std::integral_constant<int, 4>());
     else if (n_rows > 16) product(std::integral_constant<int, 2>());

@@ -46,3 +46,38 @@ def test_tiles_of_every_fill(rows, H, F, gated):
     off = F * sums * torch.einsum("nf,nhf->nh", got.abs(), down.double().abs()[e])
     off = off + half * (ref.abs() + off)
     assert bool(((out.double() - w.double() * ref).abs() <= w.double() * off + 2 * sums * ref.abs() + 1e-30).all())
+
+
+@pytest.mark.parametrize("rows", [[80, 112], [81, 79, 97], [65, 113, 64]])
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("H,F", [(136, 72), (264, 200)])
+def test_pair_outputs_at_any_address(rows, gated, H, F):
+    """Rows between the forms of wide tiles; pair outputs off 16-byte borders, which are stored element by element: the same."""
+    from cpmcu_amd import ops
+    E, n = len(rows), sum(rows)
+    g = torch.Generator(device=DEV).manual_seed(n + H)
+    idx = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(rows)]).to(DEV)[:, None].contiguous()
+    h = torch.randn(n, H, generator=g, device=DEV).to(torch.bfloat16)
+    up = torch.randn(E, F * (2 if gated else 1), H, generator=g, device=DEV).to(torch.bfloat16)
+    down = torch.randn(E, H, F, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.rand(n, 1, generator=g, device=DEV)
+    tiles = ops.moe_tiles(n, 1, E)
+    i32 = lambda k: torch.empty(k, dtype=torch.int32, device=DEV)
+
+    def run(offset):
+        act = torch.full((n, 1, F), float("nan"), dtype=torch.bfloat16, device=DEV)
+        y = torch.full((n * H + offset + 1,), float("nan"), dtype=torch.bfloat16, device=DEV)
+        out = torch.empty(n, H, device=DEV)
+        ops.moe_experts_mfma(h, up, down, idx, w, out, act, y[offset:offset + n * H].view(n, 1, H), i32(tiles * ops.MOE_TILE),
+                             i32(tiles), i32(1), gated=gated, activation="silu" if gated else "relu_squared")
+        assert bool(y[:offset].isnan().all()) and bool(y[offset + n * H:].isnan().all())
+        return out, act
+
+    (out, act), (out1, act1) = run(0), run(1)
+    assert bool(out.isfinite().all()) and torch.equal(out, out1) and torch.equal(act, act1)
+    e = idx[:, 0].long()
+    want = torch.einsum("nf,nhf->nh", act[:, 0].double(), down.double()[e])
+    mag = torch.einsum("nf,nhf->nh", act[:, 0].double().abs(), down.double().abs()[e])
+    off = F * 2.0 ** -23 * mag                                       # float sums in any order, one rounding to bf16
+    off = off + 2.0 ** -8 * (want.abs() + off)
+    assert bool(((out.double() - w.double() * want).abs() <= w.double() * off + 2.0 ** -22 * want.abs() + 1e-30).all())
