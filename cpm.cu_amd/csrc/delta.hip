@@ -195,6 +195,108 @@ __global__ __launch_bounds__(256) void delta_scan_kernel(const float* __restrict
     }
 }
 
+// The same walk where every sequence brings one token (any number is walked right): the tile's 16 or 32 rows of LDS, their
+// norms and their barriers are a token's.  A workgroup asks for its share of the state first; the decays of the key channels
+// pass through LDS, one a thread.  TPT: threads that share the norms' sums; every sum keeps the walk's order, so results are
+// the same (with a decay a head the compiler may fuse g S + k u the other way).  32 heads of 128 by 128, us, walk -> here:
+// 8 sequences in a serving, a decay a channel 26.7 -> 10.7, fixed decays 14.9 -> 10.4 (their states' 34 MB in and out take 5);
+// 24 in a chain of calls 63 -> 29, 31 -> 27, a decay a head 42 -> 28; 64, a decay a channel 153 -> 63.
+template <int NR, int TPT, int DELTA_L, typename GT, int RULE>
+__global__ __launch_bounds__(256) void delta_step_kernel(const float* __restrict__ qkv, long ld,
+                                                         const GT* __restrict__ gates, long ldg, long a_off, long b_off,
+                                                         const float* __restrict__ chan_a, long ld_a,
+                                                         const float* __restrict__ dt_bias,
+                                                         const float* __restrict__ A_log, float* __restrict__ state,
+                                                         float* __restrict__ y, const int* __restrict__ cu_q,
+                                                         const int* __restrict__ seq_slot, int heads, int kv_heads,
+                                                         int dk, int dv, float q_scale, int write_state) {
+    constexpr int NS = NR * DELTA_L;                // state values a column, padded
+    static_assert(NS <= 256, "a thread a key feature");
+    __shared__ float qs[2][NS], ks[2][NS], gcs[2][RULE == RULE_CHANNEL ? NS : 1];
+    const int b = blockIdx.x / heads, h = grouped_head(blockIdx.x % heads, heads, kv_heads);
+    const int start = cu_q[b], n_q = cu_q[b + 1] - start;
+    const int kvh = h / (heads / kv_heads);
+    const long k_col = (long)kv_heads * dk, v_col = 2L * kv_heads * dk;
+    const int l = threadIdx.x % DELTA_L, p = blockIdx.y * (256 / DELTA_L) + threadIdx.x / DELTA_L;
+    const bool p_ok = p < dv;
+    float* sp = state + (((long)seq_slot[b] * heads + h) * dv + (p_ok ? p : 0)) * dk;
+    float S[NR];
+#pragma unroll
+    for (int i = 0; i < NR; ++i) S[i] = sp[min(l + DELTA_L * i, dk - 1)];
+    const float A = RULE == RULE_DECAY ? A_log[h] : expf(A_log[h]);
+    const float bias = RULE == RULE_DELTA ? dt_bias[h] : 0.f;
+    const int n_own = min((int)threadIdx.x, dk - 1);
+    const bool own = (int)threadIdx.x < dk;
+    for (int tt = 0; tt < n_q; ++tt) {
+        const int buf = tt & 1;
+        const float* row = qkv + (long)(start + tt) * ld + (long)kvh * dk + n_own;
+        const float rq = row[0], rk = row[k_col];
+        const float vv = p_ok ? qkv[(long)(start + tt) * ld + v_col + (long)h * dv + p] : 0.f;
+        float beta = 1.0f, g = A;
+        if (RULE != RULE_DECAY) {
+            const GT* gr = gates + (long)(start + tt) * ldg;
+            beta = 1.0f / (1.0f + expf(-to_f32(gr[b_off + h])));
+            if (RULE == RULE_DELTA) g = expf(-A * delta_softplus(to_f32(gr[a_off + h]) + bias));
+        }
+        if (threadIdx.x < NS) {
+            qs[buf][threadIdx.x] = own ? rq : 0.f;
+            ks[buf][threadIdx.x] = own ? rk : 0.f;
+            if (RULE == RULE_CHANNEL) {
+                const float a = chan_a[(long)(start + tt) * ld_a + (long)h * dk + n_own] + dt_bias[(long)h * dk + n_own];
+                gcs[buf][threadIdx.x] = expf(-A * delta_softplus(own ? a : 0.f));
+            }
+        }
+        __syncthreads();
+        float sq = 0.f, sk = 0.f, dot = 0.f;
+#pragma unroll
+        for (int n = threadIdx.x % TPT; n < NS; n += TPT) {
+            const float a = qs[buf][n], c = ks[buf][n];
+            sq += a * a;
+            sk += c * c;
+            dot += a * c;
+        }
+        sq = lanes_sum<TPT>(sq);
+        sk = lanes_sum<TPT>(sk);
+        dot = lanes_sum<TPT>(dot);
+        float fq = 1.0f, fk = 1.0f, kq = dot;
+        if (RULE != RULE_DECAY) {
+            fq = q_scale / sqrtf(sq + 1e-6f);
+            fk = 1.0f / sqrtf(sk + 1e-6f);
+            kq = dot * fq * fk;
+        }
+        float kr[NR];
+        float r = 0.f, o = 0.f;
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int n = l + DELTA_L * i;
+            if (tt == 0 && !(p_ok && n < dk)) S[i] = 0.f;
+            float qr = qs[buf][n];
+            kr[i] = ks[buf][n];
+            if (RULE != RULE_DECAY) {
+                qr *= fq;
+                kr[i] *= fk;
+            }
+            if (RULE == RULE_CHANNEL) S[i] *= gcs[buf][n];
+            if (RULE != RULE_DECAY) r += S[i] * kr[i];
+            o += S[i] * qr;
+        }
+        r = lanes_sum<DELTA_L>(r);
+        o = lanes_sum<DELTA_L>(o);
+        const float gg = RULE == RULE_CHANNEL ? 1.0f : g;
+        const float u = RULE == RULE_DECAY ? vv : beta * (vv - gg * r);
+#pragma unroll
+        for (int i = 0; i < NR; ++i) S[i] = gg * S[i] + kr[i] * u;
+        if (l == 0 && p_ok) y[(long)(start + tt) * heads * dv + (long)h * dv + p] = gg * o + kq * u;
+    }
+    if (write_state && p_ok && n_q > 0) {
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            const int n = l + DELTA_L * i;
+            if (n < dk) sp[n] = S[i];
+        }
+    }
+}
+
 // ---------------------------------------------------------------------------
 // The delta rule with a decay a head (RULE_DELTA) for prompts, 64 tokens at a time on the matrix cores' float instruction
 // (v_mfma_f32_16x16x4_f32: operands as they are, sums in float).  With la_t = the sum of ln g over the chunk's tokens up to
@@ -514,7 +616,7 @@ __global__ __launch_bounds__(512) void delta_chunk_kernel(const float* __restric
 extern "C" const char* cpmcu_delta_scan(const float* qkv, long ld, const void* gates, long ldg, int gate_dtype,
                                         long a_off, long b_off, const float* chan_a, long ld_a, const float* dt_bias,
                                         const float* A_log, float* state, float* y, const int* cu_q,
-                                        const int* seq_slot, int n_seqs, int heads, int kv_heads, int dk, int dv,
+                                        const int* seq_slot, int n_rows, int n_seqs, int heads, int kv_heads, int dk, int dv,
                                         float q_scale, int write_state, int lanes, int rule, int chunk_from,
                                         int n_chunked, hipStream_t stream) {
     CPMCU_REQUIRE(rule == RULE_DELTA || rule == RULE_CHANNEL || rule == RULE_DECAY, "delta_scan: unknown rule %d", rule);
@@ -568,25 +670,30 @@ extern "C" const char* cpmcu_delta_scan(const float* qkv, long ld, const void* g
     CPMCU_REQUIRE(pb <= 65535, "delta_scan: shape exceeds the launch grid");
     dim3 grid(heads * n_walked, pb);
     const int need = (dk + lanes - 1) / lanes;
+    const bool one = n_rows == n_seqs && n_chunked == 0;                // as a step of decoding does
 #define LAUNCH(NRv, TTv, Lv, GTv, Rv)                                                                                \
-    delta_scan_kernel<NRv, TTv, Lv, GTv, Rv><<<grid, 256, 0, stream>>>(qkv, ld, (const GTv*)gates, ldg, a_off, b_off, \
+    if (one)                                                                                                          \
+        delta_step_kernel<NRv, 256 / TTv, Lv, GTv, Rv><<<grid, 256, 0, stream>>>(qkv, ld, (const GTv*)gates, ldg, a_off, b_off, \
+                                                                                 chan_a, ld_a, dt_bias, A_log, state, y, cu_q, \
+                                                                                 seq_slot, heads, kv_heads, dk, dv, q_scale, write_state); \
+    else delta_scan_kernel<NRv, TTv, Lv, GTv, Rv><<<grid, 256, 0, stream>>>(qkv, ld, (const GTv*)gates, ldg, a_off, b_off, \
                                                                        chan_a, ld_a, dt_bias, A_log, state, y, cu_q,  \
                                                                        seq_slot, heads, kv_heads, dk, dv, q_scale,    \
                                                                        write_state, n_seqs, lo, hi)
-#define BY_NR(GTv, Rv)                                        \
-    do {                                                      \
-        if (lanes == 16) {                                    \
-            if (need <= 2) LAUNCH(2, 32, 16, GTv, Rv);        \
-            else if (need <= 4) LAUNCH(4, 32, 16, GTv, Rv);   \
-            else if (need <= 8) LAUNCH(8, 32, 16, GTv, Rv);   \
-            else LAUNCH(16, 16, 16, GTv, Rv);                 \
-        } else {                                              \
-            if (need <= 2) LAUNCH(2, 32, 8, GTv, Rv);         \
-            else if (need <= 4) LAUNCH(4, 32, 8, GTv, Rv);    \
-            else if (need <= 8) LAUNCH(8, 32, 8, GTv, Rv);    \
-            else if (need <= 16) LAUNCH(16, 32, 8, GTv, Rv);  \
-            else LAUNCH(32, 16, 8, GTv, Rv);                  \
-        }                                                     \
+#define BY_NR(GTv, Rv)                                              \
+    do {                                                            \
+        if (lanes == 16) {                                          \
+            if (need <= 2) { LAUNCH(2, 32, 16, GTv, Rv); }          \
+            else if (need <= 4) { LAUNCH(4, 32, 16, GTv, Rv); }     \
+            else if (need <= 8) { LAUNCH(8, 32, 16, GTv, Rv); }     \
+            else { LAUNCH(16, 16, 16, GTv, Rv); }                   \
+        } else {                                                    \
+            if (need <= 2) { LAUNCH(2, 32, 8, GTv, Rv); }           \
+            else if (need <= 4) { LAUNCH(4, 32, 8, GTv, Rv); }      \
+            else if (need <= 8) { LAUNCH(8, 32, 8, GTv, Rv); }      \
+            else if (need <= 16) { LAUNCH(16, 32, 8, GTv, Rv); }    \
+            else { LAUNCH(32, 16, 8, GTv, Rv); }                    \
+        }                                                           \
     } while (0)
     if (rule == RULE_DECAY) BY_NR(float, RULE_DECAY);
     else if (gate_dtype == CPMCU_F32 && rule == RULE_DELTA) BY_NR(float, RULE_DELTA);

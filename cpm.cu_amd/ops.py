@@ -1330,7 +1330,7 @@ def delta_scan(qkv: torch.Tensor, gates: Optional[torch.Tensor], a_off: int, b_o
     _check(_fn("delta", "cpmcu_delta_scan")(_p(qkv), c_long(qkv.shape[1]), _p(gates), c_long(ldg),
                                             c_int(_code(gates) if gates is not None else 0), c_long(a_off), c_long(b_off),
                                             _p(channel_decay), c_long(ld_a), _p(dt_bias), _p(A_log), _p(state), _p(y),
-                                            _p(cu_q), _p(seq_slot), c_int(B), c_int(heads), c_int(kv_heads), c_int(dk),
+                                            _p(cu_q), _p(seq_slot), c_int(n), c_int(B), c_int(heads), c_int(kv_heads), c_int(dk),
                                             c_int(dv), c_float(q_scale), c_int(1 if write_state else 0), c_int(lanes),
                                             c_int(DELTA_RULES[rule]), *_chunk_args("delta", chunks, max_q, B), _stream()))
 
