@@ -15,7 +15,7 @@
 //     16 g + r holding row r, columns 32 i + 8 g ..), then the R - 16 further rows packed as [i][g][row][8].
 // One workgroup of 4 wavefronts: the wavefronts take a quarter of the columns each (x straight from global
 // memory into the B operand, asked for together with the weight's block), add their results through LDS, and
-// the first wavefront rotates and writes: queries to q_out [token][head][d], keys and values into the cache
+// a wavefront a tile of 16 tokens rotates and writes: queries to q_out [token][head][d], keys and values into the cache
 // pages in the matrix cores' order (common.h: key_index, value_index).
 // theta = pos * inv_freq[c]; (a, b) = (x[c], x[c+hd/2]) -> (a cos - b sin, a sin + b cos), cos and sin times
 // `mscale` (reference: src/model/rotary.cuh:7-34; cache rows src/model/attn.cuh:14-21; the fused decode
@@ -34,7 +34,8 @@ __global__ __launch_bounds__(NW * 64) void qkv_rope_kernel(
     const float* __restrict__ inv_freq, float mscale, bf16_t* __restrict__ kpool, bf16_t* __restrict__ vpool,
     PagedView pv, const float* __restrict__ row_ss, int ss_slices, float eps, bf16_t* __restrict__ ckpool,
     int ck_size, int ck_stride) {
-    __shared__ float red[NW - 1][MT][TILES][4][64];
+    static_assert(MT <= NW, "a wavefront a tile of tokens at the end");
+    __shared__ float red[NW][MT][TILES][4][64];
     __shared__ float rs_s[MT * 16];            // the norm's row factors (common.h: row_scales), if x lacks them
     const int wg = blockIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -84,15 +85,10 @@ __global__ __launch_bounds__(NW * 64) void qkv_rope_kernel(
     // frequencies) is asked for first: it is there when the products are, instead of costing three trips to
     // memory after them.  A lane holds, per tile, rows 4g .. 4g+3 of the workgroup's: two pairs (or 4 rows of v).
     const int total_rows = (nh + 2 * nkv) * hd;
-    int tok_pos[MT];
-    long tok_row[MT];
     const bool has_kv = (long)(wg + 1) * R > (long)nh * hd;      // some row of this workgroup goes into the cache
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int tok = min(t * 16 + r, M - 1);
-        tok_pos[t] = positions[tok];
-        tok_row[t] = has_kv ? paged_row(pv, tok_slot[tok], tok_pos[t]) : 0;
-    }
+    const int tok = min(wave, MT - 1) * 16 + r;                  // whose results this lane finishes
+    const int tok_in = min(tok, M - 1), tok_pos = positions[tok_in];
+    const long tok_row = has_kv ? paged_row(pv, tok_slot[tok_in], tok_pos) : 0;
     // row P of the re-laid weight: head P / hd; inside a q or k head, pair (P % hd) / 2, half (P % hd) % 2
     int pair_head[TILES][2], pair_in[TILES][2];                  // head and first row inside it (even) of a lane's pairs
     bool pair_ok[TILES][2];
@@ -121,21 +117,19 @@ __global__ __launch_bounds__(NW * 64) void qkv_rope_kernel(
 #pragma unroll
     for (int j = 0; j < PF; ++j) load_block(kb0 + j, a[j], bx[j]);
     // the pairs' cosines and sines are formed while the first blocks are on their way
-    float rot_cs[MT][TILES][2], rot_sn[MT][TILES][2];
+    float rot_cs[TILES][2], rot_sn[TILES][2];
 #pragma unroll
-    for (int t = 0; t < MT; ++t)
+    for (int T = 0; T < TILES; ++T)
 #pragma unroll
-        for (int T = 0; T < TILES; ++T)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                rot_cs[t][T][j] = 1.f;
-                rot_sn[t][T][j] = 0.f;
-                if (inv_freq && pair_head[T][j] < nh + nkv) {
-                    const float ang = (float)tok_pos[t] * freq[T][j];
-                    rot_cs[t][T][j] = cosf(ang) * mscale;
-                    rot_sn[t][T][j] = sinf(ang) * mscale;
-                }
+        for (int j = 0; j < 2; ++j) {
+            rot_cs[T][j] = 1.f;
+            rot_sn[T][j] = 0.f;
+            if (inv_freq && pair_head[T][j] < nh + nkv && wave < MT) {
+                const float ang = (float)tok_pos * freq[T][j];
+                rot_cs[T][j] = cosf(ang) * mscale;
+                rot_sn[T][j] = sinf(ang) * mscale;
             }
+        }
     if (row_ss && wave < 4) row_scales<256, MT * 16>(row_ss, ss_slices, M, 1.0f / (float)K, eps, rs_s);
     int kb = kb0;
     for (; kb + 2 * PF <= kb1; kb += PF) {           // every block and every block asked for exists
@@ -152,91 +146,75 @@ __global__ __launch_bounds__(NW * 64) void qkv_rope_kernel(
             if (kb + j + PF < kb1) load_block(kb + j + PF, a[j], bx[j]);
         }
     }
-    // lane (token r, g) of tile t: acc[t][T][i] is row 16T + 4g + i of the workgroup; the other wavefronts hand
-    // theirs to the first
-    if (wave > 0) {
+    // lane (token r, g) of tile t: acc[t][T][i] is row 16T + 4g + i of the workgroup; tile t's results meet in wavefront t,
+    // in the wavefronts' order
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
-#pragma unroll
-            for (int T = 0; T < TILES; ++T)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) red[wave - 1][t][T][i][lane] = acc[t][T][i];
-    }
-    __syncthreads();
-    if (wave > 0) return;
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
+    for (int t = 0; t < MT; ++t)
 #pragma unroll
         for (int T = 0; T < TILES; ++T)
 #pragma unroll
             for (int i = 0; i < 4; ++i)
+                if (MT > 1 || wave > 0) red[wave][t][T][i][lane] = acc[t][T][i];
+    __syncthreads();
+    if (wave >= MT && !ckpool) return;
+    const bool tok_ok = wave < MT && tok < M;
+    const float rs = row_ss && wave < MT ? rs_s[tok] : 1.0f;      // X was x * w of a norm whose row factor comes now
+    float own[TILES][2][2];                        // a key head's values as the cache holds them: [pair][half]
 #pragma unroll
-                for (int w = 0; w < NW - 1; ++w) acc[t][T][i] += red[w][t][T][i][lane];
-        if (row_ss) {          // X was x * w of a norm whose row factor comes now
-            const float rs = rs_s[t * 16 + r];
+    for (int T = 0; T < TILES; ++T)
 #pragma unroll
-            for (int T = 0; T < TILES; ++T)
+        for (int j = 0; j < 2; ++j) {
+            own[T][j][0] = own[T][j][1] = 0.f;
+            if (!pair_ok[T][j] || wave >= MT) continue;
+            const int head = pair_head[T][j], in = pair_in[T][j];
+            float lo = MT > 1 ? red[0][wave][T][2 * j][lane] : acc[0][T][2 * j];
+            float hi = MT > 1 ? red[0][wave][T][2 * j + 1][lane] : acc[0][T][2 * j + 1];
 #pragma unroll
-                for (int i = 0; i < 4; ++i) acc[t][T][i] *= rs;
-        }
-    }
-
-    float own[MT][TILES][2][2];                    // a key head's values as the cache holds them: [pair][half]
-#pragma unroll
-    for (int t = 0; t < MT; ++t) {
-        const int tok = t * 16 + r;
-        const bool tok_ok = tok < M;
-#pragma unroll
-        for (int T = 0; T < TILES; ++T)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) {
-                own[t][T][j][0] = own[t][T][j][1] = 0.f;
-                if (!pair_ok[T][j]) continue;
-                const int head = pair_head[T][j], in = pair_in[T][j];
-                const float lo = acc[t][T][2 * j], hi = acc[t][T][2 * j + 1];
-                if (head < nh + nkv) {
-                    const int c = in >> 1;
-                    const float cs = rot_cs[t][T][j], sn = rot_sn[t][T][j];
-                    const bf16_t v0 = f32_to_bf16(lo * cs - hi * sn), v1 = f32_to_bf16(lo * sn + hi * cs);
-                    own[t][T][j][0] = to_f32(v0);
-                    own[t][T][j][1] = to_f32(v1);
-                    if (!tok_ok) continue;
-                    if (head < nh) {
-                        bf16_t* dst = q_out + ((long)tok * nh + head) * hd;
-                        dst[c] = v0;
-                        dst[c + hd / 2] = v1;
-                    } else {
-                        bf16_t* dst = kpool + key_index(tok_row[t], head - nh, nkv, hd);
-                        dst[key_d_offset(c)] = v0;
-                        dst[key_d_offset(c + hd / 2)] = v1;
-                    }
-                } else if (tok_ok) {
-                    bf16_t* dst = vpool + value_index(tok_row[t], head - nh - nkv, nkv, hd);
-                    dst[value_d_offset(in)] = f32_to_bf16(lo);
-                    dst[value_d_offset(in + 1)] = f32_to_bf16(hi);
-                }
+            for (int w = 1; w < NW; ++w) {
+                lo += red[w][wave][T][2 * j][lane];
+                hi += red[w][wave][T][2 * j + 1][lane];
             }
-    }
+            if (row_ss) {
+                lo *= rs;
+                hi *= rs;
+            }
+            if (head < nh + nkv) {
+                const int c = in >> 1;
+                const float cs = rot_cs[T][j], sn = rot_sn[T][j];
+                const bf16_t v0 = f32_to_bf16(lo * cs - hi * sn), v1 = f32_to_bf16(lo * sn + hi * cs);
+                own[T][j][0] = to_f32(v0);
+                own[T][j][1] = to_f32(v1);
+                if (!tok_ok) continue;
+                if (head < nh) {
+                    bf16_t* dst = q_out + ((long)tok * nh + head) * hd;
+                    dst[c] = v0;
+                    dst[c + hd / 2] = v1;
+                } else {
+                    bf16_t* dst = kpool + key_index(tok_row, head - nh, nkv, hd);
+                    dst[key_d_offset(c)] = v0;
+                    dst[key_d_offset(c + hd / 2)] = v1;
+                }
+            } else if (tok_ok) {
+                bf16_t* dst = vpool + value_index(tok_row, head - nh - nkv, nkv, hd);
+                dst[value_d_offset(in)] = f32_to_bf16(lo);
+                dst[value_d_offset(in + 1)] = f32_to_bf16(hi);
+            }
+        }
 
     // Compressed keys (sparse.hip: compress_keys_kernel, the same sums in the same order): the token at position
     // p completes the mean of the keys p+1-ck_size .. p when p+1-ck_size is a non-negative multiple of ck_stride.
     // This workgroup wrote its features of all the step's keys itself; the fence makes them readable, and is
     // paid only in the steps in which a token completes one.
     if (ckpool && has_kv) {
-        bool mine[MT], any = false;
-#pragma unroll
-        for (int t = 0; t < MT; ++t) {
-            const int p1 = tok_pos[t] + 1;
-            mine[t] = t * 16 + r < M && p1 >= ck_size && (p1 - ck_size) % ck_stride == 0;
-            any = any || mine[t];
-        }
-        if (__any(any)) {
+        const int p1 = tok_pos + 1;
+        const bool mine = tok_ok && p1 >= ck_size && (p1 - ck_size) % ck_stride == 0;
+        // (all wavefronts come here: a step's other tokens, whose keys a mean may hold, belong to other wavefronts)
+        if (__syncthreads_or(mine)) {
             __threadfence();
-#pragma unroll
-            for (int t = 0; t < MT; ++t) {
-                if (!mine[t]) continue;
-                const int slot = tok_slot[t * 16 + r];
-                const int first = tok_pos[t] + 1 - ck_size;
+            __syncthreads();
+            if (mine) {
+                const int slot = tok_slot[tok];
+                const int first = tok_pos + 1 - ck_size;
                 const int page = pv.page_table[(long)slot * pv.table_width + first / pv.page_size];
                 const int rpp = pv.page_size / ck_stride;
 #pragma unroll
@@ -254,8 +232,8 @@ __global__ __launch_bounds__(NW * 64) void qkv_rope_kernel(
                             s1 += to_f32(src[key_d_offset(c + hd / 2)]);
                         }
                         bf16_t* dst = ckpool + ck_index(page, (first % pv.page_size) / ck_stride, kvh, nkv, hd, rpp);
-                        dst[ck_d_offset(c, rpp)] = f32_to_bf16((s0 + own[t][T][j][0]) / (float)ck_size);
-                        dst[ck_d_offset(c + hd / 2, rpp)] = f32_to_bf16((s1 + own[t][T][j][1]) / (float)ck_size);
+                        dst[ck_d_offset(c, rpp)] = f32_to_bf16((s0 + own[T][j][0]) / (float)ck_size);
+                        dst[ck_d_offset(c + hd / 2, rpp)] = f32_to_bf16((s1 + own[T][j][1]) / (float)ck_size);
                     }
             }
         }
@@ -310,10 +288,13 @@ extern "C" const char* cpmcu_qkv_rope(const void* X, long ldx, const void* W, in
                                                            (bf16_t*)ckpool, ck_size, ck_stride)
     // more tokens hold more of x in registers for every block in flight: fewer blocks then
     // K up to 1,024 has 8 blocks: one for each of 8 wavefronts, where 4 asked for 4 each and had 2 (1,280 x 1,024 in a chain of
-    // launches over weights that no cache holds, 1 / 8 / 32 tokens: 4.92/5.48/8.84 -> 4.28/4.56/6.74 us)
+    // launches over weights that no cache holds, captured, 1 / 8 / 32 / 64 tokens: 4.44/5.02/8.22/10.29 -> 3.92/4.24/5.48/7.40 us,
+    // a wavefront a tile of tokens finishing instead of one for all in it; 4,608 x 4,096 9.94/10.21/15.80/26.40 ->
+    // 9.68/9.69/14.20/21.48).  With 33 to 64 tokens the product in shares and the rotary kernel took 7.8 + 5.0.
     if (R == 16) {
         if (M <= 16 && K <= 1024) LAUNCH_OF(1, 8, 1, 1);
         else if (M <= 32 && M > 16 && K <= 1024) LAUNCH_OF(1, 8, 2, 1);
+        else if (M > 32 && K <= 1024) LAUNCH_OF(1, 8, 4, 1);
         else if (M <= 16) LAUNCH(4, 1, 1);
         else if (M <= 32) LAUNCH(4, 2, 1);
         else LAUNCH(2, 4, 1);

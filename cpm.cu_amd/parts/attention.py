@@ -86,7 +86,7 @@ class GQAAttention(Mixer):
     def _fused_projection(self, n: int, dtype, cache: Optional[CacheView], writes_cache: bool) -> bool:
         """Decode steps: projection, rotation and cache write in one kernel (one kernel of the chain less)."""
         plain_rotation = self._kernel_rotates()
-        return (writes_cache and cache is not None and plain_rotation and n <= ops.QKV_ROPE_MAX_ROWS
+        return (writes_cache and cache is not None and plain_rotation and ops.qkv_rope_faster(n, self.qkv.in_features)
                 and dtype == torch.bfloat16 and self.qkv.tiled is not None and self.hd % 16 == 0
                 and self.hidden_size % 8 == 0 and cache.page_size % 32 == 0)
 

@@ -63,3 +63,19 @@ def test_products_of_one_wavefront_a_strip(n, N, K, mode, dtype):
             kw = {"activation": "relu_squared"} if mode == "act" else {}
             ops.gemm_skinny(x, weight, out, 0.75, mode=mode, row_scale=rs, **kw)
         assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("n,H", [(33, 1024), (48, 1000), (49, 136), (64, 1024), (64, 8), (64, 1032)])
+@pytest.mark.parametrize("scaled", [False, True])
+def test_fused_projection_of_many_tokens(n, H, scaled):
+    """33 to 64 tokens: 8 wavefronts a workgroup up to 1,024 columns, tile t of the tokens finished by wavefront t."""
+    from test_kernels_gpu import test_fused_projection_rotation_and_cache_write as check
+    for nh, nkv, hd in ((3, 1, 16), (2, 2, 64)):
+        check(n, nh, nkv, hd, H, True, scaled, None)
+
+
+@pytest.mark.parametrize("n,ks,st", [(64, 32, 16), (40, 12, 4)])
+def test_compressed_keys_of_many_tokens(n, ks, st):
+    """A mean's keys of this step may come from several wavefronts."""
+    from test_kernels_gpu import test_fused_projection_completes_compressed_keys as check
+    check(n, ks, st, None)
