@@ -14,6 +14,7 @@
 //    and softmax, both element types; one wavefront a (token, head).
 //
 // Keys and values lie in their pages as common.h says (key_index, value_index), each with its own head size.
+#include "cache_order.h"
 #include "common.h"
 #include "vec4.h"
 
@@ -953,7 +954,7 @@ __global__ __launch_bounds__(64) void qkv_rotate_store_kernel(const T* __restric
                                                               const float* __restrict__ inv_freq, float mag,
                                                               T* __restrict__ kpool, T* __restrict__ vpool, PagedView pv,
                                                               int pool_hdk, int pool_hdv, int interleaved) {
-    const long t = blockIdx.x;
+    const long t = cache_order(blockIdx.x, gridDim.x);
     const int y = blockIdx.y, lane = threadIdx.x;
     const int pos = positions[t];
     const T* row = qkv + t * ld;
@@ -1029,7 +1030,7 @@ __global__ __launch_bounds__(64) void qkv_norm_rotate_store_kernel(
     int pool_hdk, int pool_hdv, int norm_after, int interleaved, const float* __restrict__ q_scale,
     const float* __restrict__ v_inv_freq, float temp_coef, int temp_every) {
     __shared__ float hs[AG_MAX_HD];
-    const long t = blockIdx.x;
+    const long t = cache_order(blockIdx.x, gridDim.x);
     const int y = blockIdx.y, lane = threadIdx.x;
     const int pos = positions[t];
     const bool is_q = y < nh, is_k = !is_q && y < nh + nkv;
@@ -1151,7 +1152,7 @@ __global__ __launch_bounds__(1024) void qkv_row_norm_store_kernel(
     long gate_col, T* __restrict__ gate_out) {
     extern __shared__ __attribute__((aligned(16))) float row_s[];
     __shared__ float red[17];
-    const long t = blockIdx.x;
+    const long t = cache_order(blockIdx.x, gridDim.x);
     const int what = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
     const int pos = positions[t];
     const int heads = what == 0 ? nh : nkv, hd = what == 2 ? dv : dk;
@@ -1283,7 +1284,7 @@ __global__ __launch_bounds__(256) void latent_store_kernel(const T* __restrict__
                                                            T* __restrict__ kpool, T* __restrict__ vpool, PagedView pv,
                                                            int pool_hdk, int pool_hdv) {
     __shared__ float red[17];
-    const long t = blockIdx.x;
+    const long t = cache_order(blockIdx.x, gridDim.x);
     int y = blockIdx.y;
     const int pos = positions[t];
     const int qw = dim + rot, dk = rank + rot;

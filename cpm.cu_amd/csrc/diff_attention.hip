@@ -11,6 +11,7 @@
 //    grouping; k goes into the key pages as 2 G heads, v into the value pages as G heads.
 //  * diff_combine_kernel: from the attention's output in that order, per (token, head):
 //    o = a1 - lambda a2; o / sqrt(mean(o^2) + eps) * post, written head by head in the design's order.
+#include "cache_order.h"
 #include "common.h"
 
 template <typename IT, typename T>
@@ -20,7 +21,7 @@ __global__ __launch_bounds__(64) void diff_qkv_store_kernel(const IT* __restrict
                                                             const int* __restrict__ tok_slot, T* __restrict__ kpool,
                                                             T* __restrict__ vpool, PagedView pv, int pool_hdk,
                                                             int pool_hdv) {
-    const long t = blockIdx.x;
+    const long t = cache_order(blockIdx.x, gridDim.x);
     const int y = blockIdx.y, lane = threadIdx.x;
     const int pos = positions[t];
     const IT* row = src + t * ld;

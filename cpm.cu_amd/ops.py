@@ -128,7 +128,7 @@ NORM_SLICE = 64        # columns a slice of add_norm_columns (common.h)
 # Up to 16 rows they win at every width measured (MI355X, 4,096 columns: norm 4.7 against 6.6 us at 8 rows).
 # qkv_rope (workgroups spread evenly over the CUs) wins up to 32 rows (4,096 columns, q/k/v + rotary: 11.7
 # against 18.2 us at 16 rows, 15.6 against 19.7 at 24, 16.5 against 21.3 at 32; it loses beyond: 24.6 against
-# 21.3 at 48, 27.2 against 23.2 at 64; with 1,024 columns it wins there too, 7 against 7.8 + 5.0 at 64), and proj_add_norm wins beyond 16 rows only while a workgroup's copy of
+# 21.3 at 48, 27.2 against 23.2 at 64; see qkv_rope_faster for fewer columns), and proj_add_norm wins beyond 16 rows only while a workgroup's copy of
 # x stays small (1,024 columns, 64 rows: 8.6 against 8.9 + 4.2 us).
 STRIP_ROWS = 16
 STRIP_MAX_ROWS = 64
@@ -143,8 +143,10 @@ def strip_kernels_ok(n: int, K: int) -> bool:
 
 
 def qkv_rope_faster(n: int, K: int) -> bool:
-    """Whether a step of n rows of K columns takes qkv_rope rather than the product and the rotary kernel."""
-    return n <= QKV_ROPE_MAX_ROWS or (n <= 64 and K <= 1024)
+    """Whether a step of n rows of K columns takes qkv_rope rather than the product in shares and the rotary kernel.  In a
+    chain of launches over weights that no cache holds, us, qkv_rope / the two kernels at 33, 48, 64 rows: 2,560 x 1,536
+    8.3/11.8, 9.3/12.4, 10.1/13.1; 2,560 x 2,048 9.6/9.7, 10.4/10.4, 11.6/11.5; 4,608 x 4,096 17.8/16.6, 19.5/17.4, 21.6/18.5."""
+    return n <= QKV_ROPE_MAX_ROWS or (n <= 64 and K < 2048)
 
 
 class RowScale:
