@@ -668,7 +668,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
 // Two pieces on their way at once: one made no difference beyond 300 tokens, at 24 it took 234 + 122 us.
 // Of 128-row tiles there is a form for every 16 rows, and results leave through LDS as whole lines (every lane stored its
 // 2 bytes): 2,048 tokens, both products and the sum, us: 64 experts of 1,408, 6 of 80 (16 identity) 791 -> 748, of 64 864
-// -> 802; of 2,112 without a gate 831 -> 774; 512 tokens 513 -> 496, 1,024 of 2,112 621 -> 588.
+// -> 802; of 2,112 without a gate 831 -> 774; 512 tokens 513 -> 496, 1,024 of 2,112 621 -> 588 (the sum unchanged there).
 // What bounds the wide tiles is the stream of pieces: products without stores or multiplications take 80% of the time, and
 // 256 rows or 256 weight rows a workgroup of 8 wavefronts, with half of the LDS reads, were no faster (449 to 540 us for 420).
 // The grid is dealt to the 8 XCDs in turn; each takes one run of the tasks, ordered expert by expert and within an expert
@@ -877,6 +877,60 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16_t* __restri
     }
 }
 
+// The same sums for up to 8 experts a token, a workgroup 2,048 columns of a token, 8 neighbouring ones a thread: the token's
+// experts and weights are scalars, and all TOP rows are asked for before the first is added (the kernel above has two in flight).
+// 2,048 tokens, 6 experts, width 4,096: 39.3 -> 22.5 us (100 MB of rows in, 34 out: 6 TB/s).
+template <typename ST, int TOP>
+__global__ __launch_bounds__(256) void moe_combine_token_kernel(const bf16_t* __restrict__ y, const float* __restrict__ w,
+                                                                const ST* __restrict__ shared, int shared_parts,
+                                                                long shared_stride, const float* __restrict__ sg,
+                                                                const int* __restrict__ idx, const bf16_t* __restrict__ h, long ldh,
+                                                                int E, float* __restrict__ out, int H, int pieces, Join join) {
+    const long t = blockIdx.x / pieces;
+    const int c = (int)(blockIdx.x % pieces) * 2048 + threadIdx.x * 8;
+    if (c >= H) return;
+    const long at = t * H + c;
+    mu32x4_t v[TOP];
+#pragma unroll
+    for (int k = 0; k < TOP; ++k)
+        v[k] = *(const mu32x4_t*)(idx[t * TOP + k] < E ? y + (t * TOP + k) * H + c : h + t * ldh + c);
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = 0.f;
+#pragma unroll
+    for (int k = 0; k < TOP; ++k) {
+        const float wk = w[t * TOP + k];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += wk * __uint_as_float(e & 1 ? v[k][e / 2] & 0xffff0000u : v[k][e / 2] << 16);
+    }
+    if (shared) {
+        const float g = sg ? sg[t] : 1.0f;
+        float a[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a[e] = 0.f;
+        for (int p = 0; p < shared_parts; ++p)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) a[e] += to_f32(shared[(long)p * shared_stride + at + e]);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += g * a[e];
+    }
+    if (join.x) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += join.x[at + e] + (join.a_bias ? join.a_bias[c + e] : 0.f);
+        for (int p = 0; p < join.a_parts; ++p)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) s[e] += join_part(join, p, at + e);
+    }
+    float* dst = (join.x ? join.x : out) + at;
+    *(float4*)dst = make_float4(s[0], s[1], s[2], s[3]);
+    *(float4*)(dst + 4) = make_float4(s[4], s[5], s[6], s[7]);
+    if (join.copy) {
+        bf16_t* copy = (bf16_t*)join.copy + at;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) copy[e] = f32_to_bf16(s[e]);
+    }
+}
+
 // scratch: rows int [max_tiles * 64] (the pairs by expert; its last E + 1 words are the experts' offsets), tile_expert int
 // [max_tiles], n_tiles int [1], y bf16 [n * top, H];
 // max_tiles = ceil(n * top / 64) + E
@@ -937,6 +991,23 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     const bool vec = H % 4 == 0 && ldh % 4 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)(x ? x : out) % 16 == 0;
     const long work = vec ? total / 4 : total;
     const int blocks = (int)((work + 255) / 256 < 8192 ? (work + 255) / 256 : 8192);
+    // (the token kernel's rows start on 16-byte borders: H % 8 == 0, and y and the result are looked at here)
+    if (top <= 8 && (uintptr_t)y % 16 == 0 && (uintptr_t)(x ? x : out) % 16 == 0 && (long)n * ((H + 2047) / 2048) < (1L << 31)) {
+        const int pieces = (H + 2047) / 2048;
+#define TOKENS(STv, TOPv)                                                                                                  \
+    case TOPv:                                                                                                             \
+        moe_combine_token_kernel<STv, TOPv><<<(unsigned)((long)n * pieces), 256, 0, stream>>>(                             \
+            (const bf16_t*)y, w, (const STv*)shared, shared_parts, shared_stride, sg, idx, (const bf16_t*)h, ldh, E, out, H, pieces, join); \
+        break
+#define BY_TOP(STv)                                                                                                        \
+    switch (top) { TOKENS(STv, 1); TOKENS(STv, 2); TOKENS(STv, 3); TOKENS(STv, 4); TOKENS(STv, 5); TOKENS(STv, 6); TOKENS(STv, 7); TOKENS(STv, 8); }
+        if (!shared || shared_dtype == CPMCU_F32) BY_TOP(float)
+        else BY_TOP(bf16_t)
+#undef BY_TOP
+#undef TOKENS
+        CPMCU_LAUNCH_CHECK("moe_combine");
+        return nullptr;
+    }
 #define COMBINE(STv, Vv)                                                                                              \
     moe_combine_kernel<STv, Vv><<<blocks, 256, 0, stream>>>((const bf16_t*)y, w, (const STv*)shared, shared_parts,   \
                                                             shared_stride, sg, idx, (const bf16_t*)h, ldh, E, out,  \

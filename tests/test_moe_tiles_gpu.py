@@ -81,3 +81,46 @@ def test_pair_outputs_at_any_address(rows, gated, H, F):
     off = F * 2.0 ** -23 * mag                                       # float sums in any order, one rounding to bf16
     off = off + 2.0 ** -8 * (want.abs() + off)
     assert bool(((out.double() - w.double() * want).abs() <= w.double() * off + 2.0 ** -22 * want.abs() + 1e-30).all())
+
+
+@pytest.mark.parametrize("top", [1, 2, 3, 4, 5, 6, 7, 8, 9])
+@pytest.mark.parametrize("H", [8, 2048, 2056])
+@pytest.mark.parametrize("shared_dtype", [None, torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("joined", [False, True])
+def test_sum_of_a_tokens_experts(top, H, shared_dtype, joined):
+    """The sum over a token's experts (identity experts among them), the shared expert and the layer's other result, for every
+    number that has its own form; pair outputs off 16-byte borders take the general one: the same."""
+    from cpmcu_amd import ops
+    E, F, n = 5, 16, 33
+    g = torch.Generator(device=DEV).manual_seed(top + H)
+    rnd = lambda *shape, dtype=torch.bfloat16: torch.randn(*shape, generator=g, device=DEV).to(dtype)
+    h, up, down = rnd(n, H), rnd(E, 2 * F, H) * 0.1, rnd(E, H, F)
+    idx = torch.randint(0, E + 2, (n, top), generator=torch.Generator().manual_seed(top), dtype=torch.int32).to(DEV)
+    w = torch.rand(n, top, generator=g, device=DEV)
+    shared = None if shared_dtype is None else rnd(2, n, H, dtype=shared_dtype) if shared_dtype == torch.float32 else rnd(n, H)
+    sg = None if shared is None else torch.rand(n, generator=g, device=DEV)
+    x0, a, bias = rnd(n, H, dtype=torch.float32), rnd(3, n, H, dtype=torch.float32), rnd(H, dtype=torch.float32)
+    tiles = ops.moe_tiles(n, top, E)
+    i32 = lambda k: torch.empty(k, dtype=torch.int32, device=DEV)
+
+    def run(offset):
+        act = torch.empty(n, top, F, dtype=torch.bfloat16, device=DEV)
+        y = torch.full((n * top * H + offset,), float("nan"), dtype=torch.bfloat16, device=DEV)[offset:].view(n, top, H)
+        x, copy, out = x0.clone(), torch.empty(n, H, dtype=torch.bfloat16, device=DEV), torch.empty(n, H, device=DEV)
+        join = ops.Join(x, a, bias, copy) if joined else None
+        ops.moe_experts_mfma(h, up, down, idx, w, None if joined else out, act, y, i32(tiles * ops.MOE_TILE), i32(tiles), i32(1), shared, sg, join=join)
+        return (x if joined else out), copy, y
+
+    got, copy, y = run(0)
+    other, copy1, _ = run(1)
+    assert torch.equal(got, other)
+    rows = torch.where((idx < E)[..., None], y.double(), h.double()[:, None])
+    terms = [w.double()[..., None] * rows]
+    if shared is not None:
+        terms.append((sg.double()[:, None] * (shared.double().sum(0) if shared.dim() == 3 else shared.double()))[:, None])
+    if joined:
+        terms += [x0.double()[:, None], a.double().transpose(0, 1), bias.double().expand(n, H)[:, None]]
+        assert torch.equal(copy, got.to(torch.bfloat16)) and torch.equal(copy, copy1)
+    terms = torch.cat(terms, 1)
+    mag = terms.abs().sum(1) + (0 if shared is None or shared.dim() < 3 else sg.double()[:, None] * shared.double().abs().sum(0))
+    assert bool(((got.double() - terms.sum(1)).abs() <= (terms.shape[1] + 3) * 2.0 ** -23 * mag).all())
