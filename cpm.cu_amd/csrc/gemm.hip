@@ -59,8 +59,8 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const XT* __restrict__ 
 
 // ---------------------------------------------------------------------------
 // The 32-bit product on the matrix cores.  v_mfma_f32_16x16x4_f32 takes float operands as they are and adds in float
-// (32 multiply-adds a cycle and SIMD, 157 TFLOP/s on the chip); v_mfma_f32_16x16x32_bf16 does 16 times as many, so that six
-// of its products, which a float as three bf16 asks for (below), still are 2.7 times as fast.
+// (32 multiply-adds a cycle and SIMD, 157 TFLOP/s on the chip); v_mfma_f32_16x16x32_bf16 does 16 times as many, so that eight
+// of its products, which a float as three bf16 asks for (below), still are twice as fast.
 //
 // gemm_f32_mfma_kernel: the float instruction, for few columns and for few rows of very many outputs.  256 threads, a
 // wavefront 16 x 16 of a 32 x 32 tile; 64 columns of both operands go through LDS in two buffers, the next ones on their way
@@ -136,31 +136,33 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 
 // ---------------------------------------------------------------------------
 // The same product with every float as the sum of three bf16, x = h + m + l: the upper 8 bits, the upper 8 of what is left
-// and the rest, exact for all that a float holds (down to 2^-110, where the last part ends below the smallest bf16).  Six of
-// the nine products, hh, hm, mh, mm, hl, lh, go through v_mfma_f32_16x16x32_bf16, whose sums are float, the small ones first;
-// the other three are below 2^-21 of a product at most and 2^-24 of it on average.  With a sum every 32 columns instead of
-// every 4 the result is nearer to a product in double than the float instruction's (relative error, before -> now: 1,024
-// columns 5.7e-7 -> 4.9e-7 and, with the columns shared out, 1.7e-7; 4,096 columns 1.15e-6 -> 1.0e-6 and 3.5e-7).
+// and the rest, exact for all that a float holds (down to 2^-110, where the last part ends below the smallest bf16).  Eight of
+// the nine products go through v_mfma_f32_16x16x32_bf16; the last parts' own, below 2^-30 of a product, is left out.  That
+// instruction cuts its sums' last bits where a float addition rounds them (all terms into one accumulator: sums of positive
+// products 4e-7 too small), so a piece of 32 columns has two sums that start from zero, hh and the seven others, which end 2^-7
+// below it, and meets the sum of the pieces in float additions.  Distance from a product in double, float instruction -> here:
+// 1,024 columns 5.7e-7 -> 1.1e-7 and, with the columns shared out, 7.9e-8; 4,096 columns 1.15e-6 -> 2.1e-7 and 1.0e-7; positive
+// numbers 4.9e-7 -> 9.0e-8; rows of which one element is not zero 2.5e-8 in both, four 4.0e-8 -> 2.7e-8.
 // Infinities, NaNs and results so small that the parts' own limit may show are worked out on the float instruction
 // (f32_finish_tile).
 //
 // gemm_f32_split_kernel: 64 rows against 64 TN outputs a workgroup.  X's piece of 32 columns is split once and its parts go
 // through LDS in two buffers; a wavefront splits its own 16 TN rows of W in registers, which nobody else needs.  Two pieces on
-// their way to registers.
+// their way to registers (of 48 outputs a wavefront one).
 // gemm_f32_shares_kernel: for outputs that give too few such workgroups: every one of 8 wavefronts has the whole tile of
 // 16 TM x 16 TN outputs and every eighth piece of the columns, no barrier until their sums meet in LDS.  Pieces are brought
 // whole lines a row (8 lanes each) and turned into operands through the wavefront's own LDS: loads straight into the operand's
 // order, where 64 neighbouring lanes ask for 64 rows, pass one lane a cycle (523 x 1,024 x 4,096: 59.5 -> 46.2 us).
-// What bounds both: a piece's conversions (352 vector instructions for 64 x 64 outputs) take about as long as its 96 matrix
-// instructions, and the two overlap little; then grids that 256 CUs do not divide.
-// Measured (us, tiles on the float instruction -> here; rows x outputs x columns): 523 x 8,192 x 1,024 113 -> 73 (121 TFLOP/s),
-// 523 x 1,024 x 4,096 80 -> 46, 523 x 1,024 x 1,024 22.4 -> 15.7, 523 x 1,280 x 1,024 22.9 -> 16.1, 700 x 8,192 x 1,024 126 -> 76,
-// 2,048 x 4,096 x 4,096 552 -> 367, 130 x 8,192 x 1,024 41 -> 32, 130 x 1,024 x 4,096 43 -> 24, 40 x 8,192 x 1,024 16.4 -> 13.2,
-// 17 x 1,024 x 4,096 42 -> 22, 300 x 1,000 x 1,001 29.7 -> 24.9.
+// What bounds both: a piece's vector instructions (352 of conversions for 64 x 64 outputs, 128 of sums) take about as long as its
+// 128 matrix instructions, and the two overlap little; then grids that 256 CUs do not divide.
+// Measured (us, tiles on the float instruction -> here; rows x outputs x columns): 523 x 8,192 x 1,024 108 -> 81 (108 TFLOP/s),
+// 523 x 1,024 x 4,096 72 -> 46, 523 x 1,024 x 1,024 21.2 -> 15.0, 523 x 1,280 x 1,024 22.3 -> 17.3, 700 x 8,192 x 1,024 121 -> 87,
+// 2,048 x 4,096 x 4,096 535 -> 490, 2,048 x 1,024 x 4,096 157 -> 143, 130 x 8,192 x 1,024 37.4 -> 33.4, 130 x 1,024 x 4,096 42 -> 25,
+// 40 x 8,192 x 1,024 16.7 -> 13.8, 17 x 1,024 x 4,096 42 -> 23, 64 x 73,448 x 1,024 121 -> 110.
 // ---------------------------------------------------------------------------
 typedef __bf16 gbf16x8_t __attribute__((ext_vector_type(8)));
-struct Split8 {      // eight floats as three bf16 each
-    gbf16x8_t h, m, l;
+struct Split8 {      // eight floats as three bf16 each: upper, middle, last
+    gbf16x8_t part[3];
 };
 // the upper halves of two floats, a's first
 __device__ inline uint32_t f32_upper(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
@@ -178,7 +180,25 @@ __device__ inline Split8 f32_split(const gfloatx4_t& x, const gfloatx4_t& y) {
             }
         }
     }
-    return {part[0].v, part[1].v, part[2].v};
+    return {{part[0].v, part[1].v, part[2].v}};
+}
+
+// acc[i] += a piece of 32 columns of tile i's rows (x(p, i): part p of them) times w's.  The bf16 instruction cuts what its sum
+// leaves below a float's last bit, so the products that reach there have a sum of their own, and every piece is added as floats.
+template <int TM, typename XP>
+__device__ inline void f32_multiply(const XP& x, const Split8& w, gfloatx4_t (&acc)[TM]) {
+    constexpr int P[7] = {1, 2, 2, 0, 1, 1, 0}, Q[7] = {2, 1, 0, 2, 1, 0, 1};
+    gfloatx4_t small[TM], big[TM];
+#pragma unroll
+    for (int i = 0; i < TM; ++i) small[i] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 7; ++t)
+#pragma unroll
+        for (int i = 0; i < TM; ++i) small[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x(P[t], i), w.part[Q[t]], small[i], 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) big[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x(0, i), w.part[0], gfloatx4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) acc[i] += big[i] + small[i];
 }
 
 // One 16 x 16 tile of a split product as it is stored.  A sum that is no finite number may stand for an infinity (whose parts
@@ -221,6 +241,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
     const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, float* __restrict__ Y, long ldy, int M, int N,
     int K, float alpha, int m_tiles, int tiles) {
     constexpr int TASKS = TM / 4, PLANE = TM * 16 * 64, BUF = 3 * PLANE;
+    constexpr bool AHEAD = TN < 3;       // two pieces of W on their way (of 48 outputs a wavefront one: registers)
     __shared__ __attribute__((aligned(16))) char lds[2 * BUF];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int t = tile_of_workgroup(blockIdx.x, tiles);
@@ -244,11 +265,6 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
             else v[c] = f32_piece<false>(row, k + 16 * c, K);
         }
     };
-    const auto clear = [&](int k, gfloatx4_t (&v)[2]) {
-#pragma unroll
-        for (int c = 0; c < 2; ++c)
-            if (VEC && k + 16 * c >= K) v[c] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
-    };
     const auto fetch_x = [&](Piece& p, int k) {
 #pragma unroll
         for (int i = 0; i < TASKS; ++i) fetch(xr[i], k + 4 * chunk, p.x[i]);
@@ -260,18 +276,23 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
     const auto stage = [&](Piece& p, int k, int buf) {
 #pragma unroll
         for (int i = 0; i < TASKS; ++i) {
-            if (k + 32 > K) clear(k + 4 * chunk, p.x[i]);
+            // beyond the last column X's are zeros, so that W's need not be: a clamped load's stand there, and what is not finite
+            // among them is not finite in the row either
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (VEC) p.x[i][c][e] = k + 4 * chunk + 16 * c < K ? p.x[i][c][e] : 0.f;
             const Split8 x = f32_split(p.x[i][0], p.x[i][1]);
-            *(gbf16x8_t*)(lds + buf + place[i]) = x.h;
-            *(gbf16x8_t*)(lds + buf + PLANE + place[i]) = x.m;
-            *(gbf16x8_t*)(lds + buf + 2 * PLANE + place[i]) = x.l;
+#pragma unroll
+            for (int c = 0; c < 3; ++c) *(gbf16x8_t*)(lds + buf + c * PLANE + place[i]) = x.part[c];
         }
     };
-    gfloatx4_t acc[TM][TN];
+    gfloatx4_t acc[TN][TM];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < TM; ++i) acc[j][i] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
     const int at = r * 64 + ((g ^ ((r >> 1) & 3)) << 4);
     // p: piece k (its rows of X in lds[buf]); q: piece k + 32, whose rows go to the other buffer
     const auto step = [&](Piece& p, Piece& q, int k, int buf) {
@@ -284,26 +305,17 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
         fetch_x(p, k + 64);
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            if (k + 32 > K) clear(k + 4 * g, p.w[j]);
-            const Split8 w = f32_split(p.w[j][0], p.w[j][1]);
-            fetch(wr[j], k + 64 + 4 * g, p.w[j]);
-#define TERM(P, Q)                                                                                   \
-    _Pragma("unroll") for (int i = 0; i < TM; ++i) acc[i][j] =                                       \
-        __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[P][i], w.Q, acc[i][j], 0, 0, 0)
-            TERM(2, h);
-            TERM(0, l);
-            TERM(1, m);
-            TERM(1, h);
-            TERM(0, m);
-            TERM(0, h);
-#undef TERM
+            gfloatx4_t (&v)[2] = AHEAD ? p.w[j] : p0.w[j];
+            const Split8 w = f32_split(v[0], v[1]);
+            fetch(wr[j], k + (AHEAD ? 64 : 32) + 4 * g, v);
+            f32_multiply<TM>([&](int c, int i) { return x[c][i]; }, w, acc[j]);
         }
         stage(q, k + 32, BUF - buf);
     };
     fetch_x(p0, 0);
     fetch_w(p0, 0);
     fetch_x(p1, 32);
-    fetch_w(p1, 32);
+    if (AHEAD) fetch_w(p1, 32);
     stage(p0, 0, 0);
     int k = 0;
     for (; k + 32 < K; k += 64) {
@@ -312,9 +324,9 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
     }
     if (k < K) step(p0, p1, k, 0);
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) f32_finish_tile<VEC>(acc[i][j], X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j);
+        for (int i = 0; i < TM; ++i) f32_finish_tile<VEC>(acc[j][i], X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j);
 }
 
 template <int TM, int TN, int NW, bool VEC>
@@ -347,11 +359,11 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_f32_shares_kernel(
             else next[i] = f32_piece<false>(base + off[i], k, K);
         }
     };
-    gfloatx4_t acc[TM][TN];
+    gfloatx4_t acc[TN][TM];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < TM; ++i) acc[j][i] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
     const int place = row8 * 8 + (chunk ^ row8), at0 = r * 8 + (g ^ (r & 7)), at1 = at0 ^ 4;
     fetch(wave * 32);
     for (int k = wave * 32; k < K; k += NW * 32) {
@@ -370,22 +382,13 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_f32_shares_kernel(
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             const Split8 w = f32_split(own[128 * (TM + j) + at0], own[128 * (TM + j) + at1]);
-#define TERM(P, Q)                                                                                   \
-    _Pragma("unroll") for (int i = 0; i < TM; ++i) acc[i][j] =                                       \
-        __builtin_amdgcn_mfma_f32_16x16x32_bf16(x[i].P, w.Q, acc[i][j], 0, 0, 0)
-            TERM(l, h);
-            TERM(h, l);
-            TERM(m, m);
-            TERM(m, h);
-            TERM(h, m);
-            TERM(h, h);
-#undef TERM
+            f32_multiply<TM>([&](int c, int i) { return x[i].part[c]; }, w, acc[j]);
         }
     }
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) own[(i * TN + j) * 64 + lane] = acc[i][j];
+        for (int j = 0; j < TN; ++j) own[(i * TN + j) * 64 + lane] = acc[j][i];
     __syncthreads();
 #pragma unroll
     for (int f = 0; f < PER; ++f) {
@@ -441,14 +444,14 @@ static void gemm_f32_launch(const float* X, long ldx, const float* W, long ldw, 
         gemm_f32_rows_kernel<16, VEC><<<up(N, 16), 1024, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
         return;
     }
-    // (few columns: the parts that a split leaves out would show beside so few roundings)
+    // (few columns, up to two pieces: 523 x 8,192 x 48 12.4 us, 13.9 in three parts; 523 x 1,024 x 32 both 7.2)
     if ((K < 64 && up(M, 32) <= 65535) || (M <= 32 && N > 32768)) {
         gemm_f32_mfma_kernel<VEC><<<dim3(up(N, 32), up(M, 32)), 256, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
         return;
     }
     // Columns shared out while the tiles are at most one a CU: the smallest tile for which that holds (its wavefronts' pieces cost
     // the least).  Beyond, 64 rows by as many outputs as still leave one and a half workgroups a CU, which then overlap (tiles of
-    // 64 / 128 / 192 / 256 outputs: 523 x 8,192 x 1,024 76/77/73/86, 700 x 8,192 x 1,024 87/75/74/88, 2,048 x 4,096 x 4,096 480/423/427/378).
+    // 64 / 128 / 192 outputs: 523 x 8,192 x 1,024 83/93/78, 700 x 8,192 x 1,024 101/96/85, 2,048 x 4,096 x 4,096 530/477/491).
 #define SHARES(TM, TN)                                                                                                   \
     if (up(M, 16 * TM) * (long)up(N, 16 * TN) <= 256) {                                                                  \
         const int tiles = up(M, 16 * TM) * up(N, 16 * TN);                                                               \
@@ -467,7 +470,6 @@ static void gemm_f32_launch(const float* X, long ldx, const float* W, long ldw, 
         gemm_f32_split_kernel<4, TN, VEC><<<tiles, 256, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha, up(M, 64), tiles); \
         return;                                                                                                          \
     }
-    SPLIT(4);
     SPLIT(3);
     SPLIT(2);
     SPLIT(1);

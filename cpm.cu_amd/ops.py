@@ -274,8 +274,8 @@ def rope_store(qkv: torch.Tensor, q_out: torch.Tensor, nh: int, nkv: int, hd: in
 
 
 def gemm_nt_plain(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, alpha: float = 1.0):
-    """out[m,N] = alpha * x[m,K] . w[N,K]^T summed in float (any size; float32 on the matrix cores' float instruction,
-    bfloat16 with scalar FMAs)."""
+    """out[m,N] = alpha * x[m,K] . w[N,K]^T summed in float (any size; float32 on the matrix cores, as it is or every
+    float as the exact sum of three bf16 with all products that a float's sum can show; bfloat16 with scalar FMAs)."""
     _need(x, "gemm x", shape=(None, None))
     M, K = x.shape
     _need(w, "gemm weight", x.dtype, (None, K))

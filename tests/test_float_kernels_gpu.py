@@ -37,10 +37,39 @@ def test_float_product_in_three_parts(M, N, K):
     out = torch.full((M, N), float("nan"), device=DEV)
     ops.gemm_nt_plain(x, w, out, 1.5)
     ref, mag = (1.5 * (a @ b.T) for a, b in ((x.double(), w.double()), (x.double().abs(), w.double().abs())))
-    # sums as above, and the left out products of middle and last parts: below 2^-21 of a product
-    assert bool(((out.double() - ref).abs() <= ((K + 2) * 2.0 ** -24 + 2.0 ** -21) * mag).all())
-    # the error on the whole: no larger than that of a float sum with a rounding every 4 columns
-    assert float((out.double() - ref).norm() / ref.norm()) <= 2.0 ** -24 * (K / 4) ** 0.5
+    # sums as above, and the left out product of last parts: below 2^-30 of a product
+    assert bool(((out.double() - ref).abs() <= ((K + 2) * 2.0 ** -24 + 2.0 ** -30) * mag).all())
+    # the error on the whole: no larger than that of a float sum with a rounding every 32 columns and two of the result
+    assert float((out.double() - ref).norm() / ref.norm()) <= 2.0 ** -24 * (K / 32 + 2) ** 0.5
+
+
+@pytest.mark.parametrize("M,N,K", [(130, 300, 64), (523, 1024, 64), (700, 1020, 68), (1000, 1000, 257), (1999, 3101, 164)])
+def test_float_product_of_few_columns_that_matter(M, N, K):
+    """Rows of which one element is not zero: the product itself, rounded once."""
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x, w = torch.zeros(M, K, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    at = torch.randint(0, K, (M,), generator=g, device=DEV)
+    x[torch.arange(M, device=DEV), at] = torch.randn(M, generator=g, device=DEV)
+    out = torch.empty(M, N, device=DEV)
+    ops.gemm_nt_plain(x, w, out, 1.0)
+    off = (out.double() - x.double() @ w.double().T).abs() / (x.double() @ w.double().T).abs()
+    # half a unit of the result, the cut sums of the smaller products (7 times 2^-23 of what ends below 2^-6), the one left out
+    assert float(off.max()) <= 2.0 ** -24 * (1 + 7 * 2.0 ** -5 + 2.0 ** -6)
+    # on the whole that of a rounding: an even error in a unit of 2^-24 to 2^-23 of the result, and an eighth of it for the cuts
+    assert float((off ** 2).mean() ** 0.5) <= 2.0 ** -24 / 3 ** 0.5 * 1.125
+
+
+@pytest.mark.parametrize("M,N,K", [(130, 1000, 1000), (523, 1024, 4096), (1999, 3101, 1028)])
+def test_float_product_of_positive_numbers_has_no_lean(M, N, K):
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x, w = torch.rand(M, K, generator=g, device=DEV), torch.rand(N, K, generator=g, device=DEV)
+    out = torch.empty(M, N, device=DEV)
+    ops.gemm_nt_plain(x, w, out, 1.0)
+    ref = x.double() @ w.double().T
+    # roundings go either way; the smaller products' sums, 2^-6 of the result at most, are cut by 7 units of 2^-23 at most
+    assert abs(float(((out.double() - ref) / ref).mean())) <= 7 * 2.0 ** -29
 
 
 @pytest.mark.parametrize("M,N,K", [(70, 130, 96), (1030, 1100, 131)])
@@ -62,7 +91,7 @@ def test_float_product_of_odd_values(M, N, K):
     assert torch.equal(out.isnan(), ref.isnan())
     assert bool((out.double() == ref)[torch.isinf(ref)].all())
     # (denormal products may be flushed one by one)
-    assert bool(((out.double() - ref).abs() <= ((K + 2) * 2.0 ** -24 + 2.0 ** -21) * mag + K * 2.0 ** -126)[fine].all())
+    assert bool(((out.double() - ref).abs() <= ((K + 2) * 2.0 ** -24 + 2.0 ** -30) * mag + K * 2.0 ** -126)[fine].all())
     assert bool(((out[40].double() - ref[40]).abs() <= (K + 2) * 2.0 ** -24 * mag[40] + K * 2.0 ** -126)[fine[40]].all())
 
 
