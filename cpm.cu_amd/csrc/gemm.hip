@@ -143,7 +143,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 // below it, and meets the sum of the pieces in float additions.  Distance from a product in double, float instruction -> here:
 // 1,024 columns 5.7e-7 -> 1.1e-7 and, with the columns shared out, 7.9e-8; 4,096 columns 1.15e-6 -> 2.1e-7 and 1.0e-7; positive
 // numbers 4.9e-7 -> 9.0e-8; rows of which one element is not zero 2.5e-8 in both, four 4.0e-8 -> 2.7e-8.
-// Infinities, NaNs and results so small that the parts' own limit may show are worked out on the float instruction
+// Infinities, NaNs, inputs whose parts do not hold all of them and very small results are worked out on the float instruction
 // (f32_finish_tile).
 //
 // gemm_f32_split_kernel: 64 rows against 64 TN outputs a workgroup.  X's piece of 32 columns is split once and its parts go
@@ -155,10 +155,10 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 // order, where 64 neighbouring lanes ask for 64 rows, pass one lane a cycle (523 x 1,024 x 4,096: 59.5 -> 46.2 us).
 // What bounds both: a piece's vector instructions (352 of conversions for 64 x 64 outputs, 128 of sums) take about as long as its
 // 128 matrix instructions, and the two overlap little; then grids that 256 CUs do not divide.
-// Measured (us, tiles on the float instruction -> here; rows x outputs x columns): 523 x 8,192 x 1,024 108 -> 81 (108 TFLOP/s),
-// 523 x 1,024 x 4,096 72 -> 46, 523 x 1,024 x 1,024 21.2 -> 15.0, 523 x 1,280 x 1,024 22.3 -> 17.3, 700 x 8,192 x 1,024 121 -> 87,
-// 2,048 x 4,096 x 4,096 535 -> 490, 2,048 x 1,024 x 4,096 157 -> 143, 130 x 8,192 x 1,024 37.4 -> 33.4, 130 x 1,024 x 4,096 42 -> 25,
-// 40 x 8,192 x 1,024 16.7 -> 13.8, 17 x 1,024 x 4,096 42 -> 23, 64 x 73,448 x 1,024 121 -> 110.
+// Measured (us, tiles on the float instruction -> here; rows x outputs x columns): 523 x 8,192 x 1,024 108 -> 80 (110 TFLOP/s),
+// 523 x 1,024 x 4,096 72 -> 50, 523 x 1,024 x 1,024 21.2 -> 16.1, 523 x 1,280 x 1,024 22.3 -> 17.9, 700 x 8,192 x 1,024 121 -> 87,
+// 2,048 x 4,096 x 4,096 535 -> 499, 2,048 x 1,024 x 4,096 157 -> 149, 130 x 8,192 x 1,024 37.4 -> 36.9, 130 x 1,024 x 4,096 42 -> 27,
+// 40 x 8,192 x 1,024 16.7 -> 14.3, 17 x 1,024 x 4,096 42 -> 24, 64 x 73,448 x 1,024 121 -> 103.
 // ---------------------------------------------------------------------------
 typedef __bf16 gbf16x8_t __attribute__((ext_vector_type(8)));
 struct Split8 {      // eight floats as three bf16 each: upper, middle, last
@@ -166,7 +166,8 @@ struct Split8 {      // eight floats as three bf16 each: upper, middle, last
 };
 // the upper halves of two floats, a's first
 __device__ inline uint32_t f32_upper(uint32_t a, uint32_t b) { return __builtin_amdgcn_perm(b, a, 0x07060302u); }
-__device__ inline Split8 f32_split(const gfloatx4_t& x, const gfloatx4_t& y) {
+// (lost: its lower half gathers what a last part has no room for)
+__device__ inline Split8 f32_split(const gfloatx4_t& x, const gfloatx4_t& y, uint32_t& lost) {
     union { uint32_t u[4]; gbf16x8_t v; } part[3];
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
@@ -179,6 +180,7 @@ __device__ inline Split8 f32_split(const gfloatx4_t& x, const gfloatx4_t& y) {
                 b = __float_as_uint(__uint_as_float(b) - __uint_as_float(b & 0xffff0000u));
             }
         }
+        lost |= a | b;
     }
     return {{part[0].v, part[1].v, part[2].v}};
 }
@@ -201,14 +203,15 @@ __device__ inline void f32_multiply(const XP& x, const Split8& w, gfloatx4_t (&a
     for (int i = 0; i < TM; ++i) acc[i] += big[i] + small[i];
 }
 
-// One 16 x 16 tile of a split product as it is stored.  A sum that is no finite number may stand for an infinity (whose parts
-// are an infinity and no numbers), and one below 2^-64 for inputs whose last parts fall below the smallest bf16: those tiles
-// are worked out again on the float instruction.
+// One 16 x 16 tile of a split product as it is stored.  It is worked out again on the float instruction if an input of the
+// workgroup's tile has bits that its last part has no room for (odd), if a sum is no finite number, which may stand for an infinity
+// (whose parts are an infinity and no numbers), and if one is below 2^-64, where a product of parts may lie below the smallest
+// float.  (A sum of exactly 0 is taken as it is: K 2^-126 at most are lost.)
 template <bool VEC>
 __device__ inline void f32_finish_tile(gfloatx4_t sum, const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw,
-                                       float* __restrict__ Y, long ldy, int M, int N, int K, float alpha, int m0, int n0) {
+                                       float* __restrict__ Y, long ldy, int M, int N, int K, float alpha, int m0, int n0,
+                                       bool odd) {
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    bool odd = false;
 #pragma unroll
     for (int e = 0; e < 4; ++e) odd |= !(fabsf(sum[e]) < __builtin_inff()) || (fabsf(sum[e]) < 0x1p-64f && sum[e] != 0.f);
     if (__any(odd)) {
@@ -273,6 +276,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
 #pragma unroll
         for (int j = 0; j < TN; ++j) fetch(wr[j], k + 4 * g, p.w[j]);
     };
+    uint32_t lost = 0;
     const auto stage = [&](Piece& p, int k, int buf) {
 #pragma unroll
         for (int i = 0; i < TASKS; ++i) {
@@ -283,7 +287,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     if (VEC) p.x[i][c][e] = k + 4 * chunk + 16 * c < K ? p.x[i][c][e] : 0.f;
-            const Split8 x = f32_split(p.x[i][0], p.x[i][1]);
+            const Split8 x = f32_split(p.x[i][0], p.x[i][1], lost);
 #pragma unroll
             for (int c = 0; c < 3; ++c) *(gbf16x8_t*)(lds + buf + c * PLANE + place[i]) = x.part[c];
         }
@@ -306,7 +310,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
             gfloatx4_t (&v)[2] = AHEAD ? p.w[j] : p0.w[j];
-            const Split8 w = f32_split(v[0], v[1]);
+            const Split8 w = f32_split(v[0], v[1], lost);
             fetch(wr[j], k + (AHEAD ? 64 : 32) + 4 * g, v);
             f32_multiply<TM>([&](int c, int i) { return x[c][i]; }, w, acc[j]);
         }
@@ -323,10 +327,11 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
         step(p1, p0, k + 32, BUF);
     }
     if (k < K) step(p0, p1, k, 0);
+    const bool odd = __syncthreads_or(lost & 0xffff);
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < TM; ++i) f32_finish_tile<VEC>(acc[j][i], X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j);
+        for (int i = 0; i < TM; ++i) f32_finish_tile<VEC>(acc[j][i], X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j, odd);
 }
 
 template <int TM, int TN, int NW, bool VEC>
@@ -365,6 +370,7 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_f32_shares_kernel(
 #pragma unroll
         for (int i = 0; i < TM; ++i) acc[j][i] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
     const int place = row8 * 8 + (chunk ^ row8), at0 = r * 8 + (g ^ (r & 7)), at1 = at0 ^ 4;
+    uint32_t lost = 0;
     fetch(wave * 32);
     for (int k = wave * 32; k < K; k += NW * 32) {
         if (VEC && k + 32 > K && k + 4 * chunk >= K) {
@@ -378,10 +384,10 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_f32_shares_kernel(
         fetch(k + NW * 32);
         Split8 x[TM];
 #pragma unroll
-        for (int i = 0; i < TM; ++i) x[i] = f32_split(own[128 * i + at0], own[128 * i + at1]);
+        for (int i = 0; i < TM; ++i) x[i] = f32_split(own[128 * i + at0], own[128 * i + at1], lost);
 #pragma unroll
         for (int j = 0; j < TN; ++j) {
-            const Split8 w = f32_split(own[128 * (TM + j) + at0], own[128 * (TM + j) + at1]);
+            const Split8 w = f32_split(own[128 * (TM + j) + at0], own[128 * (TM + j) + at1], lost);
             f32_multiply<TM>([&](int c, int i) { return x[i].part[c]; }, w, acc[j]);
         }
     }
@@ -389,7 +395,7 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_f32_shares_kernel(
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j) own[(i * TN + j) * 64 + lane] = acc[j][i];
-    __syncthreads();
+    const bool odd = __syncthreads_or(lost & 0xffff);
 #pragma unroll
     for (int f = 0; f < PER; ++f) {
         const int tile = wave * PER + f, i = tile / TN, j = tile % TN;
@@ -397,7 +403,7 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_f32_shares_kernel(
         gfloatx4_t sum = lds[tile * 64 + lane];
 #pragma unroll
         for (int w = 1; w < NW; ++w) sum += lds[w * REGION + tile * 64 + lane];
-        f32_finish_tile<VEC>(sum, X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j);
+        f32_finish_tile<VEC>(sum, X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j, odd);
     }
 }
 

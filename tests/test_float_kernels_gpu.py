@@ -72,6 +72,24 @@ def test_float_product_of_positive_numbers_has_no_lean(M, N, K):
     assert abs(float(((out.double() - ref) / ref).mean())) <= 7 * 2.0 ** -29
 
 
+@pytest.mark.parametrize("M,N,K", [(70, 130, 96), (130, 1000, 100), (1030, 1100, 131), (1999, 3101, 164)])
+@pytest.mark.parametrize("down,up", [(-118, 80), (-122, 60), (-125, 90), (-135, 100)])
+@pytest.mark.parametrize("which", ["rows", "weights"])
+def test_float_product_of_values_that_three_parts_do_not_hold(M, N, K, down, up, which):
+    """Elements below 2^-110, whose last part is below the smallest bf16, against large ones: results of ordinary size."""
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M + K)
+    x, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    small, large = (x, w) if which == "rows" else (w, x)
+    small[small.shape[0] // 2] *= 2.0 ** down
+    small[-1, 3] *= 2.0 ** down
+    large[:, ::2] *= 2.0 ** up
+    out = torch.empty(M, N, device=DEV)
+    ops.gemm_nt_plain(x, w, out, 1.0)
+    ref, mag = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    assert bool(((out.double() - ref).abs() <= (K + 2) * 2.0 ** -24 * mag + K * 2.0 ** -126).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 130, 96), (1030, 1100, 131)])
 def test_float_product_of_odd_values(M, N, K):
     """Infinities, NaNs, the largest floats and floats whose last parts no bf16 holds: the float instruction's results."""
