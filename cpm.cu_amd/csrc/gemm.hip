@@ -62,12 +62,12 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const XT* __restrict__ 
 // (32 multiply-adds a cycle and SIMD, 157 TFLOP/s on the chip); v_mfma_f32_16x16x32_bf16 does 16 times as many, so that eight
 // of its products, which a float as three bf16 asks for (below), still are twice as fast.
 //
-// gemm_f32_mfma_kernel: the float instruction, for few columns and for few rows of very many outputs.  256 threads, a
+// gemm_f32_mfma_kernel: the float instruction, for few columns.  256 threads, a
 // wavefront 16 x 16 of a 32 x 32 tile; 64 columns of both operands go through LDS in two buffers, the next ones on their way
 // to registers meanwhile, one barrier a piece.  A row of a piece is 16 chunks of 16 bytes, chunk c of row r at place
 // c ^ (r % 8), so that 8 neighbouring lanes (8 rows, one chunk) read all banks.  A lane's 16 bytes serve four instructions: in
 // instruction s, lane group g stands for column 4 g + s of the 16, in both operands alike (a sum over columns may take them
-// in any order).  16 x 73,448 x 1,024 takes 70 us; its distance from a product in double is a float sum's.
+// in any order).
 // ---------------------------------------------------------------------------
 typedef float gfloatx4_t __attribute__((ext_vector_type(4)));
 
@@ -141,8 +141,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 // instruction cuts its sums' last bits where a float addition rounds them (all terms into one accumulator: sums of positive
 // products 4e-7 too small), so a piece of 32 columns has two sums that start from zero, hh and the seven others, which end 2^-7
 // below it, and meets the sum of the pieces in float additions.  Distance from a product in double, float instruction -> here:
-// 1,024 columns 5.7e-7 -> 1.1e-7 and, with the columns shared out, 7.9e-8; 4,096 columns 1.15e-6 -> 2.1e-7 and 1.0e-7; positive
-// numbers 4.9e-7 -> 9.0e-8; rows of which one element is not zero 2.5e-8 in both, four 4.0e-8 -> 2.7e-8.
+// 1,024 columns 5.7e-7 -> 7.9e-8, 4,096 columns 1.15e-6 -> 1.0e-7; positive numbers 4.9e-7 -> 5.2e-8; rows of which one element is not zero 2.5e-8 in both, four 4.0e-8 -> 2.7e-8.
 // Infinities, NaNs, inputs whose parts do not hold all of them and very small results are worked out on the float instruction
 // (f32_finish_tile).
 //
@@ -150,15 +149,15 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 // through LDS in two buffers; a wavefront splits its own 16 TN rows of W in registers, which nobody else needs.  Two pieces on
 // their way to registers (of 48 outputs a wavefront one).
 // gemm_f32_shares_kernel: for outputs that give too few such workgroups: every one of 8 wavefronts has the whole tile of
-// 16 TM x 16 TN outputs and every eighth piece of the columns, no barrier until their sums meet in LDS.  Pieces are brought
+// 16 TM x 16 TN outputs and an eighth of the columns, no barrier until their sums meet in LDS.  Pieces are brought
 // whole lines a row (8 lanes each) and turned into operands through the wavefront's own LDS: loads straight into the operand's
 // order, where 64 neighbouring lanes ask for 64 rows, pass one lane a cycle (523 x 1,024 x 4,096: 59.5 -> 46.2 us).
 // What bounds both: a piece's vector instructions (352 of conversions for 64 x 64 outputs, 128 of sums) take about as long as its
 // 128 matrix instructions, and the two overlap little; then grids that 256 CUs do not divide.
-// Measured (us, tiles on the float instruction -> here; rows x outputs x columns): 523 x 8,192 x 1,024 108 -> 80 (110 TFLOP/s),
-// 523 x 1,024 x 4,096 72 -> 50, 523 x 1,024 x 1,024 21.2 -> 16.1, 523 x 1,280 x 1,024 22.3 -> 17.9, 700 x 8,192 x 1,024 121 -> 87,
-// 2,048 x 4,096 x 4,096 535 -> 499, 2,048 x 1,024 x 4,096 157 -> 149, 130 x 8,192 x 1,024 37.4 -> 36.9, 130 x 1,024 x 4,096 42 -> 27,
-// 40 x 8,192 x 1,024 16.7 -> 14.3, 17 x 1,024 x 4,096 42 -> 24, 64 x 73,448 x 1,024 121 -> 103.
+// Measured (us, tiles on the float instruction -> here; rows x outputs x columns): 523 x 8,192 x 1,024 108 -> 87 (101 TFLOP/s),
+// 523 x 1,024 x 4,096 72 -> 52, 523 x 1,024 x 1,024 21.2 -> 16.5, 523 x 1,280 x 1,024 22.3 -> 18.0, 700 x 8,192 x 1,024 121 -> 94,
+// 2,048 x 4,096 x 4,096 535 -> 517, 2,048 x 1,024 x 4,096 157 -> 149, 130 x 8,192 x 1,024 37.4 -> 38.1, 130 x 1,024 x 4,096 42 -> 27,
+// 40 x 8,192 x 1,024 16.7 -> 14.1, 17 x 1,024 x 4,096 42 -> 24, 64 x 73,448 x 1,024 121 -> 105, 1 x 73,448 x 1,024 66 -> 60.
 // ---------------------------------------------------------------------------
 typedef __bf16 gbf16x8_t __attribute__((ext_vector_type(8)));
 struct Split8 {      // eight floats as three bf16 each: upper, middle, last
@@ -203,25 +202,50 @@ __device__ inline void f32_multiply(const XP& x, const Split8& w, gfloatx4_t (&a
     for (int i = 0; i < TM; ++i) acc[i] += big[i] + small[i];
 }
 
-// One 16 x 16 tile of a split product as it is stored.  It is worked out again on the float instruction if an input of the
-// workgroup's tile has bits that its last part has no room for (odd), if a sum is no finite number, which may stand for an infinity
-// (whose parts are an infinity and no numbers), and if one is below 2^-64, where a product of parts may lie below the smallest
-// float.  (A sum of exactly 0 is taken as it is: K 2^-126 at most are lost.)
+// One 16 x 16 tile of a split product as it is stored.  A result is worked out again on the float instruction if an input of its
+// rows has bits that its last part has no room for (odd: some row of the workgroup's has), if it is no finite number, which may
+// stand for an infinity (whose parts are an infinity and no numbers), and if it is below 2^-64, where a product of parts may lie
+// below the smallest float.  (A sum of exactly 0 is taken as it is: K 2^-126 at most are lost.)  The other results of the tile
+// stay, so that none depends on its neighbours.
+__device__ inline uint32_t f32_rest(float x) {
+#pragma unroll
+    for (int p = 0; p < 2; ++p) x -= __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+    return __float_as_uint(x) & 0xffff;
+}
 template <bool VEC>
 __device__ inline void f32_finish_tile(gfloatx4_t sum, const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw,
                                        float* __restrict__ Y, long ldy, int M, int N, int K, float alpha, int m0, int n0,
                                        bool odd) {
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    bool again[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) odd |= !(fabsf(sum[e]) < __builtin_inff()) || (fabsf(sum[e]) < 0x1p-64f && sum[e] != 0.f);
+    for (int e = 0; e < 4; ++e) {
+        again[e] = !(fabsf(sum[e]) < __builtin_inff()) || (fabsf(sum[e]) < 0x1p-64f && sum[e] != 0.f);
+        odd |= again[e];
+    }
     if (__any(odd)) {
         const float* xr = X + (long)min(m0 + r, M - 1) * ldx;
         const float* wr = W + (long)min(n0 + r, N - 1) * ldw;
-        sum = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+        gfloatx4_t whole = {0.f, 0.f, 0.f, 0.f};
+        uint32_t rest_x = 0, rest_w = 0;                             // of row r of each
         for (int k = 0; k < K; k += 16) {
             const gfloatx4_t a = f32_piece<VEC>(xr, k + 4 * g, K), b = f32_piece<VEC>(wr, k + 4 * g, K);
 #pragma unroll
-            for (int s = 0; s < 4; ++s) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], sum, 0, 0, 0);
+            for (int s = 0; s < 4; ++s) {
+                whole = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], whole, 0, 0, 0);
+                rest_x |= f32_rest(a[s]);
+                rest_w |= f32_rest(b[s]);
+            }
+        }
+#pragma unroll
+        for (int d = 16; d < 64; d *= 2) {
+            rest_x |= __shfl_xor(rest_x, d);
+            rest_w |= __shfl_xor(rest_w, d);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t rest = rest_w | __shfl(rest_x, 4 * g + e);        // (by all lanes)
+            if (again[e] || rest) sum[e] = whole[e];
         }
     }
     // lane (column r, g): sum[e] is row 4 g + e
@@ -239,6 +263,10 @@ __device__ inline int tile_of_workgroup(int wg, int tiles) {
     return x * per + min(x, more) + wg / 8;
 }
 
+// The pieces of a share of the columns, an eighth.  Every kernel here adds a share's pieces in their order and then the shares, and
+// so a row's result does not depend on how many rows there are.
+__device__ inline int f32_share(int K) { return ((K + 31) / 32 + 7) / 8; }
+
 template <int TM, int TN, bool VEC>
 __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
     const float* __restrict__ X, long ldx, const float* __restrict__ W, long ldw, float* __restrict__ Y, long ldy, int M, int N,
@@ -246,6 +274,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
     constexpr int TASKS = TM / 4, PLANE = TM * 16 * 64, BUF = 3 * PLANE;
     constexpr bool AHEAD = TN < 3;       // two pieces of W on their way (of 48 outputs a wavefront one: registers)
     __shared__ __attribute__((aligned(16))) char lds[2 * BUF];
+    __shared__ gfloatx4_t total[TN * TM][256];               // the sum of whole shares, a thread's own
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int t = tile_of_workgroup(blockIdx.x, tiles);
     const int m0 = t % m_tiles * 16 * TM, n0 = (t / m_tiles * 4 + wave) * 16 * TN;
@@ -293,10 +322,15 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
         }
     };
     gfloatx4_t acc[TN][TM];
+    const auto start = [&]() {
 #pragma unroll
-    for (int j = 0; j < TN; ++j)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < TM; ++i) acc[j][i] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+            for (int i = 0; i < TM; ++i) acc[j][i] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    };
+    start();
+    const int per = f32_share(K);
+    int shares = 0, left = per;
     const int at = r * 64 + ((g ^ ((r >> 1) & 3)) << 4);
     // p: piece k (its rows of X in lds[buf]); q: piece k + 32, whose rows go to the other buffer
     const auto step = [&](Piece& p, Piece& q, int k, int buf) {
@@ -313,6 +347,18 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
             const Split8 w = f32_split(v[0], v[1], lost);
             fetch(wr[j], k + (AHEAD ? 64 : 32) + 4 * g, v);
             f32_multiply<TM>([&](int c, int i) { return x[c][i]; }, w, acc[j]);
+        }
+        if (--left == 0 && k + 32 < K) {                     // (the last share stays in registers)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int i = 0; i < TM; ++i) {
+                    gfloatx4_t& sum = total[j * TM + i][threadIdx.x];
+                    sum = shares ? sum + acc[j][i] : acc[j][i];
+                }
+            start();
+            ++shares;
+            left = per;
         }
         stage(q, k + 32, BUF - buf);
     };
@@ -331,7 +377,10 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_split_kernel(
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int i = 0; i < TM; ++i) f32_finish_tile<VEC>(acc[j][i], X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j, odd);
+        for (int i = 0; i < TM; ++i) {
+            const gfloatx4_t sum = shares ? total[j * TM + i][threadIdx.x] + acc[j][i] : acc[j][i];
+            f32_finish_tile<VEC>(sum, X, ldx, W, ldw, Y, ldy, M, N, K, alpha, m0 + 16 * i, n0 + 16 * j, odd);
+        }
 }
 
 template <int TM, int TN, int NW, bool VEC>
@@ -371,8 +420,10 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_f32_shares_kernel(
         for (int i = 0; i < TM; ++i) acc[j][i] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
     const int place = row8 * 8 + (chunk ^ row8), at0 = r * 8 + (g ^ (r & 7)), at1 = at0 ^ 4;
     uint32_t lost = 0;
-    fetch(wave * 32);
-    for (int k = wave * 32; k < K; k += NW * 32) {
+    static_assert(NW == 8, "a share a wavefront");
+    const int per = f32_share(K) * 32, end = min((wave + 1) * per, K);
+    fetch(wave * per);
+    for (int k = wave * per; k < end; k += 32) {
         if (VEC && k + 32 > K && k + 4 * chunk >= K) {
 #pragma unroll
             for (int i = 0; i < LOADS; ++i) next[i] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
@@ -381,7 +432,7 @@ __global__ __launch_bounds__(NW * 64, 2) void gemm_f32_shares_kernel(
 #pragma unroll
         for (int i = 0; i < LOADS; ++i) own[64 * i + place] = next[i];
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        fetch(k + NW * 32);
+        fetch(k + 32);
         Split8 x[TM];
 #pragma unroll
         for (int i = 0; i < TM; ++i) x[i] = f32_split(own[128 * i + at0], own[128 * i + at1], lost);
@@ -444,22 +495,24 @@ static void gemm_f32_launch(const float* X, long ldx, const float* W, long ldw, 
                             float alpha, hipStream_t stream) {
     const auto up = [](int a, int b) { return (a + b - 1) / b; };
     // Up to 16 rows the weight's bytes bound the product: every workgroup takes 16 outputs over all of K (1 x 1,024 x
-    // 4,096: 12 us, 43 us in tiles of 32 x 32).  Beyond 32,768 outputs there are tiles enough, and those read x once for
-    // 32 outputs instead of 16 (16 x 73,448 x 1,024: 70 against 83 us).
+    // 4,096: 12 us, 43 us in tiles of 32 x 32).  Beyond 32,768 outputs there are tiles enough, and the kernels for
+    // more rows read x once for 32 outputs instead of 16 (16 x 73,448 x 1,024: 66 against 83 us).
     if (M <= 16 && N <= 32768) {
         gemm_f32_rows_kernel<16, VEC><<<up(N, 16), 1024, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
         return;
     }
     // (few columns, up to two pieces: 523 x 8,192 x 48 12.4 us, 13.9 in three parts; 523 x 1,024 x 32 both 7.2)
-    if ((K < 64 && up(M, 32) <= 65535) || (M <= 32 && N > 32768)) {
+    if (K < 64 && up(M, 32) <= 65535) {
         gemm_f32_mfma_kernel<VEC><<<dim3(up(N, 32), up(M, 32)), 256, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
         return;
     }
     // Columns shared out while the tiles are at most one a CU: the smallest tile for which that holds (its wavefronts' pieces cost
     // the least).  Beyond, 64 rows by as many outputs as still leave one and a half workgroups a CU, which then overlap (tiles of
-    // 64 / 128 / 192 outputs: 523 x 8,192 x 1,024 83/93/78, 700 x 8,192 x 1,024 101/96/85, 2,048 x 4,096 x 4,096 530/477/491).
+    // 64 / 128 / 192 outputs: 523 x 8,192 x 1,024 88/98/87, 700 x 8,192 x 1,024 107/101/93, 2,048 x 4,096 x 4,096 549/486/518).
+    // (up to 32 rows of very many outputs: the weight's bytes are the bound, 32 x 73,448 x 1,024 70 us in the smallest tile, 86 in 64 rows)
+    const int few = N > 32768 ? 32 : 0;
 #define SHARES(TM, TN)                                                                                                   \
-    if (up(M, 16 * TM) * (long)up(N, 16 * TN) <= 256) {                                                                  \
+    if (up(M, 16 * TM) * (long)up(N, 16 * TN) <= 256 || M <= few) {                                                      \
         const int tiles = up(M, 16 * TM) * up(N, 16 * TN);                                                               \
         gemm_f32_shares_kernel<TM, TN, 8, VEC><<<tiles, 512, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha, up(M, 16 * TM), tiles); \
         return;                                                                                                          \

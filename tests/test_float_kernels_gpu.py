@@ -90,6 +90,26 @@ def test_float_product_of_values_that_three_parts_do_not_hold(M, N, K, down, up,
     assert bool(((out.double() - ref).abs() <= (K + 2) * 2.0 ** -24 * mag + K * 2.0 ** -126).all())
 
 
+@pytest.mark.parametrize("N,K,rows", [(1000, 1028, (17, 33, 130, 300, 523, 1100)), (1024, 64, (17, 600, 2100)), (300, 257, (20, 64, 4000)),
+                                      (8192, 320, (40, 130, 700)), (33000, 96, (1, 16, 17, 32, 33, 100))])
+def test_float_rows_do_not_depend_on_the_others(N, K, rows):
+    """Beyond 16 rows (or 32,768 outputs) a row's result is the same to the last bit whatever tile the rule takes, beside
+    infinities, NaNs and very small numbers too."""
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    x, w = torch.randn(max(rows), K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    x[0, 5], x[7, 0], x[16, K - 1] = float("inf"), float("nan"), 2.0 ** -130
+    x[20 % max(rows)] *= 2.0 ** -90
+    w[13, 1], w[200, 2] = float("-inf"), 2.0 ** -125
+    out = []
+    for n in rows:
+        y = torch.full((n, N), 7.0, device=DEV)
+        ops.gemm_nt_plain(x[:n].contiguous(), w, y, 1.0)
+        out.append(y.view(torch.int32))
+    for y in out[:-1]:
+        assert torch.equal(y, out[-1][:y.shape[0]])
+
+
 @pytest.mark.parametrize("M,N,K", [(70, 130, 96), (1030, 1100, 131)])
 def test_float_product_of_odd_values(M, N, K):
     """Infinities, NaNs, the largest floats and floats whose last parts no bf16 holds: the float instruction's results."""
