@@ -511,8 +511,9 @@ static void gemm_f32_launch(const float* X, long ldx, const float* W, long ldw, 
     // 64 / 128 / 192 outputs: 523 x 8,192 x 1,024 88/98/87, 700 x 8,192 x 1,024 107/101/93, 2,048 x 4,096 x 4,096 549/486/518).
     // (up to 32 rows of very many outputs: the weight's bytes are the bound, 32 x 73,448 x 1,024 70 us in the smallest tile, 86 in 64 rows)
     const int few = N > 32768 ? 32 : 0;
+    const bool near = 80 * (ldx > ldw ? ldx : ldw) < (1L << 32);      // (a tile's rows are within reach of 32-bit offsets)
 #define SHARES(TM, TN)                                                                                                   \
-    if (up(M, 16 * TM) * (long)up(N, 16 * TN) <= 256 || M <= few) {                                                      \
+    if (near && (up(M, 16 * TM) * (long)up(N, 16 * TN) <= 256 || M <= few)) {                                            \
         const int tiles = up(M, 16 * TM) * up(N, 16 * TN);                                                               \
         gemm_f32_shares_kernel<TM, TN, 8, VEC><<<tiles, 512, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha, up(M, 16 * TM), tiles); \
         return;                                                                                                          \

@@ -163,3 +163,19 @@ def test_float_attention_ignores_what_lies_behind_the_token(nh, nkv, hd):
         w = torch.softmax(torch.einsum("hd,jhd->hj", q[0].double().cpu(), rep(k)) * hd ** -0.5, -1)
         ref = torch.einsum("hj,jhd->hd", w, rep(v))
         assert float((out.double().cpu().view(nh, hd) - ref).abs().max()) <= 2e-6, pos
+
+
+def test_float_product_of_rows_far_apart():
+    """Rows 2^28 floats apart: the last of 17 lies beyond what 32-bit offsets reach."""
+    from cpmcu_amd import ops
+    M, N, K, ld = 17, 40, 128, 2 ** 28
+    g = torch.Generator(device=DEV).manual_seed(1)
+    rows, w = torch.randn(M, K, generator=g, device=DEV), torch.randn(N, K, generator=g, device=DEV)
+    x = torch.empty((M - 1) * ld + K, device=DEV).as_strided((M, K), (ld, 1))
+    x.copy_(rows)
+    out, want = torch.full((M, N), float("nan"), device=DEV), torch.empty(M, N, device=DEV)
+    ops.gemm_nt_plain(rows, w, want, 1.0)
+    ops._check(ops._fn("gemm", "cpmcu_gemm_nt_plain")(ops._p(x), ops.c_long(ld), ops._p(w), ops.c_long(K), ops._p(out), ops.c_long(N),
+                                                      ops.c_int(ops._code(x)), ops.c_int(ops._code(out)), ops.c_int(M), ops.c_int(N),
+                                                      ops.c_int(K), ops.c_float(1.0), ops._stream()))
+    assert torch.equal(out, want)
