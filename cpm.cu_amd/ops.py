@@ -2378,6 +2378,10 @@ def attention_any(q, out, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, pa
             and kpool.shape[2] == nkv * hdk and v_share == 1 and not softcap and out.dtype == q.dtype):
         attention(q, out, nh, nkv, hdk, scale, kpool, vpool, page_table, page_size, ctx)
         return False
+    # (as the kernels ask, but of the mask as it is given: a step at small positions is refused like those that follow)
+    if chunk < 0 or window < 0 or keep_first < 0 or (chunk and window) or (keep_first and not window):
+        raise KernelError(f"attention: mask chunk {chunk}, window {window}, keep_first {keep_first} (a chunk, or a window with or "
+                          f"without kept first tokens)")
     if not ctx.single_token:
         # a mask that cuts nothing off at the step's positions is none
         if ctx.max_pos < chunk:
