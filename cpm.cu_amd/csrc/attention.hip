@@ -1095,9 +1095,11 @@ __global__ __launch_bounds__(NW * 64) void attention_prefill_mfma_kernel(
 #pragma unroll
                 for (int r = 0; r < R; ++r) {
                     const float om = ml_s[r][n][0], ol = ml_s[r][n][1];
-                    if (ol > 0.f) {
+                    // (a wavefront without keys for the row has a sum of 0; one that saw a score that is no number has none either, and
+                    // must be told from it: bits are compared, floats as if there were no NaN)
+                    if (__float_as_uint(ol)) {
                         const float m_new = fmaxf(m[r], om);
-                        const float sa = l[r] > 0.f ? fast_exp2(m[r] - m_new) : 0.f;
+                        const float sa = __float_as_uint(l[r]) ? fast_exp2(m[r] - m_new) : 0.f;
                         const float sb = fast_exp2(om - m_new);
                         l[r] = l[r] * sa + ol * sb;
                         m[r] = m_new;

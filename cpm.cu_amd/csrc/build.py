@@ -55,8 +55,9 @@ HIPCC_FLAGS = [
 
 # extra flags of single libraries
 #   attention: matrix-core results stay in ordinary vector registers (with the accumulation registers the
-#   compiler moves the running output there and back around every rescale); no score is ever NaN, which
-#   spares a canonicalising instruction before every max
+#   compiler moves the running output there and back around every rescale); floats are compared as if there were no
+#   NaN, which spares a canonicalising instruction before every max (a score that is no number still makes its row none:
+#   it passes through sums and products, and where the prompt kernel asks for a share it asks for bits)
 MODULE_FLAGS: Dict[str, List[str]] = {
     "attention": ["-mllvm", "-amdgpu-mfma-vgpr-form", "-fno-honor-nans"],
 }

@@ -89,6 +89,44 @@ def test_prompts_with_masks_sinks_and_gates(nh, nkv, hd, opt, waves):
         assert bool(((got[t] - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-5)[fine[t]].all()), (t, p, s)
 
 
+@pytest.mark.parametrize("waves", [1, 2, 4])
+@pytest.mark.parametrize("nh,nkv,hd,opt", [
+    (32, 8, 128, {}), (4, 4, 64, {"window": 37}), (8, 2, 80, {"chunk": 48, "sink": True, "gate": True}), (16, 1, 32, {"window": 70, "out": torch.float32}),
+])
+def test_infinities_and_nans_in_queries_and_keys(nh, nkv, hd, opt, waves):
+    """Scores that are infinite or no numbers: the general kernel's results (with one wavefront a group to the last bit), and
+    rows that see none of them beside rows that do."""
+    from cpmcu_amd import ops
+    page, g = 64, torch.Generator().manual_seed(nh + hd)
+    odd = [(37, 5, math.inf), (60, 2, -math.inf), (90, 1, math.nan), (130, 0, math.inf), (64, 3, -math.nan)]
+    table, kpool, _ = cached(SPANS, nkv, hd, page, g, True, odd)
+    _, vpool, _ = cached(SPANS, nkv, hd, page, g, False)
+    pos, slot = tokens(SPANS)
+    n, scale = pos.numel(), 1.3 * hd ** -0.5
+    q = torch.randn(n, nh, hd, generator=g).to(torch.bfloat16)
+    for t, value in ((3, math.nan), (17, math.inf), (18, -math.inf), (n - 2, math.nan), (n - 60, math.inf)):
+        q[t, t % nh, t % hd] = value
+    q[25, :, 1] = math.inf
+    sink = torch.randn(nh, generator=g) if opt.get("sink") else None
+    gate = torch.randn(n, nh * hd, generator=g).to(torch.bfloat16) if opt.get("gate") else None
+    dev = lambda t: None if t is None else t.to(DEV)
+    out, other = (torch.full((n, nh * hd), 7.0, dtype=opt.get("out", torch.bfloat16), device=DEV) for _ in range(2))
+    rows, shape = dev(q.view(n, -1)), (scale, kpool, vpool, table, page, pos, slot)
+    tiles = ops.prefill_tiles([b - a for a, b in SPANS], ops.attention_prefill_tokens_per_wave(nh, nkv, 2), DEV)
+    ops.attention_prefill_mfma(rows, out, tiles, nh, nkv, hd, *shape, 2, waves, opt.get("chunk", 0), opt.get("window", 0), dev(sink), dev(gate), True)
+    tpt = ops.attention_general_tokens_per_tile(n, nh, nkv, hd)
+    ops.attention_general_mfma(rows, other, nh, nkv, hd, hd, *shape, opt.get("chunk", 0),
+                               tiles=ops.prefill_tiles([b - a for a, b in SPANS], tpt, DEV) if tpt > 1 else None, tokens_per_tile=tpt,
+                               window=opt.get("window", 0), sink=dev(sink), gate=dev(gate))
+    assert torch.equal(out.isnan(), other.isnan()) and torch.equal(out.isinf(), other.isinf())
+    assert bool(out.isnan().any()) and bool(out.isfinite().any())
+    if waves == 1:
+        assert torch.equal(out.nan_to_num(7.0), other.nan_to_num(7.0))
+    else:       # another order of the same sums: weights of half an ulp and the output's rounding, values of about 4 at most
+        fine = other.isfinite()
+        assert float((out - other)[fine].abs().max()) <= 2.0 ** -8 * 8
+
+
 @pytest.mark.parametrize("spread", [1.0, 3.0])
 def test_weights_round_no_worse_than_in_the_general_kernel(spread):
     from cpmcu_amd import ops
