@@ -1102,6 +1102,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_skinny_kernel(const bf16_t* __re
 // Measured in a chain of launches over weights that no cache holds (us at 1 / 8 / 16 rows, above -> here):
 //   4,096 x 4,096 13.4/13.9/14.3 -> 8.0/8.4/9.7     6,144 x 4,096 16.3/16.6/17.0 -> 11.0/12.1/14.4     9,280 x 4,096 17.2/18.0/19.0 -> 16.5/17.0/18.8
 //   16,384 x 4,096 25.9/26.2/26.7 -> 24.5/24.5/27.5 73,448 x 4,096 101/102/105 -> 92.6/100/122         4,096 x 16,384 45.8/47.1/49.2 -> 24.2/25.3/29.7
+//   1,024 x 1,024 4.2/4.4/4.8 -> 2.9/3.2/3.6        8,192 x 1,024 5.1/5.2/5.5 -> 4.5/4.7/5.3           73,448 x 1,024 25.3/26.2 -> 23.8/26.1
+//   1,024 x 128 3.0/3.2/3.5 -> 2.5/2.9/3.2          8,192 x 128 3.2/3.3/3.6 -> 2.7/3.0/3.5             4,096 x 2,048 7.1/7.3/7.8 -> 4.7/5.0/5.5
 // K is a multiple of 128 (nothing is padded).  ACT: Y (bf16) = act(alpha * product).
 template <int PF, typename OT, bool ACT>
 __global__ __launch_bounds__(64) void gemm_strip_kernel(const bf16_t* __restrict__ X, long ldx, const bf16_t* __restrict__ W,
@@ -1190,9 +1192,10 @@ extern "C" const char* cpmcu_gemm_skinny(const void* X, long ldx, const void* W,
     const int I = N / 2;
     const long part_stride = (long)M * ldy;
     // One wavefront a strip where that is the faster one: up to 8 rows everywhere, up to 16 where the kernel below leaves CUs
-    // without a workgroup of 64 weight rows (beyond, every strip's own copy of x costs more).  Blocks in flight: 8 where a CU has few
-    // strips, and where so many weights are streamed that only memory counts.
-    if (tiled && M <= (N <= 8192 ? 16 : 8) && (out_mode == 0 || out_mode == 3) && K % 128 == 0 &&
+    // without a workgroup of 64 weight rows (beyond, every strip's own copy of x costs more, and with few columns, where a wavefront's
+    // strip is short, its start does: 40,000 x 256 6.8 -> 10.3, 32,768 x 512 7.1 -> 7.3, 16,384 x 1,024 7.0 in both).  Blocks in flight:
+    // 8 where a CU has few strips, and where so many weights are streamed that only memory counts.
+    if (tiled && M <= (N <= 8192 ? 16 : K >= 1024 ? 8 : 0) && (out_mode == 0 || out_mode == 3) && K % 128 == 0 &&
         (out_mode == 3 || out_dtype == CPMCU_F32 || out_dtype == CPMCU_BF16)) {
 #define STRIPS(PFv, OT, ACTv)                                                                                        \
     gemm_strip_kernel<PFv, OT, ACTv><<<(N + 15) / 16, 64, 0, stream>>>((const bf16_t*)X, ldx, (const bf16_t*)W, (OT*)Y, ldy, M, \

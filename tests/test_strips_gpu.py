@@ -49,7 +49,7 @@ def test_residual_products_at_the_borders_of_the_wavefronts_shares(n, K):
     assert float((sums.double().sum(1) - (want ** 2).sum(1)).abs().max()) <= 1e-5 * float((want ** 2).sum(1).max())
 
 
-@pytest.mark.parametrize("n,N,K", [(1, 16, 128), (8, 100, 1152), (16, 8192, 256), (9, 2000, 384), (3, 9000, 640), (8, 33000, 128), (16, 40, 4096)])
+@pytest.mark.parametrize("n,N,K", [(1, 16, 128), (8, 100, 1152), (16, 8192, 256), (9, 2000, 384), (3, 9000, 640), (8, 33000, 128), (16, 40, 4096), (2, 9000, 1024), (8, 33000, 1152)])
 @pytest.mark.parametrize("mode,dtype", [("plain", torch.float32), ("plain", torch.bfloat16), ("act", torch.bfloat16)])
 def test_products_of_one_wavefront_a_strip(n, N, K, mode, dtype):
     """Fewer blocks than are asked for ahead, one more, many; columns that end inside a strip: the results of the product that
