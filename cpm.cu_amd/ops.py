@@ -2022,13 +2022,14 @@ def gated_strip_ok(n: int, K: int) -> bool:
 
 def gated_strip(x: torch.Tensor, w: "TiledWeight", out: torch.Tensor, row_scale: Optional[RowScale] = None,
                 activation="silu", most: int = STRIP_ROWS):
-    """out = act(x . Wg^T) * (x . Wu^T) (act as in silu_mul) for a step of at most ``most`` tokens (16; up to 64 where
-    gated_strip_ok says so), w tiled with the gate rows first (a multiple of 16 of them); out bfloat16 [n, N/2].  With
-    row_scale as in gemm_skinny."""
+    """out = act(x . Wg^T) * (x . Wu^T) (act as in silu_mul) for a step that gated_strip_ok takes, of at most ``most`` tokens (a
+    caller that goes by that rule says STRIP_MAX_ROWS), w tiled with the gate rows first (a multiple of 16 of them); out
+    bfloat16 [n, N/2].  With row_scale as in gemm_skinny."""
     _need(x, "gated x", torch.bfloat16, (None, None))
     n, K = x.shape
-    if n > most:
-        raise KernelError(f"gated_strip: {n} tokens (1..{most} are taken; more go through the skinny product)")
+    if n > most or not gated_strip_ok(n, K):
+        raise KernelError(f"gated_strip: {n} tokens of {K} columns (1..{min(most, STRIP_ROWS)} are taken, {most} of up to 1,024; more go "
+                          f"through the skinny product)")
     if not isinstance(w, TiledWeight) or w.K != K or w.N % 32:
         raise KernelError(f"gated_strip: the weight must be tiled for K = {K} with a multiple of 16 gate rows")
     _need(out, "gated out", torch.bfloat16, (n, w.N // 2))

@@ -123,7 +123,7 @@ class Linear(Part):
         act = ctx.ws.get(tag + ".act", (n, half), x.dtype)
         if (ops.gated_strip_ok(n, self.in_features) and x.dtype == torch.bfloat16 and self.tiled is not None and half % 16 == 0
                 and self.in_features % 8 == 0):
-            ops.gated_strip(x, self.tiled, act, row_scale=row_scale, activation=activation, most=n)   # a strip of columns a workgroup
+            ops.gated_strip(x, self.tiled, act, row_scale=row_scale, activation=activation, most=ops.STRIP_MAX_ROWS)   # a strip of columns a workgroup
         elif self._gated_skinny(n, x.dtype):
             ops.gemm_skinny(x, self.tiled if self.tiled is not None else self.weight, act, mode="gated",
                             row_scale=row_scale, activation=activation)
