@@ -124,3 +124,43 @@ def test_sum_of_a_tokens_experts(top, H, shared_dtype, joined):
     terms = torch.cat(terms, 1)
     mag = terms.abs().sum(1) + (0 if shared is None or shared.dim() < 3 else sg.double()[:, None] * shared.double().abs().sum(0))
     assert bool(((got.double() - terms.sum(1)).abs() <= (terms.shape[1] + 3) * 2.0 ** -23 * mag).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_gated_experts_of_more_pairs_than_a_grid_dimension(dtype):
+    """33,003 pairs: the launch has two layers of 32,768; identity experts write nothing."""
+    from cpmcu_amd import ops
+    n, top, E, H, F = 11001, 3, 7, 16, 24
+    g = torch.Generator(device=DEV).manual_seed(3)
+    h, gu = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((n, H), (E, 2 * F, H)))
+    idx = torch.randint(0, E + 2, (n, top), generator=torch.Generator().manual_seed(4), dtype=torch.int32).to(DEV)
+    act = torch.full((n, top, F), float("nan"), dtype=dtype, device=DEV)
+    ops.moe_gated(h, gu, idx, act)
+    real = idx < E
+    assert torch.equal(act.isnan(), ~real[..., None].expand_as(act))
+    y = torch.matmul(gu.double(), h.double().T).permute(2, 0, 1)                          # [n, E, 2F]
+    y = torch.gather(y, 1, idx.long().clamp(max=E - 1)[..., None].expand(n, top, 2 * F))
+    want = torch.nn.functional.silu(y[..., :F]) * y[..., F:]
+    # H float sums of both factors, and the output's own rounding
+    mag = torch.gather(torch.matmul(gu.double().abs(), h.double().abs().T).permute(2, 0, 1), 1, idx.long().clamp(max=E - 1)[..., None].expand(n, top, 2 * F))
+    off = (H + 6) * 2.0 ** -24 * (1.1 * mag[..., :F] * y[..., F:].abs() + mag[..., F:] * y[..., :F].abs() + want.abs()) + 1e-30
+    off = off + (2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -23) * want.abs()
+    assert bool(((act.double() - want).abs() <= off)[real].all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n", [1, 3, 16, 37])
+@pytest.mark.parametrize("H", [8, 120, 128, 136, 264, 1000])
+def test_down_products_of_any_number_of_column_blocks(n, H, dtype):
+    """Blocks of 16 columns are dealt to the XCDs by eights, what is left over in order: 1, 8, 9, 17 and 63 blocks, all written."""
+    from cpmcu_amd import ops
+    E, F, top = 5, 40, 3
+    g = torch.Generator(device=DEV).manual_seed(n + H)
+    act, down = (torch.randn(*s, generator=g, device=DEV).to(dtype) for s in ((n, top, F), (E, H, F)))
+    idx = torch.randint(0, E, (n, top), generator=torch.Generator().manual_seed(n), dtype=torch.int32).to(DEV)
+    w = torch.rand(n, top, generator=g, device=DEV)
+    out = torch.full((n, H), float("nan"), device=DEV)
+    ops.moe_down(act, down, idx, w, out)
+    terms = w.double()[..., None] * torch.matmul(down.double()[idx.long()], act.double()[..., None])[..., 0]
+    mag = w.double()[..., None] * torch.matmul(down.double().abs()[idx.long()], act.double().abs()[..., None])[..., 0]
+    assert bool(((out.double() - terms.sum(1)).abs() <= (F + top + 2) * 2.0 ** -24 * mag.sum(1)).all())
