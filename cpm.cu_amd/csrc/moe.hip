@@ -666,7 +666,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
 // With up to 64 rows a tile, where most weights are read once, they are streamed past the caches: both products of 24
 // tokens 338 -> 322 us, of 300 tokens 433 -> 403; with more tokens tiles share weights.
 // Two pieces on their way at once: one made no difference beyond 300 tokens, at 24 it took 234 + 122 us.
-// Of 128-row tiles there is a form for every 16 rows, and results leave through LDS as whole lines (every lane stored its
+// Of 128-row tiles there is a form for every 16 rows beyond 64 (and one each for up to 16, 32 and 64), and results leave through LDS as whole lines (every lane stored its
 // 2 bytes): 2,048 tokens, both products and the sum, us: 64 experts of 1,408, 6 of 80 (16 identity) 791 -> 748, of 64 864
 // -> 802; of 2,112 without a gate 831 -> 774; 512 tokens 513 -> 496, 1,024 of 2,112 621 -> 588 (the sum unchanged there).
 // What bounds the wide tiles is the stream of pieces: products without stores or multiplications take 80% of the time, and
@@ -879,7 +879,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const bf16_t* __restri
 
 // The same sums for up to 8 experts a token, a workgroup 2,048 columns of a token, 8 neighbouring ones a thread: the token's
 // experts and weights are scalars, and all TOP rows are asked for before the first is added (the kernel above has two in flight).
-// 2,048 tokens, 6 experts, width 4,096: 39.3 -> 22.5 us (100 MB of rows in, 34 out: 6 TB/s).
+// 2,048 tokens, 6 experts, width 4,096: 39.3 -> 22.5 us (100 MB of rows in, 34 out: 6 TB/s); in a pass that joins the shared
+// experts' result and the residual, read and written, on its way 47 to 50.
 template <typename ST, int TOP>
 __global__ __launch_bounds__(256) void moe_combine_token_kernel(const bf16_t* __restrict__ y, const float* __restrict__ w,
                                                                 const ST* __restrict__ shared, int shared_parts,

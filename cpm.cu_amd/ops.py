@@ -126,10 +126,10 @@ NORM_SLICE = 64        # columns a slice of add_norm_columns (common.h)
 # The kernels of decode steps that own a strip of output columns over all of K (qkv_rope, proj_add_norm) and
 # the norm cut by columns (add_norm_columns) save kernels of the chain, but every workgroup reads all of x.
 # Up to 16 rows they win at every width measured (MI355X, 4,096 columns: norm 4.7 against 6.6 us at 8 rows).
-# qkv_rope (workgroups spread evenly over the CUs) wins up to 32 rows (4,096 columns, q/k/v + rotary: 11.7
-# against 18.2 us at 16 rows, 15.6 against 19.7 at 24, 16.5 against 21.3 at 32; it loses beyond: 24.6 against
-# 21.3 at 48, 27.2 against 23.2 at 64; see qkv_rope_faster for fewer columns), and proj_add_norm wins beyond 16 rows only while a workgroup's copy of
-# x stays small (1,024 columns, 64 rows: 8.6 against 8.9 + 4.2 us).
+# qkv_rope (workgroups spread evenly over the CUs) wins up to 32 rows (4,096 columns, q/k/v + rotary, as the kernels were when
+# the line was drawn: 11.7 against 18.2 us at 16 rows, 15.6 against 19.7 at 24, 16.5 against 21.3 at 32); beyond it loses there
+# and wins with fewer columns (qkv_rope_faster).  proj_add_norm wins beyond 16 rows only while a workgroup's copy of x stays
+# small (1,024 columns, 64 rows: 8.6 against 8.9 + 4.2 us).
 STRIP_ROWS = 16
 STRIP_MAX_ROWS = 64
 STRIP_X_BYTES = 160 * 1024
@@ -2353,15 +2353,19 @@ class HeadFinish:
         self.out, self.inv_freq, self.gate, self.interleaved = out, inv_freq, gate, bool(interleaved)
 
 
-def attention_prompt_pays(n_tokens: int, max_pos: int) -> bool:
+def attention_prompt_pays(n_tokens: int) -> bool:
     """Whether attention_any's prompts of heads up to 128 features go to the prompt kernel, whose wavefronts load the keys for
-    two tiles of 16 columns instead of one.  Measured (us, general kernel / the prompt kernel with 1, 2 wavefronts sharing a
+    two tiles of 16 columns instead of one.  Measured (us, general kernel / the prompt kernel with 1, 2, 4 wavefronts sharing a
     group of tiles; 32 heads on 8 of 128; tokens + tokens of history):
-      2,048 + 0 214/98/88, 2,048 + 2,048 in a window of 2,048 311/185/124 and in chunks of 2,048 202/92/80, 1,500 + 0 114/54/54,
-      4 x 479 68/35/38, 8 x 200 40/27/28, 347 + 0 26/17/17, 300 + 0 beside 8 x 1 + 4,000 282/99/56;
-      12 heads on 4 of 64, 1,000 39/32/27; 32 heads of their own, 700 61/29/24.
-    Up to 256 tokens the two are level.  With one wavefront a group the results are the general kernel's to the last bit, and up to
-    2,048 positions that costs little."""
+      2,048 + 0 205/94/82/87, 1,500 + 0 112/53/53/57, 4 x 479 67/34/37/51, 8 x 200 38/25/27/38, 347 + 0 25/17/17/16;
+      2,048 + 2,048 in a window of 2,048 315/193/124/121 and in chunks of 2,048 196/90/78/83, 300 + 0 beside 8 x 1 + 4,000
+      282/88/51/36, 300 + 3,000 228/79/63/44 and in a window of 1,024 78/33/29/24, 1,000 + 2,500 258/89/80/88 and 91/41/38/44,
+      600 + 8,000 608/185/146/143;
+      12 heads on 4 of 64, 1,000 + 0 38/32/28/30, 300 + 3,000 110/61/48/38; 32 heads of their own, 700 + 0 61/27/23/29.
+    Up to 256 tokens the two are level.  attention_any takes one wavefront a group up to 2,048 positions, with which the results are
+    the general kernel's to the last bit where 16 is a multiple of the heads a key head, and from there on
+    attention_prefill_shape's 4 (up to 1,024 tokens), 2 or 1.  Two would be up to 15% faster than one for a single prompt and up
+    to 9% slower for several short ones."""
     return n_tokens > 256
 
 
@@ -2390,7 +2394,7 @@ def attention_any(q, out, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, pa
         if ctx.max_pos < window:
             window = keep_first = 0
         if (hdk == hdv and keep_first == 0 and not softcap and v_share == 1 and kpool.shape[2] == nkv * hdk
-                and vpool.shape[2] == nkv * hdv and attention_mfma_ok(q, hdk, page_size) and attention_prompt_pays(q.shape[0], ctx.max_pos)):
+                and vpool.shape[2] == nkv * hdv and attention_mfma_ok(q, hdk, page_size) and attention_prompt_pays(q.shape[0])):
             attention_prompt(q, out, nh, nkv, hdk, scale, kpool, vpool, page_table, page_size, ctx, chunk=chunk, window=window,
                              sink=sink, gate=gate, general=True, waves=1 if ctx.max_pos < 2048 else 0)
             return gate is not None
