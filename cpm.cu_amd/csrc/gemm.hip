@@ -62,12 +62,12 @@ __global__ __launch_bounds__(256) void gemm_tiled_kernel(const XT* __restrict__ 
 // (32 multiply-adds a cycle and SIMD, 157 TFLOP/s on the chip); v_mfma_f32_16x16x32_bf16 does 16 times as many, so that eight
 // of its products, which a float as three bf16 asks for (below), still are twice as fast.
 //
-// gemm_f32_mfma_kernel: the float instruction, for few columns.  256 threads, a
-// wavefront 16 x 16 of a 32 x 32 tile; 64 columns of both operands go through LDS in two buffers, the next ones on their way
-// to registers meanwhile, one barrier a piece.  A row of a piece is 16 chunks of 16 bytes, chunk c of row r at place
-// c ^ (r % 8), so that 8 neighbouring lanes (8 rows, one chunk) read all banks.  A lane's 16 bytes serve four instructions: in
-// instruction s, lane group g stands for column 4 g + s of the 16, in both operands alike (a sum over columns may take them
-// in any order).
+// gemm_f32_mfma_kernel: the float instruction, for few columns.  256 threads, 2 x 2 wavefronts of 32 x 32 outputs each; 32 columns
+// of both operands go through LDS in two buffers, the next ones on their way to registers meanwhile, one barrier a piece.  A row
+// of a piece is 8 chunks of 16 bytes, chunk c of row r at place c ^ (r % 8), so that 8 neighbouring lanes (8 rows, one chunk) read
+// all banks.  A lane's 16 bytes serve four instructions: in instruction s, lane group g stands for column 4 g + s of the 16, in
+// both operands alike (a sum over columns may take them in any order).  Tiles of 32 x 32 outputs and 64 columns are level up to
+// 130 x 8,192 and slower beyond (us, rows x outputs x columns: 2,048 x 4,096 x 32 22.3 -> 12.7, 523 x 8,192 x 48 12.4 -> 11.2).
 // ---------------------------------------------------------------------------
 typedef float gfloatx4_t __attribute__((ext_vector_type(4)));
 
@@ -90,7 +90,7 @@ template <bool VEC>
 __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ X, long ldx,
                                                             const float* __restrict__ W, long ldw, float* __restrict__ Y,
                                                             long ldy, int M, int N, int K, float alpha) {
-    constexpr int BM = 32, BN = 32, BK = 64, CH = BK / 4, PIECES = (BM + BN) * CH / 256;
+    constexpr int TM = 2, TN = 2, BK = 32, BM = 32 * TM, BN = 32 * TN, CH = BK / 4, PIECES = (BM + BN) * CH / 256;
     __shared__ float lds[2][(BM + BN) * BK];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
@@ -107,8 +107,12 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
     gfloatx4_t next[PIECES];
 #pragma unroll
     for (int i = 0; i < PIECES; ++i) next[i] = f32_piece<VEC>(src[i], chunk * 4, K);
-    gfloatx4_t acc = {0.f, 0.f, 0.f, 0.f};
-    const int row_a = (wave & 1) * 16 + r, row_b = BM + (wave >> 1) * 16 + r;
+    gfloatx4_t acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    const int row_a = (wave & 1) * 16 * TM + r, row_b = BM + (wave >> 1) * 16 * TN + r;
     int buf = 0;
     for (int k0 = 0; k0 < K; k0 += BK, buf ^= 1) {
 #pragma unroll
@@ -121,17 +125,33 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 #pragma unroll
         for (int kb = 0; kb < BK / 16; ++kb) {
             const int at = ((kb * 4 + g) ^ (r & 7)) << 2;
-            const gfloatx4_t a = *(const gfloatx4_t*)&lds[buf][row_a * BK + at], b = *(const gfloatx4_t*)&lds[buf][row_b * BK + at];
+            gfloatx4_t a[TM], b[TN];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[s], b[s], acc, 0, 0, 0);
+            for (int i = 0; i < TM; ++i) a[i] = *(const gfloatx4_t*)&lds[buf][(row_a + 16 * i) * BK + at];
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[j] = *(const gfloatx4_t*)&lds[buf][(row_b + 16 * j) * BK + at];
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][s], b[j][s], acc[i][j], 0, 0, 0);
         }
     }
-    // lane (column r, g): acc[e] is row 4 g + e of its 16 x 16 outputs
+    // lane (column r, g): acc[i][j][e] is row 4 g + e of its 16 x 16 outputs
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int m = m0 + (wave & 1) * 16 + 4 * g + e, n = n0 + (wave >> 1) * 16 + r;
-        if (m < M && n < N) Y[(long)m * ldy + n] = alpha * acc[e];
-    }
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + (wave & 1) * 16 * TM + 16 * i + 4 * g + e;
+            if (m >= M) continue;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const int n = n0 + (wave >> 1) * 16 * TN + 16 * j + r;
+                if (n < N) Y[(long)m * ldy + n] = alpha * acc[i][j][e];
+            }
+        }
 }
 
 // ---------------------------------------------------------------------------
@@ -501,9 +521,9 @@ static void gemm_f32_launch(const float* X, long ldx, const float* W, long ldw, 
         gemm_f32_rows_kernel<16, VEC><<<up(N, 16), 1024, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
         return;
     }
-    // (few columns, up to two pieces: 523 x 8,192 x 48 12.4 us, 13.9 in three parts; 523 x 1,024 x 32 both 7.2)
-    if (K < 64 && up(M, 32) <= 65535) {
-        gemm_f32_mfma_kernel<VEC><<<dim3(up(N, 32), up(M, 32)), 256, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
+    // (few columns, up to two pieces: 523 x 8,192 x 48 11.2 us, 13.9 in three parts; 2,048 x 4,096 x 32 12.7, 16.4; 523 x 1,024 x 32 6.8, 7.2)
+    if (K < 64) {
+        gemm_f32_mfma_kernel<VEC><<<dim3(up(N, 64), up(M, 64)), 256, 0, stream>>>(X, ldx, W, ldw, Y, ldy, M, N, K, alpha);
         return;
     }
     // Columns shared out while the tiles are at most one a CU: the smallest tile for which that holds (its wavefronts' pieces cost
