@@ -588,14 +588,14 @@ extern "C" const char* cpmcu_moe_down(const void* act, int dtype, const void* wd
 
 // ===========================================================================
 // The same experts for steps of many tokens, bf16 on the matrix cores (v_mfma_f32_16x16x32_bf16): the (token,
-// chosen expert) pairs are grouped by expert into tiles of up to MOE_TILE or 2 MOE_TILE rows, and every tile is a
+// chosen expert) pairs are grouped by expert into tiles of up to MOE_TILE or MOE_WIDE rows, and every tile is a
 // product with its expert's weights.
 //
 //  * moe_group_kernel (one workgroup): counts the pairs of every expert and lists them expert by expert: rows[offs[e] ..
 //    offs[e + 1]) are expert e's pairs, tile_expert[tile] = e + 1024 * (the tile's number among its expert's), n_tiles the
 //    number of tiles.  Which row of its expert's tiles a pair gets depends on timing; its result does not (a row's sums
 //    are its own).
-//  * moe_tile_kernel: GATED act[pair] = act(Wg_e h_t) * (Wu_e h_t), PLAIN act[pair] = act(Wu_e h_t), DOWN y[pair] =
+//  * moe_tile_kernel, moe_wide_kernel: GATED act[pair] = act(Wg_e h_t) * (Wu_e h_t), PLAIN act[pair] = act(Wu_e h_t), DOWN y[pair] =
 //    Wd_e act[pair] (bf16).
 //  * moe_combine_kernel: out[t] = sum_k w[t, k] y[t, k] (h_t where the chosen expert is an identity expert) (+ sg[t] * shared[t]) in float, k in order.
 // ===========================================================================
@@ -603,7 +603,8 @@ typedef __bf16 mbf16x8_t __attribute__((ext_vector_type(8)));
 typedef float mfloatx4_t __attribute__((ext_vector_type(4)));
 typedef unsigned mu32x4_t __attribute__((ext_vector_type(4)));
 
-#define MOE_TILE 64
+#define MOE_TILE 64                            // rows of a tile of moe_tile_kernel at most
+#define MOE_WIDE 128                           // of moe_wide_kernel
 enum { MOE_GATED = 0, MOE_PLAIN = 1, MOE_DOWN = 2 };
 
 // tile_rows: rows a tile at most; an expert's pairs are spread evenly over as few tiles as hold them (moe_tile_kernel)
@@ -654,32 +655,25 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
     }
 }
 
-// Workgroups of 4 wavefronts; a tile of up to 16 RT rows against 128 weight rows (GATED: 64 features, gate and up row of
+// Workgroups of 4 wavefronts; a tile of up to 64 rows against 128 weight rows (GATED: 64 features, gate and up row of
 // each), a wavefront all rows and 32 weight rows (GATED: 16 features).  Pieces of 64 columns of both go through LDS in
 // two buffers, the next piece on its way to registers meanwhile (with both operands straight from memory every wavefront
 // fetched all of the rows for itself, 16 bytes of a row an access, and the address unit, not HBM or the matrix cores,
 // was the bound).  A piece's row is 8 chunks of 16 bytes, chunk c of row r at place c ^ (r % 8): 8 neighbouring lanes
-// then read all banks.  The tile's rows beyond the last 16 in use are neither loaded nor multiplied.
+// then read all banks.  The tile's rows beyond the last 16 (beyond 32: 32) in use are neither loaded nor multiplied.
 // K is the rows' width, N the number of features; in: h rows by token (GATED, PLAIN: pair / top) or act rows by pair.
-// Measured (64 experts, width 4,096, 6 a token; us, before -> now): gated experts of 1,408, 2,048 tokens 1,250 -> 464
-// and 612 -> 278 (down), 24 tokens 303 -> 222 and 169 -> 116 (their 58 experts' matrices at 6 TB/s); 8 tokens 129 + 67.
-// With up to 64 rows a tile, where most weights are read once, they are streamed past the caches: both products of 24
-// tokens 338 -> 322 us, of 300 tokens 433 -> 403; with more tokens tiles share weights.
-// Two pieces on their way at once: one made no difference beyond 300 tokens, at 24 it took 234 + 122 us.
-// Of 128-row tiles there is a form for every 16 rows beyond 64 (and one each for up to 16, 32 and 64), and results leave through LDS as whole lines (every lane stored its
-// 2 bytes): 2,048 tokens, both products and the sum, us: 64 experts of 1,408, 6 of 80 (16 identity) 791 -> 748, of 64 864
-// -> 802; of 2,112 without a gate 831 -> 774; 512 tokens 513 -> 496, 1,024 of 2,112 621 -> 588 (the sum unchanged there).
-// What bounds the wide tiles is the stream of pieces: products without stores or multiplications take 80% of the time, and
-// 256 rows or 256 weight rows a workgroup of 8 wavefronts, with half of the LDS reads, were no faster (449 to 540 us for 420).
+// Measured (64 experts, width 4,096, 6 a token; us): 24 tokens, gated experts of 1,408 182 + 93 (their 58 experts' matrices
+// at 6 to 7 TB/s); most weights are read once and streamed past the caches.  Two pieces on their way at once: one took 234 +
+// 122.  Results leave through LDS as whole lines.
 // The grid is dealt to the 8 XCDs in turn; each takes one run of the tasks, ordered expert by expert and within an expert
 // weight rows by weight rows, so that the tiles that share weights meet in one L2.
-template <int KIND, int RT>
+template <int KIND>
 __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restrict__ in, long ldi,
                                                           const bf16_t* __restrict__ w, const int* __restrict__ rows,
                                                           const int* __restrict__ offs, const int* __restrict__ tile_expert,
-                                                          const int* __restrict__ n_tiles, bf16_t* __restrict__ out, int K, int N, int top, int act_fn,
-                                                          float act_limit) {
-    constexpr int BM = 16 * RT, FEATURES = KIND == MOE_GATED ? 64 : 128;
+                                                          const int* __restrict__ n_tiles, bf16_t* __restrict__ out, int K, int N, int top, int tile_rows,
+                                                          int act_fn, float act_limit) {
+    constexpr int BM = MOE_TILE, FEATURES = KIND == MOE_GATED ? 64 : 128;
     __shared__ mu32x4_t lds[2][(BM + 128) * 8];
     const int nts = (N + FEATURES - 1) / FEATURES;
     const int tasks = *n_tiles * nts, per = (tasks + 7) / 8;
@@ -687,7 +681,7 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
     if ((int)(blockIdx.x >> 3) >= per || task >= tasks) return;
     const int q = task / nts, te = tile_expert[q], e = te & 1023;
     const int start = offs[e], cnt = offs[e + 1] - start;
-    const int m = (cnt + BM - 1) / BM, rpt = ((cnt + m - 1) / m + 15) & ~15;
+    const int m = (cnt + tile_rows - 1) / tile_rows, rpt = ((cnt + m - 1) / m + 15) & ~15;
     const int local = task - (q - (te >> 10)) * nts, mt = local % m, f0 = local / m * FEATURES;
     const int row0 = start + mt * rpt, n_rows = min(rpt, cnt - mt * rpt);
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -716,10 +710,7 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
         auto fetch = [&](Piece& p, int k0) {
             const int k = min(k0, K - 8 - chunk * 8);                 // beyond the row's end: its last columns, zeroed below
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (RT == 4) p.w[i] = __builtin_nontemporal_load((const mu32x4_t*)(wp[i] + k));
-                else p.w[i] = *(const mu32x4_t*)(wp[i] + k);
-            }
+            for (int i = 0; i < 4; ++i) p.w[i] = __builtin_nontemporal_load((const mu32x4_t*)(wp[i] + k));
 #pragma unroll
             for (int i = 0; i < AP; ++i) p.a[i] = *(const mu32x4_t*)(ap[i] + k);
         };
@@ -758,18 +749,6 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
                 for (int rt = 0; rt < NRT; ++rt)
 #pragma unroll
                     for (int j = 0; j < 2; ++j) acc[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][rt], b[kk][j], acc[rt][j], 0, 0, 0);
-            if constexpr (NRT > 4) {
-                // the order to keep: the first half's operands, then the second half's one by one between the first half's
-                // matrix instructions; left alone, the scheduler reads each operand just before its use (2,048 tokens: 495
-                // against 464 us).  With few rows, where memory is the bound, it is left alone.
-                __builtin_amdgcn_sched_group_barrier(0x100, NRT + 4, 0);
-#pragma unroll
-                for (int rt = 0; rt < NRT; ++rt) {
-                    __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x008, 2, 0);
-                }
-                __builtin_amdgcn_sched_group_barrier(0x008, 2 * NRT, 0);
-            }
         };
         fetch(p0, 0);
         fetch(p1, 64);
@@ -815,15 +794,216 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
                 }
             }
     };
-    if constexpr (RT > 4) {
-        if (n_rows > 112) { product(std::integral_constant<int, 8>()); return; }
-        if (n_rows > 96) { product(std::integral_constant<int, 7>()); return; }
-        if (n_rows > 80) { product(std::integral_constant<int, 6>()); return; }
-        if (n_rows > 64) { product(std::integral_constant<int, 5>()); return; }
-    }
     if (n_rows > 32) product(std::integral_constant<int, 4>());
     else if (n_rows > 16) product(std::integral_constant<int, 2>());
     else product(std::integral_constant<int, 1>());
+}
+
+// 64 lanes' 16 bytes straight from memory to LDS, one behind the other from byte `to` on.  Nothing waits for them but
+// landed(): the compiler does not count loads of an asm block (those of the builtin it does, and before every LDS read).
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"                      // m0 on the clobber list
+__device__ inline void bring16(const void* from, unsigned to) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(from) : "memory", "m0");
+}
+__device__ inline void stream16(const void* from, unsigned to) {      // the same past the caches
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(to), "v"(from) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+// all but this wavefront's last N loads have landed and what it read from LDS has arrived; then the workgroup meets
+template <int N>
+__device__ inline void landed() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// The same products for steps that give an expert many rows: tiles of up to 128 rows against 128 weight rows (GATED: 64
+// features), workgroups of 4 wavefronts, two a CU, a wavefront half of the rows and 64 weight rows.  Pieces of 64 columns go
+// from memory to LDS without passing registers, the weights in three buffers and the rows in two (80 KB), with the swizzle of
+// the kernel above in the column that each lane asks for.  The workgroup meets once a piece, in the middle of its products:
+// what the second half multiplies has been read by then, and while it does, the next piece's first operands are read and the
+// pieces behind it are on their way.  (Through registers, with the meeting before the products, LDS reads and matrix
+// instructions took turns.)  An expert whose rows fill one tile streams its weights past the caches; where tiles share
+// them they stay (all past the caches: 476 instead of 407 us; none: the passes of 347 tokens 282 instead of 254).
+// What bounds it: weights alone take 290 us of about 400 at 2,048 tokens and even routing (5.1 TB/s), products alone 250,
+// rows alone 130; a CU is busy 75 to 80% of the time, since experts' tiles are uneven.
+// Kernel times, us, up + down, the kernel through registers (tiles of 128, under 48 pairs an expert of 64) -> this:
+//   64 experts of 1,408 gated at width 4,096, routers with random weights (from none to 2,000 of 2,048 tokens an expert):
+//     2,048 tokens 465 + 270 -> 424 + 246, 16 of 80 identity 427 + 246 -> 407 + 230, 347 tokens 275 + 157 -> 254 + 145
+//   even routing: 2,048 477 + 269 -> 443 + 252, 768 317 + 177 -> 306 + 167, 512 298 + 167 -> 269 + 156, 280 256 + 146 -> 241 +
+//     132; of 2,112 without a gate, 2,048 372 + 372 -> 350 + 344, 512 246 + 240 -> 229 + 226
+//   64 of 1,024 gated at 1,024, 2,048 tokens with 4 each 89 + 52 -> 75 + 45; 16 of 768 at 2,048 85 + 51 -> 75 + 47
+// Taken back: workgroups of 8 wavefronts, one a CU, with tiles of 256 weight rows and 128, 192 or 256 rows (LDS reads a
+// fifth fewer, weights asked for once: as fast with even routing, 0 to 5% slower with a router's); every XCD a share of all
+// experts' features, for balance (rows no longer meet in an L2: 5% slower).
+template <int KIND>
+__global__ __launch_bounds__(256, 2) void moe_wide_kernel(const bf16_t* __restrict__ in, long ldi,
+                                                          const bf16_t* __restrict__ w, const int* __restrict__ rows,
+                                                          const int* __restrict__ offs, const int* __restrict__ tile_expert,
+                                                          const int* __restrict__ n_tiles, bf16_t* __restrict__ out, int K, int N, int top, int tile_rows,
+                                                          int act_fn, float act_limit) {
+    constexpr int BM = MOE_WIDE, FEATURES = KIND == MOE_GATED ? 64 : 128;
+    constexpr int WSTAGE = 128 * 8;                                   // 16-byte chunks of a piece's weights; three pieces
+    __shared__ mu32x4_t lds[3 * WSTAGE + 2 * BM * 8];
+    const int nts = (N + FEATURES - 1) / FEATURES;
+    const int tasks = *n_tiles * nts, per = (tasks + 7) / 8;
+    const int task = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || task >= tasks) return;
+    const int q = task / nts, te = tile_expert[q], e = te & 1023;
+    const int start = offs[e], cnt = offs[e + 1] - start;
+    const int m = (cnt + tile_rows - 1) / tile_rows, rpt = ((cnt + m - 1) / m + 31) & ~31;
+    const int local = task - (q - (te >> 10)) * nts, mt = local % m, f0 = local / m * FEATURES;
+    const int row0 = start + mt * rpt, n_rows = min(rpt, cnt - mt * rpt);     // (never empty: rpt <= tile_rows)
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int chunk = ((lane & 7) ^ (lane >> 3)) * 8;                 // a lane brings place lane % 8 of row lane / 8 of 8 rows
+    const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+    const int half = wave & 1, side = wave >> 1;
+    const bool whole = (uintptr_t)out % 16 == 0;
+    const bf16_t* wp[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = wave * 32 + i * 8 + (lane >> 3);              // weight row 32 w + 16 j + x, as above
+        const int f = min(f0 + (KIND == MOE_GATED ? (row >> 5) * 16 + (row & 15) : row), N - 1);
+        wp[i] = w + ((long)e * (KIND == MOE_GATED ? 2 : 1) * N + (KIND == MOE_GATED && (row & 16) ? N : 0) + f) * K;
+    }
+    auto product = [&](auto groups) {
+        constexpr int NRT = decltype(groups)::value, HRT = NRT / 2;
+        constexpr int AP = NRT / 2;                                   // groups of 8 rows a wavefront brings
+        constexpr int RSTAGE = 16 * NRT * 8, ROWS = 3 * WSTAGE;
+        const bf16_t* ap[AP];
+#pragma unroll
+        for (int i = 0; i < AP; ++i) {
+            const int pair = rows[row0 + min((i * 4 + wave) * 8 + (lane >> 3), n_rows - 1)];
+            ap[i] = in + (long)(KIND == MOE_DOWN ? pair : pair / top) * ldi;
+        }
+        auto fetch_w = [&](int p, int stage) {
+            const int k = min(p * 64 + chunk, K - 8);
+            const unsigned to = base + (stage * WSTAGE + wave * 256) * 16;
+            if (m == 1) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) stream16(wp[i] + k, to + i * 1024);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) bring16(wp[i] + k, to + i * 1024);
+            }
+        };
+        auto fetch_r = [&](int p) {
+            const int k = min(p * 64 + chunk, K - 8);
+            const unsigned to = base + (ROWS + (p & 1) * RSTAGE) * 16;
+#pragma unroll
+            for (int i = 0; i < AP; ++i) bring16(ap[i] + k, to + (i * 4 + wave) * 1024);
+        };
+        mfloatx4_t acc[HRT][4];
+#pragma unroll
+        for (int rt = 0; rt < HRT; ++rt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[rt][j] = mfloatx4_t{0.f, 0.f, 0.f, 0.f};
+        const int pieces = (K + 63) / 64;
+        mbf16x8_t a[2][HRT], b[2][4];
+        auto read = [&](int p, int stage, int kk) {
+            const int at = (kk * 4 + g) ^ (r & 7);
+            const mu32x4_t* ws = lds + stage * WSTAGE + side * 512;
+            const mu32x4_t* rs = lds + ROWS + (p & 1) * RSTAGE + half * (HRT * 128);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[kk][j] = *(const mbf16x8_t*)&ws[(j * 16 + r) * 8 + at];
+#pragma unroll
+            for (int rt = 0; rt < HRT; ++rt) a[kk][rt] = *(const mbf16x8_t*)&rs[(rt * 16 + r) * 8 + at];
+        };
+        auto multiply = [&](int kk) {
+#pragma unroll
+            for (int rt = 0; rt < HRT; ++rt)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[rt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[kk][rt], b[kk][j], acc[rt][j], 0, 0, 0);
+        };
+        // columns beyond the row's end (K % 8 == 0: whole chunks) are nothing; asked for were the row's last ones
+        auto blank = [&](int p, int stage) {
+            if (p + 1 < pieces || K % 64 == 0) return;
+            for (int i = threadIdx.x; i < WSTAGE + RSTAGE; i += 256) {
+                mu32x4_t* to = i < WSTAGE ? lds + stage * WSTAGE + i : lds + ROWS + (p & 1) * RSTAGE + i - WSTAGE;
+                if (((i & 7) ^ (i >> 3 & 7)) >= K % 64 / 8) *to = mu32x4_t{0u, 0u, 0u, 0u};
+            }
+            __syncthreads();
+        };
+        fetch_w(0, 0);
+        fetch_r(0);
+        if (pieces > 1) {
+            fetch_w(1, 1);
+            fetch_r(1);
+        }
+        if (pieces > 2) {
+            fetch_w(2, 2);
+            landed<8 + AP>();                                         // behind the first piece: w, rows, w
+        } else {
+            landed<0>();
+        }
+        blank(0, 0);
+        read(0, 0, 0);
+        int p = 0, stage = 0;
+        for (; p + 2 < pieces; ++p) {
+            read(p, stage, 1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(0);
+            landed<4>();                                              // behind piece p + 1: the weights of p + 2; p is free
+            fetch_r(p + 2);
+            if (p + 3 < pieces) fetch_w(p + 3, stage);
+            stage = stage == 2 ? 0 : stage + 1;
+            read(p + 1, stage, 0);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(1);
+        }
+        for (; p < pieces; ++p) {
+            read(p, stage, 1);
+            multiply(0);
+            if (p + 1 < pieces) {
+                landed<0>();
+                stage = stage == 2 ? 0 : stage + 1;
+                blank(p + 1, stage);
+                read(p + 1, stage, 0);
+            }
+            multiply(1);
+        }
+        constexpr int LINE = FEATURES + 8;
+        bf16_t* out_stage = (bf16_t*)lds;
+        __syncthreads();
+#pragma unroll
+        for (int rt = 0; rt < HRT; ++rt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                bf16_t* to = out_stage + ((half * HRT + rt) * 16 + 4 * g + i) * LINE + side * (FEATURES / 2) + r;
+                if (KIND == MOE_GATED) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        float gt = acc[rt][2 * j][i], up = acc[rt][2 * j + 1][i];
+                        gate_prepare(gt, up, act_fn, act_limit);
+                        to[j * 16] = f32_to_bf16(gate_act(gt, act_fn) * up);
+                    }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j)
+                        to[j * 16] = f32_to_bf16(KIND == MOE_PLAIN ? plain_act(acc[rt][j][i], act_fn) : acc[rt][j][i]);
+                }
+            }
+        __syncthreads();
+        constexpr int CHUNKS = FEATURES / 8;
+        const int c = threadIdx.x % CHUNKS * 8;
+        if (f0 + c < N)
+            for (int row = threadIdx.x / CHUNKS; row < n_rows; row += 256 / CHUNKS) {
+                bf16_t* to = out + (long)rows[row0 + row] * N + f0 + c;
+                const bf16_t* from = out_stage + row * LINE + c;
+                if (whole) {
+                    *(mu32x4_t*)to = *(const mu32x4_t*)from;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) to[j] = from[j];
+                }
+            }
+    };
+    if (n_rows > 96) product(std::integral_constant<int, 8>());
+    else if (n_rows > 64) product(std::integral_constant<int, 6>());
+    else if (n_rows > 32) product(std::integral_constant<int, 4>());
+    else product(std::integral_constant<int, 2>());
 }
 
 // V neighbouring columns a thread (4: 8-byte loads of a pair's row)
@@ -953,39 +1133,33 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     const long pairs = (long)n * top;
     CPMCU_REQUIRE(max_tiles >= (pairs + MOE_TILE - 1) / MOE_TILE + E && max_tiles <= 65535,
                   "moe_experts_mfma: %d tiles of scratch for %ld pairs of %d experts (at most 65535)", max_tiles, pairs, E);
-    // Tiles of 128 rows where experts have many: once most have more than 64 pairs, tiles of 64 read their weights twice.  Both
-    // products and the sum in us, tiles of 64 / 128 rows, at 32, 40, 48, 56, 64, 96 pairs an expert; experts chosen evenly, and
-    // unevenly (logits with a normal bias of 0.5 an expert), as routers do, for which the line lies where it does:
-    //   64 experts of 1,408 at width 4,096  even    401/446  415/451  432/452  479/470  573/482  782/541
-    //                                       uneven  410/443  448/457  490/473  531/480  578/498  771/555
-    //   64 experts of 2,112 at width 4,096  even    567/624  588/637  615/649  633/658  858/678  1,137/749
-    //                                       uneven  593/633  652/659  706/669  762/698  863/712  1,087/802
-    //   16 experts of 512 at width 1,024    even    32/30    33/31    35/32    35/35    36/38    36/43
-    //                                       uneven  32/36    34/35    34/42    34/36    35/42    44/43
+    // moe_wide_kernel from 24 pairs an expert on.  Up + down in us, moe_tile_kernel / moe_wide_kernel: 64 experts of 1,408 gated
+    // at width 4,096 at 9 pairs an expert 228 + 114 / 226 + 111, 19 236 + 129 / 234 + 124, 26 256 + 146 / 241 + 132, 32 273 +
+    // 157 / 258 + 139; of 2,112 without a gate 9 167 + 162 / 176 + 163, 19 182 + 181 / 195 + 182, 48 (tiles of 128 through
+    // registers) 246 + 240 / 229 + 226; 16 of 512 at 1,024, 37 15 + 10 / 15 + 10.  Steps of up to 64 tokens: gated 24 182 + 93 / 201
+    // + 94, 40 197 + 96 / 228 + 100; without a gate 24 145 + 132 / 130 + 136, 48 153 + 139 / 138 + 148, so that there the first
+    // product alone takes it, on the tiles of the other.
     // The scratch is sized for tiles of 64: it holds the pairs without gaps and, at its end, the experts' offsets.
-    const bool wide = pairs >= 48L * E;
-    const int tile_rows = wide ? 2 * MOE_TILE : MOE_TILE;
+    const bool wide = pairs >= 24L * E, wide_up = wide || (!gated && n <= MOE_TILE);
+    const int tile_rows = wide ? MOE_WIDE : MOE_TILE;
     const long tiles = (pairs + tile_rows - 1) / tile_rows + E;
     const long behind = (long)max_tiles * MOE_TILE - (E + 1);         // pairs <= behind: max_tiles covers 64 E rows more
     int* offs = rows + behind;
     CPMCU_REQUIRE(pairs <= behind && (long)max_tiles * MOE_TILE < (1L << 31), "moe_experts_mfma: scratch of %d tiles for %ld pairs", max_tiles, pairs);
     moe_group_kernel<<<1, 1024, 0, stream>>>(idx, (int)pairs, E, tile_rows, rows, offs, tile_expert, n_tiles);
     CPMCU_LAUNCH_CHECK("moe_group");
-#define TILES(KIND, in, ldi, w, out, K, N, act, limit)                                                                    \
-    do {                                                                                                                      \
+#define TILES(KIND, wide, in, ldi, w, out, K, N, act, limit)                                                              \
+    do {                                                                                                                  \
         const long blocks = (tiles * (((N) + (KIND == MOE_GATED ? 63 : 127)) / (KIND == MOE_GATED ? 64 : 128)) + 7) / 8 * 8;   \
-        CPMCU_REQUIRE(blocks < (1L << 31), "moe_experts_mfma: %ld workgroups exceed the launch grid", blocks);                 \
-        if (wide)                                                                                                             \
-            moe_tile_kernel<KIND, 8><<<(unsigned)blocks, 256, 0, stream>>>(in, ldi, (const bf16_t*)(w), rows, offs, tile_expert, \
-                                                                               n_tiles, (bf16_t*)(out), K, N, top, act, limit);         \
-        else                                                                                                                  \
-            moe_tile_kernel<KIND, 4><<<(unsigned)blocks, 256, 0, stream>>>(in, ldi, (const bf16_t*)(w), rows, offs, tile_expert, \
-                                                                               n_tiles, (bf16_t*)(out), K, N, top, act, limit);         \
+        CPMCU_REQUIRE(blocks < (1L << 31), "moe_experts_mfma: %ld workgroups exceed the launch grid", blocks);             \
+        auto* const kernel = wide ? moe_wide_kernel<KIND> : moe_tile_kernel<KIND>;                                         \
+        kernel<<<(unsigned)blocks, 256, 0, stream>>>(in, ldi, (const bf16_t*)(w), rows, offs, tile_expert, n_tiles,        \
+                                                     (bf16_t*)(out), K, N, top, tile_rows, act, limit);                    \
     } while (0)
-    if (gated) TILES(MOE_GATED, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
-    else TILES(MOE_PLAIN, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
+    if (gated) TILES(MOE_GATED, wide, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
+    else TILES(MOE_PLAIN, wide_up, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
     CPMCU_LAUNCH_CHECK("moe_up_tiles");
-    TILES(MOE_DOWN, (const bf16_t*)act, (long)F, wd, y, F, H, 0, 0.f);
+    TILES(MOE_DOWN, wide, (const bf16_t*)act, (long)F, wd, y, F, H, 0, 0.f);
     CPMCU_LAUNCH_CHECK("moe_down_tiles");
 #undef TILES
     const long total = (long)n * H;

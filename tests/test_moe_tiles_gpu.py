@@ -48,6 +48,83 @@ def test_tiles_of_every_fill(rows, H, F, gated):
     assert bool(((out.double() - w.double() * ref).abs() <= w.double() * off + 2 * sums * ref.abs() + 1e-30).all())
 
 
+@pytest.mark.parametrize("H,F", [(8, 64), (64, 104), (72, 200), (128, 128), (200, 264), (264, 72)])
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_tiles_of_128_rows(H, F, gated, offset):
+    """Steps of 24 pairs an expert or more: fills at the edges of every form (the last expert none), one, two, three and more
+    pieces of 64 columns, whole and ragged, features that end inside a tile; pair outputs off 16-byte borders, and a row that
+    is no number, which reaches no other."""
+    from cpmcu_amd import ops
+    rows = [1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 256, 257, 300, 513]
+    E, n = len(rows) + 1, sum(rows)
+    assert n >= 24 * E
+    g = torch.Generator(device=DEV).manual_seed(H + F)
+    idx = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(rows)])
+    idx = idx[torch.randperm(n, generator=torch.Generator().manual_seed(n))].to(DEV)[:, None].contiguous()
+    h = torch.randn(n, H, generator=g, device=DEV).to(torch.bfloat16)
+    h[7] = float("nan")
+    up = torch.randn(E, F * (2 if gated else 1), H, generator=g, device=DEV).to(torch.bfloat16)
+    down = torch.randn(E, H, F, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.rand(n, 1, generator=g, device=DEV)
+    tiles = ops.moe_tiles(n, 1, E)
+    i32 = lambda k: torch.empty(k, dtype=torch.int32, device=DEV)
+    act = torch.full((n, 1, F), 7.0, dtype=torch.bfloat16, device=DEV)
+    y = torch.full((n * H + offset + 1,), 7.0, dtype=torch.bfloat16, device=DEV)
+    out = torch.empty(n, H, device=DEV)
+    ops.moe_experts_mfma(h, up, down, idx, w, out, act, y[offset:offset + n * H].view(n, 1, H), i32(tiles * ops.MOE_TILE), i32(tiles),
+                         i32(1), gated=gated, activation="silu" if gated else "relu_squared")
+    assert bool((y[:offset] == 7).all()) and bool((y[offset + n * H:] == 7).all())
+    assert not gated or (bool(act[7].isnan().all()) and bool(out[7].isnan().all()))      # (max(z, 0) of no number is 0)
+    half, sums = 2.0 ** -8, 2.0 ** -23
+    for e in range(E):
+        mine = (idx[:, 0] == e).nonzero()[:, 0]
+        mine = mine[mine != 7]
+        x, u = h[mine].double(), up[e].double()
+        z, off = x @ u.T, H * sums * (x.abs() @ u.abs().T)           # float sums in any order
+        if gated:
+            a, b = z[:, :F], z[:, F:]
+            want = torch.nn.functional.silu(a) * b
+            off = 1.1 * off[:, :F] * b.abs() + (a.abs() + off[:, :F]) * off[:, F:]      # |silu'| <= 1.1
+        else:
+            want, off = torch.relu(z) ** 2, 2 * z.abs() * off + off ** 2
+        got = act[mine, 0].double()
+        assert bool(((got - want).abs() <= off + (half + 8 * sums) * want.abs() + 1e-30).all()), (e, rows[e] if e < len(rows) else 0)
+        ref, off = got @ down[e].double().T, F * sums * (got.abs() @ down[e].double().abs().T)
+        off = off + half * (ref.abs() + off)
+        v = w[mine].double()
+        assert bool(((out[mine].double() - v * ref).abs() <= v * off + 2 * sums * ref.abs() + 1e-30).all()), e
+
+
+@pytest.mark.parametrize("H,F", [(72, 136), (200, 56)])
+def test_experts_without_a_gate_of_few_tokens(H, F):
+    """Up to 64 tokens, whose first product runs on tiles of 64 rows of another kernel; an expert that is every choice of every
+    token has more rows than there are tokens."""
+    from cpmcu_amd import ops
+    E, n, top = 9, 40, 3
+    g = torch.Generator(device=DEV).manual_seed(H)
+    idx = torch.randint(0, E, (n, top), generator=torch.Generator().manual_seed(1), dtype=torch.int32)
+    idx[:31] = 4
+    idx = idx.to(DEV)
+    h = torch.randn(n, H, generator=g, device=DEV).to(torch.bfloat16)
+    up = torch.randn(E, F, H, generator=g, device=DEV).to(torch.bfloat16)
+    down = torch.randn(E, H, F, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.rand(n, top, generator=g, device=DEV)
+    tiles = ops.moe_tiles(n, top, E)
+    i32 = lambda k: torch.empty(k, dtype=torch.int32, device=DEV)
+    act, y = (torch.full((n, top, k), float("nan"), dtype=torch.bfloat16, device=DEV) for k in (F, H))
+    ops.moe_experts_mfma(h, up, down, idx, w, torch.empty(n, H, device=DEV), act, y, i32(tiles * ops.MOE_TILE), i32(tiles), i32(1),
+                         gated=False, activation="relu_squared")
+    e = idx.long()
+    z = torch.einsum("nh,nkfh->nkf", h.double(), up.double()[e])
+    off = H * 2.0 ** -23 * torch.einsum("nh,nkfh->nkf", h.double().abs(), up.double().abs()[e])
+    want, off = torch.relu(z) ** 2, 2 * z.abs() * off + off ** 2
+    assert bool(((act.double() - want).abs() <= off + (2.0 ** -8 + 2.0 ** -20) * want.abs() + 1e-30).all())
+    ref = torch.einsum("nkf,nkhf->nkh", act.double(), down.double()[e])
+    off = F * 2.0 ** -23 * torch.einsum("nkf,nkhf->nkh", act.double().abs(), down.double().abs()[e])
+    assert bool(((y.double() - ref).abs() <= off + 2.0 ** -8 * (ref.abs() + off) + 1e-30).all())
+
+
 @pytest.mark.parametrize("rows", [[80, 112], [81, 79, 97], [65, 113, 64]])
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("H,F", [(136, 72), (264, 200)])
