@@ -24,6 +24,8 @@ from typing import Dict, List, Optional, Sequence, Tuple
 
 import torch
 
+from ..ops import upload
+
 
 class CacheError(RuntimeError):
     pass
@@ -376,7 +378,7 @@ class SequenceCache:
         after a forward pass that advanced the state and then failed."""
         if not self.has_state:
             return None
-        idx = torch.tensor(list(slots), dtype=torch.long).to(self.device)
+        idx = upload(list(slots), torch.long, self.device)
         return idx, [[(t, t.index_select(0, idx)) for t in g.state[e].values()] for g in self.groups for e in g.entries]
 
     def restore_state(self, snapshot):
@@ -405,8 +407,9 @@ class SequenceCache:
                 g.table.copy_(g.table_host)
             else:
                 rows = sorted(g.dirty)
-                idx = torch.tensor(rows, dtype=torch.long)
-                g.table.index_copy_(0, idx.to(self.device), g.table_host[idx].to(self.device))
+                new = torch.empty((len(rows), g.table_host.shape[1]), dtype=g.table_host.dtype, pin_memory=True)
+                torch.index_select(g.table_host, 0, torch.tensor(rows, dtype=torch.long), out=new)
+                g.table.index_copy_(0, upload(rows, torch.long, self.device), new.to(self.device, non_blocking=True))
             g.dirty.clear()
 
     # ---- views ----

@@ -19,6 +19,7 @@ import torch
 
 from ..cache.paged import CacheError, SequenceCache
 from ..config.base import ModelConfig, architecture_name, read_config_json
+from ..ops import upload
 from ..parts.base import Runtime, StepContext, Workspace
 from ..registry import get_architecture
 from ..weights.loader import checkpoint_names, load_tensors
@@ -287,7 +288,11 @@ class Engine:
             if have + n > self.max_seq_len:
                 raise StepError(f"slot {e.slot}: {have} cached + {n} new tokens exceed the longest sequence "
                                 f"this engine holds ({self.max_seq_len})")
-            bad = [t for t in e.tokens if not 0 <= int(t) < V]
+            tok = np.asarray(e.tokens)
+            if tok.dtype.kind in "iu" and tok.ndim == 1 and 0 <= int(tok.min()) and int(tok.max()) < V:
+                bad = []
+            else:
+                bad = [t for t in e.tokens if not 0 <= int(t) < V]
             if bad:
                 raise StepError(f"slot {e.slot}: token id {bad[0]} is outside the vocabulary [0, {V})")
             for w in e.want:
@@ -407,7 +412,7 @@ class Engine:
         if not want_rows:
             return None
         if graph and want_rows != list(range(B)):
-            return logits.index_select(0, torch.tensor(want_rows, dtype=torch.long).to(self.device, non_blocking=True))
+            return logits.index_select(0, upload(want_rows, torch.long, self.device))
         return logits.clone()
 
     def _graph_key(self, B: int, max_pos: int) -> Tuple[int, int]:
@@ -517,7 +522,7 @@ class Engine:
             self._roll_back([entries[i].slot for i, _, _ in chunk], before, state)
             raise
         if rows:
-            dest_t = torch.tensor([dest, rows], dtype=torch.long).to(self.device, non_blocking=True)
+            dest_t = upload([dest, rows], torch.long, self.device)
             if graph:
                 result.index_copy_(0, dest_t[0], logits.index_select(0, dest_t[1]))
             else:

@@ -64,15 +64,20 @@ class Workspace:
     def __init__(self, device):
         self.device = torch.device(device)
         self._buf: Dict[str, torch.Tensor] = {}
+        self._last: Dict[str, tuple] = {}     # (shape, dtype, tensor) that a name was last asked for: layers ask alike
         self.generation = 0           # counts the times a buffer moved (captured graphs hold the old address)
         self.sealed = False           # set by the engine once it is built: what is asked for later is noted
         self.grown: List[str] = []    # names of buffers made or enlarged after that
 
     def get(self, name: str, shape: Sequence[int], dtype: torch.dtype) -> torch.Tensor:
+        shape = tuple(shape)
+        last = self._last.get(name)
+        if last is not None and last[0] == shape and last[1] == dtype:
+            return last[2]
         n = 1
         for s in shape:
             n *= int(s)
-        nbytes = n * torch.empty((), dtype=dtype).element_size()
+        nbytes = n * dtype.itemsize
         buf = self._buf.get(name)
         if buf is None or buf.numel() < nbytes:
             if buf is not None:
@@ -81,7 +86,9 @@ class Workspace:
             self._buf[name] = buf
             if self.sealed and name not in self.grown:
                 self.grown.append(name)
-        return buf[:nbytes].view(dtype).view(*shape)
+        t = buf[:nbytes].view(dtype).view(shape)
+        self._last[name] = (shape, dtype, t)
+        return t
 
     def bytes(self) -> int:
         return sum(b.numel() for b in self._buf.values())

@@ -245,3 +245,28 @@ def test_state_snapshot_and_restore():
     h[b] = 9.0
     c.restore_state(snap)
     assert float(h[b].min()) == float(h[b].max()) == -2.0 and float(h[a].min()) == 7.0
+
+
+def test_workspace_gives_the_same_memory_in_every_shape_asked_for():
+    """A name's buffer grows and keeps its place otherwise; what a name was last asked for is not handed out for another
+    shape or type, nor after the buffer has moved."""
+    from cpmcu_amd.parts.base import Workspace
+    ws = Workspace("cpu")
+    a = ws.get("a", (4, 6), torch.float32)
+    assert ws.get("a", (4, 6), torch.float32).data_ptr() == a.data_ptr() and ws.generation == 0
+    b = ws.get("a", [6, 4], torch.float32)
+    assert tuple(b.shape) == (6, 4) and b.data_ptr() == a.data_ptr()
+    c = ws.get("a", (6, 4), torch.bfloat16)
+    assert c.dtype == torch.bfloat16 and c.data_ptr() == a.data_ptr()
+    d = ws.get("a", (600, 4), torch.float32)
+    assert ws.generation == 1 and ws.bytes() == 600 * 4 * 4
+    e = ws.get("a", (4, 6), torch.float32)
+    assert e.data_ptr() == d.data_ptr() and tuple(e.shape) == (4, 6) and ws.generation == 1
+
+
+def test_uploaded_values():
+    from cpmcu_amd.ops import upload
+    assert upload([[3, 1], [2, 7]], torch.int32, "cpu").tolist() == [[3, 1], [2, 7]]
+    if torch.cuda.is_available():
+        t = upload([[3, 1], [2, 7]], torch.int32, "cuda:0")
+        assert t.is_cuda and t.dtype == torch.int32 and t.cpu().tolist() == [[3, 1], [2, 7]]
