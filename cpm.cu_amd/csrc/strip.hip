@@ -13,7 +13,7 @@
 // The weight is tiled as for the skinny product ([strip of 16 rows][128-column block][i][lane][8],
 // ops.TiledWeight).  The NW wavefronts of a workgroup take a contiguous share of the K blocks each (a straight
 // from global memory into the B operand, asked for together with the weight's block), add their results
-// through LDS, and the first wavefront finishes.
+// through LDS, and wavefront t finishes tile t of 16 tokens.
 //
 // (reference: the output projections src/model/minicpm4/minicpm4_attn.cuh:205, 319 and src/model/ffn.cuh:77-84
 // followed by add + norm src/model/norm.cuh:53-99)
@@ -28,7 +28,9 @@ __global__ __launch_bounds__(NW * 64) void proj_add_norm_kernel(
     const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict__ W, int M, int N, int K, float alpha,
     float* __restrict__ x, const float* __restrict__ w_norm, bf16_t* __restrict__ out, float* __restrict__ row_ss,
     int n_strips) {
-    __shared__ float red[NW - 1][MT][4][64];
+    static_assert(MT <= NW, "a wavefront finishes a tile");
+    constexpr int KEPT = MT == 1;                          // a first wavefront that finishes alone keeps its own sums
+    __shared__ float red[NW - KEPT][MT][4][64];
     const int strip = blockIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
@@ -89,22 +91,25 @@ __global__ __launch_bounds__(NW * 64) void proj_add_norm_kernel(
             if (kb + j + PF < kb1) load_block(kb + j + PF, wv[j], av[j]);
         }
     }
-    // lane (token r, g) of tile t: acc[t][i] is column 16 * strip + 4g + i; the other wavefronts hand theirs
-    // to the first, which adds them in the order of the wavefronts
-    if (wave > 0) {
+    // lane (token r, g) of tile t: acc[t][i] is column 16 * strip + 4g + i; wavefront t adds tile t's, in the order of the
+    // wavefronts (one wavefront that finished all four tiles of 64 tokens was the last third of the kernel's time)
+    if (wave >= KEPT) {
 #pragma unroll
         for (int t = 0; t < MT; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) red[wave - 1][t][i][lane] = acc[t][i];
+            for (int i = 0; i < 4; ++i) red[wave - KEPT][t][i][lane] = acc[t][i];
     }
     __syncthreads();
-    if (wave > 0) return;
+    if (wave >= MT) return;
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
+        if (MT > 1 && t != wave) continue;
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 4; ++i) {
+            if (!KEPT) acc[t][i] = red[0][t][i][lane];
 #pragma unroll
-            for (int w = 0; w < NW - 1; ++w) acc[t][i] += red[w][t][i][lane];
+            for (int w = 1; w < NW; ++w) acc[t][i] += red[w - KEPT][t][i][lane];
+        }
         const int tok = t * 16 + r;
         const bool ok = tok < M && col_ok;
         const long off = (long)min(tok, M - 1) * N + min(col, N - 4);
@@ -144,10 +149,11 @@ extern "C" const char* cpmcu_proj_add_norm(const void* A, long lda, const void* 
     //   1,024 x 4,096   5.73/6.72  5.98/6.50  5.74/6.35  5.75/6.60     4,096 x 11,008  18.0/19.8  18.0/18.6  17.7/18.7  18.1/19.4
     //   4,096 x 16,384  26.0/26.7 (2 x 8)  25.9/27.2  30.7/31.6
     // (more tokens hold more of a in registers for every block in flight: fewer blocks then)
+    // A wavefront a tile at the end, 1,024 x 1,024: 24, 32, 48, 64 tokens 4.99, 5.26, 6.63, 7.68 -> 4.49, 4.86, 5.94, 6.74.
     if (M <= 16 && K <= 1024) LAUNCH(2, 4, 1);
     else if (M <= 16 && K < 12288) LAUNCH(1, 8, 1);
     else if (M <= 16) LAUNCH(2, 8, 1);
-    else if (M <= 32 && K <= 1024) LAUNCH(1, 8, 2);       // 1,024 x 1,024 at 32 tokens 7.3 -> 5.4 us
+    else if (M <= 32 && K <= 1024) LAUNCH(1, 8, 2);       // 1,024 x 1,024 at 32 tokens 5.4 us, by 4 x 4 7.3
     else if (M <= 32) LAUNCH(4, 4, 2);
     else LAUNCH(2, 4, 4);
 #undef LAUNCH
@@ -170,7 +176,9 @@ __global__ __launch_bounds__(NW * 64) void gated_strip_kernel(
     const bf16_t* __restrict__ A, long lda, const bf16_t* __restrict__ W, int M, int I, int K,
     bf16_t* __restrict__ out, const float* __restrict__ row_ss, int ss_slices, float eps, int act,
     float act_limit) {
-    __shared__ float red[NW - 1][2][MT][4][64];
+    static_assert(MT <= NW, "a wavefront finishes a tile");
+    constexpr int KEPT = MT == 1;
+    __shared__ float red[NW - KEPT][2][MT][4][64];
     __shared__ float rs_s[MT * 16];
     const int strip = blockIdx.x;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -227,29 +235,30 @@ __global__ __launch_bounds__(NW * 64) void gated_strip_kernel(
             if (kb + j + PF < kb1) load_block(kb + j + PF, wv[j], av[j]);
         }
     }
-    if (wave > 0) {
+    if (wave >= KEPT) {
 #pragma unroll
         for (int s = 0; s < 2; ++s)
 #pragma unroll
             for (int t = 0; t < MT; ++t)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) red[wave - 1][s][t][i][lane] = acc[s][t][i];
+                for (int i = 0; i < 4; ++i) red[wave - KEPT][s][t][i][lane] = acc[s][t][i];
     }
     __syncthreads();
-    if (wave > 0) return;
+    if (wave >= MT) return;
     const int col = strip * 16 + 4 * g;
 #pragma unroll
     for (int t = 0; t < MT; ++t) {
+        if (MT > 1 && t != wave) continue;                            // wavefront t finishes tile t
         const int tok = t * 16 + r;
         const float rs = row_ss ? rs_s[tok] : 1.0f;
         uint32_t o[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            float gt = acc[0][t][i], up = acc[1][t][i];
+            float gt = KEPT ? acc[0][t][i] : red[0][0][t][i][lane], up = KEPT ? acc[1][t][i] : red[0][1][t][i][lane];
 #pragma unroll
-            for (int w = 0; w < NW - 1; ++w) {
-                gt += red[w][0][t][i][lane];
-                up += red[w][1][t][i][lane];
+            for (int w = 1; w < NW; ++w) {
+                gt += red[w - KEPT][0][t][i][lane];
+                up += red[w - KEPT][1][t][i][lane];
             }
             gt *= rs; up *= rs;
             gate_prepare(gt, up, act, act_limit);
@@ -279,8 +288,11 @@ extern "C" const char* cpmcu_gated_strip(const void* A, long lda, const void* W,
     //   4,096 x 1,024 7.51/7.91 -> 5.57/5.78 (a wavefront of 4 has 2 blocks there and asked for 4), 16,384 x 4,096 47.9/47.3 ->
     //   45.8/45.2 (5.9 TB/s); level between: 11,008 x 4,096 32.6/32.7 -> 31.8/32.7, 2,816 x 4,096 11.1/12.2 -> 11.3/12.4
     // More than 16 tokens, where every workgroup reads up to four times as much of a: it pays while K is short and a wavefront
-    // has all of its blocks in flight (4,096 x 1,024, skinny product -> here: 32 tokens 9.3 -> 7.9 us, 64 tokens 15.4 -> 11.6).
-    if (M > 32) LAUNCH(2, 4, 4);
+    // has all of its blocks in flight (4,096 x 1,024, skinny product -> here: 32 tokens 9.3 -> 7.1 us, 64 tokens 15.4 -> 9.2).
+    // A wavefront a tile at the end: 48 and 64 tokens 10.5, 11.4 -> 8.6, 9.6 (24 and 32 7.3, 7.7 -> 6.7, 7.1); of more than 32
+    // tokens 8 wavefronts of one block instead of 4 of two 8.2, 9.2 (2,816 x 1,024 at 40 and 64: 8.0, 9.1 -> 7.3, 8.5; at 24
+    // and 32 tokens they are 0.1 slower).
+    if (M > 32) LAUNCH(1, 8, 4);
     else if (M > 16) LAUNCH(2, 4, 2);
     else if (K <= 1024 || I >= 16384) LAUNCH(1, 8, 1);
     else LAUNCH(4, 4, 1);

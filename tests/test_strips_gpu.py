@@ -49,6 +49,12 @@ def test_residual_products_at_the_borders_of_the_wavefronts_shares(n, K):
     assert float((sums.double().sum(1) - (want ** 2).sum(1)).abs().max()) <= 1e-5 * float((want ** 2).sum(1).max())
 
 
+@pytest.mark.parametrize("n,K", [(17, 1024), (33, 8), (33, 1024), (48, 1000), (49, 136), (64, 1024)])
+def test_residual_products_that_every_wavefront_finishes(n, K):
+    """Up to four tiles of 16 tokens, one a wavefront at the end: the last one full, or one token of it."""
+    test_residual_products_at_the_borders_of_the_wavefronts_shares(n, K)
+
+
 @pytest.mark.parametrize("n,N,K", [(1, 16, 128), (8, 100, 1152), (16, 8192, 256), (9, 2000, 384), (3, 9000, 640), (8, 33000, 128), (16, 40, 4096), (2, 9000, 1024), (8, 33000, 1152)])
 @pytest.mark.parametrize("mode,dtype", [("plain", torch.float32), ("plain", torch.bfloat16), ("act", torch.bfloat16)])
 def test_products_of_one_wavefront_a_strip(n, N, K, mode, dtype):
