@@ -16,6 +16,7 @@
 // Keys and values lie in their pages as common.h says (key_index, value_index), each with its own head size.
 #include "cache_order.h"
 #include "common.h"
+#include "lds_direct.h"
 #include "vec4.h"
 
 enum { DST_ROWS = 0, DST_KEYS = 1, DST_VALUES = 2 };
@@ -643,6 +644,37 @@ struct WideLate {
     float scale_log2e, cap_in, cap_out;
 };
 
+// A column's output once more, over the keys that it sees, feature f of a lane: l its weights' sum without the sink.
+__device__ inline void wide_sum_again(const WideLate& a, long t1, int pos1, int kvh, int head1, float m1, float l1, int f, bool mine,
+                                      int nh, int hdv, const float* sink, const bf16_t* gate, long ld_gate, void* out, int out_f32, int lane) {
+    const int first1 = a.chunk > 0 ? pos1 - pos1 % a.chunk : (a.window > 0 ? max(pos1 - a.window + 1, 0) : 0);
+    if (sink) l1 += exp2f(sink[head1] * 1.4426950408889634f - m1);
+    mine = mine && f < hdv;
+    const bf16_t* q1 = a.q + (t1 * nh + head1) * a.hdk;
+    float o = 0.f;
+    for (int c = 0; c < a.total; ++c) {
+        const int key0 = (c < a.ckeep ? c : a.cfirst + (c - a.ckeep)) << 5;
+        const long row0 = paged_row(a.pv, a.slot, key0);
+        for (int i = 0; i < 32; ++i) {
+            const int key = key0 + i;
+            if (key > pos1 || (key < first1 && key >= a.keep_first)) continue;
+            const bf16_t* k1 = a.kpool + key_index(row0 + i, kvh, a.nkv, a.pool_hdk);
+            float s = 0.f;
+            for (int d = lane; d < a.hdk; d += 64) s += to_f32(q1[d]) * to_f32(k1[key_d_offset(d)]);
+            s = wave_sum(s);
+            if (a.cap_out > 0.f) s = a.cap_out * tanhf(s * a.cap_in);
+            const float p = to_f32(f32_to_bf16(__builtin_amdgcn_exp2f(__builtin_fmaf(s, a.scale_log2e, -m1))));
+            if (mine) o += p * to_f32(a.vtpool[value_index(row0 + i, kvh / a.v_share, a.nkv / a.v_share, a.pool_hdv) + value_d_offset(f)]);
+        }
+    }
+    if (!mine) return;
+    o /= l1;
+    if (gate) o /= 1.0f + expf(-to_f32(gate[t1 * ld_gate + (long)head1 * hdv + f]));
+    const long at = (t1 * nh + head1) * hdv + f;
+    if (out_f32) ((float*)out)[at] = o;
+    else ((bf16_t*)out)[at] = f32_to_bf16(o);
+}
+
 template <int PK, int DTW, bool EXACT>
 __global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
     const bf16_t* __restrict__ q, void* __restrict__ out, int out_f32, const bf16_t* __restrict__ kpool,
@@ -840,49 +872,221 @@ __global__ __launch_bounds__(512) void attention_wide_prefill_kernel(
     const WideLate a = late_s;
     for (; again; again &= again - 1) {
         const int col = (int)__builtin_ctzll(again);
-        const long t1 = t0 + col / G;
-        const int pos1 = pos_min + col / G, head1 = kvh * G + col % G;
-        const int first1 = a.chunk > 0 ? pos1 - pos1 % a.chunk : (a.window > 0 ? max(pos1 - a.window + 1, 0) : 0);
         const float m_of = col < 16 ? m[0] : (col < 32 ? m[1] : (col < 48 ? m[2] : m[3]));
-        const float m1 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(m_of), col & 15));
-        float l1 = sum_s[0][col] + sum_s[1][col];
-        if (sink) l1 += exp2f(sink[head1] * 1.4426950408889634f - m1);
-        const int f = wave * DTW * 16 + lane;                       // this lane's feature
-        const bool mine = lane < DTW * 16 && f < hdv;
-        const bf16_t* q1 = a.q + (t1 * nh + head1) * a.hdk;
-        float o = 0.f;
-        for (int c = 0; c < a.total; ++c) {
-            const int key0 = (c < a.ckeep ? c : a.cfirst + (c - a.ckeep)) << 5;
-            const long row0 = paged_row(a.pv, a.slot, key0);
-            for (int i = 0; i < 32; ++i) {
-                const int key = key0 + i;
-                if (key > pos1 || (key < first1 && key >= a.keep_first)) continue;
-                const bf16_t* k1 = a.kpool + key_index(row0 + i, kvh, a.nkv, a.pool_hdk);
-                float s = 0.f;
-                for (int d = lane; d < a.hdk; d += 64) s += to_f32(q1[d]) * to_f32(k1[key_d_offset(d)]);
-                s = wave_sum(s);
-                if (a.cap_out > 0.f) s = a.cap_out * tanhf(s * a.cap_in);
-                const float p = to_f32(f32_to_bf16(__builtin_amdgcn_exp2f(__builtin_fmaf(s, a.scale_log2e, -m1))));
-                if (mine) o += p * to_f32(a.vtpool[value_index(row0 + i, kvh / a.v_share, a.nkv / a.v_share, a.pool_hdv) + value_d_offset(f)]);
-            }
-        }
-        if (!mine) continue;
-        o /= l1;
-        if (gate) o /= 1.0f + expf(-to_f32(gate[t1 * ld_gate + (long)head1 * hdv + f]));
-        const long at = (t1 * nh + head1) * hdv + f;
-        if (out_f32) ((float*)out)[at] = o;
-        else ((bf16_t*)out)[at] = f32_to_bf16(o);
+        wide_sum_again(a, t0 + col / G, pos_min + col / G, kvh, kvh * G + col % G, __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(m_of), col & 15)),
+                       sum_s[0][col] + sum_s[1][col], wave * DTW * 16 + lane, lane < DTW * 16, nh, hdv, sink, gate, ld_gate, out, out_f32, lane);
     }
 }
 
-// tiles: runs of at most 64 * nkv / nh consecutive tokens of one sequence, int [n_tiles][2] (first packed token, tokens)
+// The same for steps of many tokens over a latent (64 PK key features as cached, up to 128 DTW value features): 128 columns a
+// workgroup, so that L2 hands every CU a key and a value once for twice as many.  A wavefront owns a tile of 16 columns for the scores
+// and DTW tiles of 16 value features of all 128 columns for the output; 32 keys a round.  They come straight to LDS, in two
+// buffers, the next round's while this round's are read.  A column's scores are all one wavefront's, so its maximum needs no
+// meeting; the one of a round hands over weights and the factors by which a moved maximum scales the columns' sums.
+// QL of Q's operands stand in LDS: with all in registers the output's 128 would not fit beside them (QL = 4 180 us at 2,048
+// tokens, 6 184, 2 217).  The order to keep: 8 LDS reads ahead of the scores' matrix instructions (left alone 187, 12 ahead
+// 220).
+// What bounds it: a workgroup alone on its CU takes 2.3 us a round whatever else runs, of which the LDS reads of the
+// keys by 8 wavefronts are 1.2 and the matrix instructions 0.9, one behind the other; the products with the values put between the
+// next round's scores took 196 us.  attention_wide_prefill_kernel, 64 columns -> this, 32 heads over 512 + 64, us: 2,048
+// tokens 231 -> 180, behind as many 566 -> 440, in a window of 2,048 405 -> 321, 1,500 152 -> 117.
+// Taken back there: keys straight to LDS in two buffers (235 -> 248).
+template <int PK, int DTW, int QL>
+__global__ __launch_bounds__(512) void attention_latent_prefill_kernel(
+    const bf16_t* __restrict__ q, void* __restrict__ out, int out_f32, const bf16_t* __restrict__ kpool,
+    const bf16_t* __restrict__ vtpool, PagedView pv, const int* __restrict__ positions, const int* __restrict__ tok_slot,
+    int nh, int nkv, int hdk, int hdv, int pool_hdv, float scale_log2e, int chunk, int window, int keep_first,
+    const float* __restrict__ sink, const int* __restrict__ tiles, int v_share, const bf16_t* __restrict__ gate, long ld_gate,
+    float cap_in, float cap_out) {
+    constexpr int KS = 2 * PK, QR = KS - QL, CHUNK = 256 * PK;       // 16-byte pieces of 32 keys
+    __shared__ gu32x4_t keys_s[2][CHUNK];
+    __shared__ gbf16x8_t p_s[2][8][64];                             // weights [round % 2][column tile][lane]
+    __shared__ gbf16x8_t q_s[QL][8][64];
+    __shared__ float corr_s[2][128], sum_s[128], m_s[128];
+    __shared__ WideLate late_s;
+    const int tile = gridDim.x - 1 - blockIdx.x;                   // later tiles of a prompt see more keys: they start first
+    const int kvh = blockIdx.y;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
+    const int G = nh / nkv, dtn = pool_hdv >> 4;
+    const int t0 = tiles[2 * tile], n_tok = tiles[2 * tile + 1], slot = tok_slot[t0];
+    const int pos_min = positions[t0], pos_max = pos_min + n_tok - 1;
+    auto token_of = [&](int c) { const int k = (c * 16 + n) / G; return k < n_tok ? k : 0; };    // of column tile c
+    auto head_of = [&](int c) { return kvh * G + (c * 16 + n) % G; };
+    const int pos = pos_min + token_of(wave);                      // a tile's tokens are consecutive
+    const int first_key = chunk > 0 ? pos - pos % chunk : (window > 0 ? max(pos - window + 1, 0) : 0);
+    const int first_min = chunk > 0 ? pos_min - pos_min % chunk : (window > 0 ? max(pos_min - window + 1, 0) : 0);
+    const int first_max = chunk > 0 ? pos_max - pos_max % chunk : (window > 0 ? max(pos_max - window + 1, 0) : 0);
+    const int cfirst = first_min >> 5, ckeep = min((keep_first + 31) >> 5, cfirst);
+    const int total = ckeep + (pos_max >> 5) + 1 - cfirst;
+    if (threadIdx.x == 0)
+        late_s = {q, kpool, vtpool, pv, hdk, 64 * PK, pool_hdv, nkv, v_share, chunk, window, keep_first, slot, ckeep, cfirst, total,
+                  scale_log2e, cap_in, cap_out};
+    auto key0_of = [&](int c) { return (c < ckeep ? c : cfirst + (c - ckeep)) << 5; };
+    auto place_of = [&](int c) { return (int)(paged_row(pv, slot, key0_of(min(c, total - 1))) >> 5); };
+    const long kchunk = 32L * 64 * PK, vchunk = 32L * pool_hdv;
+    const unsigned keys_b = lds_byte(keys_s);
+    auto bring_keys = [&](int place, int buf) {                     // 4 PK pieces of 1 KiB among 8 wavefronts
+        const gu32x4_t* from = (const gu32x4_t*)(kpool + ((long)place * nkv + kvh) * kchunk) + lane;
+#pragma unroll
+        for (int i = 0; i < (4 * PK + 7) / 8; ++i)
+            if (i * 8 + wave < 4 * PK) bring16(from + (i * 8 + wave) * 64, keys_b + (buf * CHUNK + (i * 8 + wave) * 64) * 16);
+    };
+    int place = place_of(0), next = place_of(1);
+    bring_keys(place, 0);
+    gbf16x8_t qf[QR];
+    {
+        const bf16_t* qr = q + ((long)(t0 + token_of(wave)) * nh + head_of(wave)) * hdk;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const int d = ks * 32 + g * 8;
+            gbf16x8_t v = *(const gbf16x8_t*)(qr + min(d, hdk - 8));
+            if (d >= hdk) v = gbf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+            if (ks < QR) qf[ks < QR ? ks : 0] = v;
+            else q_s[ks - QR][wave][lane] = v;
+        }
+    }
+    gfloatx4_t acc[DTW][8];
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int d = 0; d < DTW; ++d)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) acc[d][c] = gfloatx4_t{0.f, 0.f, 0.f, 0.f};
+    landed<0>();
+    for (int it = 0; it < total; ++it) {
+        if (it + 1 < total) bring_keys(next, (it + 1) & 1);          // (its buffer was read for the last time before the meeting)
+        gbf16x8_t vf[DTW];
+        {
+            const bf16_t* vp = vtpool + ((long)place * (nkv / v_share) + kvh / v_share) * vchunk + (g * 16 + n) * 8;
+#pragma unroll
+            for (int d = 0; d < DTW; ++d) vf[d] = *(const gbf16x8_t*)(vp + min(wave * DTW + d, dtn - 1) * 512);
+        }
+        place = next;
+        next = place_of(it + 2);
+        const gu32x4_t* const keys = keys_s[it & 1];
+        gfloatx4_t st[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            const gbf16x8_t qv = ks < QR ? qf[ks < QR ? ks : 0] : q_s[ks < QR ? 0 : ks - QR][wave][lane];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                const gbf16x8_t kf = *(const gbf16x8_t*)&keys[(u * 2 * PK + ks) * 64 + lane];
+                st[u] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qv, st[u], 0, 0, 0);
+            }
+        }
+        __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
+#pragma unroll
+        for (int i = 0; i < KS / 2; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
+        }
+        // lane (column n, g): st[u][e] is key key0 + 8 g + 4 u + e
+        if (cap_out > 0.f) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) st[u][e] = cap_out * tanhf(st[u][e] * cap_in);
+        }
+        const int key0 = key0_of(it);
+        if (key0 + 31 > pos_min || (key0 < first_max && key0 + 31 >= keep_first)) {
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int key = key0 + 8 * g + 4 * u + e;
+                    if (key > pos || (key < first_key && key >= keep_first)) st[u][e] = -INFINITY;
+                }
+        }
+        float mx = fmaxf(fmaxf(fmaxf(st[0][0], st[0][1]), fmaxf(st[0][2], st[0][3])),
+                         fmaxf(fmaxf(st[1][0], st[1][1]), fmaxf(st[1][2], st[1][3])));
+        mx = rows_max(mx);
+        const float to_m = fmaxf(m, mx * scale_log2e);
+        const bool up = to_m > m;
+        const float corr = up ? __builtin_amdgcn_exp2f(m - to_m) : 1.0f;              // (m = -inf: 0)
+        m = up ? to_m : m;
+        const float ref = m == -INFINITY ? 0.f : m;                                  // nothing seen yet: all weights 0
+        float rs = 0.f;
+        gbf16x8_t pb;
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float p = __builtin_amdgcn_exp2f(__builtin_fmaf(st[u][e], scale_log2e, -ref));
+                pb[u * 4 + e] = (__bf16)p;
+                rs += (float)pb[u * 4 + e];                                      // the weights as the products take them
+            }
+        l = l * corr + rows_sum(rs);
+        p_s[it & 1][wave][lane] = pb;
+        if (g == 0) corr_s[it & 1][wave * 16 + n] = corr;
+        landed<0>();                                                // the next keys, these values; weights and factors of all
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const float c = corr_s[it & 1][k * 16 + n];
+            const gbf16x8_t pf = p_s[it & 1][k][lane];
+            if (__builtin_amdgcn_ballot_w64(c != 1.0f)) {
+#pragma unroll
+                for (int d = 0; d < DTW; ++d) acc[d][k] *= c;
+            }
+#pragma unroll
+            for (int d = 0; d < DTW; ++d) acc[d][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d], pf, acc[d][k], 0, 0, 0);
+        }
+    }
+    if (g == 0) {
+        sum_s[wave * 16 + n] = l;
+        m_s[wave * 16 + n] = m;
+    }
+    __syncthreads();
+    // lane (column n of tile k, g): acc[d][k][i] is value feature (wave * DTW + d) * 16 + 4 g + i
+    unsigned long long again[2] = {0, 0};                          // bit c: column c (64 + c) is to be added up again
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+        const bool live = (k * 16 + n) / G < n_tok;
+        const long t = t0 + token_of(k);
+        const int head = head_of(k);
+        float total_l = sum_s[k * 16 + n];
+        if (sink) total_l += exp2f(sink[head] * 1.4426950408889634f - m_s[k * 16 + n]);
+        const float inv = 1.0f / total_l;
+        float odd = 0.f;
+#pragma unroll
+        for (int d = 0; d < DTW; ++d) odd += acc[d][k][0] * 0.f + acc[d][k][1] * 0.f + acc[d][k][2] * 0.f + acc[d][k][3] * 0.f;
+        unsigned long long bad = __builtin_amdgcn_ballot_w64(live && odd != 0.f && total_l * 0.f == 0.f);
+        bad |= bad >> 32;
+        again[k / 4] |= ((bad | bad >> 16) & 0xffff) << (16 * (k & 3));
+        if (!live) continue;
+#pragma unroll
+        for (int d = 0; d < DTW; ++d) {
+            const int f = (wave * DTW + d) * 16 + 4 * g;
+            if (f >= hdv) continue;
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                v[i] = acc[d][k][i] * inv;
+                if (gate) v[i] /= 1.0f + expf(-to_f32(gate[t * ld_gate + (long)head * hdv + f + i]));
+            }
+            const long at = (t * nh + head) * hdv + f;
+            if (out_f32) store4((float*)out + at, v[0], v[1], v[2], v[3]);
+            else store4((bf16_t*)out + at, v[0], v[1], v[2], v[3]);
+        }
+    }
+    if (!(again[0] | again[1])) return;
+    __builtin_amdgcn_s_waitcnt(0);                                 // what is stored below comes behind the stores above
+    const WideLate a = late_s;
+    for (int half = 0; half < 2; ++half)
+        for (unsigned long long left = again[half]; left; left &= left - 1) {
+            const int col = half * 64 + (int)__builtin_ctzll(left);
+            wide_sum_again(a, t0 + col / G, pos_min + col / G, kvh, kvh * G + col % G, m_s[col], sum_s[col], wave * DTW * 16 + lane,
+                           lane < DTW * 16, nh, hdv, sink, gate, ld_gate, out, out_f32, lane);
+        }
+}
+
+// tiles: runs of at most columns * nkv / nh (columns: 64 or 128) consecutive tokens of one sequence, int [n_tiles][2] (first packed token, tokens)
 extern "C" const char* cpmcu_attention_wide_prefill(const void* q, void* out, int out_f32, int nh, int nkv, int hdk, int hdv,
                                                     int pool_hdk, int pool_hdv, float scale, int chunk, int window,
                                                     int keep_first, const float* sink, const void* kpool, const void* vtpool,
                                                     const int* page_table, int table_width, int page_size,
                                                     const int* positions, const int* tok_slot, const int* tiles, int n_tiles,
                                                     int v_share, const void* gate, long ld_gate, float softcap,
-                                                    hipStream_t stream) {
+                                                    int columns, hipStream_t stream) {
     CPMCU_REQUIRE(nh > 0 && nkv > 0 && nh % nkv == 0 && 64 % (nh / nkv) == 0 && nkv <= 65535,
                   "attention_wide_prefill: %d heads in %d groups (1, 2, 4 ... 64 heads a group are taken)", nh, nkv);
     CPMCU_REQUIRE(hdk >= 8 && hdk % 8 == 0 && pool_hdk >= hdk && pool_hdk % 64 == 0 && pool_hdk <= 576,
@@ -895,10 +1099,19 @@ extern "C" const char* cpmcu_attention_wide_prefill(const void* q, void* out, in
     CPMCU_REQUIRE(!gate || ld_gate >= (long)nh * hdv, "attention_wide_prefill: gate rows of %ld elements for %d heads of %d", ld_gate, nh, hdv);
     CPMCU_REQUIRE((((uintptr_t)q | (uintptr_t)out | (uintptr_t)kpool | (uintptr_t)vtpool) & 15) == 0,
                   "attention_wide_prefill: operands must start on 16-byte borders");
+    CPMCU_REQUIRE(columns == 64 || (columns == 128 && pool_hdk == 576 && pool_hdv > 256 && 128 % (nh / nkv) == 0),
+                  "attention_wide_prefill: %d columns a workgroup (64, or 128 for keys of 576 and values beyond 256)", columns);
     PagedView pv{page_table, table_width, page_size};
     const float sl = softcap > 0.f ? 1.0f : scale * 1.4426950408889634f;
     const float cap_in = softcap > 0.f ? scale / softcap : 0.f, cap_out = softcap > 0.f ? softcap * 1.4426950408889634f : 0.f;
     const dim3 grid(n_tiles, nkv);
+    if (columns == 128) {
+        attention_latent_prefill_kernel<9, 4, 4><<<grid, 512, 0, stream>>>(
+            (const bf16_t*)q, out, out_f32, (const bf16_t*)kpool, (const bf16_t*)vtpool, pv, positions, tok_slot, nh, nkv, hdk, hdv,
+            pool_hdv, sl, chunk, window, keep_first, sink, tiles, v_share, (const bf16_t*)gate, ld_gate, cap_in, cap_out);
+        CPMCU_LAUNCH_CHECK("attention_latent_prefill");
+        return nullptr;
+    }
 #define LAUNCH(PKv, DTWv, EXACTv)                                                                                       \
     attention_wide_prefill_kernel<PKv, DTWv, EXACTv><<<grid, 512, 0, stream>>>(                                                 \
         (const bf16_t*)q, out, out_f32, (const bf16_t*)kpool, (const bf16_t*)vtpool, pv, positions, tok_slot, nh, nkv,  \

@@ -22,7 +22,7 @@
 //
 // A wavefront owns output rows and its lanes stride over the input features (16-byte loads when the rows are
 // aligned), so an expert's weights stream once for every token that chose it: the form for steps of few tokens.
-#include "common.h"
+#include "lds_direct.h"
 
 #include <type_traits>
 
@@ -944,25 +944,6 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
     else product(std::integral_constant<int, 1>());
 }
 
-// 64 lanes' 16 bytes straight from memory to LDS, one behind the other from byte `to` on.  Nothing waits for them but
-// landed(): the compiler does not count loads of an asm block (those of the builtin it does, and before every LDS read).
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"                      // m0 on the clobber list
-__device__ inline void bring16(const void* from, unsigned to) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(to), "v"(from) : "memory", "m0");
-}
-__device__ inline void stream16(const void* from, unsigned to) {      // the same past the caches
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(to), "v"(from) : "memory", "m0");
-}
-#pragma clang diagnostic pop
-// all but this wavefront's last N loads have landed and what it read from LDS has arrived; then the workgroup meets
-template <int N>
-__device__ inline void landed() {
-    __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"i"(N) : "memory");
-    __builtin_amdgcn_sched_barrier(0);
-}
-
 // The same products for steps that give an expert many rows: tiles of up to 128 rows against 128 weight rows (GATED: 64
 // features), workgroups of 4 wavefronts, two a CU, a wavefront half of the rows and 64 weight rows.  Pieces of 64 columns go
 // from memory to LDS without passing registers, the weights in three buffers and the rows in two (80 KB), with the swizzle of
@@ -1003,7 +984,7 @@ __global__ __launch_bounds__(256, 2) void moe_wide_kernel(const bf16_t* __restri
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int chunk = ((lane & 7) ^ (lane >> 3)) * 8;                 // a lane brings place lane % 8 of row lane / 8 of 8 rows
-    const unsigned base = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+    const unsigned base = lds_byte(lds);
     const int half = wave & 1, side = wave >> 1;
     const bool whole = (uintptr_t)out % 16 == 0;
     const bf16_t* wp[4];

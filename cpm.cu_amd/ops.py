@@ -2311,13 +2311,26 @@ def attention_wide_prefill_pays(n_tokens: int, nh: int, nkv: int, max_keys: int)
     return group < 2 or n_tokens > 256 or n_tokens * nkv * -(-group // 16) > 512 or max_keys > 160
 
 
+def attention_wide_columns(q_lens: Sequence[int], nh: int, nkv: int, pool_hdk: int, pool_hdv: int) -> int:
+    """Columns (heads of consecutive tokens) a workgroup of attention_wide_prefill takes.  128 halve what L2 hands out, for keys
+    cached as 576 features and values of more than 256, but make half as many workgroups, one a CU: from one and a quarter for
+    every CU on.  Measured, 32 heads over a latent of 512 + 64, 64 / 128 columns, us (workgroups of 128): 1,000 tokens 77/91 (250),
+    prompts of 77, 300 and 613 61/67 (249), 16 heads 2,048 133/172 (256), 20 x 64 53/50 (320), 1,500 152/117 (375), 8 x 200 70/62
+    (400), 4 x 479 98/89 (480), 2,048 231/180 (512)."""
+    if pool_hdk != 576 or pool_hdv <= 256 or 128 % (nh // nkv):
+        return ATTENTION_WIDE_COLUMNS
+    per = 128 * nkv // nh
+    return 128 if 4 * nkv * sum(-(-n // per) for n in q_lens) >= 5 * compute_units() else ATTENTION_WIDE_COLUMNS
+
+
 def attention_wide_prefill(q: torch.Tensor, out: torch.Tensor, tiles: torch.Tensor, nh: int, nkv: int, hdk: int, hdv: int,
                            scale: float, kpool: torch.Tensor, vpool: torch.Tensor, page_table: torch.Tensor, page_size: int,
                            positions: torch.Tensor, tok_slot: torch.Tensor, chunk: int = 0, window: int = 0,
                            keep_first: int = 0, sink: Optional[torch.Tensor] = None, v_share: int = 1,
-                           gate: Optional[torch.Tensor] = None, softcap: float = 0.0):
+                           gate: Optional[torch.Tensor] = None, softcap: float = 0.0, columns: int = 64):
     """attention_general_mfma for prompts with wide values (attention_wide_prefill_ok): tiles int32 [T, 2] = (first packed
-    token, tokens), each a run of at most 64 * nkv / nh consecutive tokens of one sequence."""
+    token, tokens), each a run of at most ``columns`` * nkv / nh consecutive tokens of one sequence (columns: 64, or 128 where
+    attention_wide_columns says so)."""
     _need(q, "attention q", torch.bfloat16, (None, nh * hdk))
     n = q.shape[0]
     if out.dtype not in (torch.bfloat16, torch.float32):
@@ -2344,7 +2357,7 @@ def attention_wide_prefill(q: torch.Tensor, out: torch.Tensor, tiles: torch.Tens
         c_int(kpool.shape[2] // nkv), c_int(vpool.shape[2] // nvh), c_float(scale), c_int(chunk), c_int(window),
         c_int(keep_first), _p(sink), _p(kpool), _p(vpool), _p(page_table), c_int(page_table.shape[1]), c_int(page_size),
         _p(positions), _p(tok_slot), _p(tiles), c_int(tiles.shape[0]), c_int(v_share), _p(gate), c_long(ld_gate),
-        c_float(softcap or 0.0), _stream()))
+        c_float(softcap or 0.0), c_int(columns), _stream()))
 
 
 def attention_general_tokens_per_tile(n_tokens: int, nh: int, nkv: int, pool_hdv: int) -> int:
@@ -2427,13 +2440,14 @@ def attention_any(q, out, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, pa
     if (not ctx.single_token and attention_wide_prefill_ok(q, nh, nkv, hdk, hdv, kpool.shape[2] // nkv, pool_hdv, page_size)
             and (q.data_ptr() | out.data_ptr() | kpool.data_ptr() | vpool.data_ptr()) % 16 == 0
             and attention_wide_prefill_pays(q.shape[0], nh, nkv, min(ctx.max_pos + 1, chunk or window + keep_first or 1 << 30))):
-        per = ATTENTION_WIDE_COLUMNS * nkv // nh
+        columns = attention_wide_columns(ctx.q_lens, nh, nkv, kpool.shape[2] // nkv, pool_hdv)
+        per = columns * nkv // nh
         key = ("prefill_tiles", per)
         tiles = ctx.extras.get(key)
         if tiles is None:
             tiles = ctx.extras[key] = prefill_tiles(ctx.q_lens, per, q.device)
         attention_wide_prefill(q, out, tiles, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, page_size, ctx.positions,
-                               ctx.tok_slot, chunk, window, keep_first, sink, v_share, gate, softcap)
+                               ctx.tok_slot, chunk, window, keep_first, sink, v_share, gate, softcap, columns)
         return gate is not None
     if attention_general_mfma_ok(q, hdk, hdv, page_size):
         n = q.shape[0]

@@ -205,6 +205,50 @@ def test_infinities_reach_only_tokens_that_see_them(nh, nkv, hdk, hdv, opt):
         assert bool(((got[t] - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 1e-5)[fine].all()), t
 
 
+@pytest.fixture
+def columns_128(monkeypatch):
+    """Workgroups of 128 columns, tiles of twice the tokens."""
+    from cpmcu_amd import ops
+    wide, tiles = ops.attention_wide_prefill, ops.prefill_tiles
+    monkeypatch.setattr(ops, "attention_wide_prefill", lambda *a, **k: wide(*a, **k, columns=128))
+    monkeypatch.setattr(ops, "prefill_tiles", lambda lens, per, device: tiles(lens, 2 * per, device))
+
+
+@pytest.mark.parametrize("nh,nkv,hdk,hdv,v_share,opt", [
+    (32, 1, 576, 512, 1, {}), (32, 1, 576, 512, 1, {"window": 37, "sink": True, "gate": True}), (8, 2, 576, 260, 2, {"chunk": 48}),
+    (64, 1, 520, 512, 1, {"softcap": 3.0, "out": torch.float32}), (6, 3, 568, 272, 3, {"window": 20, "keep_first": 5, "page": 32}),
+    (2, 2, 576, 384, 1, {"page": 96, "sink": True})])
+def test_wide_prompt_attention_of_128_columns(nh, nkv, hdk, hdv, v_share, opt, columns_128):
+    """1 to 64 tokens a workgroup, tiles that end early, keys and values beside the cached sizes, every mask."""
+    test_wide_prompt_attention(nh, nkv, hdk, 576, hdv, v_share, opt)
+
+
+@pytest.mark.parametrize("spread", [1.0, 3.0])
+def test_weights_of_128_columns_round_no_worse(spread, columns_128):
+    test_weights_round_no_worse_than_token_by_token(spread)
+
+
+@pytest.mark.parametrize("nh,nkv,hdk,hdv,opt", [(32, 1, 576, 512, {}), (8, 2, 520, 272, {"window": 40, "keep_first": 3, "gate": True}),
+                                                (4, 4, 576, 260, {"sink": True, "softcap": 4.0}), (2, 1, 576, 512, {"chunk": 48, "out": torch.bfloat16})])
+def test_infinities_in_128_columns(nh, nkv, hdk, hdv, opt, columns_128):
+    test_infinities_reach_only_tokens_that_see_them(nh, nkv, hdk, hdv, opt)
+
+
+def test_the_rule_of_128_columns():
+    from cpmcu_amd import ops
+    cus = ops.compute_units()
+    most = -(-5 * cus // 4)                                                  # workgroups of 4 tokens of 32 heads
+    assert ops.attention_wide_columns([4 * most], 32, 1, 576, 512) == 128 and ops.attention_wide_columns([4 * most - 4], 32, 1, 576, 512) == 64
+    assert ops.attention_wide_columns([1] * most, 32, 1, 576, 512) == 128
+    for other in ((32, 1, 512, 512), (32, 1, 576, 256), (6, 2, 576, 512)):
+        assert ops.attention_wide_columns([4 * most * 4], *other) == 64
+    with pytest.raises(ops.KernelError, match="128 columns|columns a workgroup"):
+        x = lambda *shape: torch.zeros(*shape, dtype=torch.bfloat16, device=DEV)
+        i = lambda *shape: torch.zeros(*shape, dtype=torch.int32, device=DEV)
+        ops.attention_wide_prefill(x(1, 128), x(1, 256), torch.tensor([[0, 1]], dtype=torch.int32, device=DEV), 1, 1, 128, 256, 1.0, x(1, 64, 128), x(1, 64, 256),
+                                   i(1, 1), 64, i(1), i(1), columns=128)
+
+
 def test_outputs_off_16_byte_borders_take_the_general_kernel():
     from types import SimpleNamespace
     from cpmcu_amd import ops
