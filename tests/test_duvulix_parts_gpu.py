@@ -376,3 +376,34 @@ def test_products_head_by_head_on_the_matrix_cores(shape):
             close(out[:, h * (N + 3):h * (N + 3) + N], want, "bfloat16")
             assert float(out[:, h * (N + 3) + N:(h + 1) * (N + 3)].abs().max()) == 0.0
         assert float((out.float() - twin.float()).abs().max()) <= 0.02 * float(twin.float().abs().max())
+
+
+@pytest.mark.parametrize("n,groups,W", [(3, 5, 4), (1, 2, 128), (5, 3, 252), (2, 3, 256), (3, 1, 260), (7, 3, 512), (2, 5, 516), (3, 2, 1024), (2, 3, 1028),
+                                        (3, 1, 4096), (2, 2, 4100), (3, 3, 130)])
+@pytest.mark.parametrize("gate", ["none", "before", "sigmoid", "silu"])
+@pytest.mark.parametrize("types", [("float32", "float32", "float32"), ("float32", "bfloat16", "bfloat16"), ("bfloat16", "bfloat16", "float32")])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_group_norms_of_every_width(n, groups, W, gate, types, shift):
+    """Groups at the borders of the wavefronts' and workgroups' forms, with every gate and a divisor; rows that start off the
+    16-byte borders which those ask for go through the general kernel."""
+    from cpmcu_amd import ops
+    xt, zt, ot = (getattr(torch, t) for t in types)
+    g = torch.Generator().manual_seed(W + n)
+    width = groups * W
+    wide = lambda t: torch.randn(n, width + 8, generator=g).to(t).to(DEV)[:, shift:shift + width]
+    x, z = wide(xt), None if gate == "none" else wide(zt)
+    w, den = torch.randn(width, generator=g).to(DEV), (0.5 + torch.rand(n, groups, generator=g)).to(DEV)
+    for divisor, weight in ((None, w), (den, w), (None, None)):
+        out = torch.full((n, width + 8), 7.0, dtype=ot, device=DEV)
+        ops.rms_norm_groups(x, weight, 1e-3, out[:, shift:shift + width], groups=groups, gate=z,
+                            gate_after={"none": False, "before": False, "sigmoid": True, "silu": "silu"}[gate], divisor=divisor)
+        assert bool((out[:, :shift] == 7).all()) and bool((out[:, shift + width:] == 7).all())
+        v = x.double().view(n, groups, W) if divisor is None else x.double().view(n, groups, W) / den.double()[..., None]
+        zd = None if z is None else z.double().reshape(n, groups, W)
+        v = v * torch.nn.functional.silu(zd) if gate == "before" else v
+        v = v / torch.sqrt((v * v).mean(-1, keepdim=True) + 1e-3)
+        v = v if weight is None else v * w.double().view(groups, W)
+        v = v * torch.sigmoid(zd) if gate == "sigmoid" else v * torch.nn.functional.silu(zd) if gate == "silu" else v
+        # a float's operations one by one (exponentials among them), the result's own rounding
+        off = ((2.0 ** -8 if ot == torch.bfloat16 else 0.0) + 2.0 ** -18) * v.abs() + 1e-30
+        assert bool(((out[:, shift:shift + width].double().view(n, groups, W) - v).abs() <= off).all())
