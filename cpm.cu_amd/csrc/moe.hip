@@ -555,131 +555,6 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const T* __restrict__ act
     }
 }
 
-// y[pair][c] = Wd_e[c] . act[pair] in float, every expert's rows read once for all of its pairs (of a run of MOE_RUN, four at a
-// time), as moe_gated_kernel reads them: grid (ceil(H / 32), pairs), a wavefront 8 columns.  moe_combine_token_kernel
-// adds a token's up.  moe_down_kernel reads a row once for every pair, and the second time finds it in no cache.
-template <int NT>
-__device__ inline void down_rows(const bf16_t* __restrict__ act, const bf16_t* __restrict__ wd, const long (&pair)[4],
-                                 float* __restrict__ y, int H, int F, int c0, int lane) {
-    const bf16_t *wr[8], *ar[NT];
-#pragma unroll
-    for (int r = 0; r < 8; ++r) wr[r] = wd + (long)min(c0 + r, H - 1) * F;
-#pragma unroll
-    for (int i = 0; i < NT; ++i) ar[i] = act + pair[i] * F;
-    float s[NT][8];
-#pragma unroll
-    for (int i = 0; i < NT; ++i)
-#pragma unroll
-        for (int r = 0; r < 8; ++r) s[i][r] = 0.f;
-    for (int c = lane * 8; c < F; c += 64 * 8) {
-        float w[8][8];
-#pragma unroll
-        for (int r = 0; r < 8; ++r) stream8(wr[r] + c, w[r]);
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-            float x[8];
-            load8<bf16_t>(ar[i] + c, x);
-#pragma unroll
-            for (int r = 0; r < 8; ++r)
-#pragma unroll
-                for (int k = 0; k < 8; ++k) s[i][r] += w[r][k] * x[k];
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < NT; ++i) {
-        float v = 0.f;
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            const float t = wave_sum(s[i][r]);
-            if (lane == r) v = t;
-        }
-        if (lane < 8 && c0 + lane < H) y[pair[i] * H + c0 + lane] = v;
-    }
-}
-
-__global__ __launch_bounds__(256) void moe_down_rows_kernel(const bf16_t* __restrict__ act, const bf16_t* __restrict__ wd,
-                                                            const int* __restrict__ idx, float* __restrict__ y, int H, int F, int E,
-                                                            int n_pairs) {
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int run0 = blockIdx.y / MOE_RUN * MOE_RUN, own = blockIdx.y - run0;
-    const int a = run0 + lane < n_pairs ? idx[run0 + lane] : -1, b = run0 + 64 + lane < n_pairs ? idx[run0 + 64 + lane] : -1;
-    const int e = own < 64 ? __builtin_amdgcn_readlane(a, own & 63) : __builtin_amdgcn_readlane(b, own & 63);
-    if (e >= E) return;                 // an identity expert
-    unsigned long long first = __builtin_amdgcn_ballot_w64(a == e), second = __builtin_amdgcn_ballot_w64(b == e);
-    if ((first ? __builtin_ctzll(first) : 64 + __builtin_ctzll(second)) != own) return;
-    const int c0 = (blockIdx.x * 4 + wave) * 8;
-    if (c0 >= H) return;
-    const bf16_t* we = wd + (long)e * H * F;
-    auto next = [&]() {
-        unsigned long long& from = first ? first : second;
-        const int at = __builtin_ctzll(from) + (first ? 0 : 64);
-        from &= from - 1;
-        return (long)(run0 + at);
-    };
-    while (first | second) {
-        long pair[4];
-        int count = 0;
-        pair[0] = pair[1] = pair[2] = pair[3] = next();
-        for (count = 1; count < 4 && (first | second); ++count) {
-            const long p = next();
-            if (count == 1) pair[1] = pair[2] = pair[3] = p;
-            else if (count == 2) pair[2] = pair[3] = p;
-            else pair[3] = p;
-        }
-        if (count == 1) down_rows<1>(act, we, pair, y, H, F, c0, lane);
-        else if (count == 2) down_rows<2>(act, we, pair, y, H, F, c0, lane);
-        else down_rows<4>(act, we, pair, y, H, F, c0, lane);
-    }
-}
-
-// out[t] = sum_k w[t, k] y[t, k] and what else moe_down_kernel's end adds, from moe_down_rows_kernel's rows: grid (tokens, ceil(H /
-// 64)), 16 lanes four columns, each an expert and a part of every other sum, so that all come back in one trip to memory.
-template <typename ST>
-__global__ __launch_bounds__(256) void moe_sum_pairs_kernel(const float* __restrict__ y, const int* __restrict__ idx,
-                                                            const float* __restrict__ w, const ST* __restrict__ shared,
-                                                            int shared_parts, long shared_stride, const float* __restrict__ sg,
-                                                            const bf16_t* __restrict__ h, long ldh, int E, float* __restrict__ out,
-                                                            int H, int top, Join join) {
-    const long t = blockIdx.x;
-    const int p0 = threadIdx.x & 15, c = (blockIdx.y * 16 + (threadIdx.x >> 4)) * 4;
-    if (c >= H) return;                                              // (all 16 lanes of the columns)
-    const long at = t * H + c;
-    float v[4] = {0.f, 0.f, 0.f, 0.f};
-    if (p0 < top) {
-        const int e = idx[t * top + p0];
-        const float wk = w[t * top + p0];
-        if (e < E) {
-            const float4 u = *(const float4*)(y + (t * top + p0) * H + c);
-            v[0] = wk * u.x; v[1] = wk * u.y; v[2] = wk * u.z; v[3] = wk * u.w;
-        } else if (h) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = wk * to_f32(h[t * ldh + c + i]);
-        }
-    }
-    if (shared) {
-        const float g = sg ? sg[t] : 1.0f;
-        for (int p = p0; p < shared_parts; p += 16)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] += g * to_f32(shared[(long)p * shared_stride + at + i]);
-    }
-    if (join.x) {
-        for (int p = p0; p < join.a_parts; p += 16)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] += join_part(join, p, at + i);
-        if (p0 == 15)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] += join.x[at + i] + (join.a_bias ? join.a_bias[c + i] : 0.f);
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v[i] = row16_sum(v[i]);
-    if (p0) return;
-    *(float4*)((join.x ? join.x : out) + at) = make_float4(v[0], v[1], v[2], v[3]);
-    if (join.copy) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) ((bf16_t*)join.copy)[at + i] = f32_to_bf16(v[i]);
-    }
-}
-
 static const char* join_check(const Join& j, const float* out) {
     CPMCU_REQUIRE(j.x || out, "experts: nowhere to write");
     CPMCU_REQUIRE(!j.x || (j.a_parts >= 0 && j.a_parts <= 32 && (j.a != nullptr) == (j.a_parts > 0)),
@@ -691,30 +566,10 @@ extern "C" const char* cpmcu_moe_down(const void* act, int dtype, const void* wd
                                       const void* shared, int shared_dtype, int shared_parts, long shared_stride,
                                       const float* sg, const void* h, long ldh, int E, float* out, int n, int H, int F,
                                       int top, float* x, const void* a, int a_dtype, int a_parts, long a_stride,
-                                      const float* a_bias, void* copy, float* y, hipStream_t stream) {
+                                      const float* a_bias, void* copy, hipStream_t stream) {
     const Join join{x, a, a_dtype == CPMCU_BF16, a ? a_parts : 0, a_stride, a_bias, copy};
     if (const char* m = join_check(join, out)) return m;
     CPMCU_REQUIRE(n > 0 && H > 0 && F > 0 && top > 0 && E > 0, "moe_down: empty shape");
-    // An expert's rows once for all of its pairs, where they are too many for a cache to keep them until the next token asks
-    // (8 MiB an expert) and 18 pairs or more make up for a second kernel (n * top pairs of 64 experts, a router's uneven choice; us,
-    // row by row / here): 1,408 x 4,096 12 23.0/23.5, 18 32.2/30.9, 24 41.6/35.8, 48 64/49, 90 101/74 (even choice 48 77/60,
-    // 90 126/92); 2,112 x 4,096 12 36/34, 48 104/72; 1,024 x 2,048 (4 MiB, 32 experts) 32 17.6/18.8, 64 26.2/27.6; 512 x 1,024
-    // 16 4.5/10.4.
-    if (y && dtype == CPMCU_BF16 && (long)n * top >= 18 && (long)H * F >= 4L << 20 && top <= 16 && F % 8 == 0 && H % 4 == 0 && (long)n * top <= 65535 && H <= 64 * 65535 &&
-        (((uintptr_t)act | (uintptr_t)wd | (uintptr_t)y | (uintptr_t)(x ? x : out)) & 15) == 0 &&
-        (!shared || shared_dtype == CPMCU_F32 || shared_dtype == CPMCU_BF16)) {
-        moe_down_rows_kernel<<<dim3((H + 31) / 32, n * top), 256, 0, stream>>>((const bf16_t*)act, (const bf16_t*)wd, idx, y, H, F, E, n * top);
-        CPMCU_LAUNCH_CHECK("moe_down_rows");
-        const dim3 cells(n, (H + 63) / 64);
-        if (shared && shared_dtype == CPMCU_BF16)
-            moe_sum_pairs_kernel<bf16_t><<<cells, 256, 0, stream>>>(y, idx, w, (const bf16_t*)shared, shared_parts, shared_stride, sg,
-                                                                    (const bf16_t*)h, ldh, E, out, H, top, join);
-        else
-            moe_sum_pairs_kernel<float><<<cells, 256, 0, stream>>>(y, idx, w, (const float*)shared, shared_parts, shared_stride, sg,
-                                                                   (const bf16_t*)h, ldh, E, out, H, top, join);
-        CPMCU_LAUNCH_CHECK("moe_sum_pairs");
-        return nullptr;
-    }
     const int hy = (H + 4 * MOE_ROWS - 1) / (4 * MOE_ROWS);
     CPMCU_REQUIRE(hy <= 65535, "moe_down: a width of %d exceeds the launch grid", H);
     dim3 grid(n, hy);

@@ -1644,13 +1644,11 @@ def _join_args(join: Optional[Join], n: int, H: int, dtype: torch.dtype):
 
 def moe_down(act: torch.Tensor, down: torch.Tensor, idx: torch.Tensor, weights: torch.Tensor, out: Optional[torch.Tensor],
              shared: Optional[torch.Tensor] = None, shared_gate: Optional[torch.Tensor] = None,
-             h: Optional[torch.Tensor] = None, join: Optional[Join] = None, pair_out: Optional[torch.Tensor] = None):
+             h: Optional[torch.Tensor] = None, join: Optional[Join] = None):
     """out[t] = sum_k weights[t, k] * Wd_e act[t, k] (+ shared_gate[t] * shared[t]); down [E, H, F]; out float32
     [n, H]; shared [n, H] or float partial sums [P, n, H].  h [n, H]: the experts' input, which is the output of an
     identity expert (idx[t, k] >= E; without h such pairs add nothing).  With ``join`` the result goes into the
-    residual instead of ``out`` (which may be None).  With ``pair_out`` (float32 scratch [n, top, H]) steps of many pairs of
-    large experts (the line stands in csrc/moe.hip) read an expert's rows once for all tokens that chose it and add a token's up
-    afterwards; sums in another order."""
+    residual instead of ``out`` (which may be None)."""
     _need(act, "experts act", shape=(None, None, None))
     n, top, F = act.shape
     _need(down, "experts down", act.dtype, (None, None, F))
@@ -1665,12 +1663,10 @@ def moe_down(act: torch.Tensor, down: torch.Tensor, idx: torch.Tensor, weights: 
     sp, sstr = _parts_of(shared, n, H, "shared expert") if shared is not None else (0, 0)
     if shared_gate is not None:
         _need(shared_gate, "shared gate", torch.float32, (n,))
-    if pair_out is not None:
-        _need(pair_out, "pair outputs", torch.float32, (n, top, H))
     _check(_fn("moe", "cpmcu_moe_down")(_p(act), c_int(_code(act)), _p(down), _p(idx), _p(weights), _p(shared),
                                         c_int(_code(shared) if shared is not None else 0), c_int(sp), c_long(sstr),
                                         _p(shared_gate), _p(h), c_long(ldh), c_int(E), _p(out), c_int(n), c_int(H),
-                                        c_int(F), c_int(top), *_join_args(join, n, H, act.dtype), _p(pair_out), _stream()))
+                                       c_int(F), c_int(top), *_join_args(join, n, H, act.dtype), _stream()))
 
 
 MOE_TILE = 64

@@ -213,12 +213,6 @@ class RoutedExpertsFFN(FeedForward):
 
     can_join = True
 
-    def reserve_workspace(self, ws, rt: Runtime, max_step_tokens: int, max_slots: int):
-        # the largest step that is not grouped lies between the sizes that the engine rehearses
-        few = min(max_step_tokens, ops.SKINNY_MAX_ROWS, -(-3 * self.experts // (2 * self.top)) - 1)
-        if rt.dtype == torch.bfloat16 and few > 0:
-            ws.get("moe.pair_sums", (few, self.top, self.hidden_size), torch.float32)
-
     def joins(self, other) -> bool:
         return other is None or other.dim() == 2 or other.shape[0] <= ops.JOIN_MAX_PARTS
 
@@ -258,6 +252,5 @@ class RoutedExpertsFFN(FeedForward):
                     ops.moe_gated(h, self.gate_up, idx, act, activation=self.activation)
                 else:
                     ops.moe_up(h, self.gate_up, idx, act, self.activation)
-                sums = ctx.ws.get("moe.pair_sums", (n, self.top, self.hidden_size), torch.float32) if self.rt.dtype == torch.bfloat16 else None
-                ops.moe_down(act, self.down, idx, wts, out, shared, sg, h=h, join=join, pair_out=sums)
+                ops.moe_down(act, self.down, idx, wts, out, shared, sg, h=h, join=join)
         return out
