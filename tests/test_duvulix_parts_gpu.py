@@ -407,3 +407,24 @@ def test_group_norms_of_every_width(n, groups, W, gate, types, shift):
         # a float's operations one by one (exponentials among them), the result's own rounding
         off = ((2.0 ** -8 if ot == torch.bfloat16 else 0.0) + 2.0 ** -18) * v.abs() + 1e-30
         assert bool(((out[:, shift:shift + width].double().view(n, groups, W) - v).abs() <= off).all())
+
+
+@pytest.mark.parametrize("n,H", [(256, 4), (257, 1028), (256, 2048), (300, 2052), (256, 4096), (259, 4100), (256, 8192), (256, 8196), (300, 130)])
+@pytest.mark.parametrize("branch_type,out_type", [("float32", "bfloat16"), ("bfloat16", "bfloat16"), ("bfloat16", "float32"), ("bfloat16", None)])
+def test_branch_norms_of_many_rows(n, H, branch_type, out_type):
+    """Widths at the borders of the forms for many rows and beyond them; without a second norm too."""
+    from cpmcu_amd import ops
+    g = torch.Generator().manual_seed(n + H)
+    x0, b = torch.randn(n, H, generator=g).to(DEV), torch.randn(n, H, generator=g).to(getattr(torch, branch_type)).to(DEV)
+    wb, w = (torch.randn(H, generator=g).to(DEV) for _ in range(2))
+    x, out = x0.clone(), None if out_type is None else torch.empty(n, H, dtype=getattr(torch, out_type), device=DEV)
+    ops.branch_norm_add_norm(x, b, wb, 1e-3, None if out is None else w, 1e-5, out)
+    bd = b.double()
+    add = bd / torch.sqrt((bd * bd).mean(-1, keepdim=True) + 1e-3) * wb.double()
+    want = x0.double() + add
+    assert bool(((x.double() - want).abs() <= 2.0 ** -20 * (add.abs() + want.abs()) + 1e-30).all())
+    if out is not None:
+        xd = x.double()
+        want = xd / torch.sqrt((xd * xd).mean(-1, keepdim=True) + 1e-5) * w.double()
+        off = ((2.0 ** -8 if out.dtype == torch.bfloat16 else 0.0) + 2.0 ** -20) * want.abs() + 1e-30
+        assert bool(((out.double() - want).abs() <= off).all())
