@@ -62,13 +62,14 @@ __global__ __launch_bounds__(1024) void rms_norm_groups_kernel(const XT* __restr
 // The same with 16-byte accesses and a group's values kept in registers between the sum and the result, 4 NQ a thread: THREADS 64
 // (up to 1,024 columns): a wavefront a group, four groups a workgroup, no barrier; 256 (up to 4,096): a workgroup a group.  All of a
 // group's loads are in flight at once.  The bytes bound it: 2,048 rows of 8 groups of 1,024, float in, bf16 gate and result,
-// 84 -> 28 us (134 MB); 1,500 rows of 16 groups of 256 25 -> 14.
+// 65 -> 32 us (134 MB); 1,500 rows of 16 groups of 256 31 -> 15, 2,048 rows of 4,096 27 -> 19.
 template <typename XT, typename ZT, typename OT, int THREADS, int NQ>
 __global__ __launch_bounds__(256) void rms_norm_groups_vec_kernel(const XT* __restrict__ x, long ldx, const ZT* __restrict__ z,
                                                                   long ldz, const float* __restrict__ weight, OT* __restrict__ out,
                                                                   long ldo, int W, int groups, int total, float eps, int gate_after,
                                                                   const float* __restrict__ divisor) {
     __shared__ float red[17];
+    __shared__ float4 held[THREADS == 64 ? 4 : 1][64 * NQ * (THREADS / 64)];     // the groups' values
     const int at = THREADS == 64 ? blockIdx.x * 4 + (threadIdx.x >> 6) : blockIdx.x, t = threadIdx.x % THREADS;
     if (at >= total) return;
     const long r = at / groups;
@@ -93,10 +94,30 @@ __global__ __launch_bounds__(256) void rms_norm_groups_vec_kernel(const XT* __re
         for (int j = 0; j < 4; ++j) {
             e[j] *= pre;
             if (before) e[j] *= silu_f(q[j]);
-            if ((t + i * THREADS) * 4 < W) ss += e[j] * e[j];
         }
     }
-    ss = THREADS == 64 ? wave_sum(ss) : block_sum(ss, red);
+    // the squares are added as rms_norm_groups_kernel's 256 threads add them, to the last bit
+    float4* const own = held[THREADS == 64 ? threadIdx.x >> 6 : 0];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) own[t + i * THREADS] = v[i];
+    const float* const vs = (const float*)own;
+    if (THREADS == 64) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");       // (a wavefront's LDS accesses keep their order)
+#pragma unroll
+        for (int part = 0; part < 4; ++part) {
+            float sq = 0.f;
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                const int c = 64 * part + t + 256 * i;
+                if (c < W) sq += vs[c] * vs[c];
+            }
+            ss += wave_sum(sq);
+        }
+    } else {
+        __syncthreads();
+        for (int c = t; c < W; c += 256) ss += vs[c] * vs[c];
+        ss = block_sum(ss, red);
+    }
     const float rs = 1.0f / sqrtf(ss / (float)W + eps);
     OT* orow = out + r * ldo + (long)g * W;
 #pragma unroll
@@ -131,9 +152,8 @@ extern "C" const char* cpmcu_rms_norm_groups(const void* x, long ldx, int x_dtyp
     const int block = (W >= 2048 && (long)n * groups < 1024) ? 1024 : (W >= 256 ? 256 : 64);
     const int zd = z ? z_dtype : x_dtype;
     const auto off = [](const void* p, int dtype) { return (uintptr_t)p % (dtype == CPMCU_F32 ? 16 : 8) != 0; };
-    // (narrower groups keep the general kernel: 2,048 rows of 32 groups of 128 would take 27 us instead of 33, with sums in another
-    // order ahead of routers whose near ties see it)
-    const bool vec = W % 4 == 0 && W >= 256 && W <= 4096 && ldx % 4 == 0 && ldo % 4 == 0 && (!z || ldz % 4 == 0) && (long)n * groups < (1L << 31) &&
+    // (narrower groups, and few wide ones, which have 1,024 threads, keep the general kernel; the others' results are its own)
+    const bool vec = W % 4 == 0 && W >= 256 && W <= 4096 && block == 256 && ldx % 4 == 0 && ldo % 4 == 0 && (!z || ldz % 4 == 0) && (long)n * groups < (1L << 31) &&
                      !off(x, x_dtype) && !off(out, out_dtype) && !(z && off(z, zd)) && (uintptr_t)weight % 16 == 0;
     const int total = vec ? n * groups : 0;
 #define VEC(XT, ZT, OT, THREADS, NQ)                                                                          \
