@@ -416,3 +416,35 @@ def test_a_step_that_mixes_running_sequences_with_a_fresh_prompt(model_dirs, ref
     for s in (s1, s2, s3):
         eng.release(s)
     eng.cache.check()
+
+
+@pytest.mark.parametrize("name,dtype", [("A", "bfloat16"), ("B", "float32")])
+def test_a_pass_is_reported_when_the_one_before_has_ended(model_dirs, name, dtype):
+    """The host queues passes without waiting for them; its reports of a step's progress do not run ahead with it: with work
+    of many milliseconds behind every pass, each report still finds the pass before ended, and one comes after every pass."""
+    from cpmcu_amd import StepEntry
+    eng = engine_for(model_dirs, name, dtype, max_step_tokens=16)
+    tokens = [(7 * i) % 50 for i in range(75)]
+    a = torch.ones(2048, 2048, device=eng.device)
+    ended, reports, forward = [], [], eng._forward
+
+    def slow(*args):
+        forward(*args)
+        for _ in range(100):
+            torch.mm(a, a)
+        ended.append(torch.cuda.Event())
+        ended[-1].record()
+
+    eng._forward = slow
+    eng.on_pass = lambda done, total: reports.append((done, total, len(ended), all(e.query() for e in ended[:-1])))
+    slot = eng.acquire()
+    try:
+        got = eng.step([StepEntry(slot, tokens, [74])])
+    finally:
+        eng.on_pass = None
+        del eng._forward
+    eng.release(slot)
+    assert reports == [(min(16 * (i + 1), 75), 75, i + 1, True) for i in range(5)]
+    slot = eng.acquire()
+    assert torch.equal(got, eng.step([StepEntry(slot, tokens, [74])]))
+    eng.release(slot)
