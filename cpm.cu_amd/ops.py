@@ -2307,16 +2307,36 @@ def attention_wide_prefill_pays(n_tokens: int, nh: int, nkv: int, max_keys: int)
     return group < 2 or n_tokens > 256 or n_tokens * nkv * -(-group // 16) > 512 or max_keys > 160
 
 
-def attention_wide_columns(q_lens: Sequence[int], nh: int, nkv: int, pool_hdk: int, pool_hdv: int) -> int:
-    """Columns (heads of consecutive tokens) a workgroup of attention_wide_prefill takes.  128 halve what L2 hands out, for keys
-    cached as 576 features and values of more than 256, but make half as many workgroups, one a CU: from one and a quarter for
-    every CU on.  Measured, 32 heads over a latent of 512 + 64, 64 / 128 columns, us (workgroups of 128): 1,000 tokens 77/91 (250),
-    prompts of 77, 300 and 613 61/67 (249), 16 heads 2,048 133/172 (256), 20 x 64 53/50 (320), 1,500 152/117 (375), 8 x 200 70/62
-    (400), 4 x 479 98/89 (480), 2,048 231/180 (512)."""
+def attention_wide_columns(q_lens: Sequence[int], nh: int, nkv: int, pool_hdk: int, pool_hdv: int,
+                           kv_lens: Optional[Sequence[int]] = None, chunk: int = 0, window: int = 0, keep_first: int = 0) -> int:
+    """Columns (heads of consecutive tokens) a workgroup of attention_wide_prefill takes, for sequences of kv_lens tokens (None:
+    q_lens) whose last q_lens are the step's, under that mask.  128 halve what L2 hands out, for keys cached as 576 features and
+    values of more than 256, but make half as many workgroups, one a CU, and each of them takes longer: they pay from one and a
+    quarter for every CU on, where all keys they read are at least 0.6 times what the CUs would read if each read the longest
+    workgroup's.  Measured, 32 heads over a latent of 512 + 64, 64 / 128 columns, us (workgroups of 128, that share): 1,000 tokens
+    77/91 (250, 0.5), prompts of 77, 300 and 613 61/67 (249, 0.4), 16 heads 2,048 133/172 (256, 0.5), 20 x 64 53/50 (320, 0.6), 1,500
+    152/117 (375, 0.7), 8 x 200 70/62 (400, 0.8), 4 x 479 98/89 (480, 0.9), 2,048 231/180 (512, 1.0).  Few tokens behind a
+    long history beside many without: 1,424 in 8 sequences of 49 to 422, of which 49 behind 2,423 and 202 behind 2,617, 173/214 (358,
+    0.3), 1,762 in 16, two behind 3,300, 172/224 (446, 0.25).  Of 103 batches drawn (16 to 64 heads, 1 to 24 sequences, histories, chunks,
+    windows) all 45 above 0.6 were faster with 128, by 7 to 27%, and 41 of the 58 below slower, by up to 46%."""
     if pool_hdk != 576 or pool_hdv <= 256 or 128 % (nh // nkv):
         return ATTENTION_WIDE_COLUMNS
-    per = 128 * nkv // nh
-    return 128 if 4 * nkv * sum(-(-n // per) for n in q_lens) >= 5 * compute_units() else ATTENTION_WIDE_COLUMNS
+    per, most = 128 * nkv // nh, window + keep_first if window else 1 << 60
+
+    def read(x):                                # keys that a sequence's first x tokens see, in all
+        if chunk:
+            return x // chunk * (chunk * (chunk + 1) // 2) + x % chunk * (x % chunk + 1) // 2
+        y = min(x, most)
+        return y * (y + 1) // 2 + (x - y) * y
+
+    workgroups, keys, longest = 0, 0.0, 0
+    for n, end in zip(q_lens, q_lens if kv_lens is None else kv_lens):
+        tiles = -(-n // per)
+        workgroups += tiles
+        keys += tiles * (read(end) - read(end - n)) / n
+        longest = max(longest, min(end, most) if not chunk else chunk if (end - 1) // chunk > (end - n) // chunk else (end - 1) % chunk + 1)
+    pays = 4 * nkv * workgroups >= 5 * compute_units() and nkv * keys >= 0.6 * compute_units() * longest
+    return 128 if pays else ATTENTION_WIDE_COLUMNS
 
 
 def attention_wide_prefill(q: torch.Tensor, out: torch.Tensor, tiles: torch.Tensor, nh: int, nkv: int, hdk: int, hdv: int,
@@ -2436,7 +2456,11 @@ def attention_any(q, out, nh, nkv, hdk, hdv, scale, kpool, vpool, page_table, pa
     if (not ctx.single_token and attention_wide_prefill_ok(q, nh, nkv, hdk, hdv, kpool.shape[2] // nkv, pool_hdv, page_size)
             and (q.data_ptr() | out.data_ptr() | kpool.data_ptr() | vpool.data_ptr()) % 16 == 0
             and attention_wide_prefill_pays(q.shape[0], nh, nkv, min(ctx.max_pos + 1, chunk or window + keep_first or 1 << 30))):
-        columns = attention_wide_columns(ctx.q_lens, nh, nkv, kpool.shape[2] // nkv, pool_hdv)
+        key = ("wide_columns", nh, nkv, kpool.shape[2] // nkv, pool_hdv, chunk, window, keep_first)
+        columns = ctx.extras.get(key)
+        if columns is None:
+            columns = ctx.extras[key] = attention_wide_columns(ctx.q_lens, nh, nkv, kpool.shape[2] // nkv, pool_hdv,
+                                                               getattr(ctx, "kv_lens", None), chunk, window, keep_first)
         per = columns * nkv // nh
         key = ("prefill_tiles", per)
         tiles = ctx.extras.get(key)

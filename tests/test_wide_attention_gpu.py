@@ -249,6 +249,46 @@ def test_the_rule_of_128_columns():
                                    i(1, 1), 64, i(1), i(1), columns=128)
 
 
+@pytest.mark.parametrize("spans,mask,columns", [
+    ([(0, 161 + s) for s in range(8)], {}, 128), ([(0, 163)] * 7, {}, 64),                       # 331 and 287 workgroups of 4 tokens
+    ([(0, 161 + s) for s in range(8)] + [(900, 905)], {}, 64), ([(400, 563)] * 8, {"window": 130, "keep_first": 3}, 128)])
+def test_columns_and_tiles_of_a_step_go_together(spans, mask, columns, monkeypatch):
+    """A step over a latent on both sides of the rule of 128 columns: the tiles are cut for the columns that the kernel is
+    launched with, so that every token's output is written."""
+    from types import SimpleNamespace
+    from cpmcu_amd import ops
+    nh, hdk, hdv, page = 32, 576, 512, 64
+    monkeypatch.setattr(ops, "_cu_count", 256)
+    g = torch.Generator().manual_seed(len(spans))
+    width = max(-(-b // page) for _, b in spans)
+    pools, kept = [torch.zeros(len(spans), width * page * hd, dtype=torch.bfloat16) for hd in (hdk, hdv)], []
+    for s, (_, b) in enumerate(spans):
+        kept.append([torch.randn(b, 1, hd, generator=g).to(torch.bfloat16) for hd in (hdk, hdv)])
+        for pool, x, keys in zip(pools, kept[-1], (True, False)):
+            pool[s, element_order(b, 1, x.shape[-1], keys).flatten()] = x.flatten()
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    ctx = SimpleNamespace(single_token=False, max_pos=max(b for _, b in spans) - 1, q_lens=[b - a for a, b in spans],
+                          kv_lens=[b for _, b in spans], extras={}, positions=i32([t for a, b in spans for t in range(a, b)]),
+                          tok_slot=i32([s for s, (a, b) in enumerate(spans) for _ in range(a, b)]))
+    n, launched, wide = sum(ctx.q_lens), [], ops.attention_wide_prefill
+    monkeypatch.setattr(ops, "attention_wide_prefill", lambda *a: (launched.append((int(a[2][:, 1].max()), a[-1])), wide(*a)))
+    q, out = torch.randn(n, nh, hdk, generator=g).to(torch.bfloat16), torch.full((n, nh * hdv), float("nan"), device=DEV)
+    ops.attention_any(q.view(n, -1).to(DEV), out, nh, 1, hdk, hdv, hdk ** -0.5, *(p.view(-1, page, p.shape[1] // (width * page)).to(DEV) for p in pools),
+                      torch.arange(width * len(spans), dtype=torch.int32, device=DEV).view(len(spans), width), page, ctx, **mask)
+    assert launched == [(columns // nh, columns)]
+    at = 0
+    for s, (a, b) in enumerate(spans):
+        k, v = (x[:, 0].double().to(DEV) for x in kept[s])
+        sc = (q[at:at + b - a].double().to(DEV).view(-1, hdk) @ k.T).view(b - a, nh, b) * hdk ** -0.5
+        p, j = torch.arange(a, b, device=DEV)[:, None], torch.arange(b, device=DEV)[None]
+        hidden = (j > p) | ((p - j >= mask["window"]) & (j >= mask["keep_first"]) if mask else False)
+        w = torch.softmax(sc.masked_fill(hidden[:, None], -math.inf), -1)
+        want, size = ((w.view(-1, b) @ x).view(b - a, nh * hdv) for x in (v, v.abs()))
+        # weights rounded to bf16 (half an ulp each) against values of that size
+        assert bool(((out[at:at + b - a].double() - want).abs() <= 2.0 ** -8 * size + 1e-5).all()), s
+        at += b - a
+
+
 def test_outputs_off_16_byte_borders_take_the_general_kernel():
     from types import SimpleNamespace
     from cpmcu_amd import ops
