@@ -799,7 +799,7 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
     else product(std::integral_constant<int, 1>());
 }
 
-// The same products for steps that give an expert many rows: tiles of up to 128 rows against 128 weight rows (GATED: 64
+// The same products for steps that give an expert many rows (cpmcu_moe_experts_mfma has the rule): tiles of up to 128 rows against 128 weight rows (GATED: 64
 // features), workgroups of 4 wavefronts, two a CU, a wavefront half of the rows and 64 weight rows.  Pieces of 64 columns go
 // from memory to LDS without passing registers, the weights in three buffers and the rows in two (80 KB), with the swizzle of
 // the kernel above in the column that each lane asks for.  The workgroup meets once a piece, in the middle of its products:
@@ -1114,14 +1114,23 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     const long pairs = (long)n * top;
     CPMCU_REQUIRE(max_tiles >= (pairs + MOE_TILE - 1) / MOE_TILE + E && max_tiles <= 65535,
                   "moe_experts_mfma: %d tiles of scratch for %ld pairs of %d experts (at most 65535)", max_tiles, pairs, E);
-    // moe_wide_kernel from 24 pairs an expert on.  Up + down in us, moe_tile_kernel / moe_wide_kernel: 64 experts of 1,408 gated
-    // at width 4,096 at 9 pairs an expert 228 + 114 / 226 + 111, 19 236 + 129 / 234 + 124, 26 256 + 146 / 241 + 132, 32 273 +
-    // 157 / 258 + 139; of 2,112 without a gate 9 167 + 162 / 176 + 163, 19 182 + 181 / 195 + 182, 48 (tiles of 128 through
-    // registers) 246 + 240 / 229 + 226; 16 of 512 at 1,024, 37 15 + 10 / 15 + 10.  Steps of up to 64 tokens: gated 24 182 + 93 / 201
-    // + 94, 40 197 + 96 / 228 + 100; without a gate 24 145 + 132 / 130 + 136, 48 153 + 139 / 138 + 148, so that there the first
-    // product alone takes it, on the tiles of the other.
+    // moe_wide_kernel from 48 pairs an expert on, and from 24 where the first product has four workgroups a CU (experts x blocks of 128 weight
+    // rows).  Up + down in us, moe_tile_kernel / moe_wide_kernel; experts of width x size, gated unless said otherwise:
+    //   from 48 on, against the tiles of 128 rows through registers that it replaced: 7% faster in the mean of 308 shapes (4 to 64
+    //     experts, 512 x 256 to 4,096 x 2,112); the worst 32 of 2,048 x 1,408 at 100 pairs 131/142 (rows in steps of 32 instead of 16)
+    //   24 to 47 pairs, four workgroups a CU or more: 64 of 4,096 x 1,408 even routing 28 pairs 375/371, 36 389/390; 64 of
+    //     4,096 x 2,112 uneven 28 553/495; the same without a gate 28 390/341, 36 442/377, even 24 381/391
+    //   fewer: one round of 512 workgroups where moe_tile_kernel has one of 768, and tiles of up to 128 rows behind which the CUs
+    //     are idle.  32 of 4,096 x 1,408 28 pairs 201/228; 32 of 1,024 x 512 44 pairs 35/41, without a gate 30/35, 8 of them 26/32;
+    //     32 of 512 x 256 without a gate 24 to 44 pairs 19/25
+    // Without a gate the first product of up to 64 tokens alone takes it, on the tiles of the other, where every CU has one workgroup
+    // at most and pieces enough to be ahead (1,024 columns): 8 of 4,096 x 1,408 at 6 pairs 37.2/32.2, 16 of 2,048 x 768 21.9/19.6, 4 of
+    // 1,024 x 512 at 16 13.3/12.0.  With more workgroups it was slower: 64 of 4,096 x 2,112 at 1.5 pairs 108/125, 4 even 176/194, 6
+    // 166/177 (3 uneven 151/137: one round more or less), 16 of 4,096 x 2,112 at 8 62.9/68.0, 32 at 6 126/131; 512 x 256 at 2 8.0/8.4.
     // The scratch is sized for tiles of 64: it holds the pairs without gaps and, at its end, the experts' offsets.
-    const bool wide = pairs >= 24L * E, wide_up = wide || (!gated && n <= MOE_TILE);
+    const long fb = (F + 127) / 128, up_blocks = (gated ? (F + 63) / 64 : fb) * E;
+    const bool wide = pairs >= 48L * E || (pairs >= 24L * E && up_blocks >= 1024);
+    const bool wide_up = wide || (!gated && n <= MOE_TILE && H >= 1024 && fb * (pairs < E ? pairs : E) <= 256);
     const int tile_rows = wide ? MOE_WIDE : MOE_TILE;
     const long tiles = (pairs + tile_rows - 1) / tile_rows + E;
     const long behind = (long)max_tiles * MOE_TILE - (E + 1);         // pairs <= behind: max_tiles covers 64 E rows more

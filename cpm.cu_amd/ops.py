@@ -1690,7 +1690,7 @@ def moe_experts_mfma(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor,
                      gated: bool = True):
     """moe_gated (without ``gated`` moe_up; gate_up is then [E, F, H]) + moe_down for steps of many tokens, bf16 on the matrix
     cores: the (token, expert) pairs are listed expert by expert, and an expert's are spread evenly over tiles of at most
-    MOE_TILE rows, or 2 * MOE_TILE from 24 pairs an expert on (pairs of identity experts, idx >= E, have none: they add h).
+    MOE_TILE rows, or 2 * MOE_TILE where experts have many (pairs of identity experts, idx >= E, have none: they add h).
     Scratch: act bf16 [n, top, F], y bf16 [n, top, H], rows int32 [tiles * MOE_TILE] (the list; its last E + 1 words are the
     experts' borders in it), tile_expert int32 [tiles] (expert + 1024 * the tile's number among its expert's), n_tiles int32 [1]
     (tiles in use), tiles >= moe_tiles(n, top, E)."""

@@ -1,5 +1,6 @@
 """Experts grouped into tiles: row counts at the edges of tiles, of 16 rows and of the rule for wide tiles; widths that end
 inside a piece of 64 columns or a tile of features (GPU)."""
+import launched
 import pytest
 import torch
 
@@ -48,17 +49,17 @@ def test_tiles_of_every_fill(rows, H, F, gated):
     assert bool(((out.double() - w.double() * ref).abs() <= w.double() * off + 2 * sums * ref.abs() + 1e-30).all())
 
 
-@pytest.mark.parametrize("H,F", [(8, 64), (64, 104), (72, 200), (128, 128), (200, 264), (264, 72)])
+@pytest.mark.parametrize("H,F", [(8, 64), (64, 104), (72, 200), (128, 128), (200, 264), (264, 72), (192, 320)])
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("offset", [0, 1])
 def test_tiles_of_128_rows(H, F, gated, offset):
-    """Steps of 24 pairs an expert or more: fills at the edges of every form (the last expert none), one, two, three and more
+    """Steps of 48 pairs an expert or more: fills at the edges of every form (the last expert none), one, two, three and more
     pieces of 64 columns, whole and ragged, features that end inside a tile; pair outputs off 16-byte borders, and a row that
     is no number, which reaches no other."""
     from cpmcu_amd import ops
     rows = [1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 160, 161, 192, 193, 256, 257, 300, 513]
     E, n = len(rows) + 1, sum(rows)
-    assert n >= 24 * E
+    assert n >= 48 * E
     g = torch.Generator(device=DEV).manual_seed(H + F)
     idx = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(rows)])
     idx = idx[torch.randperm(n, generator=torch.Generator().manual_seed(n))].to(DEV)[:, None].contiguous()
@@ -96,9 +97,9 @@ def test_tiles_of_128_rows(H, F, gated, offset):
         assert bool(((out[mine].double() - v * ref).abs() <= v * off + 2 * sums * ref.abs() + 1e-30).all()), e
 
 
-@pytest.mark.parametrize("H,F", [(72, 136), (200, 56)])
+@pytest.mark.parametrize("H,F", [(72, 136), (200, 56), (1024, 136), (1096, 264)])
 def test_experts_without_a_gate_of_few_tokens(H, F):
-    """Up to 64 tokens, whose first product runs on tiles of 64 rows of another kernel; an expert that is every choice of every
+    """Up to 64 tokens, whose first product of 1,024 columns and more runs on tiles of 64 rows of another kernel; an expert that is every choice of every
     token has more rows than there are tokens."""
     from cpmcu_amd import ops
     E, n, top = 9, 40, 3
@@ -123,6 +124,74 @@ def test_experts_without_a_gate_of_few_tokens(H, F):
     ref = torch.einsum("nkf,nkhf->nkh", act.double(), down.double()[e])
     off = F * 2.0 ** -23 * torch.einsum("nkf,nkhf->nkh", act.double().abs(), down.double().abs()[e])
     assert bool(((y.double() - ref).abs() <= off + 2.0 ** -8 * (ref.abs() + off) + 1e-30).all())
+
+
+def forms(E, pairs, H, F, gated, top=1):
+    """(first product's, second's) kernel of a step of so many pairs, one more of the first expert than of others at most."""
+    from cpmcu_amd import ops
+    n = pairs // top
+    assert n * top == pairs
+    idx = (torch.arange(pairs, dtype=torch.int32, device=DEV) % E).view(n, top)
+    rnd = lambda *shape: torch.randn(*shape, device=DEV).to(torch.bfloat16)
+    h, up, down, w = rnd(n, H), rnd(E, F * (2 if gated else 1), H), rnd(E, H, F), torch.rand(n, top, device=DEV)
+    tiles = ops.moe_tiles(n, top, E)
+    i32 = lambda k: torch.empty(k, dtype=torch.int32, device=DEV)
+    scratch = rnd(n, top, F), rnd(n, top, H), i32(tiles * ops.MOE_TILE), i32(tiles), i32(1)
+    names = launched.kernels(lambda: ops.moe_experts_mfma(h, up, down, idx, w, torch.empty(n, H, device=DEV), *scratch, gated=gated,
+                                                          activation="silu" if gated else "relu_squared"))
+    return tuple("wide" if "moe_wide" in name else "tile" for name in names if "moe_wide" in name or "moe_tile" in name)
+
+
+@pytest.mark.parametrize("E,pairs,F,gated,want", [
+    (8, 384, 72, True, "wide"), (8, 383, 72, True, "tile"), (8, 383, 72, False, "tile"),
+    (64, 1536, 1024, True, "wide"), (64, 1535, 1024, True, "tile"), (64, 1536, 960, True, "tile"), (64, 1536, 2048, False, "wide"),
+    (64, 1536, 1920, False, "tile"), (32, 1408, 512, True, "tile"), (8, 352, 512, False, "tile")])
+def test_the_rule_of_wide_tiles(E, pairs, F, gated, want):
+    """48 pairs an expert, or 24 where the first product has 1,024 workgroups."""
+    assert forms(E, pairs, 64, F, gated) == (want, want)
+
+
+@pytest.mark.parametrize("E,n,top,H,F,want", [
+    (8, 64, 2, 1024, 512, "wide"), (8, 64, 2, 1016, 512, "tile"), (8, 65, 2, 1024, 512, "tile"), (16, 64, 1, 1024, 2048, "wide"),
+    (16, 64, 1, 1024, 2056, "tile"), (64, 24, 6, 1024, 2112, "tile"), (64, 4, 6, 1024, 1280, "wide"), (64, 4, 6, 1024, 1408, "tile")])
+def test_the_rule_of_first_products_without_a_gate(E, n, top, H, F, want):
+    """Up to 64 tokens of 1,024 columns or more, a workgroup a CU at most."""
+    assert forms(E, n * top, H, F, False, top) == (want, "tile")
+
+
+@pytest.mark.parametrize("H,F", [(72, 136), (264, 72)])
+@pytest.mark.parametrize("gated", [True, False])
+def test_full_and_split_tiles_of_64_rows(H, F, gated):
+    """Experts of 64 to 300 rows among others without any: below the rule of wide tiles, a tile of 64 rows full, two and
+    three of them."""
+    from cpmcu_amd import ops
+    rows = [64, 65, 63, 129, 128, 300] + [0] * 12
+    E, n = len(rows), sum(rows)
+    assert n < 48 * E
+    g = torch.Generator(device=DEV).manual_seed(H)
+    idx = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(rows)])
+    idx = idx[torch.randperm(n, generator=torch.Generator().manual_seed(n))].to(DEV)[:, None].contiguous()
+    h, up, down = (torch.randn(*s, generator=g, device=DEV).to(torch.bfloat16) for s in ((n, H), (E, F * (2 if gated else 1), H), (E, H, F)))
+    w = torch.rand(n, 1, generator=g, device=DEV)
+    tiles = ops.moe_tiles(n, 1, E)
+    i32 = lambda k: torch.empty(k, dtype=torch.int32, device=DEV)
+    act, y = (torch.full((n, 1, k), float("nan"), dtype=torch.bfloat16, device=DEV) for k in (F, H))
+    ops.moe_experts_mfma(h, up, down, idx, w, torch.empty(n, H, device=DEV), act, y, i32(tiles * ops.MOE_TILE), i32(tiles), i32(1),
+                         gated=gated, activation="silu" if gated else "relu_squared")
+    half, sums = 2.0 ** -8, 2.0 ** -23
+    for e in range(6):
+        mine = (idx[:, 0] == e).nonzero()[:, 0]
+        x, u, got = h[mine].double(), up[e].double(), act[mine, 0].double()
+        z, off = x @ u.T, H * sums * (x.abs() @ u.abs().T)           # float sums in any order
+        if gated:
+            a, b = z[:, :F], z[:, F:]
+            want = torch.nn.functional.silu(a) * b
+            off = 1.1 * off[:, :F] * b.abs() + (a.abs() + off[:, :F]) * off[:, F:]      # |silu'| <= 1.1
+        else:
+            want, off = torch.relu(z) ** 2, 2 * z.abs() * off + off ** 2
+        assert bool(((got - want).abs() <= off + (half + 8 * sums) * want.abs() + 1e-30).all()), rows[e]
+        ref, off = got @ down[e].double().T, F * sums * (got.abs() @ down[e].double().abs().T)
+        assert bool(((y[mine, 0].double() - ref).abs() <= off + half * (ref.abs() + off) + 1e-30).all()), rows[e]
 
 
 @pytest.mark.parametrize("rows", [[80, 112], [81, 79, 97], [65, 113, 64]])
