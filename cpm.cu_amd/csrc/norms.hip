@@ -152,8 +152,14 @@ extern "C" const char* cpmcu_rms_norm_groups(const void* x, long ldx, int x_dtyp
     const int block = (W >= 2048 && (long)n * groups < 1024) ? 1024 : (W >= 256 ? 256 : 64);
     const int zd = z ? z_dtype : x_dtype;
     const auto off = [](const void* p, int dtype) { return (uintptr_t)p % (dtype == CPMCU_F32 ? 16 : 8) != 0; };
-    // (narrower groups, and few wide ones, which have 1,024 threads, keep the general kernel; the others' results are its own)
-    const bool vec = W % 4 == 0 && W >= 256 && W <= 4096 && block == 256 && ldx % 4 == 0 && ldo % 4 == 0 && (!z || ldz % 4 == 0) && (long)n * groups < (1L << 31) &&
+    // The vector kernel where it was the faster one.  256 columns at any number of groups (us, general / here: 5 groups 2.8/2.2, 160
+    // 3.1/3.2, 2,200 5.2/4.1) and more than 1,024 (7 groups of 1,280 5.4/4.8, 380 of 1,536 9.2/5.1).  Between, a wavefront's own chain
+    // is longer than a workgroup's of one load a lane, and only many groups make up for it: 24 of 768 4.2/5.3, 224 of 320 3.6/4.4, 823 of
+    // 264 4.2/5.4, 1,176 of 516 5.6/8.2, 1,336 of 516 6.1/7.2; 1,560 and more level (1,568 of 1,024 9.2/9.0) to 2.7 times
+    // as fast, 1,128 of 448 to 1,376 of 1,024 on both sides.  Groups under 256 columns would leave lanes of their wavefront idle and
+    // few wide ones have 1,024 threads: the general kernel's.  The others' results are its own.
+    const bool pays = W == 256 || W > 1024 || (long)n * groups >= 1536;
+    const bool vec = W % 4 == 0 && W >= 256 && W <= 4096 && block == 256 && pays && ldx % 4 == 0 && ldo % 4 == 0 && (!z || ldz % 4 == 0) && (long)n * groups < (1L << 31) &&
                      !off(x, x_dtype) && !off(out, out_dtype) && !(z && off(z, zd)) && (uintptr_t)weight % 16 == 0;
     const int total = vec ? n * groups : 0;
 #define VEC(XT, ZT, OT, THREADS, NQ)                                                                          \

@@ -7,6 +7,7 @@ import math
 import pytest
 import torch
 
+import launched
 import plain_duvulix as plain
 
 pytestmark = pytest.mark.gpu
@@ -407,6 +408,40 @@ def test_group_norms_of_every_width(n, groups, W, gate, types, shift):
         # a float's operations one by one (exponentials among them), the result's own rounding
         off = ((2.0 ** -8 if ot == torch.bfloat16 else 0.0) + 2.0 ** -18) * v.abs() + 1e-30
         assert bool(((out[:, shift:shift + width].double().view(n, groups, W) - v).abs() <= off).all())
+
+
+@pytest.mark.parametrize("n,groups,W,vec", [
+    (1, 1, 256, True), (1535, 1, 260, False), (512, 3, 260, True), (192, 8, 512, True), (513, 3, 516, True), (1535, 1, 1024, False), (1536, 1, 1024, True),
+    (1, 2, 1028, True), (3, 1, 2044, True), (1024, 1, 2048, True), (1023, 1, 2048, False), (256, 4, 2052, True), (1025, 1, 4092, True), (512, 2, 4096, True),
+    (1024, 1, 4100, False), (2048, 1, 252, False)])
+@pytest.mark.parametrize("gate", ["none", "before", "sigmoid", "silu"])
+@pytest.mark.parametrize("types", [("float32", "float32", "float32"), ("float32", "bfloat16", "bfloat16"), ("bfloat16", "bfloat16", "float32")])
+def test_group_norms_are_the_general_kernels_to_the_last_bit(n, groups, W, vec, gate, types):
+    """The same values on 16-byte borders, on both sides of the rule of the vector kernel, and one element beyond them, where the
+    general kernel is: the same results, of large and tiny values and of a row that is no number too."""
+    from cpmcu_amd import ops
+    xt, zt, ot = (getattr(torch, t) for t in types)
+    g = torch.Generator(device=DEV).manual_seed(W + n)
+    width = groups * W
+    x = (torch.randn(n, width, generator=g, device=DEV) * 10.0 ** (6 * torch.rand(n, 1, generator=g, device=DEV) - 3)).to(xt)
+    x[n // 2, W // 2] = float("nan")
+    z = None if gate == "none" else torch.randn(n, width, generator=g, device=DEV).to(zt)
+    w, den = torch.randn(width, generator=g, device=DEV), 0.5 + torch.rand(n, groups, generator=g, device=DEV)
+
+    def run(shift, divisor):
+        at = lambda t: torch.empty(n, width + 8, dtype=t.dtype, device=DEV)[:, shift:shift + width].copy_(t)
+        out = at(torch.zeros(n, width, dtype=ot, device=DEV))
+        args, kw = (at(x), w, 1e-3, out), dict(groups=groups, gate=None if z is None else at(z), divisor=divisor,
+                                               gate_after={"none": False, "before": False, "sigmoid": True, "silu": "silu"}[gate])
+        return out, lambda: ops.rms_norm_groups(*args, **kw)
+
+    for divisor in (None, den):
+        (out, call), (other, general) = run(0, divisor), run(1, divisor)
+        call(), general()
+        assert torch.equal(out.nan_to_num(7.0), other.nan_to_num(7.0)) and torch.equal(out.isnan(), other.isnan())
+        assert bool(out[n // 2, :W].isnan().all())
+    if gate == "none":
+        assert [["rms_norm_groups_vec" in name for name in launched.kernels(f) if "rms_norm_groups" in name] for f in (call, general)] == [[vec], [False]]
 
 
 @pytest.mark.parametrize("n,H", [(256, 4), (257, 1028), (256, 2048), (300, 2052), (256, 4096), (259, 4100), (256, 8192), (256, 8196), (300, 130)])
