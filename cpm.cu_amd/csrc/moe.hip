@@ -799,8 +799,8 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
     else product(std::integral_constant<int, 1>());
 }
 
-// The same products for steps that give an expert many rows (cpmcu_moe_experts_mfma has the rule): tiles of up to 128 rows against 128 weight rows (GATED: 64
-// features), workgroups of 4 wavefronts, two a CU, a wavefront half of the rows and 64 weight rows.  Pieces of 64 columns go
+// The same products for steps that give an expert many rows (cpmcu_moe_experts_mfma has the rule): tiles of up to 128 rows
+// against 128 weight rows (GATED: 64 features), workgroups of 4 wavefronts, two a CU, a wavefront half of the rows and 64 weight rows.  Pieces of 64 columns go
 // from memory to LDS without passing registers, the weights in three buffers and the rows in two (80 KB), with the swizzle of
 // the kernel above in the column that each lane asks for.  The workgroup meets once a piece, in the middle of its products:
 // what the second half multiplies has been read by then, and while it does, the next piece's first operands are read and the
@@ -813,7 +813,8 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
 //   64 experts of 1,408 gated at width 4,096, routers with random weights (from none to 2,000 of 2,048 tokens an expert):
 //     2,048 tokens 465 + 270 -> 424 + 246, 16 of 80 identity 427 + 246 -> 407 + 230, 347 tokens 275 + 157 -> 254 + 145
 //   even routing: 2,048 477 + 269 -> 443 + 252, 768 317 + 177 -> 306 + 167, 512 298 + 167 -> 269 + 156, 280 256 + 146 -> 241 +
-//     132; of 2,112 without a gate, 2,048 372 + 372 -> 350 + 344, 512 246 + 240 -> 229 + 226
+//     132 (on another day and with more shapes level: see the rule); of 2,112 without a gate, 2,048 372 + 372 -> 350 + 344, 512 246 +
+//     240 -> 229 + 226
 //   64 of 1,024 gated at 1,024, 2,048 tokens with 4 each 89 + 52 -> 75 + 45; 16 of 768 at 2,048 85 + 51 -> 75 + 47
 // Taken back: workgroups of 8 wavefronts, one a CU, with tiles of 256 weight rows and 128, 192 or 256 rows (LDS reads a
 // fifth fewer, weights asked for once: as fast with even routing, 0 to 5% slower with a router's); every XCD a share of all
@@ -1125,8 +1126,10 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     //     32 of 512 x 256 without a gate 24 to 44 pairs 19/25
     // Without a gate the first product of up to 64 tokens alone takes it, on the tiles of the other, where every CU has one workgroup
     // at most and pieces enough to be ahead (1,024 columns): 8 of 4,096 x 1,408 at 6 pairs 37.2/32.2, 16 of 2,048 x 768 21.9/19.6, 4 of
-    // 1,024 x 512 at 16 13.3/12.0.  With more workgroups it was slower: 64 of 4,096 x 2,112 at 1.5 pairs 108/125, 4 even 176/194, 6
-    // 166/177 (3 uneven 151/137: one round more or less), 16 of 4,096 x 2,112 at 8 62.9/68.0, 32 at 6 126/131; 512 x 256 at 2 8.0/8.4.
+    // 1,024 x 512 at 16 13.3/12.0; 512 x 256 at 2 8.0/8.4.  With more workgroups it is slower: of 530 steps (8 to 128 experts, 1.5 to 23
+    // pairs) by 3% in the mean with 256 to 512, by 18% with 576 to 768, which moe_tile_kernel takes in one round (32 of 4,096 x 2,112 at 6
+    // 126/131, 64 at 1.5 108/125), 3% faster with 800 to 1,000 and slower again beyond (64 at 4, even, 176/194); how many there
+    // are is the router's choice.
     // The scratch is sized for tiles of 64: it holds the pairs without gaps and, at its end, the experts' offsets.
     const long fb = (F + 127) / 128, up_blocks = (gated ? (F + 63) / 64 : fb) * E;
     const bool wide = pairs >= 48L * E || (pairs >= 24L * E && up_blocks >= 1024);

@@ -153,7 +153,7 @@ extern "C" const char* cpmcu_proj_add_norm(const void* A, long lda, const void* 
     if (M <= 16 && K <= 1024) LAUNCH(2, 4, 1);
     else if (M <= 16 && K < 12288) LAUNCH(1, 8, 1);
     else if (M <= 16) LAUNCH(2, 8, 1);
-    else if (M <= 32 && K <= 1024) LAUNCH(1, 8, 2);       // 1,024 x 1,024 at 32 tokens 5.4 us, by 4 x 4 7.3
+    else if (M <= 32 && K <= 1024) LAUNCH(1, 8, 2);       // 1,024 x 1,024 at 32 tokens 4.9 us (5.3 with one wavefront at the end, by 4 x 4 so 7.3)
     else if (M <= 32) LAUNCH(4, 4, 2);
     else LAUNCH(2, 4, 4);
 #undef LAUNCH
@@ -165,8 +165,8 @@ extern "C" const char* cpmcu_proj_add_norm(const void* A, long lda, const void* 
 // silu(a . Wg^T) * (a . Wu^T) for decode steps of at most 16 tokens (64 of up to 1,024 columns), by strips: a workgroup owns a strip of 16
 // gate rows and the strip of their up rows over all of K (W holds the gate rows, then the up rows; I gate rows,
 // a multiple of 16).  Its wavefronts take a quarter of K each, with a straight from global memory into the B
-// operand as above (or an eighth: see the launcher), add up through LDS, and the first one applies the norm's row factor (if a is the x * w of a
-// norm cut by columns), the gate's nonlinearity and writes 16 columns.  1,024 small workgroups at 16,384 gate
+// operand as above (or an eighth: see the launcher), add up through LDS, and wavefront t applies the norm's row factor (if a is the x * w
+// of a norm cut by columns) and the gate's nonlinearity to tile t of 16 tokens and writes its 16 columns.  1,024 small workgroups at 16,384 gate
 // rows keep more loads in flight than the skinny product's 512 (gemm.hip), which stages a through LDS behind
 // barriers: 43.4 against 45.8 us at 8 tokens and 4,096 columns, over one weight.
 // (reference: src/model/ffn.cuh:31-59, 77-84; src/model/activation.cuh:6-18)
@@ -289,9 +289,11 @@ extern "C" const char* cpmcu_gated_strip(const void* A, long lda, const void* W,
     //   45.8/45.2 (5.9 TB/s); level between: 11,008 x 4,096 32.6/32.7 -> 31.8/32.7, 2,816 x 4,096 11.1/12.2 -> 11.3/12.4
     // More than 16 tokens, where every workgroup reads up to four times as much of a: it pays while K is short and a wavefront
     // has all of its blocks in flight (4,096 x 1,024, skinny product -> here: 32 tokens 9.3 -> 7.1 us, 64 tokens 15.4 -> 9.2).
-    // A wavefront a tile at the end: 48 and 64 tokens 10.5, 11.4 -> 8.6, 9.6 (24 and 32 7.3, 7.7 -> 6.7, 7.1); of more than 32
-    // tokens 8 wavefronts of one block instead of 4 of two 8.2, 9.2 (2,816 x 1,024 at 40 and 64: 8.0, 9.1 -> 7.3, 8.5; at 24
-    // and 32 tokens they are 0.1 slower).
+    // A wavefront a tile at the end: 48 and 64 tokens 10.5, 11.4 -> 8.6, 9.6 (24 and 32 7.3, 7.7 -> 6.7, 7.1).  Of more than 32 tokens
+    // 8 wavefronts of one block instead of 4 of two are as fast or faster at every number of rows: 33, 48 and 64 tokens of 1,408 x 1,024
+    // 6.9, 7.5, 8.1 -> 6.9, 7.2, 7.9; 4,096 7.8, 8.3, 8.9 -> 7.6, 8.1, 8.9; 8,192 14.7, 15.3, 16.6 -> 14.1, 15.1, 16.3; 16,384 27.3,
+    // 29.2, 31.8 -> 26.0, 28.4, 31.0; 32,768 51.0, 56.1, 60.6 -> 48.8, 53.9, 59.2; of 512 columns 0 to 0.4 less (at 24 and 32 tokens of
+    // 1,024 they are 0.1 slower).  With half of the chain, fewer results miss the nearest bf16: 1.1e-4 of them -> 0.9e-4.
     if (M > 32) LAUNCH(1, 8, 4);
     else if (M > 16) LAUNCH(2, 4, 2);
     else if (K <= 1024 || I >= 16384) LAUNCH(1, 8, 1);
