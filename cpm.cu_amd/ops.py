@@ -2333,7 +2333,7 @@ def attention_wide_columns(q_lens: Sequence[int], nh: int, nkv: int, pool_hdk: i
     for n, end in zip(q_lens, q_lens if kv_lens is None else kv_lens):
         tiles = -(-n // per)
         workgroups += tiles
-        keys += tiles * (read(end) - read(end - n)) / n
+        keys += tiles * (read(end) - read(end - n)) / max(n, 1)
         longest = max(longest, min(end, most) if not chunk else chunk if (end - 1) // chunk > (end - n) // chunk else (end - 1) % chunk + 1)
     pays = 4 * nkv * workgroups >= 5 * compute_units() and nkv * keys >= 0.6 * compute_units() * longest
     return 128 if pays else ATTENTION_WIDE_COLUMNS

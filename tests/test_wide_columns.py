@@ -23,6 +23,7 @@ def share(q_lens, kv_lens, per, chunk, window, keep_first):
 
 def test_a_few_tokens_behind_a_long_history_decide():
     rule = lambda q, kv, **mask: ops.attention_wide_columns(q, 32, 1, 576, 512, kv, **mask)
+    assert rule([], []) == 64 and rule([200] * 8 + [0], [200] * 9) == 128               # (a sequence without tokens brings nothing)
     assert rule([200] * 8, [200] * 8) == 128 and rule([200] * 8, [200] * 7 + [3000]) == 64
     q = [49, 202, 173, 266, 422, 26, 45, 230]
     assert rule(q, [n + h for n, h in zip(q, [2423, 2617, 0, 0, 0, 544, 1205, 0])]) == 64       # 173 us, with 128 columns 214
