@@ -27,6 +27,7 @@ ARCH = "gfx950"
 MODULES: Dict[str, List[str]] = {
     "core": ["elementwise.hip", "sampling.hip"],
     "gemm": ["gemm.hip"],
+    "product": ["product.hip"],
     "attention": ["attention.hip"],
     "sparse": ["sparse.hip"],
     "qkv": ["qkv_rope.hip", "strip.hip"],
@@ -43,7 +44,8 @@ HEADERS = ["common.h"]
 # headers of single libraries
 MODULE_HEADERS: Dict[str, List[str]] = {"attention": ["no_alloc.h"], "core": ["vec4.h"], "norms": ["vec4.h"], "rows": ["vec4.h"],
                                         "ssm": ["runs.h", "vec4.h"], "mlstm": ["runs.h", "vec4.h"], "delta": ["runs.h"],
-                                        "attention_general": ["cache_order.h", "vec4.h", "lds_direct.h"], "moe": ["lds_direct.h"]}
+                                        "attention_general": ["cache_order.h", "vec4.h", "lds_direct.h"], "moe": ["lds_direct.h"],
+                                        "product": ["lds_direct.h"]}
 
 # -packed-fp32-ops off: the compiler must not form packed float instructions on its own
 HIPCC_FLAGS = [

@@ -1,0 +1,309 @@
+// Products of steps of many tokens (bf16, from 256 rows on): out [M, N] = X [M, K] . W [N, K]^T, summed in float, written in bf16 or float,
+// or with the gate's nonlinearity on the float sums (W: gate rows, then up rows), so that neither half is rounded, written and read again.
+//
+// A workgroup of 4 wavefronts (2 x 2) holds a tile of 32 RT rows by 32 CT weight rows in its accumulators, 256 x 256 at most: 256
+// registers a lane, and as many left.  Pieces of 64 columns go from memory to LDS without passing registers (rows of X in SA stages, W in
+// SB: HBM is further away), rows of 128 bytes whose 16-byte places are swapped by the row's number, so that 16 lanes that read 16 rows
+// meet no bank twice.  A wavefront reads half a piece's operands while it multiplies the half before, a read and at most one fetch
+// for two matrix instructions; the workgroup meets once a piece, in the middle.  At most 256 workgroups, one a CU, go from tile to
+// tile: the pieces of the next tile are fetched while the last is multiplied and written.  XCD b % 8 has a run of neighbouring
+// tiles, rows fastest: 32 at a time that share their operands in its L2.
+//
+// What bounds it: with random numbers the chip's power.  Matrix instructions alone reach 2,090 TFLOP/s (2,460 with zeros), this kernel with
+// tiles of 256 x 256 in whole rounds 1,310 to 1,400 at 2.0 GHz, the library 1,430 to 1,480; on half the CUs (2,048 x 4,096 x 16,384) it
+// takes 2,600 cycles a piece for 2,048 of matrix instructions.  Smaller tiles are bound by what L2 hands a CU (32 bytes a cycle), a few
+// tiles alone by what one CU is handed of memory (about 37 GB/s of W).
+// The matrix instructions are written as asm with the accumulators in place: left to itself the compiler moved them between registers
+// in some of these loops (124 moves a piece, 281 -> 434 us).
+//
+// us, the library -> here, weights that no cache holds:
+//   2,048 rows: 22,016 x 4,096 402 -> 276, 4,096 x 4,096 59 to 75 -> 60 to 62, 4,096 x 16,384 223 -> 216, 6,176 x 4,096 89 -> 85;
+//     whole rounds of 256 x 256: 16,384 x 4,096 191 -> 203, 32,768 x 4,096 377 -> 407
+//   1,500: 22,016 x 4,096 292 -> 218, 4,096 x 11,008 128 -> 123; 1,040: 4,096 x 4,096 45.5 -> 40.3; 347: 22,016 x 4,096 75 -> 63
+//   with the gate, against the library's product and the kernel for the nonlinearity (distance from 64 bits 3.1e-3 -> 1.7e-3): 11,008 gates x
+//     4,096 at 2,048, 1,500, 1,040, 700, 480 rows 432, 309, 186, 154, 94 -> 291, 228, 184, 140, 100; 2,816 96, 73, 60, 52, 37 -> 84, 74,
+//     53, 42, 38; whole rounds: 16,384 at 2,048 422 -> 440, at 1,500 317 -> 328
+// (reference: every linear layer is its vendor's library's, src/model/linear.cuh:9-37; the gate src/model/activation.cuh:6-18)
+#include "common.h"
+#include "lds_direct.h"
+
+typedef __bf16 rbf16x8_t __attribute__((ext_vector_type(8)));
+typedef __bf16 rbf16x2_t __attribute__((ext_vector_type(2)));
+typedef float rfloatx4_t __attribute__((ext_vector_type(4)));
+typedef float rfloatx2_t __attribute__((ext_vector_type(2)));
+typedef unsigned ru32x4_t __attribute__((ext_vector_type(4)));
+
+enum { PRODUCT_PLAIN = 0, PRODUCT_GATED = 1, PRODUCT_FLOAT = 2 };
+
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"                      // m0 on the clobber list
+__device__ inline void bring16_at(const void* base, unsigned off, unsigned to) {      // as bring16, `off` bytes behind a uniform address
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(to), "v"(off), "s"(base) : "memory", "m0");
+}
+#pragma clang diagnostic pop
+__device__ inline void multiply_into(rfloatx4_t& c, rbf16x8_t a, rbf16x8_t b) {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+__device__ inline float sum_of(float c) {
+    float v;
+    asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(c));
+    return v;
+}
+__device__ inline unsigned bf16_pair(float a, float b) {             // to the nearest, ties to even
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(rfloatx2_t{a, b}, rbf16x2_t));
+}
+__device__ inline float gate_fast(float g, int act) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-gate_arg(g, act))); }
+
+template <int RT, int CT, int SA, int SB, int KIND>
+__global__ __launch_bounds__(256, 1) void product_kernel(const bf16_t* __restrict__ X, int ldx, const bf16_t* __restrict__ W, int M,
+                                                         int N, int K, void* __restrict__ out, int ldo, int mt, int nt, int act, float act_limit) {
+    constexpr int BM = 32 * RT, BN = 32 * CT;
+    constexpr int AS = BM * 8, BS = BN * 8, B0 = SA * AS;               // 16-byte chunks
+    __shared__ ru32x4_t lds[SA * AS + SB * BS];
+    const int tiles = mt * nt, per = (tiles + 7) / 8;
+    const int first = (blockIdx.x & 7) * per, last = min(first + per, tiles), stride = gridDim.x >> 3;
+    int u = first + (blockIdx.x >> 3);
+    if (u >= last) return;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int wm = wave & 1, wn = wave >> 1;
+    const unsigned base = lds_byte(lds);
+    const int pieces = K / 64;
+    unsigned ao[RT], bo[CT];
+    auto aim_a = [&](int u) {
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));                                  // (worked out again for every tile: no registers held)
+        const int m0 = u % mt * BM, chunk = (lane & 7) ^ (lane >> 3);
+#pragma unroll
+        for (int i = 0; i < RT; ++i) ao[i] = (unsigned)min(m0 + (i * 4 + wave) * 8 + (lane >> 3), M - 1) * (unsigned)(ldx * 2) + chunk * 16;
+    };
+    auto aim_b = [&](int u) {
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));
+        const int n0 = u / mt * BN, chunk = (lane & 7) ^ (lane >> 3);
+#pragma unroll
+        for (int i = 0; i < CT; ++i) {
+            const int row = (i * 4 + wave) * 8 + (lane >> 3);
+            int n;
+            if (KIND == PRODUCT_GATED) n = min(n0 / 2 + (row >> 5) * 16 + (row & 15), N - 1) + (row & 16 ? N : 0);
+            else n = min(n0 + row, N - 1);
+            bo[i] = (unsigned)n * (unsigned)(K * 2) + chunk * 16;
+        }
+    };
+    // what is fetched next: unit, piece, stage
+    int ua = u, ub = u, fa = 0, fb = 0, sa = 0, sb = 0;
+    const char* xa = (const char*)X;
+    const char* wa = (const char*)W;
+    auto fetch_a = [&](int i) { bring16_at(xa, ao[i], base + (sa * AS + (i * 4 + wave) * 64) * 16); };
+    auto fetch_b = [&](int i) { bring16_at(wa, bo[i], base + (B0 + sb * BS + (i * 4 + wave) * 64) * 16); };
+    auto next_a = [&]() {
+        sa = sa + 1 == SA ? 0 : sa + 1;
+        xa += 128;
+        if (++fa == pieces) {
+            fa = 0;
+            xa = (const char*)X;
+            if (ua + stride < last) { ua += stride; aim_a(ua); }
+        }
+    };
+    auto next_b = [&]() {
+        sb = sb + 1 == SB ? 0 : sb + 1;
+        wa += 128;
+        if (++fb == pieces) {
+            fb = 0;
+            wa = (const char*)W;
+            if (ub + stride < last) { ub += stride; aim_b(ub); }
+        }
+    };
+    rfloatx4_t acc[RT][CT];
+    rbf16x8_t a[2][RT], b[2][CT];
+    const int sw0 = r * 8 + (g ^ (r & 7)), sw1 = r * 8 + ((4 + g) ^ (r & 7));
+    auto read_one = [&](int s, int i, const ru32x4_t* as, const ru32x4_t* bs) {      // a0 b0 .. b(CT-1) a1 ..
+        const int sw = s ? sw1 : sw0;
+        if (i == 0) a[s][0] = *(const rbf16x8_t*)&as[wm * (RT * 128) + sw];
+        else if (i <= CT) b[s][i - 1] = *(const rbf16x8_t*)&bs[wn * (CT * 128) + (i - 1) * 128 + sw];
+        else a[s][i - CT] = *(const rbf16x8_t*)&as[wm * (RT * 128) + (i - CT) * 128 + sw];
+    };
+    constexpr int READS = RT + CT, MM = RT * CT, STEPS = MM / 2;
+    static_assert(READS <= STEPS && SB >= SA && SA >= 2 && CT % 2 == 0, "");
+    auto half = [&](auto S, const ru32x4_t* as, const ru32x4_t* bs) {
+        constexpr int s = decltype(S)::value;
+#pragma unroll
+        for (int i = 0; i < STEPS; ++i) {
+            if (i < READS) read_one(s ^ 1, i, as, bs);
+            if (s && i * READS / STEPS != (i + 1) * READS / STEPS) {
+                const int f = i * READS / STEPS;
+                if (f < RT) fetch_a(f);
+                else fetch_b(f - RT);
+            }
+#pragma unroll
+            for (int q = 2 * i; q < 2 * i + 2; ++q) {
+                const int x = q / CT, y = x & 1 ? CT - 1 - q % CT : q % CT;
+                multiply_into(acc[x][y], b[s][y], a[s][x]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);                            // lgkmcnt(0): here it is free, behind the next half's first read not
+    };
+    using I0 = std::integral_constant<int, 0>;
+    using I1 = std::integral_constant<int, 1>;
+    constexpr int STORES = KIND == PRODUCT_GATED ? MM / 4 : KIND == PRODUCT_PLAIN ? MM / 2 : MM;
+    constexpr int BEHIND = (SB > SA ? CT : 0) + (SA - 2) * (RT + CT);
+    constexpr int BEHIND_STORES = BEHIND + STORES < 63 ? BEHIND + STORES : 63;
+    aim_a(u);
+    aim_b(u);
+#pragma unroll
+    for (int i = 0; i < SB - SA; ++i) {
+#pragma unroll
+        for (int j = 0; j < CT; ++j) fetch_b(j);
+        next_b();
+    }
+#pragma unroll
+    for (int i = 0; i < SA; ++i) {
+#pragma unroll
+        for (int j = 0; j < RT; ++j) fetch_a(j);
+        next_a();
+#pragma unroll
+        for (int j = 0; j < CT; ++j) fetch_b(j);
+        next_b();
+    }
+    landed<BEHIND>();
+#pragma unroll
+    for (int i = 0; i < READS; ++i) read_one(0, i, lds, lds + B0);
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    bool written = false;
+    int ra = 0, rb = 0;                                                // the stages of the piece that is multiplied
+    for (;; u += stride) {
+#pragma unroll
+        for (int x = 0; x < RT; ++x)
+#pragma unroll
+            for (int y = 0; y < CT; ++y) acc[x][y] = rfloatx4_t{0.f, 0.f, 0.f, 0.f};
+        asm volatile("s_nop 7" ::: "memory");
+        int p = 0;
+        do {
+            half(I0(), lds + ra * AS, lds + B0 + rb * BS);
+            if (p == 0 && written) landed<BEHIND_STORES>();
+            else landed<BEHIND>();
+            __builtin_amdgcn_s_waitcnt(0xC07F);
+            ra = ra + 1 == SA ? 0 : ra + 1;
+            rb = rb + 1 == SB ? 0 : rb + 1;
+            half(I1(), lds + ra * AS, lds + B0 + rb * BS);
+            next_a();
+            next_b();
+        } while (++p < pieces);
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");             // the matrix instructions' results are there
+        constexpr int EB = KIND == PRODUCT_FLOAT ? 4 : 2;
+        const int m0 = u % mt * BM + wm * 16 * RT, n0 = (u / mt * BN + wn * 16 * CT) / (KIND == PRODUCT_GATED ? 2 : 1);
+        int er = m0 + r, ec = KIND == PRODUCT_FLOAT ? n0 + 4 * g : n0 + (g & 1) * 16 + (g >> 1) * 8;
+        asm volatile("" : "+v"(er), "+v"(ec));
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)(((unsigned)(M - 1) * (unsigned)ldo + (unsigned)N) * EB), 0x00020000);
+#pragma unroll
+        for (int x = 0; x < RT; ++x) {
+            const unsigned line = (unsigned)(er + x * 16) * (unsigned)ldo;
+            const bool ok = er + x * 16 < M;
+            if (KIND == PRODUCT_FLOAT) {
+#pragma unroll
+                for (int y = 0; y < CT; ++y) {
+                    rfloatx4_t v;
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) v[i] = sum_of(acc[x][y][i]);
+                    const int col = ec + y * 16;
+                    __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(ru32x4_t, v), rsrc, ok && col < N ? (line + (unsigned)col) * 4u : 0xFFFFF000u, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int y = 0; y < CT; y += KIND == PRODUCT_GATED ? 4 : 2) {
+                    unsigned d[2][2];
+#pragma unroll
+                    for (int h = 0; h < 2; ++h)
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            float v[2];
+#pragma unroll
+                            for (int j = 0; j < 2; ++j) {
+                                if (KIND == PRODUCT_GATED) {
+                                    float gt = sum_of(acc[x][y + 2 * h][2 * i + j]), up = sum_of(acc[x][y + 2 * h + 1][2 * i + j]);
+                                    gate_prepare(gt, up, act, act_limit);
+                                    v[j] = gate_fast(gt, act) * up;
+                                } else {
+                                    v[j] = sum_of(acc[x][y + h][2 * i + j]);
+                                }
+                            }
+                            d[h][i] = bf16_pair(v[0], v[1]);
+                        }
+                    const cpmcu_u32x2_t p0 = __builtin_amdgcn_permlane16_swap(d[0][0], d[1][0], false, false);
+                    const cpmcu_u32x2_t p1 = __builtin_amdgcn_permlane16_swap(d[0][1], d[1][1], false, false);
+                    const int col = ec + y * (KIND == PRODUCT_GATED ? 8 : 16);
+                    __builtin_amdgcn_raw_buffer_store_b128(ru32x4_t{p0.x, p1.x, p0.y, p1.y}, rsrc, ok && col < N ? (line + (unsigned)col) * 2u : 0xFFFFF000u, 0, 0);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (u + stride >= last) break;
+        written = true;
+    }
+    landed<0>();
+}
+
+// What a product costs with a tile of 32 RT x 32 CT, in us: the launch, what a round of 256 tiles adds, a piece of 64 columns where few
+// CUs are busy and what it takes longer with the share of them that is.  Fitted to 260 products of 65 to 2,048 rows (256 to 33,000
+// outputs, 256 to 16,512 columns, every tile): 4 to 10% off in the mean; the tile chosen by it is 0.5% slower than the fastest.
+struct ProductTile { int rt, ct; float launch, round, piece, shared; };
+#define PRODUCT_TILES(DO)                                                                                                                  \
+    DO(8, 8, 2, 3, 3.6f, 4.2f, 0.981f, 0.512f) DO(7, 8, 2, 3, 2.8f, 4.3f, 0.944f, 0.346f) DO(6, 8, 2, 3, 1.9f, 4.9f, 0.796f, 0.287f)       \
+    DO(5, 8, 3, 3, 2.1f, 4.1f, 0.740f, 0.241f) DO(4, 8, 3, 3, 2.7f, 2.8f, 0.642f, 0.206f) DO(8, 4, 3, 4, 3.2f, 2.7f, 0.579f, 0.240f)       \
+    DO(7, 4, 3, 4, 3.5f, 2.1f, 0.541f, 0.180f) DO(6, 4, 4, 4, 3.3f, 2.1f, 0.493f, 0.176f) DO(5, 4, 4, 5, 3.8f, 1.6f, 0.433f, 0.173f)       \
+    DO(4, 4, 4, 5, 3.9f, 1.1f, 0.380f, 0.154f) DO(6, 6, 3, 3, 2.8f, 3.3f, 0.644f, 0.211f) DO(8, 6, 2, 4, 2.0f, 4.8f, 0.783f, 0.288f)       \
+    DO(4, 6, 4, 4, 3.2f, 2.1f, 0.529f, 0.156f)
+#define PRODUCT_ROW(RT, CT, SA, SB, a, b, c, d) {RT, CT, a, b, c, d},
+static const ProductTile PRODUCT_SHAPES[] = {PRODUCT_TILES(PRODUCT_ROW)};
+static const int PRODUCT_COUNT = sizeof(PRODUCT_SHAPES) / sizeof(PRODUCT_SHAPES[0]);
+
+static float product_us(const ProductTile& t, long M, long rows, int K) {      // rows: of the weight
+    const long tiles = ((M + 32 * t.rt - 1) / (32 * t.rt)) * ((rows + 32 * t.ct - 1) / (32 * t.ct));
+    const long per = (tiles + 7) / 8, rounds = (per + 31) / 32;               // of an XCD with 32 CUs
+    return t.launch + rounds * t.round + K / 64 * (rounds * t.piece + per / 32.0f * t.shared);
+}
+static int product_tile(long M, long rows, int K, bool gated) {
+    int best = -1;
+    float least = 0.f;
+    for (int i = 0; i < PRODUCT_COUNT; ++i) {
+        if (gated && PRODUCT_SHAPES[i].ct % 4) continue;                          // gates and their up rows: 32 weight rows at a time
+        const float us = product_us(PRODUCT_SHAPES[i], M, rows, K);
+        if (best < 0 || us < least) best = i, least = us;
+    }
+    return best;
+}
+
+// out [M, N] = X [M, K] . W^T, W [N, K] bf16, out bf16 or (PRODUCT_FLOAT) float32; PRODUCT_GATED: W [2 N, K] holds gate rows, then up rows, out =
+// act(gate) * up in bf16.  tile: one of PRODUCT_TILES, or -1 for the rule's.
+extern "C" const char* cpmcu_product(const void* X, long ldx, const void* W, int M, int N, int K, void* out, long ldo, int kind, int act,
+                                     float act_limit, int tile, hipStream_t stream) {
+    CPMCU_REQUIRE(kind >= PRODUCT_PLAIN && kind <= PRODUCT_FLOAT, "product: unknown kind %d", kind);
+    CPMCU_REQUIRE(kind != PRODUCT_GATED || CPMCU_ACT_KNOWN(act), "product: unknown nonlinearity %d", act);
+    CPMCU_REQUIRE(M > 0 && N > 0 && K > 0 && K % 64 == 0 && N % 8 == 0, "product: K=%d must be a multiple of 64, N=%d of 8", K, N);
+    const long rows = (long)N * (kind == PRODUCT_GATED ? 2 : 1);
+    CPMCU_REQUIRE((long)M * ldo < (1L << 30) - 4096 && (long)M * ldx < (1L << 31) && rows * K < (1L << 31),
+                  "product: %d rows of %ld, %d x %d exceed 32-bit offsets", M, ldx, N, K);
+    CPMCU_REQUIRE(ldx % 8 == 0 && ldo % 8 == 0 && ldx >= K && ldo >= N && X && W && out && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0 &&
+                  (uintptr_t)out % 16 == 0, "product: rows must start on 16-byte borders");
+    if (tile < 0) tile = product_tile(M, rows, K, kind == PRODUCT_GATED);
+    CPMCU_REQUIRE(tile < PRODUCT_COUNT && (kind != PRODUCT_GATED || PRODUCT_SHAPES[tile].ct % 4 == 0), "product: no tile %d", tile);
+    const int rt = PRODUCT_SHAPES[tile].rt, ct = PRODUCT_SHAPES[tile].ct;
+    const int mt = (M + 32 * rt - 1) / (32 * rt), nt = (int)((rows + 32 * ct - 1) / (32 * ct));
+    const long blocks = ((long)mt * nt + 7) / 8 * 8;
+    const unsigned grid = (unsigned)(blocks < 256 ? blocks : 256);
+#define PRODUCT_KIND(RT, CT, SA, SB, KINDv)                                                                                                \
+    product_kernel<RT, CT, SA, SB, KINDv><<<grid, 256, 0, stream>>>((const bf16_t*)X, (int)ldx, (const bf16_t*)W, M, N, K, out, (int)ldo, mt, nt, \
+                                                                    act, act_limit)
+#define PRODUCT_LAUNCH(RT, CT, SA, SB, a, b, c, d)                                                                                         \
+    if (rt == RT && ct == CT) {                                                                                                            \
+        if (kind == PRODUCT_PLAIN) PRODUCT_KIND(RT, CT, SA, SB, PRODUCT_PLAIN);                                                            \
+        else if (kind == PRODUCT_FLOAT) PRODUCT_KIND(RT, CT, SA, SB, PRODUCT_FLOAT);                                                       \
+        else if constexpr (CT % 4 == 0) PRODUCT_KIND(RT, CT, SA, SB, PRODUCT_GATED);                                                       \
+    }
+    PRODUCT_TILES(PRODUCT_LAUNCH)
+#undef PRODUCT_LAUNCH
+#undef PRODUCT_KIND
+    CPMCU_LAUNCH_CHECK("product");
+    return nullptr;
+}

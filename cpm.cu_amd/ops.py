@@ -2135,6 +2135,48 @@ def skinny_split(M: int, N: int, K: int) -> int:
     return -(-K // ks)
 
 
+PRODUCT_MIN_ROWS = 256
+PRODUCT_MIN_RESULTS = 2 << 20
+PRODUCT_KINDS = {"plain": 0, "gated": 1, "float": 2}
+
+
+def product_takes(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str = "plain") -> bool:
+    """Whether ``product`` takes these operands at all: bfloat16 on 16-byte borders, whole pieces of 64 columns, sizes within
+    32-bit offsets."""
+    M, K = x.shape
+    rows, ldx, ldo = w.shape[0], x.stride(0), out.stride(0)
+    return (x.dtype == w.dtype == torch.bfloat16 and K > 0 and K % 64 == 0 and rows % (16 if kind == "gated" else 8) == 0
+            and x.stride(1) == 1 and out.stride(1) == 1 and w.is_contiguous()
+            and ldx % 8 == 0 and ldo % 8 == 0 and ldx >= K and ldo >= out.shape[1]
+            and (x.data_ptr() | w.data_ptr() | out.data_ptr()) % 16 == 0
+            and M * ldo < (1 << 30) - 4096 and M * ldx < 1 << 31 and rows * K < 1 << 31)
+
+
+def product_faster(M: int, N: int, K: int) -> bool:
+    """Whether ``product`` is faster than the library's product of M rows, N outputs and K columns (csrc/product.hip has the
+    figures): from 256 rows and two million results on, fewer leave too few tiles for the CUs; but not where tiles of 256 x 256
+    fill whole rounds of 256 CUs without gaps, which the library does 5 to 10% faster."""
+    if M < PRODUCT_MIN_ROWS or M * N < PRODUCT_MIN_RESULTS:
+        return False
+    tiles = -(-M // 256) * -(-N // 256)
+    return M * N < 0.93 * 65536 * 256 * -(-tiles // 256)
+
+
+def product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str = "plain", activation="silu", tile: int = -1):
+    """out = x . w^T for steps of many tokens, x [M, K] and w [N, K] bfloat16, summed in float: 'plain' out bfloat16 [M, N],
+    'float' out float32 [M, N], 'gated' w holds gate rows then up rows, out bfloat16 [M, N/2] = act(gate) * up (act as in
+    silu_mul).  tile: a form of the kernel instead of the rule's."""
+    M, K = x.shape
+    N = w.shape[0] // 2 if kind == "gated" else w.shape[0]
+    if (not (x.is_cuda and w.is_cuda and out.is_cuda) or w.shape[1] != K or out.shape != (M, N)
+            or out.dtype != (torch.float32 if kind == "float" else torch.bfloat16) or not product_takes(x, w, out, kind)):
+        raise KernelError(f"product: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype}, out {tuple(out.shape)} {out.dtype} "
+                          f"('{kind}') are not what the kernel takes")
+    _check(_fn("product", "cpmcu_product")(_p(x), c_long(x.stride(0)), _p(w), c_int(M), c_int(N), c_int(K), _p(out),
+                                           c_long(out.stride(0)), c_int(PRODUCT_KINDS[kind]),
+                                           *(_act(activation) if kind == "gated" else (c_int(0), c_float(0.0))), c_int(tile), _stream()))
+
+
 # ---------------------------------------------------------------------------
 # dispatchers: choose the kernel for a shape and element type
 # ---------------------------------------------------------------------------
@@ -2155,7 +2197,10 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, alpha: float = 1
             gemm_skinny(x, w_tiled if w_tiled is not None else w, out, alpha)
             return
         if out.dtype == torch.bfloat16 and alpha == 1.0:
-            torch.mm(x, w.t(), out=out)
+            if product_faster(M, w.shape[0], w.shape[1]) and product_takes(x, w, out):
+                product(x, w, out)
+            else:
+                torch.mm(x, w.t(), out=out)
             return
         # float output for many rows (logits of many positions): the skinny kernel, 64 rows at a time
         for r in range(0, M, SKINNY_MAX_ROWS):

@@ -1,0 +1,88 @@
+"""Products of many rows: every tile's form at the edges of tiles, rounds and pieces, results inside a wider buffer (GPU)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 8, 64), (65, 8, 128), (130, 264, 128), (257, 72, 192), (300, 1032, 320), (33, 520, 1024), (512, 512, 512),
+                                   (1040, 2048, 64), (1500, 6176, 192), (2048, 9256, 128)])
+@pytest.mark.parametrize("kind", ["plain", "gated", "float"])
+def test_every_tile(M, N, K, kind):
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = torch.randn(M, K + 16, generator=g, device=DEV).to(torch.bfloat16)[:, 8:K + 8]            # rows apart, 16 bytes in
+    w = torch.randn(N * (2 if kind == "gated" else 1), K, generator=g, device=DEV).to(torch.bfloat16)
+    if M > 2:
+        x[M // 2, 5] = float("nan")                                    # reaches its own row only
+    z = x.double() @ w.double().t()
+    off = K * 2.0 ** -23 * (x.double().abs() @ w.double().abs().t())   # float sums in any order
+    if kind == "gated":
+        a, u = z[:, :N], z[:, N:]
+        want = torch.nn.functional.silu(a) * u
+        # |silu'| <= 1.1; the exponential's argument is rounded to 2^-24 of itself (|a| e^-|a| < 0.4 of a gate's value), the rest to a few bits
+        off = 1.1 * off[:, :N] * u.abs() + (a.abs() + off[:, :N]) * off[:, N:] + 16 * 2.0 ** -23 * (1 + a.abs()) * want.abs()
+    else:
+        want = z
+    off = off + (0 if kind == "float" else 2.0 ** -8) * (want.abs() + off) + 1e-30
+    dtype = torch.float32 if kind == "float" else torch.bfloat16
+    for tile in range(13):
+        if kind == "gated" and tile >= 10:
+            continue                                                   # tiles of 192 weight rows hold no whole gates
+        wide = torch.full((M + 1, N + 8), 7.0, device=DEV, dtype=dtype)
+        out = wide[:M, :N]
+        ops.product(x, w, out, kind, tile=tile)
+        rows = torch.arange(M, device=DEV) != (M // 2 if M > 2 else -1)
+        assert bool(((out.double() - want).abs() <= off)[rows].all()), tile
+        assert M <= 2 or bool(out[M // 2].isnan().all())
+        assert bool((wide[M] == 7).all()) and bool((wide[:, N:] == 7).all())
+
+
+@pytest.mark.parametrize("activation", ["gelu_tanh", ("clamped_swish", 1.5)])
+def test_gates(activation):
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(256, 128, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(2 * 200, 128, generator=g, device=DEV) * 128 ** -0.5).to(torch.bfloat16)
+    out = torch.empty(256, 200, device=DEV, dtype=torch.bfloat16)
+    ops.product(x, w, out, "gated", activation)
+    z = x.double() @ w.double().t()
+    a, u = z[:, :200], z[:, 200:]
+    if activation == "gelu_tanh":
+        want = torch.nn.functional.gelu(a, approximate="tanh") * u
+    else:
+        a, u = a.clamp(max=1.5), u.clamp(-1.5, 1.5)
+        want = a * torch.sigmoid(1.702 * a) * (u + 1)
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all())      # sums of 128 numbers of order one
+
+
+def test_what_is_refused():
+    from cpmcu_amd import ops
+    x, w = torch.zeros(300, 128, device=DEV, dtype=torch.bfloat16), torch.zeros(64, 128, device=DEV, dtype=torch.bfloat16)
+    out = torch.empty(300, 64, device=DEV, dtype=torch.bfloat16)
+    ops.product(x, w, out)
+    for bad in [(x[:, :96], w[:, :96], out), (x[:, 4:68], w[:, :64].contiguous(), out), (x.t().contiguous().t(), w, out), (x.float(), w, out),
+                (x, w[:60], out[:, :60]), (x, w, out[:, :32]), (x, w, out.float()), (x, w[:, :64], out)]:
+        with pytest.raises(ops.KernelError):
+            ops.product(*bad)
+    with pytest.raises(ops.KernelError):
+        ops.product(x, w, out, tile=13)
+    with pytest.raises(ops.KernelError):
+        ops.product(x, w, out[:, :32], "gated", tile=12)
+
+
+@pytest.mark.parametrize("rows,columns,strided", [(300, 128, False), (300, 72, False), (300, 128, True), (255, 128, False), (2048, 64, False)])
+def test_linear_takes_what_it_took(rows, columns, strided):
+    """The dispatcher's two ways for many rows, with operands that the kernel does not take among them."""
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(rows + columns)
+    x = torch.randn(rows, columns, generator=g, device=DEV).to(torch.bfloat16)
+    if strided:
+        x = x.t().contiguous().t()
+    w = torch.randn(8192, columns, generator=g, device=DEV).to(torch.bfloat16)
+    out = torch.empty(rows, 8192, device=DEV, dtype=torch.bfloat16)
+    ops.linear(x, w, out)
+    want = x.double() @ w.double().t()
+    off = columns * 2.0 ** -23 * (x.double().abs() @ w.double().abs().t())
+    assert bool(((out.double() - want).abs() <= off + 2.0 ** -8 * (want.abs() + off)).all())
