@@ -36,7 +36,7 @@ MODULES: Dict[str, List[str]] = {
     "mlstm": ["mlstm.hip"],
     "delta": ["delta.hip"],
     "gla": ["gla.hip"],
-    "moe": ["moe.hip"],
+    "moe": ["moe.hip", "moe_product.hip"],
     "rows": ["rows.hip"],
     "attention_general": ["attention_general.hip", "diff_attention.hip"],
 }
@@ -44,8 +44,8 @@ HEADERS = ["common.h"]
 # headers of single libraries
 MODULE_HEADERS: Dict[str, List[str]] = {"attention": ["no_alloc.h"], "core": ["vec4.h"], "norms": ["vec4.h"], "rows": ["vec4.h"],
                                         "ssm": ["runs.h", "vec4.h"], "mlstm": ["runs.h", "vec4.h"], "delta": ["runs.h"],
-                                        "attention_general": ["cache_order.h", "vec4.h", "lds_direct.h"], "moe": ["lds_direct.h"],
-                                        "product": ["lds_direct.h"]}
+                                        "attention_general": ["cache_order.h", "vec4.h", "lds_direct.h"], "moe": ["lds_direct.h", "product.h", "moe_product.h"],
+                                        "product": ["lds_direct.h", "product.h"]}
 
 # -packed-fp32-ops off: the compiler must not form packed float instructions on its own
 HIPCC_FLAGS = [

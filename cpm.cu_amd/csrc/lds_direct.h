@@ -13,6 +13,9 @@ __device__ inline void bring16(const void* from, unsigned to) {
 __device__ inline void stream16(const void* from, unsigned to) {      // the same past the caches
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off nt" ::"s"(to), "v"(from) : "memory", "m0");
 }
+__device__ inline void bring4(const void* from, unsigned to) {        // 4 bytes a lane
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(to), "v"(from) : "memory", "m0");
+}
 #pragma clang diagnostic pop
 __device__ inline unsigned lds_byte(const void* p) {                  // where a shared variable lies
     return (unsigned)(uintptr_t)(__attribute__((address_space(3))) const void*)p;

@@ -23,6 +23,7 @@
 // A wavefront owns output rows and its lanes stride over the input features (16-byte loads when the rows are
 // aligned), so an expert's weights stream once for every token that chose it: the form for steps of few tokens.
 #include "lds_direct.h"
+#include "moe_product.h"
 
 #include <type_traits>
 
@@ -605,22 +606,37 @@ typedef unsigned mu32x4_t __attribute__((ext_vector_type(4)));
 
 #define MOE_TILE 64                            // rows of a tile of moe_tile_kernel at most
 #define MOE_WIDE 128                           // of moe_wide_kernel
-enum { MOE_GATED = 0, MOE_PLAIN = 1, MOE_DOWN = 2 };
 
-// tile_rows: rows a tile at most; an expert's pairs are spread evenly over as few tiles as hold them (moe_tile_kernel)
+// tile_rows: rows a tile at most; an expert's pairs are spread evenly over as few tiles as hold them (moe_tile_kernel).
+// counters: MOE_PRODUCT_COUNTERS of moe_product_kernel, set to 0.  large: the tiles are moe_product_kernel's, listed run by run of the 8 that
+// an XCD takes each, experts of many rows first and dealt to the runs in turn: what is left at the end is small
 __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__ idx, int n_pairs, int E, int tile_rows,
                                                          int* __restrict__ rows, int* __restrict__ offs,
-                                                         int* __restrict__ tile_expert, int* __restrict__ n_tiles) {
-    __shared__ int counts[MOE_MAX_EXPERTS];
+                                                         int* __restrict__ tile_expert, int* __restrict__ n_tiles,
+                                                         int* __restrict__ counters, int large) {
+    __shared__ int counts[MOE_MAX_EXPERTS], order[MOE_MAX_EXPERTS];
     __shared__ int pair_sum[16], tile_sum[16];
     const int e = threadIdx.x, lane = e & 63, wave = e >> 6;
     counts[e] = 0;
+    if (e < MOE_PRODUCT_COUNTERS) counters[e] = 0;
     __syncthreads();
     for (int p = threadIdx.x; p < n_pairs; p += 1024)
         if (idx[p] < E) atomicAdd(&counts[idx[p]], 1);              // identity experts have no tiles
     __syncthreads();
     // running sums of pairs and tiles over the experts, one expert a thread
-    const int c = counts[e], nt = (c + tile_rows - 1) / tile_rows;
+    const int c = counts[e];
+    int mine = e;                                                       // the expert whose tiles this thread lists
+    if (large) {
+        if (e < E) {
+            int rank = 0;                                               // experts with more rows, or as many and a lower number
+            for (int i = 0; i < E; ++i) rank += counts[i] > c || (counts[i] == c && i < e);
+            const int run = rank & 7, each = E / 8, more = E % 8;       // runs 0 .. more - 1 have one expert more
+            order[run * each + min(run, more) + (rank >> 3)] = e;
+        }
+        __syncthreads();
+        if (e < E) mine = order[e];
+    }
+    const int nt = (counts[mine] + tile_rows - 1) / tile_rows;
     int pairs = c, tiles = nt;
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
@@ -645,7 +661,7 @@ __global__ __launch_bounds__(1024) void moe_group_kernel(const int* __restrict__
             offs[E] = pairs;
             *n_tiles = tiles;
         }
-        for (int i = 0; i < nt; ++i) tile_expert[tiles - nt + i] = e + 1024 * i;
+        for (int i = 0; i < nt; ++i) tile_expert[tiles - nt + i] = mine + 1024 * i;
     }
     counts[e] = pairs - c;
     __syncthreads();
@@ -1134,12 +1150,23 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     const long fb = (F + 127) / 128, up_blocks = (gated ? (F + 63) / 64 : fb) * E;
     const bool wide = pairs >= 48L * E || (pairs >= 24L * E && up_blocks >= 1024);
     const bool wide_up = wide || (!gated && n <= MOE_TILE && H >= 1024 && fb * (pairs < E ? pairs : E) <= 256);
-    const int tile_rows = wide ? MOE_WIDE : MOE_TILE;
+    // moe_product_kernel from 64 pairs an expert, 16 experts and 14e9 products of a matrix's numbers with rows on, of widths that it takes.
+    // Up + down + the rest of the call, us, moe_wide_kernel / moe_product_kernel:
+    //   64 of 4,096 x 1,408 gated, 6 a token: 2,048 tokens 700/590, even routing 683/535, 16 of 80 identity 631/565, 1,200 546/512, 700 (66 an
+    //     expert) 465/456; 512 (48, even) 413/436.  Of 4,096 x 2,112 without a gate 2,048 713/630, 300 (28) 402/414
+    //   smaller: 64 of 2,048 x 512, 16 pieces and 700 tasks for 256 CUs, 144/168 at 128 an expert (8.6e9), 123/140 at 176 without a gate
+    //     (11.8e9), 2,048 x 1,408 260/237 at 87 (16e9); 16 of 1,024 x 1,536 75/89 at 180 (4.5e9)
+    //   8 experts: 264 tasks are two rounds, 4,096 x 1,408 at 455 an expert 177/210
+    const bool many = pairs >= 64L * E && E >= 16 && pairs * H >= 14000000000L / F;
+    const bool large = wide && many && moe_product_takes(H, F, gated, n, ldh, pairs, top) && moe_product_takes(F, H, false, pairs, F, pairs, top) &&
+                       (uintptr_t)y % 16 == 0;
+    const int tile_rows = large ? MOE_PRODUCT_ROWS : wide ? MOE_WIDE : MOE_TILE;
     const long tiles = (pairs + tile_rows - 1) / tile_rows + E;
-    const long behind = (long)max_tiles * MOE_TILE - (E + 1);         // pairs <= behind: max_tiles covers 64 E rows more
-    int* offs = rows + behind;
+    const long behind = (long)max_tiles * MOE_TILE - (E + 1) - MOE_PRODUCT_COUNTERS;      // pairs <= behind: max_tiles covers 64 E rows more
+    int* counters = rows + behind;
+    int* offs = counters + MOE_PRODUCT_COUNTERS;
     CPMCU_REQUIRE(pairs <= behind && (long)max_tiles * MOE_TILE < (1L << 31), "moe_experts_mfma: scratch of %d tiles for %ld pairs", max_tiles, pairs);
-    moe_group_kernel<<<1, 1024, 0, stream>>>(idx, (int)pairs, E, tile_rows, rows, offs, tile_expert, n_tiles);
+    moe_group_kernel<<<1, 1024, 0, stream>>>(idx, (int)pairs, E, tile_rows, rows, offs, tile_expert, n_tiles, counters, large);
     CPMCU_LAUNCH_CHECK("moe_group");
 #define TILES(KIND, wide, in, ldi, w, out, K, N, act, limit)                                                              \
     do {                                                                                                                  \
@@ -1149,11 +1176,18 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
         kernel<<<(unsigned)blocks, 256, 0, stream>>>(in, ldi, (const bf16_t*)(w), rows, offs, tile_expert, n_tiles,        \
                                                      (bf16_t*)(out), K, N, top, tile_rows, act, limit);                    \
     } while (0)
-    if (gated) TILES(MOE_GATED, wide, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
-    else TILES(MOE_PLAIN, wide_up, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
-    CPMCU_LAUNCH_CHECK("moe_up_tiles");
-    TILES(MOE_DOWN, wide, (const bf16_t*)act, (long)F, wd, y, F, H, 0, 0.f);
-    CPMCU_LAUNCH_CHECK("moe_down_tiles");
+    if (large) {
+        if (const char* m = moe_product(gated ? MOE_GATED : MOE_PLAIN, (const bf16_t*)h, ldh, (const bf16_t*)wgu, rows, offs, tile_expert,
+                                        n_tiles, counters, (bf16_t*)act, pairs, H, F, top, tiles, act_fn, act_limit, stream)) return m;
+        if (const char* m = moe_product(MOE_DOWN, (const bf16_t*)act, F, (const bf16_t*)wd, rows, offs, tile_expert, n_tiles,
+                                        counters + 8, (bf16_t*)y, pairs, F, H, top, tiles, 0, 0.f, stream)) return m;
+    } else {
+        if (gated) TILES(MOE_GATED, wide, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
+        else TILES(MOE_PLAIN, wide_up, (const bf16_t*)h, ldh, wgu, act, H, F, act_fn, act_limit);
+        CPMCU_LAUNCH_CHECK("moe_up_tiles");
+        TILES(MOE_DOWN, wide, (const bf16_t*)act, (long)F, wd, y, F, H, 0, 0.f);
+        CPMCU_LAUNCH_CHECK("moe_down_tiles");
+    }
 #undef TILES
     const long total = (long)n * H;
     const bool vec = H % 4 == 0 && ldh % 4 == 0 && (uintptr_t)y % 16 == 0 && (uintptr_t)(x ? x : out) % 16 == 0;
