@@ -1,4 +1,4 @@
-// Products of steps of many tokens (bf16, from 256 rows on): out [M, N] = X [M, K] . W [N, K]^T, summed in float, written in bf16 or float,
+// Products of steps of many tokens (bf16, from 65 rows on): out [M, N] = X [M, K] . W [N, K]^T, summed in float, written in bf16 or float,
 // or with the gate's nonlinearity on the float sums (W: gate rows, then up rows), so that neither half is rounded, written and read again.
 //
 // A workgroup of 4 wavefronts (2 x 2) holds a tile of 32 RT rows by 32 CT weight rows in its accumulators, 256 x 256 at most: 256
@@ -23,18 +23,28 @@
 //   with the gate, against the library's product and the kernel for the nonlinearity (distance from 64 bits 3.1e-3 -> 1.7e-3): 11,008 gates x
 //     4,096 at 2,048, 1,500, 1,040, 700, 480 rows 432, 309, 186, 154, 94 -> 291, 228, 184, 140, 100; 2,816 96, 73, 60, 52, 37 -> 84, 74,
 //     53, 42, 38; whole rounds: 16,384 at 2,048 422 -> 440, at 1,500 317 -> 328
+//
+// Up to 704 rows (few tiles for 256 CUs) K is cut into 2 or 4 equal shares where the costs below say so (cpmcu_product_plan): every share's
+// sums go out as floats, product_sum_kernel adds them in their order and applies the gate's nonlinearity.  us, the library (with the
+// kernel for the nonlinearity) -> here, in 4 shares unless said otherwise:
+//   4,096 x 16,384 at 65, 128, 256, 512, 700 rows 50, 81, 66, 103, 111 -> 42, 51, 53, 70, 95; without shares 115, 141, 139, 138, 129
+//   4,096 x 11,008 40, 59, 50, 73, 82 -> 33, 38, 40, 53, 69; 4,096 x 4,096 20, 24, 23, 30 (2 shares), 33 (1) -> 16, 18, 21, 29, 35
+//   2,816 gates x 4,096 27, 29, 45, 42 (1), 54 (1) -> 18, 21, 27, 40, 43; 12,288 x 4,096 31, 33, 51 (1), 56 (1), 78 (1) -> 31, 32, 44, 55, 67
+//   one share: 16,384 gates 67, 69, 81, 120, 180 -> 63, 64, 76, 123, 171; 11,008 gates 48 (2), 50, 67, 96, 156 -> 50, 50, 62, 100, 140
+// 8 and 16 shares are slower than 4 but for 65 and 128 rows of 4,096 x 16,384 (38 and 41 us with 16).
 // (reference: every linear layer is its vendor's library's, src/model/linear.cuh:9-37; the gate src/model/activation.cuh:6-18)
 #include "product.h"
 
-enum { PRODUCT_PLAIN = 0, PRODUCT_GATED = 1, PRODUCT_FLOAT = 2 };
+enum { PRODUCT_PLAIN = 0, PRODUCT_GATED = 1, PRODUCT_FLOAT = 2, PRODUCT_PARTS = 3 };
 
 template <int RT, int CT, int SA, int SB, int KIND>
 __global__ __launch_bounds__(256, 1) void product_kernel(const bf16_t* __restrict__ X, int ldx, const bf16_t* __restrict__ W, int M,
-                                                         int N, int K, void* __restrict__ out, int ldo, int mt, int nt, int act, float act_limit) {
+                                                         int N, int K, void* __restrict__ out, int ldo, int mt, int nt, int act, float act_limit, int parts) {
     constexpr int BM = 32 * RT, BN = 32 * CT;
     constexpr int AS = BM * 8, BS = BN * 8, B0 = SA * AS;               // 16-byte chunks
     __shared__ ru32x4_t lds[SA * AS + SB * BS];
-    const int tiles = mt * nt, per = (tiles + 7) / 8;
+    // PRODUCT_PARTS: `parts` equal shares of K, each into a buffer of its own; units run tile by tile, share by share
+    const int tiles = mt * nt * (KIND == PRODUCT_PARTS ? parts : 1), per = (tiles + 7) / 8;
     const int first = (blockIdx.x & 7) * per, last = min(first + per, tiles), stride = gridDim.x >> 3;
     int u = first + (blockIdx.x >> 3);
     if (u >= last) return;
@@ -42,19 +52,20 @@ __global__ __launch_bounds__(256, 1) void product_kernel(const bf16_t* __restric
     const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int wm = wave & 1, wn = wave >> 1;
     const unsigned base = lds_byte(lds);
-    const int pieces = K / 64;
+    const int pieces = KIND == PRODUCT_PARTS ? K / 64 / parts : K / 64;
+    auto share_of = [&](int u) { return KIND == PRODUCT_PARTS ? u / (mt * nt) : 0; };
     unsigned ao[RT], bo[CT];
     auto aim_a = [&](int u) {
         int lane = threadIdx.x & 63;
         asm volatile("" : "+v"(lane));                                  // (worked out again for every tile: no registers held)
-        const int m0 = u % mt * BM, chunk = (lane & 7) ^ (lane >> 3);
+        const int m0 = u % mt * BM, chunk = ((lane & 7) ^ (lane >> 3)) + share_of(u) * pieces * 8;
 #pragma unroll
         for (int i = 0; i < RT; ++i) ao[i] = (unsigned)min(m0 + (i * 4 + wave) * 8 + (lane >> 3), M - 1) * (unsigned)(ldx * 2) + chunk * 16;
     };
     auto aim_b = [&](int u) {
         int lane = threadIdx.x & 63;
         asm volatile("" : "+v"(lane));
-        const int n0 = u / mt * BN, chunk = (lane & 7) ^ (lane >> 3);
+        const int n0 = (u - share_of(u) * (mt * nt)) / mt * BN, chunk = ((lane & 7) ^ (lane >> 3)) + share_of(u) * pieces * 8;
 #pragma unroll
         for (int i = 0; i < CT; ++i) {
             const int row = (i * 4 + wave) * 8 + (lane >> 3);
@@ -165,16 +176,18 @@ __global__ __launch_bounds__(256, 1) void product_kernel(const bf16_t* __restric
             next_b();
         } while (++p < pieces);
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");             // the matrix instructions' results are there
-        constexpr int EB = KIND == PRODUCT_FLOAT ? 4 : 2;
-        const int m0 = u % mt * BM + wm * 16 * RT, n0 = (u / mt * BN + wn * 16 * CT) / (KIND == PRODUCT_GATED ? 2 : 1);
-        int er = m0 + r, ec = KIND == PRODUCT_FLOAT ? n0 + 4 * g : n0 + (g & 1) * 16 + (g >> 1) * 8;
+        constexpr bool FLOATS = KIND == PRODUCT_FLOAT || KIND == PRODUCT_PARTS;
+        constexpr int EB = FLOATS ? 4 : 2;
+        const int m0 = u % mt * BM + wm * 16 * RT, n0 = ((u - share_of(u) * (mt * nt)) / mt * BN + wn * 16 * CT) / (KIND == PRODUCT_GATED ? 2 : 1);
+        int er = m0 + r, ec = FLOATS ? n0 + 4 * g : n0 + (g & 1) * 16 + (g >> 1) * 8;
         asm volatile("" : "+v"(er), "+v"(ec));
-        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(out, 0, (int)(((unsigned)(M - 1) * (unsigned)ldo + (unsigned)N) * EB), 0x00020000);
+        void* const to = KIND == PRODUCT_PARTS ? (void*)((float*)out + (long)share_of(u) * M * ldo) : out;
+        const auto rsrc = __builtin_amdgcn_make_buffer_rsrc(to, 0, (int)(((unsigned)(M - 1) * (unsigned)ldo + (unsigned)N) * EB), 0x00020000);
 #pragma unroll
         for (int x = 0; x < RT; ++x) {
             const unsigned line = (unsigned)(er + x * 16) * (unsigned)ldo;
             const bool ok = er + x * 16 < M;
-            if (KIND == PRODUCT_FLOAT) {
+            if (FLOATS) {
 #pragma unroll
                 for (int y = 0; y < CT; ++y) {
                     rfloatx4_t v;
@@ -232,18 +245,58 @@ struct ProductTile { int rt, ct; float launch, round, piece, shared; };
 static const ProductTile PRODUCT_SHAPES[] = {PRODUCT_TILES(PRODUCT_ROW)};
 static const int PRODUCT_COUNT = sizeof(PRODUCT_SHAPES) / sizeof(PRODUCT_SHAPES[0]);
 
-static float product_us(const ProductTile& t, long M, long rows, int K) {      // rows: of the weight
-    const long tiles = ((M + 32 * t.rt - 1) / (32 * t.rt)) * ((rows + 32 * t.ct - 1) / (32 * t.ct));
-    const long per = (tiles + 7) / 8, rounds = (per + 31) / 32;               // of an XCD with 32 CUs
-    return t.launch + rounds * t.round + K / 64 * (rounds * t.piece + per / 32.0f * t.shared);
+// out [M, N] of `parts` buffers [M, rows] of floats, part after part: their sum in bf16, or (gated: rows = 2 N) the gate's nonlinearity on the sums
+template <bool GATED>
+__global__ __launch_bounds__(256) void product_sum_kernel(const float* __restrict__ part, int parts, int M, int N, bf16_t* __restrict__ out, long ldo,
+                                                          int act, float act_limit) {
+    const int rows = GATED ? 2 * N : N, cols = N / 8;
+    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (long)M * cols) return;
+    const int m = (int)(i / cols), c = (int)(i % cols) * 8;
+    const float* p = part + (long)m * rows + c;
+    rfloatx4_t v[GATED ? 4 : 2] = {};
+    for (int s = 0; s < parts; ++s, p += (long)M * rows)
+#pragma unroll
+        for (int j = 0; j < (GATED ? 4 : 2); ++j) v[j] += *(const rfloatx4_t*)(p + (j & 1) * 4 + (j >> 1) * N);
+    if (GATED) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                float gt = v[j][e], up = v[GATED ? j + 2 : j][e];
+                gate_prepare(gt, up, act, act_limit);
+                v[j][e] = gate_fast(gt, act) * up;
+            }
+    }
+    *(ru32x4_t*)(out + m * ldo + c) = ru32x4_t{bf16_pair(v[0][0], v[0][1]), bf16_pair(v[0][2], v[0][3]), bf16_pair(v[1][0], v[1][1]), bf16_pair(v[1][2], v[1][3])};
 }
-static int product_tile(long M, long rows, int K, bool gated) {
+
+static float product_us(const ProductTile& t, long M, long rows, int K, int parts = 1) {      // rows: of the weight
+    const long tiles = ((M + 32 * t.rt - 1) / (32 * t.rt)) * ((rows + 32 * t.ct - 1) / (32 * t.ct)) * parts;
+    const long per = (tiles + 7) / 8, rounds = (per + 31) / 32;               // of an XCD with 32 CUs
+    return t.launch + rounds * t.round + K / 64 / parts * (rounds * t.piece + per / 32.0f * t.shared);
+}
+static int product_tile(long M, long rows, int K, bool gated, int parts = 1) {
     int best = -1;
     float least = 0.f;
     for (int i = 0; i < PRODUCT_COUNT; ++i) {
         if (gated && PRODUCT_SHAPES[i].ct % 4) continue;                          // gates and their up rows: 32 weight rows at a time
-        const float us = product_us(PRODUCT_SHAPES[i], M, rows, K);
+        const float us = product_us(PRODUCT_SHAPES[i], M, rows, K, parts);
         if (best < 0 || us < least) best = i, least = us;
+    }
+    return best;
+}
+
+// In how many shares of K a product takes least: each share more is M x rows floats that are written and read again (1.4 ps each) and, the
+// first of them, a launch.
+extern "C" int cpmcu_product_plan(int M, long rows, int K, int gated) {
+    int best = 1;
+    float least = 0.f;
+    for (int parts = 1; parts <= 4; parts *= 2) {
+        if (K / 64 % parts || (parts > 1 && (K / 64 / parts < 8 || (double)M * rows * parts >= 1 << 29 || rows * K >= 1L << 30))) continue;
+        const int tile = product_tile(M, rows, K, gated && parts == 1, parts);
+        const float us = product_us(PRODUCT_SHAPES[tile], M, rows, K, parts) + (parts > 1 ? 3.5f + 1.4e-6f * parts * M * rows : 0.f);
+        if (parts == 1 || us < least) best = parts, least = us;
     }
     return best;
 }
@@ -268,7 +321,7 @@ extern "C" const char* cpmcu_product(const void* X, long ldx, const void* W, int
     const unsigned grid = (unsigned)(blocks < 256 ? blocks : 256);
 #define PRODUCT_KIND(RT, CT, SA, SB, KINDv)                                                                                                \
     product_kernel<RT, CT, SA, SB, KINDv><<<grid, 256, 0, stream>>>((const bf16_t*)X, (int)ldx, (const bf16_t*)W, M, N, K, out, (int)ldo, mt, nt, \
-                                                                    act, act_limit)
+                                                                    act, act_limit, 1)
 #define PRODUCT_LAUNCH(RT, CT, SA, SB, a, b, c, d)                                                                                         \
     if (rt == RT && ct == CT) {                                                                                                            \
         if (kind == PRODUCT_PLAIN) PRODUCT_KIND(RT, CT, SA, SB, PRODUCT_PLAIN);                                                            \
@@ -279,5 +332,37 @@ extern "C" const char* cpmcu_product(const void* X, long ldx, const void* W, int
 #undef PRODUCT_LAUNCH
 #undef PRODUCT_KIND
     CPMCU_LAUNCH_CHECK("product");
+    return nullptr;
+}
+
+// The same by shares of K: `parts` partial sums in scratch (parts x M x rows floats, rows 2 N where gated), then their sum; K / 64 in equal shares
+// of at least 4 pieces; bf16 results.
+extern "C" const char* cpmcu_product_parts(const void* X, long ldx, const void* W, int M, int N, int K, void* out, long ldo, int gated, int act,
+                                           float act_limit, float* scratch, int parts, int tile, hipStream_t stream) {
+    CPMCU_REQUIRE(!gated || CPMCU_ACT_KNOWN(act), "product_parts: unknown nonlinearity %d", act);
+    CPMCU_REQUIRE(M > 0 && N > 0 && K > 0 && K % 64 == 0 && N % 8 == 0, "product_parts: K=%d must be a multiple of 64, N=%d of 8", K, N);
+    CPMCU_REQUIRE(parts > 0 && K / 64 % parts == 0 && K / 64 / parts >= 4, "product_parts: %d shares of K=%d", parts, K);
+    const int rows = N * (gated ? 2 : 1);
+    CPMCU_REQUIRE((long)M * rows * parts < (1L << 29) && (long)M * ldx < (1L << 31) && (long)N * K < (1L << 30),
+                  "product_parts: %d rows of %ld, %d x %d exceed 32-bit offsets", M, ldx, N, K);
+    CPMCU_REQUIRE(ldx % 8 == 0 && ldo % 8 == 0 && ldx >= K && ldo >= N && X && W && out && scratch && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0 &&
+                  (uintptr_t)out % 16 == 0 && (uintptr_t)scratch % 16 == 0, "product_parts: rows must start on 16-byte borders");
+    if (tile < 0) tile = product_tile(M, rows, K, false, parts);
+    CPMCU_REQUIRE(tile < PRODUCT_COUNT, "product_parts: no tile %d", tile);
+    const int rt = PRODUCT_SHAPES[tile].rt, ct = PRODUCT_SHAPES[tile].ct;
+    const int mt = (M + 32 * rt - 1) / (32 * rt), nt = (rows + 32 * ct - 1) / (32 * ct);
+    const long blocks = ((long)mt * nt * parts + 7) / 8 * 8;
+    const unsigned grid = (unsigned)(blocks < 256 ? blocks : 256);
+#define PRODUCT_LAUNCH(RT, CT, SA, SB, a, b, c, d)                                                                                         \
+    if (rt == RT && ct == CT)                                                                                                              \
+        product_kernel<RT, CT, SA, SB, PRODUCT_PARTS><<<grid, 256, 0, stream>>>((const bf16_t*)X, (int)ldx, (const bf16_t*)W, M, rows, K, scratch, rows, \
+                                                                                mt, nt, 0, 0.f, parts);
+    PRODUCT_TILES(PRODUCT_LAUNCH)
+#undef PRODUCT_LAUNCH
+    CPMCU_LAUNCH_CHECK("product_parts");
+    const unsigned sums = (unsigned)(((long)M * (N / 8) + 255) / 256);
+    if (gated) product_sum_kernel<true><<<sums, 256, 0, stream>>>(scratch, parts, M, N, (bf16_t*)out, ldo, act, act_limit);
+    else product_sum_kernel<false><<<sums, 256, 0, stream>>>(scratch, parts, M, N, (bf16_t*)out, ldo, act, act_limit);
+    CPMCU_LAUNCH_CHECK("product_sum");
     return nullptr;
 }

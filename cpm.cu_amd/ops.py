@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import ctypes
 from ctypes import c_char_p, c_float, c_int, c_long, c_ulonglong, c_void_p
+from functools import lru_cache
 from typing import NamedTuple, Optional, Sequence, Tuple
 
 import torch
@@ -76,13 +77,16 @@ def upload(values, dtype: torch.dtype, device) -> torch.Tensor:
 _fn_cache = {}
 
 
+_RETURN_INT = {"cpmcu_product_plan"}
+
+
 def _fn(module: str, name: str):
     key = (module, name)
     f = _fn_cache.get(key)
     if f is None:
         lib = _build.load(module)
         f = getattr(lib, name)
-        f.restype = c_char_p
+        f.restype = c_int if name in _RETURN_INT else c_char_p
         _fn_cache[key] = f
     return f
 
@@ -1690,9 +1694,9 @@ def moe_experts_mfma(h: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor,
                      gated: bool = True):
     """moe_gated (without ``gated`` moe_up; gate_up is then [E, F, H]) + moe_down for steps of many tokens, bf16 on the matrix
     cores: the (token, expert) pairs are listed expert by expert, and an expert's are spread evenly over tiles of at most
-    MOE_TILE rows, or 2 * MOE_TILE where experts have many (pairs of identity experts, idx >= E, have none: they add h).
-    Scratch: act bf16 [n, top, F], y bf16 [n, top, H], rows int32 [tiles * MOE_TILE] (the list; its last E + 1 words are the
-    experts' borders in it), tile_expert int32 [tiles] (expert + 1024 * the tile's number among its expert's), n_tiles int32 [1]
+    MOE_TILE rows, or 2 * MOE_TILE or 224 where experts have many (pairs of identity experts, idx >= E, have none: they add h).
+    Scratch: act bf16 [n, top, F], y bf16 [n, top, H], rows int32 [tiles * MOE_TILE] (the list; at its end the experts'
+    borders in it and 16 counters), tile_expert int32 [tiles] (expert + 1024 * the tile's number among its expert's), n_tiles int32 [1]
     (tiles in use), tiles >= moe_tiles(n, top, E)."""
     ldh = _ld(h, "experts input")
     n, H = h.shape
@@ -2135,7 +2139,8 @@ def skinny_split(M: int, N: int, K: int) -> int:
     return -(-K // ks)
 
 
-PRODUCT_MIN_ROWS = 256
+PRODUCT_FEW_ROWS = 704
+PRODUCT_MIN_WEIGHTS = 11 << 20
 PRODUCT_MIN_RESULTS = 2 << 20
 PRODUCT_KINDS = {"plain": 0, "gated": 1, "float": 2}
 
@@ -2153,13 +2158,31 @@ def product_takes(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str
 
 
 def product_faster(M: int, N: int, K: int) -> bool:
-    """Whether ``product`` is faster than the library's product of M rows, N outputs and K columns (csrc/product.hip has the
-    figures): from 256 rows and two million results on, fewer leave too few tiles for the CUs; but not where tiles of 256 x 256
-    fill whole rounds of 256 CUs without gaps, which the library does 5 to 10% faster."""
-    if M < PRODUCT_MIN_ROWS or M * N < PRODUCT_MIN_RESULTS:
+    """Whether ``product_many`` is faster than the library's product of M rows, N outputs and K columns (csrc/product.hip has the
+    figures).  Up to 704 rows from 11 million weights on: few tiles, which shares of K deal to the CUs (smaller products end in the time
+    of their launches).  Beyond, from two million results on; but not where tiles of 256 x 256 fill whole rounds of 256 CUs without
+    gaps, which the library does 5 to 10% faster."""
+    if M <= PRODUCT_FEW_ROWS:
+        return M > SKINNY_MAX_ROWS and N * K >= PRODUCT_MIN_WEIGHTS
+    if M * N < PRODUCT_MIN_RESULTS:
         return False
     tiles = -(-M // 256) * -(-N // 256)
     return M * N < 0.93 * 65536 * 256 * -(-tiles // 256)
+
+
+@lru_cache(maxsize=4096)
+def product_plan(M: int, N: int, K: int, gated: bool) -> int:
+    """In how many shares of K (1, 2 or 4) a product takes least, by the kernel's costs; N with the gate's rows."""
+    return _fn("product", "cpmcu_product_plan")(c_int(M), c_long(N), c_int(K), c_int(1 if gated else 0))
+
+
+def product_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gated: bool = False, activation="silu"):
+    """``product``, or ``product_parts`` where that is the faster one."""
+    parts = product_plan(x.shape[0], w.shape[0], x.shape[1], gated)
+    if parts > 1:
+        product_parts(x, w, out, parts, gated, activation)
+    else:
+        product(x, w, out, "gated" if gated else "plain", activation)
 
 
 def product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str = "plain", activation="silu", tile: int = -1):
@@ -2175,6 +2198,23 @@ def product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str = "pl
     _check(_fn("product", "cpmcu_product")(_p(x), c_long(x.stride(0)), _p(w), c_int(M), c_int(N), c_int(K), _p(out),
                                            c_long(out.stride(0)), c_int(PRODUCT_KINDS[kind]),
                                            *(_act(activation) if kind == "gated" else (c_int(0), c_float(0.0))), c_int(tile), _stream()))
+
+
+def product_parts(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, parts: int, gated: bool = False, activation="silu", tile: int = -1):
+    """``product`` ('plain' or 'gated') for steps whose tiles are too few for the CUs: ``parts`` equal shares of K, each summed in float
+    in a tile of its own, then added in their order."""
+    M, K = x.shape
+    N = w.shape[0] // 2 if gated else w.shape[0]
+    if (not (x.is_cuda and w.is_cuda and out.is_cuda) or w.shape[1] != K or out.shape != (M, N) or out.dtype != torch.bfloat16
+            or not product_takes(x, w, out, "gated" if gated else "plain") or parts < 1 or K // 64 % parts or K // 64 // parts < 4
+            or parts * M * w.shape[0] >= 1 << 29 or w.shape[0] * K >= 1 << 30):
+        raise KernelError(f"product_parts: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype}, out {tuple(out.shape)} {out.dtype} "
+                          f"in {parts} parts are not what the kernel takes")
+    scratch = torch.empty(parts * M * w.shape[0], dtype=torch.float32, device=x.device)
+    _check(_fn("product", "cpmcu_product_parts")(_p(x), c_long(x.stride(0)), _p(w), c_int(M), c_int(N), c_int(K), _p(out),
+                                                 c_long(out.stride(0)), c_int(1 if gated else 0),
+                                                 *(_act(activation) if gated else (c_int(0), c_float(0.0))), _p(scratch), c_int(parts),
+                                                 c_int(tile), _stream()))
 
 
 # ---------------------------------------------------------------------------
@@ -2198,7 +2238,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, alpha: float = 1
             return
         if out.dtype == torch.bfloat16 and alpha == 1.0:
             if product_faster(M, w.shape[0], w.shape[1]) and product_takes(x, w, out):
-                product(x, w, out)
+                product_many(x, w, out)
             else:
                 torch.mm(x, w.t(), out=out)
             return

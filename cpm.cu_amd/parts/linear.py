@@ -131,7 +131,7 @@ class Linear(Part):
             if row_scale is not None:
                 raise ValueError("forward_gated: a row scale needs the few-rows kernel (gated_takes_row_scale)")
             if x.dtype == torch.bfloat16 and ops.product_faster(n, self.out_features, self.in_features) and ops.product_takes(x, self.weight, act, "gated"):
-                ops.product(x, self.weight, act, "gated", activation)           # the nonlinearity on the product's float sums
+                ops.product_many(x, self.weight, act, True, activation)         # the nonlinearity on the product's float sums
                 return act
             gu = self.forward(x, ctx, tag)
             ops.silu_mul(gu, act, activation)

@@ -86,3 +86,75 @@ def test_linear_takes_what_it_took(rows, columns, strided):
     want = x.double() @ w.double().t()
     off = columns * 2.0 ** -23 * (x.double().abs() @ w.double().abs().t())
     assert bool(((out.double() - want).abs() <= off + 2.0 ** -8 * (want.abs() + off)).all())
+
+
+@pytest.mark.parametrize("M,N,K,parts", [(1, 8, 512, 2), (65, 264, 1024, 4), (130, 72, 768, 3), (257, 520, 512, 1), (300, 1032, 2048, 8), (704, 2056, 512, 2)])
+@pytest.mark.parametrize("activation", [None, "silu", ("clamped_swish", 1.5)])
+def test_shares_of_the_columns(M, N, K, parts, activation):
+    """Every tile; sums of shares in their order, results inside a wider buffer, a row that is no number."""
+    from cpmcu_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    x = (torch.randn(M, K + 16, generator=g, device=DEV) * K ** -0.5).to(torch.bfloat16)[:, 8:K + 8]
+    w = torch.randn(N * (2 if activation else 1), K, generator=g, device=DEV).to(torch.bfloat16)
+    if M > 2:
+        x[M // 2, 5] = float("nan")
+    z = x.double() @ w.double().t()
+    off = K * 2.0 ** -23 * (x.double().abs() @ w.double().abs().t())
+    if activation:
+        a, u, slack = z[:, :N], z[:, N:], 16 * 2.0 ** -23
+        if activation != "silu":
+            a, u = a.clamp(max=1.5), u.clamp(-1.5, 1.5) + 1
+        want = a * torch.sigmoid(a if activation == "silu" else 1.702 * a) * u
+        off = 1.1 * off[:, :N] * u.abs() + (a.abs() + off[:, :N]) * off[:, N:] + slack * (1 + 1.702 * a.abs()) * want.abs()
+    else:
+        want = z
+    off = off + 2.0 ** -8 * (want.abs() + off) + 1e-30
+    rows = torch.arange(M, device=DEV) != (M // 2 if M > 2 else -1)
+    for tile in range(-1, 13):
+        wide = torch.full((M + 1, N + 8), 7.0, device=DEV, dtype=torch.bfloat16)
+        ops.product_parts(x, w, wide[:M, :N], parts, activation is not None, activation or "silu", tile=tile)
+        out = wide[:M, :N]
+        assert bool(((out.double() - want).abs() <= off)[rows].all()), tile
+        assert M <= 2 or activation not in (None, "silu") or bool(out[M // 2].isnan().all())
+        assert bool((wide[M] == 7).all()) and bool((wide[:, N:] == 7).all())
+
+
+def test_what_shares_refuse():
+    from cpmcu_amd import ops
+    x, w = torch.zeros(100, 1024, device=DEV, dtype=torch.bfloat16), torch.zeros(64, 1024, device=DEV, dtype=torch.bfloat16)
+    out = torch.empty(100, 64, device=DEV, dtype=torch.bfloat16)
+    ops.product_parts(x, w, out, 4)
+    for bad in [(x, w, out, 3), (x, w, out, 8), (x, w, out, 0), (x, w, out.float(), 2), (x[:, :96], w[:, :96], out, 1)]:
+        with pytest.raises(ops.KernelError):
+            ops.product_parts(*bad)
+
+
+@pytest.mark.parametrize("rows,outputs,columns,want", [(64, 4096, 4096, None), (65, 4096, 4096, "sum"), (704, 4096, 16384, "sum"), (705, 4096, 4096, "product"),
+                                                       (65, 2808, 4096, None), (65, 2816, 4096, "sum"), (200, 16384, 4096, "product"), (300, 4096, 4104, None)])
+def test_the_rule_of_many_rows(rows, outputs, columns, want):
+    from cpmcu_amd import ops
+    import launched
+    x, w = torch.randn(rows, columns, device=DEV).to(torch.bfloat16), torch.randn(outputs, columns, device=DEV).to(torch.bfloat16)
+    out = torch.empty(rows, outputs, device=DEV, dtype=torch.bfloat16)
+    names = launched.kernels(lambda: ops.linear(x, w, out))
+    assert any("product_kernel" in n for n in names) == (want is not None) and any("product_sum" in n for n in names) == (want == "sum")
+    z, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    off = columns * 2.0 ** -23 * size
+    assert bool(((out.double() - z).abs() <= off + 2.0 ** -8 * (z.abs() + off)).all())
+
+
+def test_shares_inside_a_captured_graph():
+    from cpmcu_amd import ops
+    x, w = torch.randn(100, 4096, device=DEV).to(torch.bfloat16), torch.randn(4096, 4096, device=DEV).to(torch.bfloat16)
+    out = torch.empty(100, 4096, device=DEV, dtype=torch.bfloat16)
+    ops.linear(x, w, out)
+    want = out.clone()
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        ops.linear(x, w, out)
+    for _ in range(4):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
