@@ -596,7 +596,7 @@ extern "C" const char* cpmcu_moe_down(const void* act, int dtype, const void* wd
 //    offs[e + 1]) are expert e's pairs, tile_expert[tile] = e + 1024 * (the tile's number among its expert's), n_tiles the
 //    number of tiles.  Which row of its expert's tiles a pair gets depends on timing; its result does not (a row's sums
 //    are its own).
-//  * moe_tile_kernel, moe_wide_kernel: GATED act[pair] = act(Wg_e h_t) * (Wu_e h_t), PLAIN act[pair] = act(Wu_e h_t), DOWN y[pair] =
+//  * moe_tile_kernel, moe_wide_kernel, moe_product_kernel (moe_product.hip): GATED act[pair] = act(Wg_e h_t) * (Wu_e h_t), PLAIN act[pair] = act(Wu_e h_t), DOWN y[pair] =
 //    Wd_e act[pair] (bf16).
 //  * moe_combine_kernel: out[t] = sum_k w[t, k] y[t, k] (h_t where the chosen expert is an identity expert) (+ sg[t] * shared[t]) in float, k in order.
 // ===========================================================================
@@ -815,7 +815,8 @@ __global__ __launch_bounds__(256, 2) void moe_tile_kernel(const bf16_t* __restri
     else product(std::integral_constant<int, 1>());
 }
 
-// The same products for steps that give an expert many rows (cpmcu_moe_experts_mfma has the rule): tiles of up to 128 rows
+// The same products for steps that give an expert many rows (cpmcu_moe_experts_mfma has the rule; the largest of them go to
+// moe_product_kernel): tiles of up to 128 rows
 // against 128 weight rows (GATED: 64 features), workgroups of 4 wavefronts, two a CU, a wavefront half of the rows and 64 weight rows.  Pieces of 64 columns go
 // from memory to LDS without passing registers, the weights in three buffers and the rows in two (80 KB), with the swizzle of
 // the kernel above in the column that each lane asks for.  The workgroup meets once a piece, in the middle of its products:
@@ -1110,7 +1111,7 @@ __global__ __launch_bounds__(256) void moe_combine_token_kernel(const bf16_t* __
     }
 }
 
-// scratch: rows int [max_tiles * 64] (the pairs by expert; its last E + 1 words are the experts' offsets), tile_expert int
+// scratch: rows int [max_tiles * 64] (the pairs by expert; at its end moe_product_kernel's counters and the experts' offsets), tile_expert int
 // [max_tiles], n_tiles int [1], y bf16 [n * top, H];
 // max_tiles = ceil(n * top / 64) + E
 extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const void* wgu, const void* wd, const int* idx,
@@ -1146,7 +1147,7 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     // pairs) by 3% in the mean with 256 to 512, by 18% with 576 to 768, which moe_tile_kernel takes in one round (32 of 4,096 x 2,112 at 6
     // 126/131, 64 at 1.5 108/125), 3% faster with 800 to 1,000 and slower again beyond (64 at 4, even, 176/194); how many there
     // are is the router's choice.
-    // The scratch is sized for tiles of 64: it holds the pairs without gaps and, at its end, the experts' offsets.
+    // The scratch is sized for tiles of 64: it holds the pairs without gaps and, at its end, the counters and the experts' offsets.
     const long fb = (F + 127) / 128, up_blocks = (gated ? (F + 63) / 64 : fb) * E;
     const bool wide = pairs >= 48L * E || (pairs >= 24L * E && up_blocks >= 1024);
     const bool wide_up = wide || (!gated && n <= MOE_TILE && H >= 1024 && fb * (pairs < E ? pairs : E) <= 256);
@@ -1154,6 +1155,7 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     // Up + down + the rest of the call, us, moe_wide_kernel / moe_product_kernel:
     //   64 of 4,096 x 1,408 gated, 6 a token: 2,048 tokens 700/590, even routing 683/535, 16 of 80 identity 631/565, 1,200 546/512, 700 (66 an
     //     expert) 465/456; 512 (48, even) 413/436.  Of 4,096 x 2,112 without a gate 2,048 713/630, 300 (28) 402/414
+    //   45 drawn steps of this rule (16 to 160 experts): 11% faster in the mean, from 27% faster to 1.5% slower
     //   smaller: 64 of 2,048 x 512, 16 pieces and 700 tasks for 256 CUs, 144/168 at 128 an expert (8.6e9), 123/140 at 176 without a gate
     //     (11.8e9), 2,048 x 1,408 260/237 at 87 (16e9); 16 of 1,024 x 1,536 75/89 at 180 (4.5e9)
     //   8 experts: 264 tasks are two rounds, 4,096 x 1,408 at 455 an expert 177/210

@@ -1,11 +1,22 @@
 // Products of routed experts of steps that give an expert many rows: the tiles of product.hip, expert by expert.
 //
 // A workgroup of 4 wavefronts (2 x 2), one a CU, holds up to 224 rows of an expert against 256 of its weight rows (GATED: gate and up
-// rows of 128 features) in its accumulators; pieces of 64 columns go from memory to LDS without passing registers, rows in 2 stages and
-// weights in 3.  A form of the loop for every 32 rows of 96 to 224.  256 workgroups go from tile to tile, the pieces of the next tile on
-// their way while the last is multiplied and written.  The tasks (expert by expert, weight rows by weight rows, an expert's tiles of
-// rows side by side) are cut into 8 runs, one an XCD, whose workgroups take the next one from a counter; a run that has ended helps
-// the run that has most left: experts' tiles are uneven.
+// rows of 128 features) in its accumulators; pieces of 64 columns go from memory to LDS without passing registers, rows in 2 stages,
+// weights, past the caches, in 3 (with 256 rows nothing would be left of LDS for the rows' list).  A form of the loop for every 32
+// rows of 96 to 224.  256 workgroups go from tile to tile, the pieces of the next tile on their way while the last is multiplied and
+// written.  The tasks (expert by expert, weight rows by weight rows, an expert's tiles of rows side by side) are cut into 8 runs, one an
+// XCD, whose workgroups take the next one from a counter; a run that has ended helps the run that has most left.  moe_group_kernel
+// deals the experts to the runs by their rows, many rows first, so that what runs last is small.
+//
+// us (64 experts of 4,096 x 1,408 gated, 2,048 tokens with 6 each), tiles of 128 x 128 two a CU -> this: even routing 424 + 245 ->
+// 290 + 205, uneven (up to 900 rows an expert) 437 + 250 -> 345 + 210, routers with random weights (two experts of 1,900 rows, 45 of fewer
+// than 100) the whole call 728 -> 672, with 16 of 80 identity 676 -> 620.  2,112 without a gate 345 + 345 -> 292 + 291.
+// What bounds it: even routing moves 1.47 + 0.74 GB of weights, a piece of 32 KB in 1.26 us a CU (6.6 TB/s together) beside
+// 1,536 cycles of matrix instructions; with all operands in caches and nothing written 246 + 137 are left.  A tile costs 7 us beside its
+// pieces (results 4, the next task and its list 2), the kernel's start 7, and at the end CUs wait for the last: a tenth of the time.
+// Taken back: weights through the caches where tiles share them (592 -> 613 for the call, even routing 540 -> 551), runs taken
+// from both ends, so that large tiles and small ones meet (594 -> 621, level with a router's load), forms for 96, 160 and 224 rows only (594 ->
+// 606), experts in the order of their numbers (first product uneven 354 -> 344, of 1,200 tokens 315 -> 292 with the order).
 #include "moe_product.h"
 #include "product.h"
 
