@@ -183,7 +183,9 @@ class Engine:
     def _rehearse(self, needs, max_slots: int):
         """One prompt pass of max_step_tokens tokens and decode passes of the largest and of small batches, on a
         scratch cache that is freed afterwards: every part asks the workspace for what its largest steps need,
-        and the product library sets itself up, before the memory figure is made."""
+        and the product library sets itself up, before the memory figure is made.  A part whose way through a pass does
+        not follow the rows (a product that is the library's at some numbers of rows between two of its kernel's) asks for the same
+        buffers whichever way it takes, or reserves them in reserve_workspace."""
         page = self.options.page_size
         n_prompt = min(self.max_step_tokens, self.max_seq_len)
         B = max(min(max_slots, self.max_step_tokens), 1)
@@ -196,7 +198,10 @@ class Engine:
             # token ids spread over the vocabulary (the product library sets itself up on ordinary rows)
             self.step([StepEntry(s, [(7919 * i) % self.vocab_size for i in range(n_prompt)], [n_prompt - 1])])
             self.release(s)
-            # kernels change with the number of rows at powers of two at most: those sizes and their successors
+            if self.dtype == torch.bfloat16:        # whether or not a rehearsed pass has a product of the library's
+                x = torch.zeros((128, 64), dtype=self.dtype, device=self.device)
+                torch.mm(x, x.t())
+            # sizes at powers of two and their successors: parts with forms for few and for many rows change there
             sizes = {1}
             b = 2
             while b < max(B, n_prompt):

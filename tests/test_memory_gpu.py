@@ -121,3 +121,50 @@ def test_an_engine_of_short_passes_lets_the_checkpoint_layout_go(model_dirs, nam
         for r, ref in refs.items():
             assert float((got[r] - ref).abs().max()) < 0.01 * float(ref.abs().max()), (what, r)
     short.cache.check()
+
+
+def wide_model(hidden=2048, ff=6144, layers=2):
+    """Two layers whose products are large enough for the kernels of many rows."""
+    return dict(tiny.tiny_a(), num_hidden_layers=layers, hidden_size=hidden, num_attention_heads=hidden // 128, num_key_value_heads=2, head_dim=128,
+                intermediate_size=ff, vocab_size=512, max_position_embeddings=4096,
+                rope_scaling={"rope_type": "longrope", "short_factor": [1.0] * 64, "long_factor": [1.0] * 64,
+                              "original_max_position_embeddings": 4096})
+
+
+def wide_engine(ff, **options):
+    from cpmcu_amd import Engine, EngineOptions, get_architecture
+    from cpmcu_amd.weights import random_tensors
+    raw = wide_model(ff=ff)
+    cfg = get_architecture(raw["architectures"][0]).config_class.from_dict(raw)
+    return Engine.from_tensors(cfg, random_tensors(cfg, 5, device="cuda:0"), EngineOptions(**options))
+
+
+def prompt(eng, n):
+    from cpmcu_amd import StepEntry
+    s = eng.acquire()
+    out = eng.step([StepEntry(s, [(31 * i) % eng.vocab_size for i in range(n)], [n - 1])])
+    eng.release(s)
+    return out
+
+
+@pytest.mark.parametrize("ff,chunk", [(6144, 2048), (16384, 1800)])
+def test_products_of_every_number_of_rows_find_their_workspace(ff, chunk):
+    """Whether a product is the library's or the kernel's goes up and down with the rows: passes on both sides of the rule, between the rehearsed
+    sizes, find the workspace as the engine left it, and the captured decode step stays."""
+    from cpmcu_amd import StepEntry, ops
+    rows = [65, 100, 300, 512, 700, 705, 769, 900, 1024, 1100, 1280, 1366, 1500, 1536, 1700, 1792, 1800, 2048]
+    ways = [ops.product_faster(n, 2 * ff, 2048) for n in rows if n <= chunk]
+    assert True in ways and False in ways
+    eng = wide_engine(ff, dtype="bfloat16", max_tokens=4096, max_slots=8, max_step_tokens=chunk, hip_graph=True)
+    held = eng.acquire()
+    prompt_of_held = [StepEntry(held, [1, 2, 3], [2])]
+    eng.step(prompt_of_held)
+    eng.step([StepEntry(held, [5], [0])])
+    graphs, ws, gen = dict(eng._graphs), eng.workspace.bytes(), eng.workspace.generation
+    assert len(graphs) == 1
+    for n in rows:
+        if n <= chunk:
+            prompt(eng, n)
+            assert eng.workspace.grown == [], n
+    eng.step([StepEntry(held, [5], [0])])
+    assert eng.workspace.bytes() == ws and eng.workspace.generation == gen and eng._graphs == graphs
