@@ -1,7 +1,8 @@
 """Python face of the HIP kernels: argument checks, then one launch each.
 
 Tensors are torch tensors on the GPU, used as typed memory only; every function
-launches on torch's current stream and allocates nothing.  Shapes are checked
+launches on torch's current stream and allocates nothing (product_parts alone does
+where it is given no scratch).  Shapes are checked
 here, on the host, before a pointer reaches a kernel; a size a kernel does not
 take is refused with an error that names it.  There is no fallback: without a
 GPU or without the built libraries these functions raise.
@@ -2176,11 +2177,36 @@ def product_plan(M: int, N: int, K: int, gated: bool) -> int:
     return _fn("product", "cpmcu_product_plan")(c_int(M), c_long(N), c_int(K), c_int(1 if gated else 0))
 
 
-def product_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gated: bool = False, activation="silu"):
-    """``product``, or ``product_parts`` where that is the faster one."""
+@lru_cache(maxsize=256)
+def product_scratch(most_rows: int, N: int, K: int, gated: bool) -> int:
+    """Bytes of partial sums that steps of up to ``most_rows`` rows have ``product_many`` keep, where the rule gives them to it."""
+    plan, most = _fn("product", "cpmcu_product_plan"), 0
+    if N % 8 or K % 64:
+        return 0
+    for M in range(SKINNY_MAX_ROWS + 1, most_rows + 1):
+        if product_faster(M, N, K):
+            parts = plan(c_int(M), c_long(N), c_int(K), c_int(1 if gated else 0))
+            if parts > 1:
+                most = max(most, parts * M * N * 4)
+    return most
+
+
+PRODUCT_ROOM = "product.shares"                # the workspace's name for those sums
+
+
+def reserve_product(ws, most_rows: int, N: int, K: int, gated: bool = False):
+    """Room in the workspace for product_many's partial sums: which step needs most does not follow the rows."""
+    need = product_scratch(most_rows, N, K, gated)
+    if need:
+        ws.room(PRODUCT_ROOM, need)
+
+
+def product_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gated: bool = False, activation="silu", ws=None):
+    """``product``, or ``product_parts`` where that is the faster one; ``ws``: the workspace that holds its partial sums."""
     parts = product_plan(x.shape[0], w.shape[0], x.shape[1], gated)
     if parts > 1:
-        product_parts(x, w, out, parts, gated, activation)
+        product_parts(x, w, out, parts, gated, activation,
+                      scratch=None if ws is None else ws.room(PRODUCT_ROOM, parts * x.shape[0] * w.shape[0] * 4))
     else:
         product(x, w, out, "gated" if gated else "plain", activation)
 
@@ -2200,9 +2226,11 @@ def product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str = "pl
                                            *(_act(activation) if kind == "gated" else (c_int(0), c_float(0.0))), c_int(tile), _stream()))
 
 
-def product_parts(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, parts: int, gated: bool = False, activation="silu", tile: int = -1):
+def product_parts(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, parts: int, gated: bool = False, activation="silu", tile: int = -1,
+                  scratch: Optional[torch.Tensor] = None):
     """``product`` ('plain' or 'gated') for steps whose tiles are too few for the CUs: ``parts`` equal shares of K, each summed in float
-    in a tile of its own, then added in their order."""
+    in a tile of its own, then added in their order.  ``scratch``: parts * M * len(w) floats or more, of any type (a caller without
+    a workspace leaves it out: the allocator's, for this call)."""
     M, K = x.shape
     N = w.shape[0] // 2 if gated else w.shape[0]
     if (not (x.is_cuda and w.is_cuda and out.is_cuda) or w.shape[1] != K or out.shape != (M, N) or out.dtype != torch.bfloat16
@@ -2210,7 +2238,12 @@ def product_parts(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, parts: in
             or parts * M * w.shape[0] >= 1 << 29 or w.shape[0] * K >= 1 << 30):
         raise KernelError(f"product_parts: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype}, out {tuple(out.shape)} {out.dtype} "
                           f"in {parts} parts are not what the kernel takes")
-    scratch = torch.empty(parts * M * w.shape[0], dtype=torch.float32, device=x.device)
+    need = parts * M * w.shape[0] * 4
+    if scratch is None:
+        scratch = torch.empty(need, dtype=torch.uint8, device=x.device)
+    elif not (scratch.is_cuda and scratch.is_contiguous() and scratch.numel() * scratch.element_size() >= need and scratch.data_ptr() % 16 == 0):
+        raise KernelError(f"product_parts: {need} contiguous bytes on a 16-byte border of the GPU are needed for the sums of {parts} shares, got "
+                          f"{tuple(scratch.shape)} {scratch.dtype} on {scratch.device}")
     _check(_fn("product", "cpmcu_product_parts")(_p(x), c_long(x.stride(0)), _p(w), c_int(M), c_int(N), c_int(K), _p(out),
                                                  c_long(out.stride(0)), c_int(1 if gated else 0),
                                                  *(_act(activation) if gated else (c_int(0), c_float(0.0))), _p(scratch), c_int(parts),
@@ -2226,8 +2259,9 @@ def library_gemm_ok(x: torch.Tensor, out_dtype: torch.dtype) -> bool:
     return x.dtype == torch.bfloat16 and out_dtype == torch.bfloat16 and x.shape[0] > SKINNY_MAX_ROWS
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, alpha: float = 1.0, w_tiled=None):
-    """out = alpha * x . w^T with the kernel that suits the element type and the number of rows."""
+def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, alpha: float = 1.0, w_tiled=None, ws=None):
+    """out = alpha * x . w^T with the kernel that suits the element type and the number of rows; ``ws``: the workspace for a product's
+    partial sums (product_many)."""
     M = x.shape[0]
     if w is None and (w_tiled is None or M > SKINNY_MAX_ROWS and out.dtype == torch.bfloat16 and alpha == 1.0):
         raise KernelError(f"linear: {M} rows need the weight in the checkpoint's layout, which this engine let go "
@@ -2238,7 +2272,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, alpha: float = 1
             return
         if out.dtype == torch.bfloat16 and alpha == 1.0:
             if product_faster(M, w.shape[0], w.shape[1]) and product_takes(x, w, out):
-                product_many(x, w, out)
+                product_many(x, w, out, ws=ws)
             else:
                 torch.mm(x, w.t(), out=out)
             return

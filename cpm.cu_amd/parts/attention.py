@@ -59,6 +59,7 @@ class GQAAttention(Mixer):
         self._qkv_fused = None               # the q/k/v weight re-laid for the fused decode kernel, made at first use
 
     def reserve_workspace(self, ws, rt: Runtime, max_step_tokens: int, max_slots: int):
+        self.qkv.reserve_sums(ws, max_step_tokens, rows=self.nh * self.hd)          # (a run that reads another run's cache)
         # the q/k/v weight in the fused decode kernel's order, if any step of this engine can run that kernel
         plain_rotation = self._kernel_rotates()
         if (self._qkv_fused is None and plain_rotation and rt.dtype == torch.bfloat16 and self.qkv.tiled is not None
@@ -380,6 +381,8 @@ class GeneralAttention(Mixer):
                           window=self.chunk or self.window or None, keep_first=self.keep_first)
 
     def reserve_workspace(self, ws, rt: Runtime, max_step_tokens: int, max_slots: int):
+        if self.gate_off is None and self.head_gate_off is None:
+            self.qkv.reserve_sums(ws, max_step_tokens, rows=self.nh * self.dk)      # (a run that reads another run's cache)
         keys = rt.max_seq_len
         if self.chunk:
             keys = min(keys, self.chunk)

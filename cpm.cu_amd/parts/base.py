@@ -78,6 +78,12 @@ class Workspace:
         for s in shape:
             n *= int(s)
         nbytes = n * dtype.itemsize
+        t = self.room(name, nbytes)[:nbytes].view(dtype).view(shape)
+        self._last[name] = (shape, dtype, t)
+        return t
+
+    def room(self, name: str, nbytes: int) -> torch.Tensor:
+        """The named buffer as bytes, at least ``nbytes`` of them."""
         buf = self._buf.get(name)
         if buf is None or buf.numel() < nbytes:
             if buf is not None:
@@ -86,9 +92,7 @@ class Workspace:
             self._buf[name] = buf
             if self.sealed and name not in self.grown:
                 self.grown.append(name)
-        t = buf[:nbytes].view(dtype).view(shape)
-        self._last[name] = (shape, dtype, t)
-        return t
+        return buf
 
     def bytes(self) -> int:
         return sum(b.numel() for b in self._buf.values())

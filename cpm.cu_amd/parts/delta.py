@@ -116,6 +116,10 @@ class GatedDeltaMixer(Mixer):
                 w[self.up_decay:, self.decay_rank:] = f("gate_up")
             self.up_w = w.to(rt.dtype).contiguous()
 
+    def reserve_workspace(self, ws, rt: Runtime, max_step_tokens: int, max_slots: int):
+        if self.low and rt.dtype == torch.bfloat16:
+            ops.reserve_product(ws, max_step_tokens, self.up_width, self.low)
+
     def cache_needs(self) -> CacheNeeds:
         state = [("delta", StateSpec((self.heads, self.dv, self.dk), torch.float32))]
         if self.taps > 1:
@@ -129,7 +133,7 @@ class GatedDeltaMixer(Mixer):
         low.copy_(u[:, self.low_off:self.low_off + self.low])
         few = n <= ops.SKINNY_MAX_ROWS or self.rt.dtype == torch.float32
         up = ctx.ws.get("delta.up", (n, self.up_width), torch.float32 if few else self.rt.dtype)
-        ops.linear(low, self.up_w, up)
+        ops.linear(low, self.up_w, up, ws=ctx.ws)
         decay = gate = None
         if self.decay_rank:
             decay = up[:, :self.up_decay]

@@ -38,6 +38,9 @@ class GatedFFN(FeedForward):
     def parts(self) -> List[Part]:
         return [self.gate_up, self.down]
 
+    def reserve_workspace(self, ws, rt: Runtime, max_step_tokens: int, max_slots: int):
+        self.gate_up.reserve_sums(ws, max_step_tokens, gated=True)
+
     def takes_row_scale(self, n: int, ctx: StepContext) -> bool:
         return self.gate_up.gated_takes_row_scale(n)
 

@@ -56,6 +56,12 @@ class Linear(Part):
         # is let go, which halves what the weights hold.
         if self.tiled is not None and max_step_tokens <= ops.SKINNY_MAX_ROWS and self.in_features % 8 == 0:
             self.weight = None
+        self.reserve_sums(ws, max_step_tokens)
+
+    def reserve_sums(self, ws, max_step_tokens: int, rows: Optional[int] = None, gated: bool = False):
+        """Room for the partial sums of products of many rows (``rows``, ``gated``: as forward and forward_gated take them)."""
+        if self.weight is not None and self.rt.dtype == torch.bfloat16:
+            ops.reserve_product(ws, max_step_tokens, self.out_features if rows is None else rows, self.in_features, gated)
 
     def forward(self, x: torch.Tensor, ctx: StepContext, tag: str, out_dtype: Optional[torch.dtype] = None,
                 alpha: float = 1.0, rows: Optional[int] = None, partials: bool = False) -> torch.Tensor:
@@ -78,7 +84,7 @@ class Linear(Part):
         if partials and alpha == 1.0 and ops.library_gemm_ok(x, x.dtype):
             out_dtype = x.dtype         # many rows: the branch comes back in bf16 from the library product
         out = ctx.ws.get(tag, (n, N), out_dtype)
-        ops.linear(x, w, out, alpha, w_tiled=wt)
+        ops.linear(x, w, out, alpha, w_tiled=wt, ws=ctx.ws)
         return out
 
     def forward_activated(self, x: torch.Tensor, ctx: StepContext, tag: str, activation: str) -> torch.Tensor:
@@ -88,7 +94,7 @@ class Linear(Part):
         if ops.skinny_ok(x):
             ops.gemm_skinny(x, self.tiled if self.tiled is not None else self.weight, act, mode="act", activation=activation)
         else:
-            ops.linear(x, self.weight, act)
+            ops.linear(x, self.weight, act, ws=ctx.ws)
             ops.activate(act, activation)
         return act
 
@@ -135,7 +141,7 @@ class Linear(Part):
             ctx.ws.get(tag, (n, self.out_features), x.dtype)
             if (x.dtype == torch.bfloat16 and self.weight is not None and ops.product_faster(n, self.out_features, self.in_features)
                     and ops.product_takes(x, self.weight, act, "gated")):
-                ops.product_many(x, self.weight, act, True, activation)         # the nonlinearity on the product's float sums
+                ops.product_many(x, self.weight, act, True, activation, ctx.ws)         # the nonlinearity on the product's float sums
                 return act
             gu = self.forward(x, ctx, tag)
             ops.silu_mul(gu, act, activation)

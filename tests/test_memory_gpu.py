@@ -168,3 +168,36 @@ def test_products_of_every_number_of_rows_find_their_workspace(ff, chunk):
             assert eng.workspace.grown == [], n
     eng.step([StepEntry(held, [5], [0])])
     assert eng.workspace.bytes() == ws and eng.workspace.generation == gen and eng._graphs == graphs
+
+
+def test_partial_sums_lie_in_the_workspace():
+    """Shares of K leave their sums in room that the engine reserved: a pass that takes them asks the allocator for nothing."""
+    from cpmcu_amd import ops
+    eng = wide_engine(6144, dtype="bfloat16", max_tokens=4096, max_slots=4, max_step_tokens=1100)
+    most = max(ops.product_plan(n, N, K, gated) * n * N * 4 for n in range(65, 1101)
+               for N, K, gated in ((12288, 2048, True), (2048, 6144, False))
+               if ops.product_plan(n, N, K, gated) > 1 and ops.product_faster(n, N, K))
+    assert most > 8 << 20 and eng.workspace.bytes() >= most
+    rows = [65, 130, 256, 300, 700, 769, 1025, 1100]
+    assert any(ops.product_plan(n, 2048, 6144, False) > 1 and ops.product_faster(n, 2048, 6144) for n in rows if n > 704)
+    assert any(ops.product_plan(n, 2048, 6144, False) > 1 and ops.product_faster(n, 2048, 6144) for n in rows if n <= 704)
+    out = [prompt(eng, n) for n in rows]                            # (what a pass uploads is allocated by now)
+    held, report = torch.cuda.memory_allocated(), eng.memory_report()
+    for n, want in zip(rows, out):
+        torch.cuda.reset_peak_memory_stats()
+        got = prompt(eng, n)
+        assert torch.cuda.max_memory_allocated() - held < 1 << 20, n
+        assert torch.equal(got, want)
+        del got
+    assert eng.workspace.grown == [] and eng.memory_report() == report
+
+
+def test_scratch_that_is_too_small_is_refused():
+    from cpmcu_amd import ops
+    x, w = torch.zeros(100, 1024, device="cuda:0", dtype=torch.bfloat16), torch.zeros(64, 1024, device="cuda:0", dtype=torch.bfloat16)
+    out = torch.empty(100, 64, device="cuda:0", dtype=torch.bfloat16)
+    room = torch.empty(2 * 100 * 64 + 1, device="cuda:0")
+    ops.product_parts(x, w, out, 2, scratch=room)
+    for bad in (room[:-2], room[1:], torch.empty(2 * 100 * 64), room[:2 * 100 * 64].view(64, 200).t()):
+        with pytest.raises(ops.KernelError, match="shares"):
+            ops.product_parts(x, w, out, 2, scratch=bad)
