@@ -204,6 +204,10 @@ __global__ __launch_bounds__(256, 1) void moe_product_kernel(const bf16_t* __res
 #pragma unroll
             for (int y = 0; y < CT; ++y) acc[x][y] = rfloatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
+        for (int x = 0; x < RT; ++x)
+#pragma unroll
+            for (int y = 0; y < CT; ++y) in_place(acc[x][y]);
+#pragma unroll
         for (int i = 0; i < READS; ++i) read_one(0, i, lds + ra * AS, lds + B0 + rb * BS);
         __builtin_amdgcn_s_waitcnt(0xC07F);
         asm volatile("s_nop 7" ::: "memory");

@@ -20,6 +20,9 @@ __device__ inline void stream16_at(const void* base, unsigned off, unsigned to) 
 __device__ inline void multiply_into(rfloatx4_t& c, rbf16x8_t a, rbf16x8_t b) {
     asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
 }
+// An accumulator is written up to here: blocks of asm keep their order, and what one takes as an operand stands before it.  (The compiler keeps
+// no distances for instructions inside asm: zeros belong in front of the wait that stands in front of the first matrix instruction.)
+__device__ inline void in_place(rfloatx4_t& c) { asm volatile("" : "+a"(c)); }
 __device__ inline float sum_of(float c) {
     float v;
     asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(c));

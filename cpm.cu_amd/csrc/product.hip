@@ -162,6 +162,10 @@ __global__ __launch_bounds__(256, 1) void product_kernel(const bf16_t* __restric
         for (int x = 0; x < RT; ++x)
 #pragma unroll
             for (int y = 0; y < CT; ++y) acc[x][y] = rfloatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int x = 0; x < RT; ++x)
+#pragma unroll
+            for (int y = 0; y < CT; ++y) in_place(acc[x][y]);
         asm volatile("s_nop 7" ::: "memory");
         int p = 0;
         do {
