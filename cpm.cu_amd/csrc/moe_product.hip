@@ -273,10 +273,10 @@ __global__ __launch_bounds__(256, 1) void moe_product_kernel(const bf16_t* __res
                                 if (KIND == MOE_GATED) {
                                     float gt = sum_of(acc[x][y + 2 * h][2 * i + j]), up = sum_of(acc[x][y + 2 * h + 1][2 * i + j]);
                                     gate_prepare(gt, up, act, act_limit);
-                                    v[j] = gate_fast(gt, act) * up;
+                                    v[j] = gate_act(gt, act) * up;
                                 } else {
                                     v[j] = sum_of(acc[x][y + h][2 * i + j]);
-                                    if (KIND == MOE_PLAIN) v[j] = act == CPMCU_ACT_RELU_SQUARED ? fmaxf(v[j], 0.f) * fmaxf(v[j], 0.f) : gate_fast(v[j], act);
+                                    if (KIND == MOE_PLAIN) v[j] = plain_act(v[j], act);
                                 }
                             }
                             d[h][i] = bf16_pair(v[0], v[1]);

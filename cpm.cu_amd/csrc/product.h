@@ -31,4 +31,3 @@ __device__ inline float sum_of(float c) {
 __device__ inline unsigned bf16_pair(float a, float b) {             // to the nearest, ties to even
     return __builtin_bit_cast(unsigned, __builtin_convertvector(rfloatx2_t{a, b}, rbf16x2_t));
 }
-__device__ inline float gate_fast(float g, int act) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-gate_arg(g, act))); }

@@ -136,3 +136,55 @@ def test_inside_a_captured_graph():
         run()
         torch.cuda.synchronize()
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("activation", ["silu", "gelu_tanh", ("clamped_swish", 7.0), "plain_silu", "plain_gelu_tanh", "relu_squared"])
+def test_the_bits_of_the_other_kernel(activation):
+    """The same sums in the same order, the same nonlinearity in float: what the tiles of 128 rows give, to the last bit."""
+    gated = not str(activation).startswith(("plain", "relu"))
+    E, n, h, up, down, idx, w = operands([260, 300, 129, 700] * 4, 2048, 1728, gated, 11)
+    h = h * 2.0 ** -4
+    act = [torch.empty(n, 1, 1728, dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    y = torch.full((2, n * 2048 + 8), 7.0, dtype=torch.bfloat16, device=DEV)
+    out = [torch.empty(n, 2048, device=DEV) for _ in range(2)]
+    for i in range(2):                                                  # off its 16-byte border y keeps the other kernel
+        run = lambda: call(E, n, h, up, down, idx, w, act[i], y[i, i:i + n * 2048].view(n, 1, 2048), out[i], gated, str(activation).removeprefix("plain_")
+                           if isinstance(activation, str) else activation)
+        assert sum("moe_product" in x for x in launched.kernels(run)) == (0 if i else 2)
+    assert torch.equal(act[0], act[1]) and torch.equal(y[0, :n * 2048], y[1, 1:n * 2048 + 1]) and torch.equal(out[0], out[1])
+
+
+def test_identity_experts():
+    """Pairs of identity experts have no tiles; the rest of an uneven load, and an expert without rows, keep their places."""
+    E, H, F, top, n = 20, 2048, 1728, 4, 1500
+    g = torch.Generator(device=DEV).manual_seed(2)
+    load = torch.cat([torch.arange(1, E + 9, device=DEV, dtype=torch.float32) ** 2])        # the last 8 columns: identity experts
+    load[7] = 0
+    idx = torch.multinomial(load.expand(n, -1), top, generator=g).to(torch.int32)
+    h = torch.randn(n, H, generator=g, device=DEV).to(torch.bfloat16)
+    up = (torch.randn(E, 2 * F, H, generator=g, device=DEV) * H ** -0.5).to(torch.bfloat16)
+    down = (torch.randn(E, H, F, generator=g, device=DEV) * F ** -0.5).to(torch.bfloat16)
+    w = torch.rand(n, top, generator=g, device=DEV)
+    act, y = (torch.full((n, top, k), 7.0, dtype=torch.bfloat16, device=DEV) for k in (F, H))
+    out = torch.empty(n, H, device=DEV)
+    names = launched.kernels(lambda: call(E, n, h, up, down, idx, w, act, y, out, True, "silu"))
+    assert sum("moe_product" in x for x in names) == 2
+    idle = idx >= E
+    assert 0 < int(idle.sum()) < n * top and bool((act[idle] == 7).all()) and bool((y[idle] == 7).all())
+    want = torch.zeros(n, H, dtype=torch.float64, device=DEV)
+    flat, size = idx.flatten(), torch.zeros(n, H, dtype=torch.float64, device=DEV)
+    for e in range(E + 8):
+        mine = (flat == e).nonzero()[:, 0]
+        t, k = mine // top, mine % top
+        x = h[t].double()
+        if e < E:
+            z = x @ up[e].double().T
+            a = torch.nn.functional.silu(z[:, :F]) * z[:, F:]
+            v, s = a @ down[e].double().T, a.abs() @ down[e].double().abs().T
+            # act is rounded to 2^-9 of itself, its float sums of 2,048 and the result's of 1,728 numbers to 2^-12 of their sizes, y to 2^-9
+            off = (2.0 ** -9 + 2.0 ** -12) * s + 2.0 ** -9 * v.abs()
+        else:
+            v, off = x, torch.zeros_like(x)
+        want.index_add_(0, t, w[t, k, None].double() * v)
+        size.index_add_(0, t, w[t, k, None].double() * off + 2.0 ** -20 * v.abs())
+    assert bool(((out.double() - want).abs() <= size).all())
