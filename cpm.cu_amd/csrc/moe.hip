@@ -1151,15 +1151,19 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     const long fb = (F + 127) / 128, up_blocks = (gated ? (F + 63) / 64 : fb) * E;
     const bool wide = pairs >= 48L * E || (pairs >= 24L * E && up_blocks >= 1024);
     const bool wide_up = wide || (!gated && n <= MOE_TILE && H >= 1024 && fb * (pairs < E ? pairs : E) <= 256);
-    // moe_product_kernel from 64 pairs an expert, 16 experts and 14e9 products of a matrix's numbers with rows on, of widths that it takes.
+    // moe_product_kernel from 64 pairs an expert, 16 experts and 14e9 products of a matrix's numbers with rows on (21e9 of narrow experts), of widths
+    // that it takes.
     // Up + down + the rest of the call, us, moe_wide_kernel / moe_product_kernel:
     //   64 of 4,096 x 1,408 gated, 6 a token: 2,048 tokens 700/590, even routing 683/535, 16 of 80 identity 631/565, 1,200 546/512, 700 (66 an
     //     expert) 465/456; 512 (48, even) 413/436.  Of 4,096 x 2,112 without a gate 2,048 713/630, 300 (28) 402/414
-    //   45 drawn steps of this rule (16 to 160 experts): 11% faster in the mean, from 27% faster to 1.5% slower
+    //   92 drawn steps of this rule (16 to 160 experts of 1,600 to 4,700 x 512 to 2,500, even routing to a few experts with most rows): 8% faster in
+    //     the mean, 25% at most; 11 slower, all but one of fewer than 20e9 products: 16 to 24 experts of which a few have most rows 2 to 34%,
+    //     others up to 11% (of 24 steps of 14e9 to 21e9 half are faster, up to 22%)
+    //   fewer than 1,600 columns (24 pieces a tile): below 21e9 level to 18% slower (64 of 1,088 x 576 at 351 an expert 184/197), above 2 to 15% faster
     //   smaller: 64 of 2,048 x 512, 16 pieces and 700 tasks for 256 CUs, 144/168 at 128 an expert (8.6e9), 123/140 at 176 without a gate
     //     (11.8e9), 2,048 x 1,408 260/237 at 87 (16e9); 16 of 1,024 x 1,536 75/89 at 180 (4.5e9)
     //   8 experts: 264 tasks are two rounds, 4,096 x 1,408 at 455 an expert 177/210
-    const bool many = pairs >= 64L * E && E >= 16 && pairs * H >= 14000000000L / F;
+    const bool many = pairs >= 64L * E && E >= 16 && pairs * H >= (H < 1600 ? 21000000000L : 14000000000L) / F;
     const bool large = wide && many && moe_product_takes(H, F, gated, n, ldh, pairs, top) && moe_product_takes(F, H, false, pairs, F, pairs, top) &&
                        (uintptr_t)y % 16 == 0;
     const int tile_rows = large ? MOE_PRODUCT_ROWS : wide ? MOE_WIDE : MOE_TILE;

@@ -21,16 +21,28 @@
 //     whole rounds of 256 x 256: 16,384 x 4,096 191 -> 203, 32,768 x 4,096 377 -> 407
 //   1,500: 22,016 x 4,096 292 -> 218, 4,096 x 11,008 128 -> 123; 1,040: 4,096 x 4,096 45.5 -> 40.3; 347: 22,016 x 4,096 75 -> 63
 //   with the gate, against the library's product and the kernel for the nonlinearity (distance from 64 bits 3.1e-3 -> 1.7e-3): 11,008 gates x
-//     4,096 at 2,048, 1,500, 1,040, 700, 480 rows 432, 309, 186, 154, 94 -> 291, 228, 184, 140, 100; 2,816 96, 73, 60, 52, 37 -> 84, 74,
-//     53, 42, 38; whole rounds: 16,384 at 2,048 422 -> 440, at 1,500 317 -> 328
+//     4,096 at 2,048, 1,500, 1,040, 704 rows 429, 308, 180, 155 -> 285, 224, 174, 136; 2,816 91, 74, 59, 53 -> 78, 72, 51, 40; whole rounds:
+//     16,384 at 2,048 397 -> 426, at 1,500 309 -> 331
 //
-// Up to 704 rows (few tiles for 256 CUs) K is cut into 2 or 4 equal shares where the costs below say so (cpmcu_product_plan): every share's
-// sums go out as floats, product_sum_kernel adds them in their order and applies the gate's nonlinearity.  us, the library (with the
-// kernel for the nonlinearity) -> here, in 4 shares unless said otherwise:
-//   4,096 x 16,384 at 65, 128, 256, 512, 700 rows 50, 81, 66, 103, 111 -> 42, 51, 53, 70, 95; without shares 115, 141, 139, 138, 129
-//   4,096 x 11,008 40, 59, 50, 73, 82 -> 33, 38, 40, 53, 69; 4,096 x 4,096 20, 24, 23, 30 (2 shares), 33 (1) -> 16, 18, 21, 29, 35
-//   2,816 gates x 4,096 27, 29, 45, 42 (1), 54 (1) -> 18, 21, 27, 40, 43; 12,288 x 4,096 31, 33, 51 (1), 56 (1), 78 (1) -> 31, 32, 44, 55, 67
-//   one share: 16,384 gates 67, 69, 81, 120, 180 -> 63, 64, 76, 123, 171; 11,008 gates 48 (2), 50, 67, 96, 156 -> 50, 50, 62, 100, 140
+// Where tiles are few for 256 CUs, K is cut into 2 or 4 equal shares if the costs below say so (cpmcu_product_plan; of up to 704 rows most
+// products, of more those of long rows): every share's sums go out as floats, product_sum_kernel adds them in their order and applies the
+// gate's nonlinearity.  us, the library (with the kernel for the nonlinearity) -> here, in 4 shares unless said otherwise:
+//   4,096 x 16,384 at 65, 128, 256, 512, 704 rows 50, 81, 65, 105, 111 -> 42, 51, 53, 72, 92; without shares 116, 145, 142, 139, 126
+//     768, 1,024 (2), 1,500 (2), 2,048 (1) 119, 143, 184, 218 -> 94, 123, 172, 222; without 142, 145, 178
+//   4,096 x 11,008 38, 58, 49, 74, 81 -> 33, 38, 40, 53, 68; 1,024 (2) 104 -> 85; 2,048 x 16,384 at 1,040, 2,048 (2) 114, 135 -> 74, 117
+//   4,096 x 4,096 16, 24, 23, 30 (2), 32 (1) -> 16, 19, 23, 30, 35; 12,288 x 4,096 at 256, 512, 704 (1) 50, 55, 77 -> 44, 54, 64
+//   2,816 gates x 4,096 26, 28, 44, 41 (1), 53 (1) -> 18, 20, 28, 39, 40
+//   one share: 16,384 gates 67, 68, 82, 117, 171 -> 63, 65, 76, 111, 163; 11,008 gates 48 (2), 51, 68, 95, 155 -> 51, 52, 63, 95, 136
+//
+// The rule (ops.product_faster) over 1,056 products of 65 to 2,048 rows (23 shapes without a gate, 9 with one; shares as planned), against the library
+// for all: without a gate 10% faster in the mean up to 704 rows and 6% beyond, with one 9% and 10%.  How fast the library is goes up and
+// down with the sizes (4,096 x 4,096 at 160, 192, 224, 320 rows 27, 33, 22, 26; 4,096 x 16,384 at 1,536, 1,579 183, 393), so it is not always the
+// slower one: 96 of the products are more than 2% slower here, half of them by up to 5%, four in five by up to 10%; the worst 128 x 2,048 x 16,384 37 -> 45,
+// 1,400 x 32,768 x 4,096 268 -> 320 (with the gate 294 -> 331), 768 and 1,500 rows of 4,096 x 2,816 and 2,048 x 4,096 26, 32 -> 30, 36.
+//   Left to the library, us there / here: 11 to 16 million weights beyond 192 rows 17/20 (4,096 x 2,816 at 256), 24/25 (2,816 x 4,096 at 448); from 8,192
+//   outputs on, up to 128 rows, 33/39 (16,384 x 4,096 at 65), 30/32 (12,288), though 38/25 (10,240); up to 1,024 outputs 58/80 (8,192 rows of
+//   1,024 x 4,096); results below 2.88 million without shares 34/38 (1,280 x 2,048 x 4,096)
+//
 // 8 and 16 shares are slower than 4 but for 65 and 128 rows of 4,096 x 16,384 (38 and 41 us with 16).
 // (reference: every linear layer is its vendor's library's, src/model/linear.cuh:9-37; the gate src/model/activation.cuh:6-18)
 #include "product.h"

@@ -2158,23 +2158,30 @@ def product_takes(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str
             and M * ldo < (1 << 30) - 4096 and M * ldx < 1 << 31 and rows * K < 1 << 31)
 
 
-def product_faster(M: int, N: int, K: int) -> bool:
-    """Whether ``product_many`` is faster than the library's product of M rows, N outputs and K columns (csrc/product.hip has the
-    figures).  Up to 704 rows from 11 million weights on: few tiles, which shares of K deal to the CUs (smaller products end in the time
-    of their launches).  Beyond, from two million results on; but not where tiles of 256 x 256 fill whole rounds of 256 CUs without
-    gaps, which the library does 5 to 10% faster."""
-    if M <= PRODUCT_FEW_ROWS:
-        return M > SKINNY_MAX_ROWS and N * K >= PRODUCT_MIN_WEIGHTS
-    if M * N < PRODUCT_MIN_RESULTS:
-        return False
-    tiles = -(-M // 256) * -(-N // 256)
-    return M * N < 0.93 * 65536 * 256 * -(-tiles // 256)
-
-
 @lru_cache(maxsize=4096)
 def product_plan(M: int, N: int, K: int, gated: bool) -> int:
     """In how many shares of K (1, 2 or 4) a product takes least, by the kernel's costs; N with the gate's rows."""
     return _fn("product", "cpmcu_product_plan")(c_int(M), c_long(N), c_int(K), c_int(1 if gated else 0))
+
+
+def product_faster(M: int, N: int, K: int, gated: bool = False) -> bool:
+    """Whether ``product_many`` is faster than the library's product (and, ``gated``, the kernel of the nonlinearity behind it) of M rows, N
+    outputs and K columns; N with the gate's rows.  csrc/product.hip has the figures.
+    Up to 704 rows (few tiles, which shares of K deal to the CUs): from 11 million weights on; smaller products end in the time of their
+    launches.  Without a gate those below 16 million up to 192 rows only, and 8,192 outputs and more from 129 rows on: few rows of wide
+    products are the time of the weights, which the library streams 5 to 15% faster.
+    Beyond: from two million results on, without a gate from 2.88 million where K stays whole and only more than 1,024 outputs; but not
+    where tiles of 256 x 256 fill whole rounds of 256 CUs without gaps, which the library does 5 to 10% faster."""
+    if M <= PRODUCT_FEW_ROWS:
+        if M <= SKINNY_MAX_ROWS or N * K < PRODUCT_MIN_WEIGHTS:
+            return False
+        return gated or not (N * K < 16 << 20 and M > 192 or N >= 8192 and M <= 128)
+    if M * N < PRODUCT_MIN_RESULTS:
+        return False
+    if not gated and (N <= 1024 or M * N < 2880000 and product_plan(M, N, K, False) == 1):
+        return False
+    tiles = -(-M // 256) * -(-N // 256)
+    return M * N < 0.93 * 65536 * 256 * -(-tiles // 256)
 
 
 @lru_cache(maxsize=256)
@@ -2184,7 +2191,7 @@ def product_scratch(most_rows: int, N: int, K: int, gated: bool) -> int:
     if N % 8 or K % 64:
         return 0
     for M in range(SKINNY_MAX_ROWS + 1, most_rows + 1):
-        if product_faster(M, N, K):
+        if product_faster(M, N, K, gated):
             parts = plan(c_int(M), c_long(N), c_int(K), c_int(1 if gated else 0))
             if parts > 1:
                 most = max(most, parts * M * N * 4)

@@ -139,7 +139,7 @@ class Linear(Part):
             # both halves' place, whichever way this pass takes: the choice goes up and down with the rows, and the largest
             # pass has to leave the workspace as large as any other needs it
             ctx.ws.get(tag, (n, self.out_features), x.dtype)
-            if (x.dtype == torch.bfloat16 and self.weight is not None and ops.product_faster(n, self.out_features, self.in_features)
+            if (x.dtype == torch.bfloat16 and self.weight is not None and ops.product_faster(n, self.out_features, self.in_features, True)
                     and ops.product_takes(x, self.weight, act, "gated")):
                 ops.product_many(x, self.weight, act, True, activation, ctx.ws)         # the nonlinearity on the product's float sums
                 return act

@@ -88,10 +88,11 @@ def test_every_fill(H, F, activation):
 
 @pytest.mark.parametrize("E,pairs,H,F,want", [
     (16, 4096, 2048, 1728, "product"), (16, 4096, 2048, 1664, "wide"), (15, 4500, 2048, 1728, "wide"), (72, 64 * 72, 2048, 1536, "product"),
-    (72, 64 * 72 - 1, 2048, 1536, "wide"), (16, 4096, 2048, 1736, "wide"), (16, 8192, 4096, 448, "wide"), (16, 8192, 4096, 512, "product")])
+    (72, 64 * 72 - 1, 2048, 1536, "wide"), (16, 4096, 2048, 1736, "wide"), (16, 8192, 4096, 448, "wide"), (16, 8192, 4096, 512, "product"),
+    (64, 7872, 1536, 1792, "product"), (64, 7552, 1536, 1792, "wide")])
 @pytest.mark.parametrize("gated", [True, False])
 def test_the_rule(E, pairs, H, F, want, gated):
-    """64 pairs an expert, 16 experts, 14e9 products; whole pieces of 64 columns, 8 of them."""
+    """64 pairs an expert, 16 experts, 14e9 products (21e9 of fewer than 1,600 columns); whole pieces of 64 columns, 8 of them."""
     rows = [pairs // E + (e < pairs % E) for e in range(E)]
     E, n, h, up, down, idx, w = operands(rows, H, F, gated, F)
     act, y = (torch.empty(n, 1, k, dtype=torch.bfloat16, device=DEV) for k in (F, H))
@@ -181,8 +182,8 @@ def test_identity_experts():
             z = x @ up[e].double().T
             a = torch.nn.functional.silu(z[:, :F]) * z[:, F:]
             v, s = a @ down[e].double().T, a.abs() @ down[e].double().abs().T
-            # act is rounded to 2^-9 of itself, its float sums of 2,048 and the result's of 1,728 numbers to 2^-12 of their sizes, y to 2^-9
-            off = (2.0 ** -9 + 2.0 ** -12) * s + 2.0 ** -9 * v.abs()
+            # act is rounded to 8 bits, 2^-8 of itself, its float sums of 2,048 and the result's of 1,728 numbers to 2^-12 of their sizes, y to 2^-8
+            off = (2.0 ** -8 + 2.0 ** -12) * s + 2.0 ** -8 * v.abs()
         else:
             v, off = x, torch.zeros_like(x)
         want.index_add_(0, t, w[t, k, None].double() * v)
