@@ -1,4 +1,4 @@
-// Products of steps of many tokens (bf16, from 65 rows on): out [M, N] = X [M, K] . W [N, K]^T, summed in float, written in bf16 or float,
+// Products of steps of many tokens (bf16, from 65 rows on): out [M, N] = X [M, K] . W [N, K]^T, summed in float, written in bf16,
 // or with the gate's nonlinearity on the float sums (W: gate rows, then up rows), so that neither half is rounded, written and read again.
 //
 // A workgroup of 4 wavefronts (2 x 2) holds a tile of 32 RT rows by 32 CT weight rows in its accumulators, 256 x 256 at most: 256
@@ -50,7 +50,7 @@
 // (as the kernel that runs behind the library's product forms it)
 __device__ inline float gate_fast(float g, int act) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-gate_arg(g, act))); }
 
-enum { PRODUCT_PLAIN = 0, PRODUCT_GATED = 1, PRODUCT_FLOAT = 2, PRODUCT_PARTS = 3 };
+enum { PRODUCT_PLAIN = 0, PRODUCT_GATED = 1, PRODUCT_PARTS = 2 };
 
 template <int RT, int CT, int SA, int SB, int KIND>
 __global__ __launch_bounds__(256, 1) void product_kernel(const bf16_t* __restrict__ X, int ldx, const bf16_t* __restrict__ W, int M,
@@ -195,7 +195,7 @@ __global__ __launch_bounds__(256, 1) void product_kernel(const bf16_t* __restric
             next_b();
         } while (++p < pieces);
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");             // the matrix instructions' results are there
-        constexpr bool FLOATS = KIND == PRODUCT_FLOAT || KIND == PRODUCT_PARTS;
+        constexpr bool FLOATS = KIND == PRODUCT_PARTS;
         constexpr int EB = FLOATS ? 4 : 2;
         const int m0 = u % mt * BM + wm * 16 * RT, n0 = ((u - share_of(u) * (mt * nt)) / mt * BN + wn * 16 * CT) / (KIND == PRODUCT_GATED ? 2 : 1);
         int er = m0 + r, ec = FLOATS ? n0 + 4 * g : n0 + (g & 1) * 16 + (g >> 1) * 8;
@@ -320,11 +320,11 @@ extern "C" int cpmcu_product_plan(int M, long rows, int K, int gated) {
     return best;
 }
 
-// out [M, N] = X [M, K] . W^T, W [N, K] bf16, out bf16 or (PRODUCT_FLOAT) float32; PRODUCT_GATED: W [2 N, K] holds gate rows, then up rows, out =
+// out [M, N] = X [M, K] . W^T, W [N, K] and out bf16; PRODUCT_GATED: W [2 N, K] holds gate rows, then up rows, out =
 // act(gate) * up in bf16.  tile: one of PRODUCT_TILES, or -1 for the rule's.
 extern "C" const char* cpmcu_product(const void* X, long ldx, const void* W, int M, int N, int K, void* out, long ldo, int kind, int act,
                                      float act_limit, int tile, hipStream_t stream) {
-    CPMCU_REQUIRE(kind >= PRODUCT_PLAIN && kind <= PRODUCT_FLOAT, "product: unknown kind %d", kind);
+    CPMCU_REQUIRE(kind == PRODUCT_PLAIN || kind == PRODUCT_GATED, "product: unknown kind %d", kind);
     CPMCU_REQUIRE(kind != PRODUCT_GATED || CPMCU_ACT_KNOWN(act), "product: unknown nonlinearity %d", act);
     CPMCU_REQUIRE(M > 0 && N > 0 && K > 0 && K % 64 == 0 && N % 8 == 0, "product: K=%d must be a multiple of 64, N=%d of 8", K, N);
     const long rows = (long)N * (kind == PRODUCT_GATED ? 2 : 1);
@@ -344,7 +344,6 @@ extern "C" const char* cpmcu_product(const void* X, long ldx, const void* W, int
 #define PRODUCT_LAUNCH(RT, CT, SA, SB, a, b, c, d)                                                                                         \
     if (rt == RT && ct == CT) {                                                                                                            \
         if (kind == PRODUCT_PLAIN) PRODUCT_KIND(RT, CT, SA, SB, PRODUCT_PLAIN);                                                            \
-        else if (kind == PRODUCT_FLOAT) PRODUCT_KIND(RT, CT, SA, SB, PRODUCT_FLOAT);                                                       \
         else if constexpr (CT % 4 == 0) PRODUCT_KIND(RT, CT, SA, SB, PRODUCT_GATED);                                                       \
     }
     PRODUCT_TILES(PRODUCT_LAUNCH)

@@ -2143,7 +2143,7 @@ def skinny_split(M: int, N: int, K: int) -> int:
 PRODUCT_FEW_ROWS = 704
 PRODUCT_MIN_WEIGHTS = 11 << 20
 PRODUCT_MIN_RESULTS = 2 << 20
-PRODUCT_KINDS = {"plain": 0, "gated": 1, "float": 2}
+PRODUCT_KINDS = {"plain": 0, "gated": 1}
 
 
 def product_takes(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str = "plain") -> bool:
@@ -2220,12 +2220,12 @@ def product_many(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, gated: boo
 
 def product(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, kind: str = "plain", activation="silu", tile: int = -1):
     """out = x . w^T for steps of many tokens, x [M, K] and w [N, K] bfloat16, summed in float: 'plain' out bfloat16 [M, N],
-    'float' out float32 [M, N], 'gated' w holds gate rows then up rows, out bfloat16 [M, N/2] = act(gate) * up (act as in
+    'gated' w holds gate rows then up rows, out bfloat16 [M, N/2] = act(gate) * up (act as in
     silu_mul).  tile: a form of the kernel instead of the rule's."""
     M, K = x.shape
     N = w.shape[0] // 2 if kind == "gated" else w.shape[0]
     if (not (x.is_cuda and w.is_cuda and out.is_cuda) or w.shape[1] != K or out.shape != (M, N)
-            or out.dtype != (torch.float32 if kind == "float" else torch.bfloat16) or not product_takes(x, w, out, kind)):
+            or kind not in PRODUCT_KINDS or out.dtype != torch.bfloat16 or not product_takes(x, w, out, kind)):
         raise KernelError(f"product: x {tuple(x.shape)} {x.dtype}, w {tuple(w.shape)} {w.dtype}, out {tuple(out.shape)} {out.dtype} "
                           f"('{kind}') are not what the kernel takes")
     _check(_fn("product", "cpmcu_product")(_p(x), c_long(x.stride(0)), _p(w), c_int(M), c_int(N), c_int(K), _p(out),
