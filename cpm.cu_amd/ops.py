@@ -2261,8 +2261,8 @@ def product_parts(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, parts: in
 # dispatchers: choose the kernel for a shape and element type
 # ---------------------------------------------------------------------------
 def library_gemm_ok(x: torch.Tensor, out_dtype: torch.dtype) -> bool:
-    """Many rows in bf16 with bf16 output: the library's matrix product (the reference calls its vendor's
-    library for every linear layer, src/model/linear.cuh:9-37)."""
+    """Many rows in bf16 with bf16 output: the library's matrix product or ``product_many``, both of which write bf16 (the reference calls
+    its vendor's library for every linear layer, src/model/linear.cuh:9-37)."""
     return x.dtype == torch.bfloat16 and out_dtype == torch.bfloat16 and x.shape[0] > SKINNY_MAX_ROWS
 
 

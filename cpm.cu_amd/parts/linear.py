@@ -52,7 +52,7 @@ class Linear(Part):
 
     def reserve_workspace(self, ws, rt: Runtime, max_step_tokens: int, max_slots: int):
         # An engine whose forward passes never carry more rows than the decode product takes reads the re-laid
-        # copy only: the checkpoint's layout (what the library's many-row product and the 32-bit kernels read)
+        # copy only: the checkpoint's layout (what the products of many rows and the 32-bit kernels read)
         # is let go, which halves what the weights hold.
         if self.tiled is not None and max_step_tokens <= ops.SKINNY_MAX_ROWS and self.in_features % 8 == 0:
             self.weight = None
@@ -82,7 +82,7 @@ class Linear(Part):
                 return out
         out_dtype = out_dtype or x.dtype
         if partials and alpha == 1.0 and ops.library_gemm_ok(x, x.dtype):
-            out_dtype = x.dtype         # many rows: the branch comes back in bf16 from the library product
+            out_dtype = x.dtype         # many rows: their products leave the branch in bf16
         out = ctx.ws.get(tag, (n, N), out_dtype)
         ops.linear(x, w, out, alpha, w_tiled=wt, ws=ctx.ws)
         return out
@@ -138,7 +138,7 @@ class Linear(Part):
                 raise ValueError("forward_gated: a row scale needs the few-rows kernel (gated_takes_row_scale)")
             # both halves' place, whichever way this pass takes: the choice goes up and down with the rows, and the largest
             # pass has to leave the workspace as large as any other needs it
-            ctx.ws.get(tag, (n, self.out_features), x.dtype)
+            ctx.ws.room(tag, n * self.out_features * x.element_size())
             if (x.dtype == torch.bfloat16 and self.weight is not None and ops.product_faster(n, self.out_features, self.in_features, True)
                     and ops.product_takes(x, self.weight, act, "gated")):
                 ops.product_many(x, self.weight, act, True, activation, ctx.ws)         # the nonlinearity on the product's float sums
