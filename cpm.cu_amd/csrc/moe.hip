@@ -1154,8 +1154,8 @@ extern "C" const char* cpmcu_moe_experts_mfma(const void* h, long ldh, const voi
     // moe_product_kernel from 64 pairs an expert, 16 experts and 14e9 products of a matrix's numbers with rows on (21e9 of narrow experts), of widths
     // that it takes.
     // Up + down + the rest of the call, us, moe_wide_kernel / moe_product_kernel:
-    //   64 of 4,096 x 1,408 gated, 6 a token: 2,048 tokens 700/590, even routing 683/535, 16 of 80 identity 631/565, 1,200 546/512, 700 (66 an
-    //     expert) 465/456; 512 (48, even) 413/436.  Of 4,096 x 2,112 without a gate 2,048 713/630, 300 (28) 402/414
+    //   64 of 4,096 x 1,408 gated, 6 a token, uneven: 2,048 tokens 670/612, even routing 688/555, 16 of 80 identity 640/542, 1,200 572/473, 700 (66 an
+    //     expert) 468/408; 512 (48, even) 413/436.  Of 4,096 x 2,112 without a gate 2,048 720/664, 300 (28) 402/414
     //   92 drawn steps of this rule (16 to 160 experts of 1,600 to 4,700 x 512 to 2,500, even routing to a few experts with most rows): 8% faster in
     //     the mean, 25% at most; 11 slower, all but one of fewer than 20e9 products: 16 to 24 experts of which a few have most rows 2 to 34%,
     //     others up to 11% (of 24 steps of 14e9 to 21e9 half are faster, up to 22%)

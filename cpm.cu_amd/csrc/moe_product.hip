@@ -8,10 +8,13 @@
 // XCD, whose workgroups take the next one from a counter; a run that has ended helps the run that has most left.  moe_group_kernel
 // deals the experts to the runs by their rows, many rows first, so that what runs last is small.
 //
-// us (64 experts of 4,096 x 1,408 gated, 2,048 tokens with 6 each), tiles of 128 x 128 two a CU -> this: even routing 424 + 245 ->
-// 290 + 205, uneven (up to 900 rows an expert) 437 + 250 -> 345 + 210, routers with random weights (two experts of 1,900 rows, 45 of fewer
-// than 100) the whole call 728 -> 672, with 16 of 80 identity 676 -> 620.  2,112 without a gate 345 + 345 -> 292 + 291.
-// What bounds it: even routing moves 1.47 + 0.74 GB of weights, a piece of 32 KB in 1.26 us a CU (6.6 TB/s together) beside
+// us (64 experts of 4,096 x 1,408 gated, 2,048 tokens with 6 each), tiles of 128 x 128 two a CU -> this, each product standing alone and the whole
+// call: even routing 447 + 263 -> 346 + 189, 688 -> 555; uneven (up to 750 rows an expert, half with fewer than 80) 452 + 259 -> 385 + 221, 670 -> 612; a
+// router with random weights (one expert of 1,700 rows, half with fewer than 10) 443 + 254 -> 366 + 214, 681 -> 604; with 16 of 80 identity 384 + 221 ->
+// 319 + 192, 640 -> 542.  2,112 without a gate 337 + 340 -> 306 + 317.  In a pass of other layers the second product gains less, or nothing
+// (Pemalorn's 2,048 tokens 214.5 -> 214).  The gate has the full precision of the other kernels; by the fast exponential and
+// reciprocal the first product takes up to 4% less.
+// What bounds it (the figures up to the end with the fast gate): even routing moves 1.47 + 0.74 GB of weights, a piece of 32 KB in 1.26 us a CU (6.6 TB/s together) beside
 // 1,536 cycles of matrix instructions; with all operands in caches and nothing written 246 + 137 are left.  A tile costs 7 us beside its
 // pieces (results 4, the next task and its list 2), the kernel's start 7, and at the end CUs wait for the last: a tenth of the time.
 // Taken back: weights through the caches where tiles share them (592 -> 613 for the call, even routing 540 -> 551), runs taken

@@ -9,10 +9,10 @@
 // tile: the pieces of the next tile are fetched while the last is multiplied and written.  XCD b % 8 has a run of neighbouring
 // tiles, rows fastest: 32 at a time that share their operands in its L2.
 //
-// What bounds it: with random numbers the chip's power.  Matrix instructions alone reach 2,090 TFLOP/s (2,460 with zeros), this kernel with
-// tiles of 256 x 256 in whole rounds 1,310 to 1,400 at 2.0 GHz, the library 1,430 to 1,480; on half the CUs (2,048 x 4,096 x 16,384) it
-// takes 2,600 cycles a piece for 2,048 of matrix instructions.  Smaller tiles are bound by what L2 hands a CU (32 bytes a cycle), a few
-// tiles alone by what one CU is handed of memory (about 37 GB/s of W).
+// What bounds it: matrix instructions alone reach 2,090 TFLOP/s with random numbers (2,460 with zeros: that part is the chip's power), this kernel
+// with tiles of 256 x 256 in whole rounds 1,310 to 1,400 at 2.0 GHz, the library 1,430 to 1,480; on half the CUs (2,048 x 4,096 x 16,384)
+// it takes 2,600 cycles a piece for 2,048 of matrix instructions.  Smaller tiles are bound by what L2 hands a CU (32 bytes a cycle; 256 x 128
+// in a prompt's pass 1,200 TFLOP/s, 192 x 128 1,050), a few tiles alone by what one CU is handed of memory (about 37 GB/s of W).
 // The matrix instructions are written as asm with the accumulators in place: left to itself the compiler moved them between registers
 // in some of these loops (124 moves a piece, 281 -> 434 us).
 //
